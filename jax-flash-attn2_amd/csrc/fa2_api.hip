@@ -268,6 +268,30 @@ static bool fwd_pack_gqa(const fa2_params* p) {
 	return p->Hkv > 0 && p->Hq % p->Hkv == 0 && p->Hq > p->Hkv && (long)(p->Hq / p->Hkv) * p->Sq <= 64;
 }
 
+// Few query rows in all, nothing but masks by position and key lengths: fwd_decode_kernel.  Returns the number of waves that
+// share the key tiles (0 = not this kernel); *whole: one (batch, kv-head) per wave, no scratch.
+static int fwd_decode_waves(const fa2_params* p, int* whole) {
+	if (p->Hkv <= 0 || p->Hq % p->Hkv || p->bias || p->p_drop > 0.f || p->softcap > 0.f || p->has_window || p->seqlens) return 0;
+	const int64_t r = p->Hq / p->Hkv, units = (int64_t)p->B * p->Hkv;
+	if (r * p->Sq > 16) return 0;  // (the columns of a 16 x 16 product)
+	// the query rows of a unit are addressed with 32-bit byte offsets from its first, the tiles are counted in 32 bits
+	if (p->q.stride_h < 0 || ((r - 1) * p->q.stride_h + (p->Sq - 1) * p->q.stride_s) * 2 > 0x7fff0000) return 0;
+	const int kt = p->D == 64 ? 64 : 32;
+	const int64_t tiles = (p->Sk + kt - 1) / kt, total = units * tiles;
+	if (total > 0x3fffffff) return 0;
+	// A wave takes about a microsecond per tile, the second launch 4.5: a unit of up to six tiles is left whole (at eight tiles of
+	// 32 keys, B1 Hkv8, 11.0 us against 10.8 in the 128-row kernel, which keeps that range; tiles of 64 keys 6.9 against 8.1),
+	// and so are the units where they fill all resident waves in whole rounds (B64 Hkv32 Sk2048: 283 us; B70, 2.2 rounds, 323 us
+	// whole) or are so many that the last round does not matter.
+	if (p->Sk <= 256 && tiles > 6) return 0;
+	*whole = p->Sk <= 256 || (units >= 2048 && (units % 1024 == 0 || units >= 16384));
+	if (*whole) return (int)units;
+	// as many waves as are resident at once, down to a tile each (B1 Hkv8 Sk1029: 8.5 us, two tiles each 10.0), at most 63 a unit
+	int64_t waves = p->D == 256 ? 512 : 1024;
+	if (waves > total) waves = total;
+	return (int)(waves < 63 * units ? waves : 63 * units);
+}
+
 static int fwd_split_plan(const fa2_params* p, int* split_len) {
 	*split_len = 0;
 	// workgroups of an unsplit launch of this kernel variant (row tiles of 64)
@@ -294,6 +318,13 @@ static size_t fwd_scratch_bytes(const fa2_params* p) {
 	if (p->B <= 0 || p->Hq <= 0 || p->Sq <= 0 || p->Sk <= 0 || p->D <= 0) return 0;
 	if (p->has_window || p->softcap > 0.f) return 0;
 	int len;
+	int whole;
+	if (int waves = fwd_decode_waves(p, &whole)) {
+		if (whole) return 0;
+		// the pieces (at most one per wave and one more per (batch, kv-head)): O and lse of a unit's rows; where they are, per unit
+		const size_t units = (size_t)p->B * (size_t)p->Hkv, rows = (waves + units) * (size_t)(p->Hq / p->Hkv) * (size_t)p->Sq;
+		return (rows * ((size_t)p->D + 1) * sizeof(float) + units * 8 + 255) & ~(size_t)255;
+	}
 	int n = fwd_split_plan(p, &len);
 	if (n <= 1) return 0;
 	size_t rows = (size_t)n * (size_t)p->B * (size_t)p->Hq * (size_t)p->Sq;
@@ -315,7 +346,17 @@ int fa2_fwd(const fa2_params* p, void* hip_stream) {
 	fill(p, a);
 	// optional scratch: with enough of it a short query over many keys runs split over key ranges
 	size_t need = fwd_scratch_bytes(p);
-	if (need && p->scratch && ((uintptr_t)p->scratch & 255) == 0 && p->scratch_bytes >= need) {
+	const bool room = need && p->scratch && ((uintptr_t)p->scratch & 255) == 0 && p->scratch_bytes >= need;
+	int whole = 0;
+	const int waves = fwd_decode_waves(p, &whole);
+	if (waves && (whole || room)) {
+		a.decode_waves = waves;
+		a.decode_whole = whole;
+		size_t rows = (waves + (size_t)p->B * (size_t)p->Hkv) * (size_t)(p->Hq / p->Hkv) * (size_t)p->Sq;
+		a.o_part = (float*)p->scratch;
+		a.lse_part = a.o_part + rows * (size_t)p->D;
+		a.decode_units = (int32_t*)(a.lse_part + rows);
+	} else if (room && !waves) {
 		a.nsplit = fwd_split_plan(p, &a.split_len);
 		a.pack_gqa = fwd_pack_gqa(p) ? 1 : 0;
 		size_t rows = (size_t)a.nsplit * (size_t)p->B * (size_t)p->Hq * (size_t)p->Sq;
