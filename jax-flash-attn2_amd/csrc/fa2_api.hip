@@ -292,15 +292,45 @@ static int fwd_decode_waves(const fa2_params* p, int* whole) {
 	return (int)(waves < 63 * units ? waves : 63 * units);
 }
 
-static int fwd_split_plan(const fa2_params* p, int* split_len) {
+static int fwd_split_plan(const fa2_params* p, int* split_len, int* tall) {
 	*split_len = 0;
+	*tall = 0;
+	if (p->D <= 128 && !p->bias && !(p->p_drop > 0.f) && !fwd_pack_gqa(p)) {
+		// Workgroups of 128 rows whose eight waves share the keys, one per CU: as many key ranges as make the estimate smallest - whole
+		// rounds of the longest workgroup (less where a causal mask makes them unequal and they even out over
+		// several rounds), plus 3 us for the second launch and the partial results written and read.  Figures measured: a tile
+		// takes such a workgroup 1.07 us (0.8 at D = 64), partial results move at 2.8 TB/s; without ranges and with more than 256 workgroups
+		// the 128-row kernel runs two workgroups a CU and needs 1.46 to 2.2 us a tile.  B1 Hq32 Hkv8 D128, 100 rows over
+		// 4000 keys: 71 us in one range, 44 in 2, 30 in 4, 24 in 8, 35 in 12 (16 ranges of the 64-row kernel: 36); B1 H4 S4096 D128
+		// causal: 61 / 42 / 54 us in 1 / 2 / 4; B2 Hq16 300 rows over 3000 keys: 55 / 36 / 44 us in 1 / 2 / 4.
+		const int64_t base = (int64_t)p->B * p->Hq * ((p->Sq + 127) / 128);
+		if (base >= 512) return 1;
+		const int tiles = (p->Sk + 63) / 64;
+		const double mean = p->causal && p->Sq <= p->Sk ? (p->Sk - 0.5 * p->Sq) / 64 : tiles;
+		const bool even = mean > 0.75 * tiles;
+		const double tile_us = p->D == 64 ? 0.8 : 1.07;
+		const double part_us = (double)p->B * p->Hq * p->Sq * p->D * 8 / 2.8e6 * (mean / tiles);
+		int best = 1;
+		double best_us = tiles * (base <= 256 ? tile_us : (1.46 + (base - 256) / 256.0 * 0.7) * (even ? 1.0 : 0.6));
+		for (int n = 2; n <= 16 && n <= tiles / 2; ++n) {
+			const int64_t rounds = (base * n + 255) / 256;
+			const double us = rounds * ((tiles + n - 1) / n) * (even || rounds == 1 ? 1.0 : 0.85) * tile_us + 3 + n * part_us;
+			if (us < best_us) {
+				best = n;
+				best_us = us;
+			}
+		}
+		const int per = (tiles + best - 1) / best;
+		*tall = 1;
+		*split_len = per * 64;
+		return (tiles + per - 1) / per;
+	}
 	// workgroups of an unsplit launch of this kernel variant (row tiles of 64)
 	long base = fwd_pack_gqa(p) ? (long)p->B * p->Hkv : (long)p->B * p->Hq * ((p->Sq + 63) / 64);
 	int tiles = (p->Sk + 63) / 64;
-	// A query longer than one row tile runs unsplit on the 128-row kernel, which a quarter of the chip's worth of
-	// units already keeps busy over a short key range: the second launch pays from 16 key tiles on up to 128 units
-	// and from 32 above (measured at D=64: 256 units over 16 tiles 0.0185 ms unsplit, 0.0203 ms split; over 32 tiles
-	// 0.0316 and 0.0235).
+	// A query longer than one row tile (with bias or dropout, or at D = 256) runs unsplit on the 128-row kernel, which a quarter of the
+	// chip's worth of units already keeps busy over a short key range: the second launch pays from 16 key tiles on up to 128 units
+	// and from 32 above.
 	int min_tiles = p->Sq <= 64 ? 8 : (base <= 128 ? 16 : 32);
 	if (base >= 512 || tiles < min_tiles) return 1;
 	long want = (1024 + base - 1) / base;
@@ -325,7 +355,7 @@ static size_t fwd_scratch_bytes(const fa2_params* p) {
 		const size_t units = (size_t)p->B * (size_t)p->Hkv, rows = (waves + units) * (size_t)(p->Hq / p->Hkv) * (size_t)p->Sq;
 		return (rows * ((size_t)p->D + 1) * sizeof(float) + units * 8 + 255) & ~(size_t)255;
 	}
-	int n = fwd_split_plan(p, &len);
+	int tall, n = fwd_split_plan(p, &len, &tall);
 	if (n <= 1) return 0;
 	size_t rows = (size_t)n * (size_t)p->B * (size_t)p->Hq * (size_t)p->Sq;
 	return (rows * ((size_t)p->D + 1) * sizeof(float) + 255) & ~(size_t)255;
@@ -357,7 +387,7 @@ int fa2_fwd(const fa2_params* p, void* hip_stream) {
 		a.lse_part = a.o_part + rows * (size_t)p->D;
 		a.decode_units = (int32_t*)(a.lse_part + rows);
 	} else if (room && !waves) {
-		a.nsplit = fwd_split_plan(p, &a.split_len);
+		a.nsplit = fwd_split_plan(p, &a.split_len, &a.tall_split);
 		a.pack_gqa = fwd_pack_gqa(p) ? 1 : 0;
 		size_t rows = (size_t)a.nsplit * (size_t)p->B * (size_t)p->Hq * (size_t)p->Sq;
 		a.o_part = (float*)p->scratch;

@@ -169,8 +169,11 @@ FA2_DEV f32x4 load_bias4(const char* rowp, int col, int dtype, bool vec_ok, int 
 // BLDS: the bias goes through LDS (the launcher has checked element type, alignment and the key
 // count); otherwise every lane loads its bias values from global memory.
 // CAP: tanh soft-capping of the scores (refrence_call.py:48-51), on the path with bias; the bias itself may be absent.
-template <typename T, int D, int NW, int QB, int WPS, bool BIAS, bool DROP, bool SPLIT = false, bool BLDS = false, bool CAP = false>
-__global__ __launch_bounds__(NW * 64, WPS) void fwd_kernel(const KArgs a) {
+// KW: this many groups of NW waves share the rows of a workgroup and take its key tiles in turn, each with tiles of its own in
+// LDS; group 0 merges their (O, maximum, sum) at the end.  For grids that would leave SIMDs with one wave or none.
+template <typename T, int D, int NW, int QB, int WPS, bool BIAS, bool DROP, bool SPLIT = false, bool BLDS = false, bool CAP = false, int KW = 1>
+__global__ __launch_bounds__(NW * 64 * KW, WPS) void fwd_kernel(const KArgs a) {
+	static_assert(KW == 1 || QB == 1, "");
 	static_assert(!CAP || (BIAS && !BLDS && !SPLIT), "soft-capping runs on the plain path with bias");
 	typedef typename T::V8 V8;
 	constexpr int BM = NW * QB * 32;
@@ -186,9 +189,9 @@ __global__ __launch_bounds__(NW * 64, WPS) void fwd_kernel(const KArgs a) {
 	constexpr bool BIAS_LDS = BIAS && BLDS && (D <= 128 || !SPLIT);
 	constexpr int BIAS_BYTES = BIAS_LDS ? BM * BN * 2 : 0;
 	static_assert(BN == 64, "bias tiles use the 64-element row geometry");
-	__shared__ __attribute__((aligned(1024))) char smem[4 * TILE_BYTES + 2 * BIAS_BYTES];
-	FA2_LDS char* lds = (FA2_LDS char*)smem;
-	// layout: K[0] K[1] V[0] V[1] bias[0] bias[1]
+	constexpr int GROUP_BYTES = 4 * TILE_BYTES + 2 * BIAS_BYTES;
+	__shared__ __attribute__((aligned(1024))) char smem[KW * GROUP_BYTES];
+	// layout (per group of waves): K[0] K[1] V[0] V[1] bias[0] bias[1]
 
 	int mt, h, b, split = 0;
 	// pack (split kernel only): the rows of the tile are the Sq rows of ALL r q-heads of one
@@ -210,10 +213,12 @@ __global__ __launch_bounds__(NW * 64, WPS) void fwd_kernel(const KArgs a) {
 		decode_block(a, mt, h, b);
 	}
 	const int hk = h / (a.Hq / a.Hkv);
-	const int tid = threadIdx.x, lane = tid & 63;
+	const int tid = KW == 1 ? threadIdx.x : threadIdx.x & (NT - 1), lane = tid & 63;  // (of the group)
 	// the wave index as an explicitly scalar value: everything derived from it (tile bounds, loop trip counts,
 	// "nothing to do for this wave") then stays in scalar registers and scalar branches
 	const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+	const int kw = KW == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)threadIdx.x / NT);
+	FA2_LDS char* lds = (FA2_LDS char*)smem + kw * GROUP_BYTES;
 	const int g = lane >> 5, c = lane & 31;
 	// dropout key: from the parameter block, or from device memory when the caller keeps it there
 	uint32_t drop_k0 = a.drop_k0, drop_k1 = a.drop_k1;
@@ -258,12 +263,16 @@ __global__ __launch_bounds__(NW * 64, WPS) void fwd_kernel(const KArgs a) {
 		int e = kv_begin + a.split_len;
 		kv_end = e < kv_end ? e : kv_end;
 		t_begin = kv_begin / BN;
-		if (kv_end <= kv_begin) kv_end = 0;
+		if (kv_end <= kv_begin) {  // nothing in this range for these rows
+			kv_end = 0;
+			t_begin = 0;
+		}
 	} else if (wl >= 0) {
 		int first_key = m0 + off - wl;  // first key the tile's first row sees
 		if (first_key > 0) t_begin = first_key / BN;
 	}
 	const int ntiles = kv_end > 0 ? (kv_end + BN - 1) / BN : 0;  // one past the last tile
+	const int t_first = KW == 1 ? t_begin : t_begin + kw;                            // this group's first tile
 
 	// per-lane first and last allowed key for each of this lane's rows
 	int jmax[QB], jmin[QB];
@@ -324,8 +333,8 @@ __global__ __launch_bounds__(NW * 64, WPS) void fwd_kernel(const KArgs a) {
 	kload.init(a.k.ss, tid);
 	vload.init(a.v.ss, tid);
 	// prologue: first K/V tile in flight while Q is fetched
-	if (ntiles > t_begin) {
-		int nb = t_begin * BN, bsel = t_begin & 1;
+	if (ntiles > t_first) {
+		int nb = t_first * BN, bsel = KW == 1 ? t_first & 1 : 0;
 		int rows = sk_eff - nb < BN ? sk_eff - nb : BN;
 		kload.load(lds + bsel * TILE_BYTES, kbase + (int64_t)nb * a.k.ss, a.k.ss, rows, tid);
 		vload.load(lds + (2 + bsel) * TILE_BYTES, vbase + (int64_t)nb * a.v.ss, a.v.ss, rows, tid);
@@ -385,11 +394,11 @@ __global__ __launch_bounds__(NW * 64, WPS) void fwd_kernel(const KArgs a) {
 		bload.init(a.bias_sm, tid, brows);
 		// this lane's row of the tile: byte offset of its chunk 0 (+ 8 bytes for the upper half-wave) and swizzle key
 		int row = w * (QB * 32) + c;
-		boff_lane = row * 128 + 8 * g + (t_begin & 1) * BIAS_BYTES;
+		boff_lane = row * 128 + 8 * g + (KW == 1 ? t_first & 1 : 0) * BIAS_BYTES;
 		bkey16 = swz<64>(row) << 4;
-		if (bias_lds && ntiles > t_begin)
-			bload.load(lds + 4 * TILE_BYTES + (t_begin & 1) * BIAS_BYTES, bias_base + (int64_t)m0 * a.bias_sm + (int64_t)t_begin * BN * 2,
-			           a.bias_sm, brows, tid, (a.Sk - t_begin * BN) >> 3);
+		if (bias_lds && ntiles > t_first)
+			bload.load(lds + 4 * TILE_BYTES + (KW == 1 ? t_first & 1 : 0) * BIAS_BYTES, bias_base + (int64_t)m0 * a.bias_sm + (int64_t)t_first * BN * 2,
+			           a.bias_sm, brows, tid, (a.Sk - t_first * BN) >> 3);
 	}
 
 	// Per-lane LDS byte offsets with the swizzle folded in, so that every fragment
@@ -398,7 +407,7 @@ __global__ __launch_bounds__(NW * 64, WPS) void fwd_kernel(const KArgs a) {
 	//   V fragment (kk, db):  rows 16kk + 4g + (lane&15)/4 (+8), 8 bytes at column 32db + 16((lane>>4)&1) + 4(lane&3)
 	// The offsets carry the buffer (K[1] / V[1] / bias[1] lie a power of two behind K[0] / V[0] / bias[0])
 	// and are flipped after every tile, so that the reads need no address arithmetic in the loop.
-	const int buf0 = t_begin & 1;
+	const int buf0 = (KW == 1 ? t_first & 1 : 0);
 	// (the swizzle touches the low four bits of the chunk index only: chunks 16 and up - head dim 256 - are the same
 	// offsets 256 bytes further on, an immediate of the read instead of eight more registers)
 	constexpr int KR = KS < 8 ? KS : 8, DR = DB < 4 ? DB : 4;
@@ -742,7 +751,7 @@ __global__ __launch_bounds__(NW * 64, WPS) void fwd_kernel(const KArgs a) {
 	// (Head dim 128 takes the same path in its four-wave workgroups, where two waves share a SIMD: B4 H32 S4096 causal forward 0.531 -> 0.511 ms,
 	// B8 S2048 0.307 -> 0.294 ms; nothing at S 8192 or without a causal mask, and the eight-wave workgroups of long context
 	// measured 0.4 % slower and stay on the plain tile body.  With dropout the generator's pieces need sixteen slots a phase.)
-	constexpr bool PIPE = (D == 256 || (D == 128 && !DROP)) && NW == 4 && QB == 1 && FOLD && !SPLIT;
+	constexpr bool PIPE = (D == 256 || (D == 128 && !DROP)) && NW == 4 && QB == 1 && FOLD && (!SPLIT || KW > 1);
 	auto tile_pipe = [&](int n0) {
 		if constexpr (PIPE) {
 			constexpr int NFR = KS;  // fragments = products of a phase: KS of K for a half, 2 sixteen-key steps x DB of V
@@ -920,14 +929,14 @@ __global__ __launch_bounds__(NW * 64, WPS) void fwd_kernel(const KArgs a) {
 		}
 	};
 
-	// One pipeline step: publish tile t, start the copies of tile t + 1, compute.
+	// One pipeline step: publish tile t, start the copies of the group's next tile, compute.
 	auto step = [&](auto masked_tag, int t) {
 		const int n0 = t * BN;
-		const int buf = t & 1;
+		const int buf = KW == 1 ? t & 1 : ((t - t_first) / KW) & 1;
 		wait_async_loads();
 		__syncthreads();
-		if (t + 1 < ntiles) {
-			int n1 = n0 + BN;
+		if (t + KW < ntiles) {
+			int n1 = n0 + KW * BN;
 			int rows = sk_eff - n1 < BN ? sk_eff - n1 : BN;
 			kload.load(lds + (buf ^ 1) * TILE_BYTES, kbase + (int64_t)n1 * a.k.ss, a.k.ss, rows, tid);
 			vload.load(lds + (2 + (buf ^ 1)) * TILE_BYTES, vbase + (int64_t)n1 * a.v.ss, a.v.ss, rows, tid);
@@ -963,9 +972,57 @@ __global__ __launch_bounds__(NW * 64, WPS) void fwd_kernel(const KArgs a) {
 	t_lo = t_lo < t_begin ? t_begin : (t_lo > ntiles ? ntiles : t_lo);
 	int t_full = (wave_jmin + 1) / BN;
 	t_full = t_full < t_lo ? t_lo : (t_full > ntiles ? ntiles : t_full);
-	for (int t = t_begin; t < t_lo; ++t) step(std::true_type{}, t);
-	for (int t = t_lo; t < t_full; ++t) step(std::false_type{}, t);
-	for (int t = t_full; t < ntiles; ++t) step(std::true_type{}, t);
+	if constexpr (KW == 1) {
+		for (int t = t_begin; t < t_lo; ++t) step(std::true_type{}, t);
+		for (int t = t_lo; t < t_full; ++t) step(std::false_type{}, t);
+		for (int t = t_full; t < ntiles; ++t) step(std::true_type{}, t);
+	} else {
+		int t = t_first;
+		for (; t < t_lo; t += KW) step(std::true_type{}, t);
+		for (; t < t_full; t += KW) step(std::false_type{}, t);
+		for (; t < ntiles; t += KW) step(std::true_type{}, t);
+		// (every step is a barrier of the workgroup: a group with a tile fewer than group 0 joins the last one)
+		if (ntiles > t_begin && (ntiles - 1 - t_begin) % KW < kw) __syncthreads();
+		// merge: the groups leave O, maximum and sum in LDS, value by value as their lanes hold them - the lane of group 0 that
+		// owns the same row and columns picks them up
+		constexpr int PIECE = NT * (DB * 16 + 2) * 4;  // bytes of a group
+		static_assert((KW - 1) * PIECE <= KW * GROUP_BYTES, "");
+		__syncthreads();
+		FA2_LDS char* mine = (FA2_LDS char*)smem + tid * 16;
+		if (kw > 0) {
+			mine += (kw - 1) * PIECE;
+#pragma unroll
+			for (int db = 0; db < DB; ++db)
+#pragma unroll
+				for (int aa = 0; aa < 4; ++aa)
+					*(FA2_LDS f32x4*)(mine + (db * 4 + aa) * (NT * 16)) =
+					    f32x4{oacc[0][db][4 * aa], oacc[0][db][4 * aa + 1], oacc[0][db][4 * aa + 2], oacc[0][db][4 * aa + 3]};
+			FA2_LDS float* ml = (FA2_LDS float*)(mine - tid * 16 + DB * 4 * (NT * 16)) + tid;
+			ml[0] = mrow[0];
+			ml[NT] = lrow[0];
+		}
+		__syncthreads();
+		if (kw > 0) return;
+		const float cm = BIAS ? kLog2e : c1;  // the reference's units -> log2 domain
+#pragma unroll
+		for (int x = 1; x < KW; ++x) {
+			const FA2_LDS char* p = mine + (x - 1) * PIECE;
+			const FA2_LDS float* ml = (const FA2_LDS float*)(p - tid * 16 + DB * 4 * (NT * 16)) + tid;
+			const float mo = ml[0], mn = __builtin_fmaxf(mrow[0], mo);
+			// (a group without keys for the row: factor 0)
+			const float f0 = mrow[0] == -INFINITY ? 0.f : exp2_fast((mrow[0] - mn) * cm), f1 = mo == -INFINITY ? 0.f : exp2_fast((mo - mn) * cm);
+			mrow[0] = mn;
+			lrow[0] = lrow[0] * f0 + ml[NT] * f1;
+#pragma unroll
+			for (int db = 0; db < DB; ++db)
+#pragma unroll
+				for (int aa = 0; aa < 4; ++aa) {
+					const f32x4 y = *(const FA2_LDS f32x4*)(p + (db * 4 + aa) * (NT * 16));
+#pragma unroll
+					for (int e = 0; e < 4; ++e) oacc[0][db][4 * aa + e] = oacc[0][db][4 * aa + e] * f0 + y[e] * f1;
+				}
+		}
+	}
 
 	// epilogue: normalise, store O (lane: row c, four consecutive d per store) and LSE
 	char* obase = a.o.ptr + (int64_t)b * a.o.sb + (int64_t)h * a.o.sh;
@@ -980,8 +1037,8 @@ __global__ __launch_bounds__(NW * 64, WPS) void fwd_kernel(const KArgs a) {
 			if (i < a.Sq) {
 				int64_t row = (((int64_t)split * a.B + b) * a.Hq + hl[qb]) * a.Sq + i;
 				float* rp = a.o_part + row * D;
-#pragma unroll
-				for (int db = 0; db < DB; ++db)
+				// (a row without keys in this range leaves its -inf only: the combine kernel does not look at its O)
+				for (int db = 0; db < DB && lt > 0.f; ++db)
 #pragma unroll
 					for (int aa = 0; aa < 4; ++aa) {
 						const f32x16& r = oacc[qb][db];
@@ -1021,8 +1078,8 @@ __global__ __launch_bounds__(NW * 64, WPS) void fwd_kernel(const KArgs a) {
 
 // O = sum_s exp(lse_s - lse) O_s, lse = log sum_s exp(lse_s) over the key ranges of a split forward.
 // A row is D / 8 threads wide and G deep: group g of the row merges the ranges g, g + G, ... and the groups meet in LDS.
-// G = 8 where there are many ranges (decoding: few rows, so a row's partial results are loaded side by side instead of one
-// after the other - B8 Hq32, 16 ranges: 10.7 us with G = 1); G = 1 where rows are plenty and ranges few (HBM-bound).
+// G = 8 where rows are few and ranges many (256 rows, 16 ranges: 10.7 us with G = 1, which loads a row's partial results one after
+// the other, 4.7 with G = 8); G = 1 where there are rows enough to fill the chip.
 template <typename T, int D, int G>
 __global__ __launch_bounds__(256) void fwd_combine_kernel(const KArgs a) {
 	constexpr int TPR = D / 8;
@@ -1037,20 +1094,36 @@ __global__ __launch_bounds__(256) void fwd_combine_kernel(const KArgs a) {
 	float m = -INFINITY, tot = 0.f;
 	float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 	if (live) {
-		// (a range's weight and values are loaded together, rescaling as the maximum rises: one memory latency, not two)
-#pragma unroll 4
-		for (int s = g; s < a.nsplit; s += G) {
-			const float lse = a.lse_part[(int64_t)s * nrows + row];
-			const float* op = a.o_part + ((int64_t)s * nrows + row) * D + part * 8;
-			f32x4 x0 = *(const f32x4*)op, x1 = *(const f32x4*)(op + 4);
-			const float mn = __builtin_fmaxf(m, lse), ref = mn > -INFINITY ? mn : 0.f;
-			const float old = exp2_fast((m - ref) * kLog2e), wgt = exp2_fast((lse - ref) * kLog2e);
-			m = mn;
-			tot = tot * old + wgt;
+		// four ranges at a time, so that their loads are on their way together; of a range without keys for the row only lse is there
+		for (int s0 = g; s0 < a.nsplit; s0 += 4 * G) {
+			float lse[4];
+			f32x4 x0[4], x1[4];
 #pragma unroll
-			for (int e = 0; e < 4; ++e) {
-				acc[e] = acc[e] * old + wgt * x0[e];
-				acc[4 + e] = acc[4 + e] * old + wgt * x1[e];
+			for (int u = 0; u < 4; ++u) lse[u] = s0 + u * G < a.nsplit ? a.lse_part[(int64_t)(s0 + u * G) * nrows + row] : -INFINITY;
+#pragma unroll
+			for (int u = 0; u < 4; ++u) {
+				x0[u] = x1[u] = f32x4{0.f, 0.f, 0.f, 0.f};
+				if (lse[u] > -INFINITY) {
+					const float* op = a.o_part + ((int64_t)(s0 + u * G) * nrows + row) * D + part * 8;
+					x0[u] = *(const f32x4*)op;
+					x1[u] = *(const f32x4*)(op + 4);
+				}
+			}
+			const float mn = __builtin_fmaxf(__builtin_fmaxf(__builtin_fmaxf(m, lse[0]), lse[1]), __builtin_fmaxf(lse[2], lse[3]));
+			const float ref = mn > -INFINITY ? mn : 0.f, old = exp2_fast((m - ref) * kLog2e);
+			m = mn;
+			tot *= old;
+#pragma unroll
+			for (int e = 0; e < 8; ++e) acc[e] *= old;
+#pragma unroll
+			for (int u = 0; u < 4; ++u) {
+				const float wgt = exp2_fast((lse[u] - ref) * kLog2e);
+				tot += wgt;
+#pragma unroll
+				for (int e = 0; e < 4; ++e) {
+					acc[e] += wgt * x0[u][e];
+					acc[4 + e] += wgt * x1[u][e];
+				}
 			}
 		}
 	}
@@ -1098,7 +1171,7 @@ template <typename T, int D>
 hipError_t launch_fwd_combine_t(KArgs& a, hipStream_t s) {
 	const int64_t nrows = (int64_t)a.B * a.Hq * a.Sq;
 	constexpr int RPB1 = 256 / (D / 8), RPB8 = 256 / (D / 8) / 8;
-	if (a.nsplit >= 4)
+	if (a.nsplit >= 4 && nrows <= 2048)
 		hipLaunchKernelGGL((fwd_combine_kernel<T, D, 8>), dim3((unsigned)((nrows + RPB8 - 1) / RPB8)), dim3(256), 0, s, a);
 	else
 		hipLaunchKernelGGL((fwd_combine_kernel<T, D, 1>), dim3((unsigned)((nrows + RPB1 - 1) / RPB1)), dim3(256), 0, s, a);
@@ -1118,6 +1191,16 @@ struct FwdCfg {
 };
 
 // Split forward: 2 waves x 32 rows per workgroup (the query is short), nsplit key ranges each.
+// Split forward of a longer query on a small grid: the 128-row workgroups of eight waves of launch_fwd_t, nsplit key ranges each.
+template <typename T, int D>
+hipError_t launch_fwd_tall_split_t(KArgs& a, hipStream_t s) {
+	a.mtiles = (a.Sq + 127) / 128;
+	a.xcd_remap = (a.B * a.Hkv % 8 == 0) ? 1 : 0;
+	a.interleave = 1;
+	hipLaunchKernelGGL((fwd_kernel<T, D, 4, 1, 1, false, false, true, false, false, 2>), dim3((unsigned)(a.mtiles * a.B * a.Hq * a.nsplit)), dim3(512), 0, s, a);
+	return launch_fwd_combine_t<T, D>(a, s);
+}
+
 template <typename T, int D>
 hipError_t launch_fwd_split_t(bool bias, bool drop, KArgs& a, hipStream_t s) {
 	constexpr int NW = D == 256 ? 4 : 2, BM = NW * 32;  // (D = 256: four waves, the tile copies need the threads)
@@ -1142,8 +1225,8 @@ hipError_t launch_fwd_split_t(bool bias, bool drop, KArgs& a, hipStream_t s) {
 	return launch_fwd_combine_t<T, D>(a, s);
 }
 
-// One tile configuration: NW waves x 32 rows per workgroup (WPS: launch bound, waves per SIMD).
-template <typename T, int D, int NW, int WPS>
+// One tile configuration: NW waves x 32 rows per workgroup (WPS: launch bound, waves per SIMD), times KW groups that share the keys.
+template <typename T, int D, int NW, int WPS, int KW = 1>
 hipError_t launch_fwd_cfg(bool bias, bool drop, KArgs& a, hipStream_t s) {
 	constexpr int QB = 1, BM = NW * QB * 32;
 	a.mtiles = (a.Sq + BM - 1) / BM;
@@ -1151,38 +1234,54 @@ hipError_t launch_fwd_cfg(bool bias, bool drop, KArgs& a, hipStream_t s) {
 	a.xcd_remap = (groups % 8 == 0) ? 1 : 0;
 	a.interleave = a.xcd_remap ? launch_order(a, a.Hq / a.Hkv, groups / 8, (int64_t)a.Sk * D * 4) : 1;
 	if (bias && a.bias_sh == 0 && a.B % 8 == 0) a.xcd_remap = a.kv_lens ? 3 : 2;
-	dim3 grid((unsigned)(a.mtiles * a.B * a.Hq)), block(NW * 64);
-	a.fold_half = fold_half_of(a, NW, (int64_t)grid.x, D == 64 || WPS == 2);
+	dim3 grid((unsigned)(a.mtiles * a.B * a.Hq)), block(NW * 64 * KW);
+	a.fold_half = KW == 1 ? fold_half_of(a, NW, (int64_t)grid.x, D == 64 || WPS == 2) : 0;
 	const bool blds = bias && a.bias_lds;
-	if (a.softcap > 0.f && drop)
-		hipLaunchKernelGGL((fwd_kernel<T, D, NW, QB, WPS, true, true, false, false, true>), grid, block, 0, s, a);
-	else if (a.softcap > 0.f)
-		hipLaunchKernelGGL((fwd_kernel<T, D, NW, QB, WPS, true, false, false, false, true>), grid, block, 0, s, a);
-	else if (blds && drop)
-		hipLaunchKernelGGL((fwd_kernel<T, D, NW, QB, WPS, true, true, false, true>), grid, block, 0, s, a);
-	else if (blds)
-		hipLaunchKernelGGL((fwd_kernel<T, D, NW, QB, WPS, true, false, false, true>), grid, block, 0, s, a);
-	else if (bias && drop)
-		hipLaunchKernelGGL((fwd_kernel<T, D, NW, QB, WPS, true, true>), grid, block, 0, s, a);
-	else if (bias)
-		hipLaunchKernelGGL((fwd_kernel<T, D, NW, QB, WPS, true, false>), grid, block, 0, s, a);
-	else if (drop)
-		hipLaunchKernelGGL((fwd_kernel<T, D, NW, QB, WPS, false, true>), grid, block, 0, s, a);
-	else
-		hipLaunchKernelGGL((fwd_kernel<T, D, NW, QB, WPS, false, false>), grid, block, 0, s, a);
+	// (head dim 128 with bias tiles has no LDS for a second group)
+	constexpr bool WITH_BIAS = D == 64 || (KW == 1 && WPS == 1);
+	if (!bias && drop)
+		hipLaunchKernelGGL((fwd_kernel<T, D, NW, QB, WPS, false, true, false, false, false, KW>), grid, block, 0, s, a);
+	else if (!bias)
+		hipLaunchKernelGGL((fwd_kernel<T, D, NW, QB, WPS, false, false, false, false, false, KW>), grid, block, 0, s, a);
+	if constexpr (WITH_BIAS) {
+		if (!bias)
+			;
+		else if (a.softcap > 0.f && drop)
+			hipLaunchKernelGGL((fwd_kernel<T, D, NW, QB, WPS, true, true, false, false, true, KW>), grid, block, 0, s, a);
+		else if (a.softcap > 0.f)
+			hipLaunchKernelGGL((fwd_kernel<T, D, NW, QB, WPS, true, false, false, false, true, KW>), grid, block, 0, s, a);
+		else if (blds && drop)
+			hipLaunchKernelGGL((fwd_kernel<T, D, NW, QB, WPS, true, true, false, true, false, KW>), grid, block, 0, s, a);
+		else if (blds)
+			hipLaunchKernelGGL((fwd_kernel<T, D, NW, QB, WPS, true, false, false, true, false, KW>), grid, block, 0, s, a);
+		else if (drop)
+			hipLaunchKernelGGL((fwd_kernel<T, D, NW, QB, WPS, true, true, false, false, false, KW>), grid, block, 0, s, a);
+		else
+			hipLaunchKernelGGL((fwd_kernel<T, D, NW, QB, WPS, true, false, false, false, false, KW>), grid, block, 0, s, a);
+	}
 	return hipGetLastError();
 }
 
 template <typename T, int D>
 hipError_t launch_fwd_t(bool bias, bool drop, KArgs& a, hipStream_t s) {
 	if (a.decode_waves) return launch_fwd_decode_t<T, D>(a, s);
+	if constexpr (D <= 128) {
+		if (a.nsplit > 1 && a.tall_split) return launch_fwd_tall_split_t<T, D>(a, s);
+	}
 	if (a.nsplit > 1) return launch_fwd_split_t<T, D>(bias, drop, a, s);
 	typedef FwdCfg<T, D> C;
 	if constexpr (C::NW == 8) {
 		// A grid that leaves at least half of the chip idle (small batch x heads, short sequences): workgroups of
 		// 128 rows instead of 256, twice as many of them, still at most one per CU.
 		int64_t wgs = (int64_t)((a.Sq + 127) / 128) * a.B * a.Hq;
-		if (wgs <= kNumCU) return launch_fwd_cfg<T, D, 4, 1>(bias, drop, a, s);
+		if (wgs <= kNumCU) {
+			// ... and two groups of four waves that take the key tiles of the workgroup's rows in turn: two waves per SIMD where
+			// there was one (B1 Hq32 Hkv8 D128, 1000 rows over 9000 keys: 233 -> 170 us; B1 H8 S4096 D128 81 -> 71 us, causal 79 -> 61;
+			// B2 H16 S1024 D64 with bias 23.4 -> 20.5; B4 H12 S197 D64 9.3 -> 8.9).  With up to three tiles the merge costs more
+			// than it saves (B1 H8 S128: 8.7 us alone, 10.1 in two groups); four groups spill.
+			if (a.Sk > 3 * kFwdBN && (D == 64 || !bias)) return launch_fwd_cfg<T, D, 4, 1, 2>(bias, drop, a, s);
+			return launch_fwd_cfg<T, D, 4, 1>(bias, drop, a, s);
+		}
 		// Larger grids: two independent 128-row workgroups per CU instead of one of 256 rows - the same eight waves, but
 		// one workgroup computes while the other loads its Q, waits for its first tiles or stores its result, and a
 		// causal tile of 128 rows wastes less on the diagonal.  They read K and V twice as often, so only where the K

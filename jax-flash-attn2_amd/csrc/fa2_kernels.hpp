@@ -55,14 +55,15 @@ struct KArgs {
 	int dq_makes_delta;  // the dQ kernel computes delta itself (and stores it for the dK/dV kernel)
 	// split forward (0 / 1 = off): key ranges of split_len keys, partial results in scratch
 	int nsplit, split_len;
+	int pack_gqa;     // split forward: one workgroup holds the rows of all q-heads of a kv-head
+	float* o_part;    // [nsplit, B, Hq, Sq, D] fp32
+	float* lse_part;  // [nsplit, B, Hq, Sq] fp32
+	int tall_split;   // split forward: of a query longer than one row tile, in workgroups of 128 rows
 	// few query rows in all (fwd_decode_kernel): number of waves that share the key tiles (0 = off);
 	// pieces of units in o_part / lse_part, and per (batch, kv-head) where its pieces are
 	// (decode_whole: one (batch, kv-head) per wave, no scratch)
 	int decode_waves, decode_whole;
 	int32_t* decode_units;
-	int pack_gqa;     // split forward: one workgroup holds the rows of all q-heads of a kv-head
-	float* o_part;    // [nsplit, B, Hq, Sq, D] fp32
-	float* lse_part;  // [nsplit, B, Hq, Sq] fp32
 };
 
 // dtype: FA2_FP16 / FA2_BF16.  Return hipError_t of the launch.
