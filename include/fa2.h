@@ -46,7 +46,7 @@ enum {
 	FA2_EINVAL_BIAS = -8,     /* bias dtype / stride invalid                     */
 	FA2_EINVAL_MASK = -9,     /* seqlens given together with bias or with Sq != Sk
 	                             (_forward_triton.py:474-481)                    */
-	FA2_EUNSUPPORTED = -10,   /* head dim not in {64, 128, 256}                  */
+	FA2_EUNSUPPORTED = -10,   /* head dim not in {64, 128, 256}, or no variant for head_dim */
 	FA2_ESCRATCH = -11,       /* backward scratch missing or too small           */
 	FA2_EHIP = -12,           /* HIP runtime reported a launch error             */
 	FA2_ESCRATCH_STATIC = -13 /* fa2_bwd_static: the call needs more than
@@ -162,6 +162,13 @@ typedef struct fa2_params {
 	 * (_flash_attention.py:88), so this has no counterpart there. */
 	float* dbias;
 	int64_t dbias_stride_b, dbias_stride_h, dbias_stride_m;
+
+	/* Optional: the columns the rows of q, k, v, o, dO, dq, dk, dv really have, where that is less than D (0 or D: D).
+	 * The kernels then read and write no more than these, and the result is that of rows padded with zeros to D
+	 * (`scale` is the caller's either way).  Built for D = 128 and 72, 80, 88 or 96 columns without bias, soft-capping and dropout;
+	 * anything else, and a forward of so few query rows that its keys are better split over workgroups (where
+	 * fa2_fwd_scratch_bytes() asks for scratch without this field), is refused with FA2_EUNSUPPORTED: pad the rows.  */
+	int32_t head_dim;
 } fa2_params;
 
 /* sizeof(fa2_params) in the first version of this header: up to and including scratch_bytes */

@@ -59,6 +59,10 @@ size_t bwd_scratch_bytes(const fa2_params* p) {
 	return (n + 255) & ~(size_t)255;
 }
 
+// rows of fewer columns than the head dim of the tiles
+bool short_rows(const fa2_params* p) { return p->head_dim > 0 && p->head_dim != p->D; }
+bool fwd_takes_ranges(const fa2_params* p);
+
 // own_scratch: the backward brings its scratch itself (fa2_bwd_static), p->scratch is not looked at
 int validate(const fa2_params* p, int which, bool own_scratch = false) {
 	if (!p) return FA2_EINVAL_STRUCT;
@@ -67,6 +71,13 @@ int validate(const fa2_params* p, int which, bool own_scratch = false) {
 	if (p->B <= 0 || p->Sq <= 0 || p->Sk <= 0 || p->Hq <= 0 || p->Hkv <= 0 || p->D <= 0) return FA2_EINVAL_SHAPE;
 	if (p->Hq % p->Hkv) return FA2_EINVAL_HEADS;
 	if (p->D != 64 && p->D != 128 && p->D != 256) return FA2_EUNSUPPORTED;
+	if (short_rows(p)) {
+		// (up to 64 columns the tiles of head dim 64 would do, from 104 on there is too little to leave out)
+		if (p->D != 128 || p->head_dim <= 64 || p->head_dim > 96 || p->head_dim % 8) return FA2_EUNSUPPORTED;
+		if (p->bias || p->softcap > 0.f || p->p_drop > 0.f) return FA2_EUNSUPPORTED;
+		// a forward for which the kernels of few query rows or the key ranges are the better ones runs on padded rows
+		if (which == 0 && fwd_takes_ranges(p)) return FA2_EUNSUPPORTED;
+	}
 	if (!(p->p_drop >= 0.f && p->p_drop < 1.f)) return FA2_EINVAL_DROPOUT;
 	if (!isfinite(p->scale) || !(p->scale > 0.f)) return FA2_EINVAL_SHAPE;
 	if (!isfinite(p->softcap) || p->softcap < 0.f) return FA2_EINVAL_SHAPE;
@@ -146,6 +157,7 @@ void fill(const fa2_params* p, KArgs& a) {
 	}
 	a.seqlens = p->seqlens;
 	a.kv_lens = p->kv_lens;
+	a.hd = short_rows(p) ? p->head_dim : p->D;
 	a.B = p->B;
 	a.Sq = p->Sq;
 	a.Sk = p->Sk;
@@ -172,6 +184,7 @@ void fill(const fa2_params* p, KArgs& a) {
 namespace fa2 {
 
 hipError_t launch_fwd(int dtype, int D, bool bias, bool drop, KArgs& a, hipStream_t s) {
+	if (a.hd != D) return dtype == FA2_BF16 ? launch_fwd_bf16_96(bias, drop, a, s) : launch_fwd_fp16_96(bias, drop, a, s);
 	if (dtype == FA2_BF16) {
 		if (D == 64) return launch_fwd_bf16_64(bias, drop, a, s);
 		if (D == 128) return launch_fwd_bf16_128(bias, drop, a, s);
@@ -183,6 +196,7 @@ hipError_t launch_fwd(int dtype, int D, bool bias, bool drop, KArgs& a, hipStrea
 }
 
 hipError_t launch_bwd(int dtype, int D, bool bias, bool drop, KArgs& a, hipStream_t s) {
+	if (a.hd != D) return dtype == FA2_BF16 ? launch_bwd_bf16_96(bias, drop, a, s) : launch_bwd_fp16_96(bias, drop, a, s);
 	if (dtype == FA2_BF16) {
 		if (D == 64) return launch_bwd_bf16_64(bias, drop, a, s);
 		if (D == 128) return launch_bwd_bf16_128(bias, drop, a, s);
@@ -361,10 +375,21 @@ static size_t fwd_scratch_bytes(const fa2_params* p) {
 	return (rows * ((size_t)p->D + 1) * sizeof(float) + 255) & ~(size_t)255;
 }
 
+}  // extern "C"
+
+namespace {
+bool fwd_takes_ranges(const fa2_params* p) {
+	int whole;
+	return fwd_decode_waves(p, &whole) || fwd_scratch_bytes(p);
+}
+}  // namespace
+
+extern "C" {
+
 size_t fa2_fwd_scratch_bytes(const fa2_params* p) {
 	fa2_params lp;
 	p = complete(p, lp);
-	return p ? fwd_scratch_bytes(p) : 0;
+	return p && !short_rows(p) ? fwd_scratch_bytes(p) : 0;
 }
 
 int fa2_fwd(const fa2_params* p, void* hip_stream) {
@@ -374,6 +399,7 @@ int fa2_fwd(const fa2_params* p, void* hip_stream) {
 	if (rc) return rc;
 	KArgs a;
 	fill(p, a);
+	if (short_rows(p)) return fa2::launch_fwd(p->dtype, p->D, false, false, a, (hipStream_t)hip_stream) == hipSuccess ? FA2_OK : FA2_EHIP;
 	// optional scratch: with enough of it a short query over many keys runs split over key ranges
 	size_t need = fwd_scratch_bytes(p);
 	const bool room = need && p->scratch && ((uintptr_t)p->scratch & 255) == 0 && p->scratch_bytes >= need;
@@ -493,7 +519,7 @@ const char* fa2_strerror(int code) {
 		case FA2_EINVAL_DROPOUT: return "dropout probability must be in [0, 1)";
 		case FA2_EINVAL_BIAS: return "bias dtype or strides invalid";
 		case FA2_EINVAL_MASK: return "Attention mask is not supported along with attention bias or with QSeq != KSeq";
-		case FA2_EUNSUPPORTED: return "head dim must be 64, 128 or 256";
+		case FA2_EUNSUPPORTED: return "head dim must be 64, 128 or 256 (and head_dim one the kernels of D have a variant for)";
 		case FA2_ESCRATCH: return "backward scratch buffer missing, misaligned or too small";
 		case FA2_EHIP: return "HIP launch failed";
 		case FA2_ESCRATCH_STATIC: return "fa2_bwd_static: B * Hq * Sq * 4 bytes exceed the 16 MiB built-in scratch";

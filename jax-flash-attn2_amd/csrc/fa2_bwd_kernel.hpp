@@ -38,15 +38,18 @@ __global__ __launch_bounds__(256) void bwd_delta_kernel(const KArgs a) {
 	int64_t nrows = (int64_t)a.B * a.Sq * a.Hq;
 	float acc = 0.f;
 	int h = 0, b = 0, i = 0;
+	const bool in = part * 8 < a.hd;
 	if (row < nrows) {
 		h = (int)(row % a.Hq);
 		int64_t r = row / a.Hq;
 		i = (int)(r % a.Sq);
 		b = (int)(r / a.Sq);
-		typename T::V8 o = *(const typename T::V8*)(a.o.ptr + b * a.o.sb + (int64_t)i * a.o.ss + (int64_t)h * a.o.sh + part * 16);
-		typename T::V8 d = *(const typename T::V8*)(a.dout.ptr + b * a.dout.sb + (int64_t)i * a.dout.ss + (int64_t)h * a.dout.sh + part * 16);
+		if (in) {
+			typename T::V8 o = *(const typename T::V8*)(a.o.ptr + b * a.o.sb + (int64_t)i * a.o.ss + (int64_t)h * a.o.sh + part * 16);
+			typename T::V8 d = *(const typename T::V8*)(a.dout.ptr + b * a.dout.sb + (int64_t)i * a.dout.ss + (int64_t)h * a.dout.sh + part * 16);
 #pragma unroll
-		for (int e = 0; e < 8; ++e) acc += (float)o[e] * (float)d[e];
+			for (int e = 0; e < 8; ++e) acc += (float)o[e] * (float)d[e];
+		}
 	}
 #pragma unroll
 	for (int sft = TPR / 2; sft >= 1; sft >>= 1) acc += __shfl_xor(acc, sft, 64);
@@ -102,25 +105,26 @@ FA2_DEV DkdvRow dkdv_row(const KArgs& a, int b) {
 }
 
 // K, V rows of this lane's key of key tile nt as B operands: the lane holds X[key][16 ks + 8 g .. + 7].
-template <typename T, int D, int NW>
-FA2_DEV void dkdv_load_kv(const KArgs& a, int nt, int hk, int b, typename T::V8 (&kf)[D / 16], typename T::V8 (&vf)[D / 16]) {
+template <typename T, int DE, int NW, bool COLS>
+FA2_DEV void dkdv_load_kv(const KArgs& a, int nt, int hk, int b, typename T::V8 (&kf)[DE / 16], typename T::V8 (&vf)[DE / 16]) {
 	typedef typename T::V8 V8;
 	const int tid = threadIdx.x, lane = tid & 63;
 	const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
 	const int g = lane >> 5, c = lane & 31;
 	const int jcol = nt * (NW * 32) + 32 * w + c;
 	int j = jcol < a.Sk ? jcol : a.Sk - 1;
-	const char* kp = a.k.ptr + (int64_t)b * a.k.sb + (int64_t)hk * a.k.sh + (int64_t)j * a.k.ss + g * 16;
-	const char* vp = a.v.ptr + (int64_t)b * a.v.sb + (int64_t)hk * a.v.sh + (int64_t)j * a.v.ss + g * 16;
+	const char* kp = a.k.ptr + (int64_t)b * a.k.sb + (int64_t)hk * a.k.sh + (int64_t)j * a.k.ss;
+	const char* vp = a.v.ptr + (int64_t)b * a.v.sb + (int64_t)hk * a.v.sh + (int64_t)j * a.v.ss;
 #pragma unroll
-	for (int ks = 0; ks < D / 16; ++ks) {
-		kf[ks] = *(const V8*)(kp + ks * 32);
-		vf[ks] = *(const V8*)(vp + ks * 32);
+	for (int ks = 0; ks < DE / 16; ++ks) {
+		kf[ks] = load_row8<V8, COLS>(kp, 16 * ks + 8 * g, a.hd);
+		vf[ks] = load_row8<V8, COLS>(vp, 16 * ks + 8 * g, a.hd);
 	}
 }
 
 // WALKS: `order` is a run-time value (the paired kernel); otherwise the tile is walked head by head and `order_rt` is not looked at.
-template <typename T, int D, int NW, int QB, bool BIAS, bool DROP, bool BIAS_T, bool CAP, bool WALKS>
+// DE: columns of the products (DE < D: rows of a.hd <= DE columns in tiles of D, see the forward kernel).
+template <typename T, int D, int NW, int QB, bool BIAS, bool DROP, bool BIAS_T, bool CAP, bool WALKS, int DE = D>
 FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int b, const int hsi, const int hsplit, const int order_rt,
                            const int rot, const DkdvRow& rw) {
 	const int order = WALKS ? order_rt : 0;
@@ -128,8 +132,10 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 	typedef typename T::V8 V8;
 	constexpr int BN = NW * 32;     // keys per workgroup
 	constexpr int BMQ = QB * 32;    // query rows per streamed tile
-	constexpr int KS = D / 16;
-	constexpr int DB = D / 32;
+	constexpr int KS = DE / 16;
+	constexpr int DB = DE / 32;
+	constexpr bool COLS = DE < D;
+	static_assert(!COLS || (!BIAS && !DROP), "");
 	constexpr int NT = NW * 64;
 	constexpr int TILE_BYTES = BMQ * D * 2;
 	constexpr int STAT_BYTES = BMQ * 4;
@@ -184,7 +190,7 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 
 	// K, V rows of this lane's key as B operands: lane holds X[jcol][16ks + 8g .. +7]
 	V8 kf[KS], vf[KS];
-	dkdv_load_kv<T, D, NW>(a, nt, hk, b, kf, vf);
+	dkdv_load_kv<T, DE, NW, COLS>(a, nt, hk, b, kf, vf);
 	// The fragments must have arrived before the loop over streamed tiles starts.  Otherwise the compiler places its
 	// waits for these loads (s_waitcnt vmcnt) at their first uses inside the loop - it does not see the wait that
 	// publishes a tile - where the same counter also counts the tile copies in flight: every step would then wait
@@ -235,9 +241,13 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 	const float c1 = BIAS ? a.scale : a.scale * kLog2e;
 	const float inv_scale = 1.f / a.scale;
 
-	TileLoader<D, BMQ, NT> qload, doload;
-	qload.init(a.q.ss, tid);
-	doload.init(a.dout.ss, tid);
+	TileLoader<D, BMQ, NT, COLS> qload, doload;
+	const int cols = COLS ? a.hd >> 3 : D / 8;  // 16-byte chunks of a row
+	qload.init(a.q.ss, tid, BMQ, cols);
+	doload.init(a.dout.ss, tid, BMQ, cols);
+	if constexpr (COLS) {
+		for (int i = 0; i < 4; ++i) zero_cols<D, BMQ, NT>(lds + i * TILE_BYTES, tid, cols, DE / 8);
+	}
 	TileLoader<128, BMQ, NT> bload;
 	if constexpr (BIAS_LDS) bload.init(a.bias_sm, tid);
 	// Streamed tile `step` in the order `order` asks for (see above).  Head by head is what a workgroup with one key
@@ -280,8 +290,8 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 	};
 	auto issue_tile = [&](int step, const TileBase& tb, int m0, FA2_LDS char* qdst, FA2_LDS char* dodst) __attribute__((always_inline)) {
 		int rows = a.Sq - m0 < BMQ ? a.Sq - m0 : BMQ;
-		qload.load(qdst, tb.q, a.q.ss, rows, tid);
-		doload.load(dodst, tb.dout, a.dout.ss, rows, tid);
+		qload.load(qdst, tb.q, a.q.ss, rows, tid, cols);
+		doload.load(dodst, tb.dout, a.dout.ss, rows, tid, cols);
 		if constexpr (BIAS_LDS) bload.load(lds_bias + ((step - s_lo) & 1) * BIAS_BYTES, tb.bias, a.bias_sm, rows, tid, (a.Sk - n0) >> 3);
 	};
 	// per-row statistics of a tile: thread t < BMQ fetches lse, t in [BMQ, 2 BMQ) fetches delta.
@@ -365,7 +375,7 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 		constexpr int NSLOT = 2 * KS;     // = 4 DB
 		constexpr int PA = 4;             // read-ahead distance in slots
 		constexpr int RING = PA + 1;
-		static_assert(NSLOT % 16 == 0 || 16 % NSLOT == 0, "");
+		static_assert(NSLOT % 16 == 0 || NSLOT == 8 || (NSLOT == 12 && FOLD), "");
 		f32x16 s[2], dp[2];
 		u32x4 pbits[2][2], sbits[2][2];   // [block parity][16-row half]: P and dS packed to 16 bits
 		V8 afr[RING];                     // fragments of Q_i / dO_i for the products of A
@@ -701,12 +711,11 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 								micro_B(k - 1, ms / 4, ms % 4, e0, e1, s[(k - 1) & 1], dp[(k - 1) & 1], pbits[(k - 1) & 1], sbits[(k - 1) & 1]);
 							}
 						} else {
-							// several quads share a slot, all in the same phase
-							constexpr int QPS = 16 / NSLOT;  // quads per slot
-							int grp = j / 4, phase = j % 4;
+							// several quads share a slot, all in the same phase (twelve slots: quads 0 and 1 the first four, then one quad each)
+							const int grp = j / 4, phase = j % 4;
+							const int q0 = NSLOT == 12 ? (grp ? grp + 1 : 0) : grp * (16 / NSLOT), q1 = NSLOT == 12 ? grp + 2 : q0 + 16 / NSLOT;
 #pragma unroll
-							for (int e = 0; e < QPS; ++e) {
-								int q = grp * QPS + e;
+							for (int q = q0; q < q1; ++q) {
 								micro_B(k - 1, q, phase, e0, e1, s[(k - 1) & 1], dp[(k - 1) & 1], pbits[(k - 1) & 1], sbits[(k - 1) & 1]);
 							}
 						}
@@ -891,6 +900,7 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 		for (int db = 0; db < DB; ++db)
 #pragma unroll
 			for (int aa = 0; aa < 4; ++aa) {
+				if (COLS && 32 * db + 8 * aa >= a.hd) continue;
 				int d0 = 32 * db + 8 * aa + 4 * g;
 				u32x2 pk = {pack2<typename T::V2>(dk[db][4 * aa] * ks_, dk[db][4 * aa + 1] * ks_),
 				            pack2<typename T::V2>(dk[db][4 * aa + 2] * ks_, dk[db][4 * aa + 3] * ks_)};
@@ -907,7 +917,7 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 // CAP: tanh soft-capping of the scores (see the forward kernel); the bias itself may then be absent
 // PAIR: the instantiation for launches that give a workgroup two key tiles (a.kv_pair); the launcher picks it only then,
 // so that every other launch runs the kernel with the one walk as a compile-time constant.
-template <typename T, int D, int NW, int QB, bool BIAS, bool DROP, bool BIAS_T, bool CAP = false, bool PAIR = false>
+template <typename T, int D, int NW, int QB, bool BIAS, bool DROP, bool BIAS_T, bool CAP = false, bool PAIR = false, int DE = D>
 __global__ __launch_bounds__(NW * 64) void bwd_dkdv_kernel(const KArgs a) {
 	// (with the steps of a key tile split over workgroups: the parts of one key tile are adjacent)
 	int hk, b, within;
@@ -947,7 +957,7 @@ __global__ __launch_bounds__(NW * 64) void bwd_dkdv_kernel(const KArgs a) {
 	const DkdvRow rw = dkdv_row<DROP>(a, b);
 	if constexpr (!PAIR) {
 		// one key tile, head by head (early key tiles see the most query rows under a causal mask: first)
-		bwd_dkdv_tile<T, D, NW, QB, BIAS, DROP, BIAS_T, CAP, false>(a, within, hk, b, hsi, hsplit, 0, 0, rw);
+		bwd_dkdv_tile<T, D, NW, QB, BIAS, DROP, BIAS_T, CAP, false, DE>(a, within, hk, b, hsi, hsplit, 0, 0, rw);
 	} else {
 		// Causal self-attention: key tile p streams every query tile from p up, so a workgroup takes tile p and tile
 		// ntiles - 1 - p one after the other - every workgroup then has the same number of steps (no CU waits for the
@@ -962,7 +972,7 @@ __global__ __launch_bounds__(NW * 64) void bwd_dkdv_kernel(const KArgs a) {
 		const int npass = partner != within ? 2 : 1;
 		const int rot = within % r;
 		for (int pass = 0; pass < npass; ++pass) {
-			bwd_dkdv_tile<T, D, NW, QB, BIAS, DROP, BIAS_T, CAP, true>(a, pass == 0 ? within : partner, hk, b, 0, 1, 2 - pass, rot, rw);
+			bwd_dkdv_tile<T, D, NW, QB, BIAS, DROP, BIAS_T, CAP, true, DE>(a, pass == 0 ? within : partner, hk, b, 0, 1, 2 - pass, rot, rw);
 			// (the LDS buffers of the first tile are free once every wave has left its last step)
 			if (pass + 1 < npass) __syncthreads();
 		}
@@ -976,8 +986,8 @@ __global__ __launch_bounds__(256) void bwd_dkdv_reduce_kernel(const KArgs a, flo
 	constexpr int CH = D / 8;  // chunks of eight per row
 	int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
 	int64_t total = (int64_t)a.B * a.Hkv * a.Sk * 2 * CH;
-	if (idx >= total) return;
 	int ch = (int)(idx % CH);
+	if (idx >= total || ch * 8 >= a.hd) return;
 	int which = (int)((idx / CH) % 2);
 	int64_t row = idx / (2 * CH);  // (b * Hkv + hk) * Sk + key
 	int key = (int)(row % a.Sk);
@@ -1009,16 +1019,19 @@ __global__ __launch_bounds__(256) void bwd_dkdv_reduce_kernel(const KArgs a, flo
 // ---------------------------------------------------------------------------
 // BLDS: the bias goes through LDS as in the forward kernel (conditions checked by the launcher)
 // DBIAS: also writes the gradient of the additive term (a.dbias); on the plain path with bias
-template <typename T, int D, int NW, int QB, int WPS, bool BIAS, bool DROP, bool BLDS = false, bool CAP = false, bool DBIAS = false>
+// DE: columns of the products (DE < D: rows of a.hd <= DE columns in tiles of D, see the forward kernel)
+template <typename T, int D, int NW, int QB, int WPS, bool BIAS, bool DROP, bool BLDS = false, bool CAP = false, bool DBIAS = false, int DE = D>
 __global__ __launch_bounds__(NW * 64, WPS) void bwd_dq_kernel(const KArgs a) {
+	constexpr bool COLS = DE < D;
+	static_assert(!COLS || (!BIAS && !DROP), "");
 	static_assert(!CAP || (BIAS && !BLDS), "soft-capping runs on the plain path with bias");
 	static_assert(!DBIAS || (BIAS && !BLDS), "the bias gradient is written on the plain path with bias");
 	typedef typename T::V8 V8;
 	constexpr int BM = NW * QB * 32;
 	constexpr int BN = kFwdBN;
 	constexpr int KB = BN / 32;
-	constexpr int KS = D / 16;
-	constexpr int DB = D / 32;
+	constexpr int KS = DE / 16;
+	constexpr int DB = DE / 32;
 	constexpr int NT = NW * 64;
 	constexpr int TILE_BYTES = BN * D * 2;
 
@@ -1121,14 +1134,18 @@ __global__ __launch_bounds__(NW * 64, WPS) void bwd_dq_kernel(const KArgs a) {
 
 	const char* kbase = a.k.ptr + (int64_t)b * a.k.sb + (int64_t)hk * a.k.sh;
 	const char* vbase = a.v.ptr + (int64_t)b * a.v.sb + (int64_t)hk * a.v.sh;
-	TileLoader<D, BN, NT> kload, vload;
-	kload.init(a.k.ss, tid);
-	vload.init(a.v.ss, tid);
+	TileLoader<D, BN, NT, COLS> kload, vload;
+	const int cols = COLS ? a.hd >> 3 : D / 8;  // 16-byte chunks of a row
+	kload.init(a.k.ss, tid, BN, cols);
+	vload.init(a.v.ss, tid, BN, cols);
+	if constexpr (COLS) {
+		for (int i = 0; i < 4; ++i) zero_cols<D, BN, NT>(lds + i * TILE_BYTES, tid, cols, DE / 8);
+	}
 	if (ntiles > t_begin) {
 		int nb = t_begin * BN, bsel = t_begin & 1;
 		int rows = sk_eff - nb < BN ? sk_eff - nb : BN;
-		kload.load(lds + bsel * TILE_BYTES, kbase + (int64_t)nb * a.k.ss, a.k.ss, rows, tid);
-		vload.load(lds + (2 + bsel) * TILE_BYTES, vbase + (int64_t)nb * a.v.ss, a.v.ss, rows, tid);
+		kload.load(lds + bsel * TILE_BYTES, kbase + (int64_t)nb * a.k.ss, a.k.ss, rows, tid, cols);
+		vload.load(lds + (2 + bsel) * TILE_BYTES, vbase + (int64_t)nb * a.v.ss, a.v.ss, rows, tid, cols);
 	}
 
 	V8 qf[QB][KS], dof[QB][KS];
@@ -1138,12 +1155,12 @@ __global__ __launch_bounds__(NW * 64, WPS) void bwd_dq_kernel(const KArgs a) {
 #pragma unroll
 		for (int qb = 0; qb < QB; ++qb) {
 			int i = qrow[qb] < a.Sq ? qrow[qb] : a.Sq - 1;
-			const char* rp = qbase + (int64_t)i * a.q.ss + g * 16;
-			const char* dp_ = dbase + (int64_t)i * a.dout.ss + g * 16;
+			const char* rp = qbase + (int64_t)i * a.q.ss;
+			const char* dp_ = dbase + (int64_t)i * a.dout.ss;
 #pragma unroll
 			for (int ks = 0; ks < KS; ++ks) {
-				qf[qb][ks] = *(const V8*)(rp + ks * 32);
-				dof[qb][ks] = *(const V8*)(dp_ + ks * 32);
+				qf[qb][ks] = load_row8<V8, COLS>(rp, 16 * ks + 8 * g, a.hd);
+				dof[qb][ks] = load_row8<V8, COLS>(dp_, 16 * ks + 8 * g, a.hd);
 			}
 		}
 	}
@@ -1156,11 +1173,11 @@ __global__ __launch_bounds__(NW * 64, WPS) void bwd_dq_kernel(const KArgs a) {
 #pragma unroll
 		for (int qb = 0; qb < QB; ++qb) {
 			int i = qrow[qb] < a.Sq ? qrow[qb] : a.Sq - 1;
-			const char* op_ = obase_ + (int64_t)i * a.o.ss + g * 16;
+			const char* op_ = obase_ + (int64_t)i * a.o.ss;
 			float acc4[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
 			for (int ks = 0; ks < KS; ++ks) {
-				V8 ov = *(const V8*)(op_ + ks * 32);
+				V8 ov = load_row8<V8, COLS>(op_, 16 * ks + 8 * g, a.hd);
 #pragma unroll
 				for (int e = 0; e < 8; ++e) acc4[e & 3] += (float)ov[e] * (float)dof[qb][ks][e];
 			}
@@ -1515,8 +1532,8 @@ __global__ __launch_bounds__(NW * 64, WPS) void bwd_dq_kernel(const KArgs a) {
 		if (t + 1 < ntiles) {
 			int n1 = n0 + BN;
 			int rows = sk_eff - n1 < BN ? sk_eff - n1 : BN;
-			kload.load(lds + (buf ^ 1) * TILE_BYTES, kbase + (int64_t)n1 * a.k.ss, a.k.ss, rows, tid);
-			vload.load(lds + (2 + (buf ^ 1)) * TILE_BYTES, vbase + (int64_t)n1 * a.v.ss, a.v.ss, rows, tid);
+			kload.load(lds + (buf ^ 1) * TILE_BYTES, kbase + (int64_t)n1 * a.k.ss, a.k.ss, rows, tid, cols);
+			vload.load(lds + (2 + (buf ^ 1)) * TILE_BYTES, vbase + (int64_t)n1 * a.v.ss, a.v.ss, rows, tid, cols);
 			if constexpr (BIAS_LDS) {
 				if (bias_lds)
 					bload.load(lds + 4 * TILE_BYTES + (buf ^ 1) * BIAS_BYTES, bias_base + (int64_t)m0 * a.bias_sm + (int64_t)n1 * 2,
@@ -1564,6 +1581,7 @@ __global__ __launch_bounds__(NW * 64, WPS) void bwd_dq_kernel(const KArgs a) {
 			for (int db = 0; db < DB; ++db)
 #pragma unroll
 				for (int aa = 0; aa < 4; ++aa) {
+					if (COLS && 32 * db + 8 * aa >= a.hd) continue;
 					const f32x16& x = dq[qb][db];
 					u32x2 pk = {pack2<typename T::V2>(x[4 * aa] * sc, x[4 * aa + 1] * sc),
 					            pack2<typename T::V2>(x[4 * aa + 2] * sc, x[4 * aa + 3] * sc)};
@@ -1586,7 +1604,7 @@ struct BwdCfg {
 	static constexpr int DQ_BM = DQ_NW * DQ_QB * 32;
 };
 
-template <typename T, int D, bool BIAS, bool DROP>
+template <typename T, int D, int DE, bool BIAS, bool DROP>
 hipError_t launch_bwd_v(KArgs& a, hipStream_t s) {
 	typedef BwdCfg<T, D> C;
 	int groups = a.B * a.Hkv;
@@ -1605,19 +1623,23 @@ hipError_t launch_bwd_v(KArgs& a, hipStream_t s) {
 	auto launch_dq_cfg = [&](auto nw_tag, auto wps_tag) {
 		constexpr int NW = decltype(nw_tag)::value, BM = NW * C::DQ_QB * 32, WPS = decltype(wps_tag)::value;
 		a.mtiles = (a.Sq + BM - 1) / BM;
-		a.interleave = a.xcd_remap == 1 ? launch_order(a, a.Hq / a.Hkv, groups / 8, (int64_t)a.Sk * D * 4) : 1;
+		a.interleave = a.xcd_remap == 1 ? launch_order(a, a.Hq / a.Hkv, groups / 8, (int64_t)a.Sk * DE * 4) : 1;
 		dim3 grid((unsigned)(a.mtiles * a.B * a.Hq)), block(NW * 64);
 		a.fold_half = fold_half_of(a, NW, (int64_t)grid.x, D == 64 || WPS == 2);
-		if (BIAS && a.dbias && a.softcap > 0.f)
-			hipLaunchKernelGGL((bwd_dq_kernel<T, D, NW, C::DQ_QB, WPS, BIAS, DROP, false, BIAS, BIAS>), grid, block, 0, s, a);
-		else if (BIAS && a.dbias)
-			hipLaunchKernelGGL((bwd_dq_kernel<T, D, NW, C::DQ_QB, WPS, BIAS, DROP, false, false, BIAS>), grid, block, 0, s, a);
-		else if (BIAS && a.softcap > 0.f)
-			hipLaunchKernelGGL((bwd_dq_kernel<T, D, NW, C::DQ_QB, WPS, BIAS, DROP, false, BIAS>), grid, block, 0, s, a);
-		else if (BIAS && a.bias_lds)
-			hipLaunchKernelGGL((bwd_dq_kernel<T, D, NW, C::DQ_QB, WPS, BIAS, DROP, BIAS>), grid, block, 0, s, a);
-		else
-			hipLaunchKernelGGL((bwd_dq_kernel<T, D, NW, C::DQ_QB, WPS, BIAS, DROP, false>), grid, block, 0, s, a);
+		if constexpr (BIAS) {
+			if (a.dbias && a.softcap > 0.f)
+				hipLaunchKernelGGL((bwd_dq_kernel<T, D, NW, C::DQ_QB, WPS, true, DROP, false, true, true>), grid, block, 0, s, a);
+			else if (a.dbias)
+				hipLaunchKernelGGL((bwd_dq_kernel<T, D, NW, C::DQ_QB, WPS, true, DROP, false, false, true>), grid, block, 0, s, a);
+			else if (a.softcap > 0.f)
+				hipLaunchKernelGGL((bwd_dq_kernel<T, D, NW, C::DQ_QB, WPS, true, DROP, false, true>), grid, block, 0, s, a);
+			else if (a.bias_lds)
+				hipLaunchKernelGGL((bwd_dq_kernel<T, D, NW, C::DQ_QB, WPS, true, DROP, true>), grid, block, 0, s, a);
+			else
+				hipLaunchKernelGGL((bwd_dq_kernel<T, D, NW, C::DQ_QB, WPS, true, DROP>), grid, block, 0, s, a);
+		} else {
+			hipLaunchKernelGGL((bwd_dq_kernel<T, D, NW, C::DQ_QB, WPS, false, DROP, false, false, false, DE>), grid, block, 0, s, a);
+		}
 	};
 	auto launch_dq = [&]() {
 		if constexpr (C::DQ_NW == 8) {
@@ -1629,7 +1651,7 @@ hipError_t launch_bwd_v(KArgs& a, hipStream_t s) {
 			// 0.784 -> 0.734 ms, B4 S4096 causal 0.770 -> 0.739 ms; D = 64 B32 S512 0.060 -> 0.051 ms); D = 128 with bias
 			// would spill within 256 registers
 			if constexpr (D == 64 || !BIAS) {
-				if ((int64_t)a.Sk * D * 4 <= (4 << 20))
+				if ((int64_t)a.Sk * DE * 4 <= (4 << 20))
 					return launch_dq_cfg(std::integral_constant<int, 4>{}, std::integral_constant<int, (D == 128 ? 2 : 1)>{});
 			}
 		}
@@ -1638,7 +1660,7 @@ hipError_t launch_bwd_v(KArgs& a, hipStream_t s) {
 	if (fused_delta) launch_dq();
 	if (a.stages & 2) {
 		a.mtiles = (a.Sk + C::KV_BN - 1) / C::KV_BN;
-		a.interleave = a.xcd_remap == 1 ? launch_order(a, 1, groups / 8, (int64_t)(a.Hq / a.Hkv) * a.Sq * D * 4) : 1;
+		a.interleave = a.xcd_remap == 1 ? launch_order(a, 1, groups / 8, (int64_t)(a.Hq / a.Hkv) * a.Sq * DE * 4) : 1;
 		const int hs = a.kv_hsplit > 1 ? a.kv_hsplit : 1;
 		// Causal self-attention on a grid that fills the chip in whole rounds: every workgroup takes the key tiles p and
 		// ntiles - 1 - p one after the other (see bwd_dkdv_kernel).  Measured on the 4096-token workload (B4 Hq32 Hkv8):
@@ -1663,15 +1685,19 @@ hipError_t launch_bwd_v(KArgs& a, hipStream_t s) {
 		if (!a.bias_lds) typed = false;
 		// with bias at D = 128 the streamed tiles are 64 rows, which leaves LDS room for the bias tiles
 		constexpr int QBV = (BIAS && D == 128) ? 2 : C::KV_QB;
-		if (BIAS && a.softcap > 0.f)
-			hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, C::KV_NW, QBV, BIAS, DROP, false, BIAS>), grid, block, 0, s, a);
-		else if (typed)
-			hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, C::KV_NW, QBV, BIAS, DROP, BIAS>), grid, block, 0, s, a);
-		else if (a.kv_pair) {
+		if constexpr (BIAS) {
+			if (a.softcap > 0.f)
+				hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, C::KV_NW, QBV, true, DROP, false, true>), grid, block, 0, s, a);
+			else if (typed)
+				hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, C::KV_NW, QBV, true, DROP, true>), grid, block, 0, s, a);
+			else
+				hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, C::KV_NW, QBV, true, DROP, false>), grid, block, 0, s, a);
+		} else if (a.kv_pair) {
 			// (only instantiated where the launcher can choose it: no bias, head dim up to 128)
-			if constexpr (D <= 128 && !BIAS) hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, C::KV_NW, QBV, BIAS, DROP, false, false, true>), grid, block, 0, s, a);
-		} else
-			hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, C::KV_NW, QBV, BIAS, DROP, false>), grid, block, 0, s, a);
+			if constexpr (D <= 128) hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, C::KV_NW, QBV, false, DROP, false, false, true, DE>), grid, block, 0, s, a);
+		} else {
+			hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, C::KV_NW, QBV, false, DROP, false, false, false, DE>), grid, block, 0, s, a);
+		}
 		if (hs > 1) {
 			int64_t total = (int64_t)a.B * a.Hkv * a.Sk * 2 * (D / 8);
 			hipLaunchKernelGGL((bwd_dkdv_reduce_kernel<T, D>), dim3((unsigned)((total + 255) / 256)), dim3(256), 0, s, a, a.scale,
@@ -1682,12 +1708,15 @@ hipError_t launch_bwd_v(KArgs& a, hipStream_t s) {
 	return hipGetLastError();
 }
 
-template <typename T, int D>
+// DE < D: without bias and dropout (the C ABI checks)
+template <typename T, int D, int DE = D>
 hipError_t launch_bwd_t(bool bias, bool drop, KArgs& a, hipStream_t s) {
-	if (bias && drop) return launch_bwd_v<T, D, true, true>(a, s);
-	if (bias) return launch_bwd_v<T, D, true, false>(a, s);
-	if (drop) return launch_bwd_v<T, D, false, true>(a, s);
-	return launch_bwd_v<T, D, false, false>(a, s);
+	if constexpr (DE == D) {
+		if (bias && drop) return launch_bwd_v<T, D, D, true, true>(a, s);
+		if (bias) return launch_bwd_v<T, D, D, true, false>(a, s);
+		if (drop) return launch_bwd_v<T, D, D, false, true>(a, s);
+	}
+	return launch_bwd_v<T, D, DE, false, false>(a, s);
 }
 
 }  // namespace fa2

@@ -252,7 +252,9 @@ FA2_DEV void lds_dma16_so(uint32_t lane_off, const char* uniform_base, FA2_LDS c
 	             : "m0");
 }
 
-template <int D, int ROWS, int NTHREADS>
+// COLS: rows in memory are shorter than the tile's (head dims that are not the tile's own): lanes whose chunk lies beyond the row
+// fetch nothing, and what the tile holds there stays as it is - zero where zero_cols() has been called.
+template <int D, int ROWS, int NTHREADS, bool COLS = false>
 struct TileLoader {
 	static constexpr int CPR = D / 8;
 	static constexpr int TOTAL = ROWS * CPR;
@@ -270,6 +272,8 @@ struct TileLoader {
 	int rows_state;  // the offsets clamp rows to [0, rows_state)
 	int cols_state;  // ... and 16-byte chunks of a row to [0, cols_state)
 	int wave_slot;   // byte offset of this wave's 64 x 16 bytes inside a piece (scalar)
+	bool lane_on;    // COLS: this lane's chunk is inside the row (the same for every piece: pieces differ by whole 16-row blocks)
+	static_assert(!COLS || (!COMPACT && RPI % 16 == 0), "");
 
 	static FA2_DEV uint32_t offset_of(int it, int64_t stride_bytes, int tid, int rows_valid, int chunks_valid) {
 		int slot = it * NTHREADS + tid;
@@ -284,6 +288,7 @@ struct TileLoader {
 		rows_state = rows_valid;
 		cols_state = chunks_valid;
 		wave_slot = __builtin_amdgcn_readfirstlane((tid >> 6) << 10);
+		if constexpr (COLS) lane_on = ((tid % CPR) ^ swz<D>(tid / CPR)) < chunks_valid;
 #pragma unroll
 		for (int it = 0; it < NP; ++it)
 			off[it] = COMPACT ? offset_of(it, stride_bytes, tid, ROWS, CPR) : offset_of(it, stride_bytes, tid, rows_valid, chunks_valid);
@@ -324,12 +329,30 @@ struct TileLoader {
 				for (int it = 0; it < NIT; ++it)
 					lds_dma16_so(offset_of(it, stride_bytes, tid, rows_state, cols_state), ub, tile + it * NTHREADS * 16 + wave_slot);
 			}
-		} else {
+		} else if (!COLS || lane_on) {
 #pragma unroll
 			for (int it = 0; it < NIT; ++it) load_one(tile, ub, it, tid);
 		}
 	}
 };
+
+// Zeroes the 16-byte chunks [c0, c1) of every row of a tile (by NTHREADS threads; the barrier that publishes the tile publishes them too).
+template <int D, int ROWS, int NTHREADS>
+FA2_DEV void zero_cols(FA2_LDS char* tile, int tid, int c0, int c1) {
+	for (int row = tid; row < ROWS; row += NTHREADS)
+		for (int ch = c0; ch < c1; ++ch) *(FA2_LDS u32x4*)(tile + tile_off<D>(row, ch)) = u32x4{0u, 0u, 0u, 0u};
+}
+
+// Eight elements of a row from column `col` on; COLS: zeros where the row (hd columns, a multiple of 8) has ended.
+template <typename V8, bool COLS>
+FA2_DEV V8 load_row8(const char* row, int col, int hd) {
+	if constexpr (!COLS) return *(const V8*)(row + col * 2);
+	const bool in = col < hd;
+	u32x4 x = *(const u32x4*)(row + (in ? col * 2 : 0));
+#pragma unroll
+	for (int e = 0; e < 4; ++e) x[e] = in ? x[e] : 0u;
+	return __builtin_bit_cast(V8, x);
+}
 
 FA2_DEV void wait_async_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 

@@ -171,16 +171,22 @@ FA2_DEV f32x4 load_bias4(const char* rowp, int col, int dtype, bool vec_ok, int 
 // CAP: tanh soft-capping of the scores (refrence_call.py:48-51), on the path with bias; the bias itself may be absent.
 // KW: this many groups of NW waves share the rows of a workgroup and take its key tiles in turn, each with tiles of its own in
 // LDS; group 0 merges their (O, maximum, sum) at the end.  For grids that would leave SIMDs with one wave or none.
-template <typename T, int D, int NW, int QB, int WPS, bool BIAS, bool DROP, bool SPLIT = false, bool BLDS = false, bool CAP = false, int KW = 1>
+// DE: columns of the products.  DE < D: rows of a.hd <= DE columns (a multiple of 8) in tiles of D; the columns from a.hd to DE are
+// zeros of the kernel's own, those beyond DE are neither copied nor multiplied.  Rows padded by a copy cost more than the kernels'
+// own work on the padding: B64 S257 H16 D80 fp16, forward and backward, 722 us of which the eight padded copies were 245; 389 us on the
+// rows as they are with three quarters of the products (the kernels alone 480 -> 385).
+template <typename T, int D, int NW, int QB, int WPS, bool BIAS, bool DROP, bool SPLIT = false, bool BLDS = false, bool CAP = false, int KW = 1, int DE = D>
 __global__ __launch_bounds__(NW * 64 * KW, WPS) void fwd_kernel(const KArgs a) {
+	static_assert(DE == D || (!BIAS && !DROP && !SPLIT && !CAP), "");
+	constexpr bool COLS = DE < D;
 	static_assert(KW == 1 || QB == 1, "");
 	static_assert(!CAP || (BIAS && !BLDS && !SPLIT), "soft-capping runs on the plain path with bias");
 	typedef typename T::V8 V8;
 	constexpr int BM = NW * QB * 32;
 	constexpr int BN = kFwdBN;
 	constexpr int KB = BN / 32;   // 32-key blocks per tile
-	constexpr int KS = D / 16;    // MFMA k-steps along D
-	constexpr int DB = D / 32;    // 32-wide blocks of the head dim
+	constexpr int KS = DE / 16;   // MFMA k-steps along D
+	constexpr int DB = DE / 32;   // 32-wide blocks of the head dim
 	constexpr int NT = NW * 64;
 	constexpr int TILE_BYTES = BN * D * 2;
 
@@ -329,15 +335,19 @@ __global__ __launch_bounds__(NW * 64 * KW, WPS) void fwd_kernel(const KArgs a) {
 	const char* kbase = a.k.ptr + (int64_t)b * a.k.sb + (int64_t)hk * a.k.sh;
 	const char* vbase = a.v.ptr + (int64_t)b * a.v.sb + (int64_t)hk * a.v.sh;
 
-	TileLoader<D, BN, NT> kload, vload;
-	kload.init(a.k.ss, tid);
-	vload.init(a.v.ss, tid);
+	TileLoader<D, BN, NT, COLS> kload, vload;
+	const int cols = COLS ? a.hd >> 3 : D / 8;  // 16-byte chunks of a row
+	kload.init(a.k.ss, tid, BN, cols);
+	vload.init(a.v.ss, tid, BN, cols);
+	if constexpr (COLS) {
+		for (int i = 0; i < 2; ++i) zero_cols<D, BN, NT>(lds + i * TILE_BYTES, tid, cols, DE / 8);  // (of V they only reach columns that are not stored)
+	}
 	// prologue: first K/V tile in flight while Q is fetched
 	if (ntiles > t_first) {
 		int nb = t_first * BN, bsel = KW == 1 ? t_first & 1 : 0;
 		int rows = sk_eff - nb < BN ? sk_eff - nb : BN;
-		kload.load(lds + bsel * TILE_BYTES, kbase + (int64_t)nb * a.k.ss, a.k.ss, rows, tid);
-		vload.load(lds + (2 + bsel) * TILE_BYTES, vbase + (int64_t)nb * a.v.ss, a.v.ss, rows, tid);
+		kload.load(lds + bsel * TILE_BYTES, kbase + (int64_t)nb * a.k.ss, a.k.ss, rows, tid, cols);
+		vload.load(lds + (2 + bsel) * TILE_BYTES, vbase + (int64_t)nb * a.v.ss, a.v.ss, rows, tid, cols);
 	}
 
 	// Q fragments (B operand of S^T): lane holds Q[row c][16ks + 8g .. +7]
@@ -347,9 +357,9 @@ __global__ __launch_bounds__(NW * 64 * KW, WPS) void fwd_kernel(const KArgs a) {
 		for (int qb = 0; qb < QB; ++qb) {
 			const char* qbase = a.q.ptr + (int64_t)b * a.q.sb + (int64_t)hl[qb] * a.q.sh;
 			int i = qrow[qb] < a.Sq ? qrow[qb] : a.Sq - 1;
-			const char* rp = qbase + (int64_t)i * a.q.ss + g * 16;
+			const char* rp = qbase + (int64_t)i * a.q.ss;
 #pragma unroll
-			for (int ks = 0; ks < KS; ++ks) qf[qb][ks] = *(const V8*)(rp + ks * 32);
+			for (int ks = 0; ks < KS; ++ks) qf[qb][ks] = load_row8<V8, COLS>(rp, 16 * ks + 8 * g, a.hd);
 		}
 	}
 
@@ -496,8 +506,9 @@ __global__ __launch_bounds__(NW * 64 * KW, WPS) void fwd_kernel(const KArgs a) {
 		// flight during the softmax, each further one during the products of the previous.
 		constexpr int KK = BN / 16;
 		constexpr int NFR = KK * DB;                                  // fragments of a tile: 16-key step fi / DB, d-block fi % DB
-		constexpr int NF = D == 256 ? 4 : (NFR < 8 ? NFR : 8);        // fragments per batch (head dim 256: registers are short)
+		constexpr int NF = D == 256 ? 4 : (NFR % 8 == 0 ? 8 : 6);     // fragments per batch (head dim 256: registers are short)
 		constexpr int NBATCH = NFR / NF;
+		static_assert(NFR % NF == 0, "");
 		u32x4 vfr[2][NF];
 		auto issue_v = [&](auto batch_tag, u32x4(&dst)[NF]) {
 			constexpr int BI = decltype(batch_tag)::value;
@@ -755,7 +766,7 @@ __global__ __launch_bounds__(NW * 64 * KW, WPS) void fwd_kernel(const KArgs a) {
 	auto tile_pipe = [&](int n0) {
 		if constexpr (PIPE) {
 			constexpr int NFR = KS;  // fragments = products of a phase: KS of K for a half, 2 sixteen-key steps x DB of V
-			constexpr int RING = 8, PA = DROP ? 4 : 7;  // (dropout: the generator needs the registers)
+			constexpr int RING = KS % 8 == 0 ? 8 : KS, PA = DROP ? 4 : RING - 1;  // (dropout: the generator needs the registers)
 			static_assert(2 * DB == KS && KS % RING == 0 && PA < RING, "");
 			u32x4 fr[RING];
 			f32x16 sc[2];
@@ -893,6 +904,11 @@ __global__ __launch_bounds__(NW * 64 * KW, WPS) void fwd_kernel(const KArgs a) {
 				constexpr int j = decltype(jt)::value;
 				if constexpr (NFR >= 10) {
 					if constexpr (j >= 2 && j < 10) soft_piece(hf, j - 2);
+				} else if constexpr (NFR == 6) {  // (six slots: two pieces behind each of the products 2 .. 5)
+					if constexpr (j >= 2) {
+						soft_piece(hf, 2 * (j - 2));
+						soft_piece(hf, 2 * (j - 2) + 1);
+					}
 				} else if constexpr (j == 2 || j == 3) {
 					soft_piece(hf, 2 * (j - 2));
 					soft_piece(hf, 2 * (j - 2) + 1);
@@ -938,8 +954,8 @@ __global__ __launch_bounds__(NW * 64 * KW, WPS) void fwd_kernel(const KArgs a) {
 		if (t + KW < ntiles) {
 			int n1 = n0 + KW * BN;
 			int rows = sk_eff - n1 < BN ? sk_eff - n1 : BN;
-			kload.load(lds + (buf ^ 1) * TILE_BYTES, kbase + (int64_t)n1 * a.k.ss, a.k.ss, rows, tid);
-			vload.load(lds + (2 + (buf ^ 1)) * TILE_BYTES, vbase + (int64_t)n1 * a.v.ss, a.v.ss, rows, tid);
+			kload.load(lds + (buf ^ 1) * TILE_BYTES, kbase + (int64_t)n1 * a.k.ss, a.k.ss, rows, tid, cols);
+			vload.load(lds + (2 + (buf ^ 1)) * TILE_BYTES, vbase + (int64_t)n1 * a.v.ss, a.v.ss, rows, tid, cols);
 			if constexpr (BIAS_LDS) {
 				if (bias_lds)
 					bload.load(lds + 4 * TILE_BYTES + (buf ^ 1) * BIAS_BYTES, bias_base + (int64_t)m0 * a.bias_sm + (int64_t)n1 * 2,
@@ -1059,6 +1075,7 @@ __global__ __launch_bounds__(NW * 64 * KW, WPS) void fwd_kernel(const KArgs a) {
 			for (int db = 0; db < DB; ++db)
 #pragma unroll
 				for (int aa = 0; aa < 4; ++aa) {
+					if (COLS && 32 * db + 8 * aa >= a.hd) continue;
 					const f32x16& r = oacc[qb][db];
 					u32x2 pk = {pack2<typename T::V2>(r[4 * aa] * inv, r[4 * aa + 1] * inv),
 					            pack2<typename T::V2>(r[4 * aa + 2] * inv, r[4 * aa + 3] * inv)};
@@ -1226,23 +1243,23 @@ hipError_t launch_fwd_split_t(bool bias, bool drop, KArgs& a, hipStream_t s) {
 }
 
 // One tile configuration: NW waves x 32 rows per workgroup (WPS: launch bound, waves per SIMD), times KW groups that share the keys.
-template <typename T, int D, int NW, int WPS, int KW = 1>
+template <typename T, int D, int DE, int NW, int WPS, int KW = 1>
 hipError_t launch_fwd_cfg(bool bias, bool drop, KArgs& a, hipStream_t s) {
 	constexpr int QB = 1, BM = NW * QB * 32;
 	a.mtiles = (a.Sq + BM - 1) / BM;
 	int groups = a.B * a.Hkv;
 	a.xcd_remap = (groups % 8 == 0) ? 1 : 0;
-	a.interleave = a.xcd_remap ? launch_order(a, a.Hq / a.Hkv, groups / 8, (int64_t)a.Sk * D * 4) : 1;
+	a.interleave = a.xcd_remap ? launch_order(a, a.Hq / a.Hkv, groups / 8, (int64_t)a.Sk * DE * 4) : 1;
 	if (bias && a.bias_sh == 0 && a.B % 8 == 0) a.xcd_remap = a.kv_lens ? 3 : 2;
 	dim3 grid((unsigned)(a.mtiles * a.B * a.Hq)), block(NW * 64 * KW);
 	a.fold_half = KW == 1 ? fold_half_of(a, NW, (int64_t)grid.x, D == 64 || WPS == 2) : 0;
 	const bool blds = bias && a.bias_lds;
 	// (head dim 128 with bias tiles has no LDS for a second group)
-	constexpr bool WITH_BIAS = D == 64 || (KW == 1 && WPS == 1);
-	if (!bias && drop)
-		hipLaunchKernelGGL((fwd_kernel<T, D, NW, QB, WPS, false, true, false, false, false, KW>), grid, block, 0, s, a);
-	else if (!bias)
-		hipLaunchKernelGGL((fwd_kernel<T, D, NW, QB, WPS, false, false, false, false, false, KW>), grid, block, 0, s, a);
+	constexpr bool WITH_BIAS = D == 64 || (DE == D && KW == 1 && WPS == 1);
+	if constexpr (DE == D) {
+		if (!bias && drop) hipLaunchKernelGGL((fwd_kernel<T, D, NW, QB, WPS, false, true, false, false, false, KW>), grid, block, 0, s, a);
+	}
+	if (!bias && !drop) hipLaunchKernelGGL((fwd_kernel<T, D, NW, QB, WPS, false, false, false, false, false, KW, DE>), grid, block, 0, s, a);
 	if constexpr (WITH_BIAS) {
 		if (!bias)
 			;
@@ -1262,13 +1279,16 @@ hipError_t launch_fwd_cfg(bool bias, bool drop, KArgs& a, hipStream_t s) {
 	return hipGetLastError();
 }
 
-template <typename T, int D>
+// DE < D: rows of a.hd <= DE columns in the tiles of head dim D, without bias and dropout, one range of keys (the C ABI checks)
+template <typename T, int D, int DE = D>
 hipError_t launch_fwd_t(bool bias, bool drop, KArgs& a, hipStream_t s) {
-	if (a.decode_waves) return launch_fwd_decode_t<T, D>(a, s);
-	if constexpr (D <= 128) {
-		if (a.nsplit > 1 && a.tall_split) return launch_fwd_tall_split_t<T, D>(a, s);
+	if constexpr (DE == D) {
+		if (a.decode_waves) return launch_fwd_decode_t<T, D>(a, s);
+		if constexpr (D <= 128) {
+			if (a.nsplit > 1 && a.tall_split) return launch_fwd_tall_split_t<T, D>(a, s);
+		}
+		if (a.nsplit > 1) return launch_fwd_split_t<T, D>(bias, drop, a, s);
 	}
-	if (a.nsplit > 1) return launch_fwd_split_t<T, D>(bias, drop, a, s);
 	typedef FwdCfg<T, D> C;
 	if constexpr (C::NW == 8) {
 		// A grid that leaves at least half of the chip idle (small batch x heads, short sequences): workgroups of
@@ -1279,8 +1299,8 @@ hipError_t launch_fwd_t(bool bias, bool drop, KArgs& a, hipStream_t s) {
 			// there was one (B1 Hq32 Hkv8 D128, 1000 rows over 9000 keys: 233 -> 170 us; B1 H8 S4096 D128 81 -> 71 us, causal 79 -> 61;
 			// B2 H16 S1024 D64 with bias 23.4 -> 20.5; B4 H12 S197 D64 9.3 -> 8.9).  With up to three tiles the merge costs more
 			// than it saves (B1 H8 S128: 8.7 us alone, 10.1 in two groups); four groups spill.
-			if (a.Sk > 3 * kFwdBN && (D == 64 || !bias)) return launch_fwd_cfg<T, D, 4, 1, 2>(bias, drop, a, s);
-			return launch_fwd_cfg<T, D, 4, 1>(bias, drop, a, s);
+			if (a.Sk > 3 * kFwdBN && (D == 64 || !bias)) return launch_fwd_cfg<T, D, DE, 4, 1, 2>(bias, drop, a, s);
+			return launch_fwd_cfg<T, D, DE, 4, 1>(bias, drop, a, s);
 		}
 		// Larger grids: two independent 128-row workgroups per CU instead of one of 256 rows - the same eight waves, but
 		// one workgroup computes while the other loads its Q, waits for its first tiles or stores its result, and a
@@ -1298,10 +1318,10 @@ hipError_t launch_fwd_t(bool bias, bool drop, KArgs& a, hipStream_t s) {
 		const int64_t kv_limit = D == 64   ? (4 << 20)
 		                         : a.causal ? ((drop && wgs > 2 * kNumCU) ? (2 << 20) : (4 << 20))
 		                                    : (drop ? 1024 * D * 4 : (2 << 20));
-		if ((int64_t)a.Sk * D * 4 <= kv_limit && (D == 64 || (!bias && !(a.softcap > 0.f))))
-			return launch_fwd_cfg<T, D, 4, (D == 128 ? 2 : 1)>(bias, drop, a, s);
+		if ((int64_t)a.Sk * DE * 4 <= kv_limit && (D == 64 || (!bias && !(a.softcap > 0.f))))
+			return launch_fwd_cfg<T, D, DE, 4, (D == 128 ? 2 : 1)>(bias, drop, a, s);
 	}
-	return launch_fwd_cfg<T, D, C::NW, C::WPS>(bias, drop, a, s);
+	return launch_fwd_cfg<T, D, DE, C::NW, C::WPS>(bias, drop, a, s);
 }
 
 }  // namespace fa2

@@ -29,6 +29,7 @@ struct KArgs {
 	const int32_t* seqlens;
 	const int32_t* kv_lens;  // [B]: keys at or beyond kv_lens[b] are masked (query rows unaffected)
 	int B, Sq, Sk, Hq, Hkv;
+	int hd;          // columns the rows of q, k, v, o and the gradients really have (kernel variants DE < D; else the head dim D)
 	int causal;      // (host side only: the kernels read win_right)
 	int win_left, win_right;  // row i sees keys i + off - win_left .. i + off + win_right; a negative bound is none; causal = win_right 0
 	float scale;
@@ -75,6 +76,11 @@ hipError_t launch_dropout_mask(uint8_t* keep, int B, int H, int Sq, int Sk, uint
 // Per-(dtype, D) translation units provide these.
 #define FA2_DECL_FWD(TAG, DD) hipError_t launch_fwd_##TAG##_##DD(bool bias, bool drop, KArgs& a, hipStream_t s);
 #define FA2_DECL_BWD(TAG, DD) hipError_t launch_bwd_##TAG##_##DD(bool bias, bool drop, KArgs& a, hipStream_t s);
+// (96: rows of 72 to 96 elements in the tiles of head dim 128, no bias, no dropout)
+FA2_DECL_FWD(bf16, 96)
+FA2_DECL_FWD(fp16, 96)
+FA2_DECL_BWD(bf16, 96)
+FA2_DECL_BWD(fp16, 96)
 FA2_DECL_FWD(bf16, 64)
 FA2_DECL_FWD(bf16, 128)
 FA2_DECL_FWD(bf16, 256)

@@ -87,6 +87,7 @@ ffi::Error fill_common(fa2_params& p, ffi::AnyBuffer q, ffi::AnyBuffer k, ffi::A
 	p.Sq = (int32_t)qd[1];
 	p.Hq = (int32_t)qd[2];
 	p.D = (int32_t)qd[3];
+	p.head_dim = p.D;  // (the JAX operator pads its rows)
 	p.Sk = (int32_t)kd[1];
 	p.Hkv = (int32_t)kd[2];
 	p.causal = at.causal ? 1 : 0;

@@ -40,7 +40,7 @@ HANDLERS = {
 
 # which field of fa2_params (include/fa2.h) each operand / attribute fills
 PARAM_FIELDS = {
-	"q": "q", "k": "k", "v": "v", "o": "o", "lse": "lse", "dout": "dout", "dq": "dq", "dk": "dk", "dv": "dv",
+	"q": "q, head_dim", "k": "k", "v": "v", "o": "o", "lse": "lse", "dout": "dout", "dq": "dq", "dk": "dk", "dv": "dv",
 	"bias": "bias, bias_dtype (FA2_MASK_U8 for a boolean / byte buffer), bias_stride_*",
 	"seqlens": "seqlens", "kv_lens": "kv_lens", "seed": "seed_dev", "scratch": "scratch, scratch_bytes",
 	"dbias": "dbias, dbias_stride_*",

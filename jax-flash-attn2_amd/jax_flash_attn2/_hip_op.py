@@ -46,6 +46,7 @@ def _t4(x: torch.Tensor) -> Fa2Tensor:
 # one, as the reference pads to the next power of two (_forward_triton.py:525-526): zero
 # columns of q / k leave the scores unchanged, zero columns of v and dO give zero columns of
 # O, dV and dQ / dK, which are cut off again.  The softmax scale keeps using the true head dim.
+# Where the kernels have a variant for the shorter rows (fa2_params.head_dim) nothing is padded.
 HEAD_DIMS = (64, 128, 256)
 
 
@@ -58,6 +59,14 @@ def _kernel_head_dim(D: int) -> int:
 
 def _pad_d(x: torch.Tensor, Dp: int) -> torch.Tensor:
 	return x if x.shape[-1] == Dp else torch.nn.functional.pad(x, (0, Dp - x.shape[-1]))
+
+
+def _runs_unpadded(lib, which, D, q, k, v, *args) -> bool:
+	"""Whether the library runs this forward (which = 0) / backward (1) on rows that are shorter than its head dim D."""
+	p = _lib.new_params()
+	_fill_common(p, q, k, v, *args)
+	p.D, p.head_dim = D, q.shape[-1]
+	return lib.fa2_validate(ctypes.byref(p), which) != _lib.FA2_EUNSUPPORTED
 
 
 def _usable(x: torch.Tensor) -> torch.Tensor:
@@ -152,14 +161,17 @@ def fwd(q, k, v, bias=None, seqlens=None, softmax_scale=None, dropout_prob=0.0, 
 	lib = _lib.load()
 	D0 = q.shape[-1]
 	D = _kernel_head_dim(D0)
-	q, k, v = _usable(_pad_d(q, D)), _usable(_pad_d(k, D)), _usable(_pad_d(v, D))
 	bias = _prep_bias(bias)
-	B, Sq, Hq, _ = q.shape
 	scale = 1.0 / math.sqrt(D0) if softmax_scale is None else softmax_scale
-	out = torch.empty((B, Sq, Hq, D), dtype=q.dtype, device=q.device)
+	call = (bias, seqlens, scale, dropout_prob, causal, dropout_seed, kv_lens, window, softcap)
+	rows = D0 if D0 != D and _runs_unpadded(lib, 0, D, q, k, v, *call) else D  # columns of the rows the library is given
+	q, k, v = (_usable(_pad_d(x, rows)) for x in (q, k, v))
+	B, Sq, Hq, _ = q.shape
+	out = torch.empty((B, Sq, Hq, rows), dtype=q.dtype, device=q.device)
 	lse = torch.empty((B, Hq, Sq), dtype=torch.float32, device=q.device)
 	p = _lib.new_params()
-	_fill_common(p, q, k, v, bias, seqlens, scale, dropout_prob, causal, dropout_seed, kv_lens, window, softcap)
+	_fill_common(p, q, k, v, *call)
+	p.D, p.head_dim = D, rows
 	p.o = _t4(out)
 	p.lse = lse.data_ptr()
 	# short query over many keys: scratch lets the library split the keys over workgroups
@@ -169,7 +181,7 @@ def fwd(q, k, v, bias=None, seqlens=None, softmax_scale=None, dropout_prob=0.0, 
 		p.scratch = scratch.data_ptr()
 		p.scratch_bytes = need
 	_lib.check(lib.fa2_fwd(ctypes.byref(p), _stream_ptr(q.device)))
-	return (out if D == D0 else out[..., :D0]), lse
+	return (out if rows == D0 else out[..., :D0]), lse
 
 
 def bwd(q, k, v, out, lse, dout, bias=None, seqlens=None, softmax_scale=None, dropout_prob=0.0, causal=False,
@@ -180,15 +192,18 @@ def bwd(q, k, v, out, lse, dout, bias=None, seqlens=None, softmax_scale=None, dr
 	lib = _lib.load()
 	D0 = q.shape[-1]
 	D = _kernel_head_dim(D0)
-	q, k, v, out, dout = (_usable(_pad_d(x, D)) for x in (q, k, v, out, dout))
 	bias = _prep_bias(bias)
-	B, Sq, Hq, _ = q.shape
 	scale = 1.0 / math.sqrt(D0) if softmax_scale is None else softmax_scale
+	call = (bias, seqlens, scale, dropout_prob, causal, dropout_seed, kv_lens, window, softcap)
+	rows = D0 if D0 != D and _runs_unpadded(lib, 1, D, q, k, v, *call) else D
+	q, k, v, out, dout = (_usable(_pad_d(x, rows)) for x in (q, k, v, out, dout))
+	B, Sq, Hq, _ = q.shape
 	dq = torch.empty_like(q, memory_format=torch.contiguous_format)
 	dk = torch.empty_like(k, memory_format=torch.contiguous_format)
 	dv = torch.empty_like(v, memory_format=torch.contiguous_format)
 	p = _lib.new_params()
-	_fill_common(p, q, k, v, bias, seqlens, scale, dropout_prob, causal, dropout_seed, kv_lens, window, softcap)
+	_fill_common(p, q, k, v, *call)
+	p.D, p.head_dim = D, rows
 	p.o = _t4(out)
 	p.lse = lse.data_ptr()
 	p.dout, p.dq, p.dk, p.dv = _t4(dout), _t4(dq), _t4(dk), _t4(dv)
@@ -211,7 +226,7 @@ def bwd(q, k, v, out, lse, dout, bias=None, seqlens=None, softmax_scale=None, dr
 		p.dbias_stride_h = 0 if bias.shape[1] == 1 else dbias.stride(1)
 		p.dbias_stride_m = dbias.stride(2)
 	_lib.check(lib.fa2_bwd(ctypes.byref(p), _stream_ptr(q.device)))
-	if D != D0:
+	if rows != D0:
 		dq, dk, dv = dq[..., :D0], dk[..., :D0], dv[..., :D0]
 	if need_dbias:
 		return dq, dk, dv, dbias

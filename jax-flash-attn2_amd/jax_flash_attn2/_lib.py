@@ -11,6 +11,7 @@ import os
 import threading
 
 FA2_FP16, FA2_BF16, FA2_FP32, FA2_MASK_U8 = 1, 2, 3, 4
+FA2_EUNSUPPORTED = -10
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(os.path.dirname(_HERE), "libfa2_hip.so")
@@ -67,6 +68,7 @@ class Fa2Params(ctypes.Structure):
 		("dbias_stride_b", ctypes.c_int64),
 		("dbias_stride_h", ctypes.c_int64),
 		("dbias_stride_m", ctypes.c_int64),
+		("head_dim", ctypes.c_int32),
 	]
 
 

@@ -1,0 +1,58 @@
+"""Head dims that run in the tiles of head dim 128 without padded copies of the operands: shortest and longest rows, query and key
+counts around the tiles, strided operands, and what surrounds the rows in memory (never read into a result, never written)."""
+
+import pytest
+import torch
+
+from jax_flash_attn2 import _hip_op as op
+import fa2_oracle as O
+from _cases import check_forward, check_grads, f64, make_inputs
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize(
+	"B,Sq,Sk,Hq,Hkv,D,dtype,causal,kv_lens,window",
+	[
+		(2, 257, 257, 2, 2, 80, torch.float16, False, None, None),   # one row and one key beyond the tiles
+		(1, 33, 31, 2, 1, 72, torch.bfloat16, False, None, None),    # a single ragged tile
+		(1, 128, 128, 4, 2, 96, torch.bfloat16, True, None, None),   # whole tiles
+		(2, 300, 430, 4, 1, 88, torch.float16, True, [430, 70], None),
+		(1, 700, 700, 2, 2, 72, torch.bfloat16, True, None, (100, 0)),
+		(3, 1030, 1030, 32, 8, 80, torch.bfloat16, True, None, None),   # grids of more than one workgroup per CU
+		(8, 520, 5600, 16, 16, 96, torch.float16, False, None, None),   # keys of a head beyond what the smaller workgroups are for
+		(1, 2050, 2050, 64, 64, 88, torch.bfloat16, True, None, None),  # key tiles in pairs
+	],
+)
+def test_short_rows_against_the_oracle(B, Sq, Sk, Hq, Hkv, D, dtype, causal, kv_lens, window):
+	q, k, v, do, _ = make_inputs(B, Sq, Sk, Hq, Hkv, D, dtype, seed=D + Sq)
+	kl = None if kv_lens is None else torch.tensor(kv_lens, dtype=torch.int32, device="cuda:0")
+
+	def inside(x):
+		# a slice of wider rows whose other columns are NaN: the kernels must not look at them
+		wide = torch.full((*x.shape[:3], D + 16), float("nan"), dtype=dtype, device="cuda:0")
+		wide[..., 8 : D + 8] = x.cuda()
+		return wide[..., 8 : D + 8]
+
+	q_, k_, v_, do_ = (inside(x) for x in (q, k, v, do))
+	args = (None, None, None, 0.0, causal, None, kl, window)
+	o, lse = op.fwd(q_, k_, v_, *args)
+	grads = op.bwd(q_, k_, v_, o, lse, do_, *args)
+	# (the last KV group of the last batch row is enough for the oracle)
+	bs, hs, kv = slice(B - 1, B), slice(Hq - Hq // Hkv, Hq), slice(Hkv - 1, Hkv)
+	ref = dict(causal=causal, kv_lens=None if kv_lens is None else kv_lens[bs], window=window)
+	a = [f64(x) for x in (q[bs, :, hs], k[bs, :, kv], v[bs, :, kv], do[bs, :, hs])]
+	name = f"B{B} Sq{Sq} Sk{Sk} Hq{Hq} Hkv{Hkv} D{D} {ref}"
+	check_forward(o[bs, :, hs], lse[bs, hs], *O.attention_fwd(*a[:3], **ref), dtype, name)
+	check_grads([x[bs, :, y] for x, y in zip(grads, (hs, kv, kv))], O.attention_bwd(*a, **ref), name)
+
+
+def test_infinite_last_column():
+	"""A key whose last column is -inf scores -inf for a positive query (probability 0); the columns that are not there add nothing to it."""
+	q, k, v, _, _ = make_inputs(1, 64, 100, 1, 1, 72, torch.bfloat16, seed=3)
+	q[..., -1] = q[..., -1].abs() + 0.1
+	k[:, 5, :, -1] = float("-inf")
+	o, lse = op.fwd(q.cuda(), k.cuda(), v.cuda())
+	keep = [j for j in range(100) if j != 5]
+	o_ref, lse_ref = O.attention_fwd(f64(q), f64(k[:, keep]), f64(v[:, keep]))
+	check_forward(o, lse, o_ref, lse_ref, torch.bfloat16, "key of -inf")
