@@ -23,7 +23,7 @@ import torch
 
 from . import _lib
 from ._checks import check_shapes  # noqa: F401  (re-exported)
-from ._lib import FA2_BF16, FA2_FP16, FA2_FP32, FA2_MASK_U8, Fa2Tensor
+from ._lib import FA2_BF16, FA2_FP16, FA2_FP32, FA2_MASK_U8
 
 _DTYPES = {torch.float16: FA2_FP16, torch.bfloat16: FA2_BF16}
 # (a uint8 / bool `bias` is a boolean mask, one byte per position: see fa2_params.bias_dtype)
@@ -31,15 +31,16 @@ _BIAS_DTYPES = {torch.float16: FA2_FP16, torch.bfloat16: FA2_BF16, torch.float32
 
 
 def _stream_ptr(device) -> int:
-	return torch.cuda.current_stream(device).cuda_stream
+	# (what torch.cuda.current_stream(device).cuda_stream gives, without building the stream object)
+	return torch._C._cuda_getCurrentRawStream(device.index)
 
 
-def _t4(x: torch.Tensor) -> Fa2Tensor:
-	"""[B, S, H, D] tensor -> pointer + element strides (D stride must be 1)."""
-	t = Fa2Tensor()
-	t.ptr = x.data_ptr()
-	t.stride_b, t.stride_s, t.stride_h = x.stride(0), x.stride(1), x.stride(2)
-	return t
+_NONE4 = (0, 0, 0, 0)  # an absent tensor
+
+
+def _t4(x) -> tuple:
+	"""[B, S, H, D] tensor -> pointer + element strides (D stride must be 1): the fields of an fa2_tensor."""
+	return (x.data_ptr(), *x.stride()[:3])
 
 
 # Head dims the kernels are built for.  Any other head dim up to 256 is zero-padded to the next
@@ -61,65 +62,60 @@ def _pad_d(x: torch.Tensor, Dp: int) -> torch.Tensor:
 	return x if x.shape[-1] == Dp else torch.nn.functional.pad(x, (0, Dp - x.shape[-1]))
 
 
-def _runs_unpadded(lib, which, D, q, k, v, *args) -> bool:
+def _runs_unpadded(lib, which, D, q, k, v, *call) -> bool:
 	"""Whether the library runs this forward (which = 0) / backward (1) on rows that are shorter than its head dim D."""
-	p = _lib.new_params()
-	_fill_common(p, q, k, v, *args)
-	p.D, p.head_dim = D, q.shape[-1]
-	return lib.fa2_validate(ctypes.byref(p), which) != _lib.FA2_EUNSUPPORTED
+	return lib.fa2_validate(ctypes.byref(_block(D, q, k, v, *call)), which) != _lib.FA2_EUNSUPPORTED
 
 
 def _usable(x: torch.Tensor) -> torch.Tensor:
 	"""Kernels read 16 bytes at a time along D: unit D stride, 16-byte aligned rows."""
-	if x.stride(3) != 1 or any(s % 8 for s in x.stride()[:3]) or x.data_ptr() % 16:
+	sb, ss, sh, sd = x.stride()
+	if sd != 1 or (sb | ss | sh) & 7 or x.data_ptr() & 15:
 		return x.contiguous()
 	return x
 
 
-def _fill_common(p, q, k, v, bias, seqlens, scale, p_drop, causal, seed, kv_lens=None, window=None, softcap=0.0):
-	B, Sq, Hq, D = q.shape
-	Sk, Hkv = k.shape[1], k.shape[2]
-	p.dtype = _DTYPES[q.dtype]
-	p.B, p.Sq, p.Sk, p.Hq, p.Hkv, p.D = B, Sq, Sk, Hq, Hkv, D
-	p.causal = 1 if causal else 0
-	p.scale = float(scale)
-	p.p_drop = float(p_drop)
-	_fill_seed(p, seed, q.device)
-	p.q, p.k, p.v = _t4(q), _t4(k), _t4(v)
+def _block(D, q, k, v, bias, seqlens, scale, p_drop, causal, seed, kv_lens=None, window=None, softcap=0.0, o=_NONE4, lse=None,
+           backward=(_NONE4, _NONE4, _NONE4, _NONE4)):
+	"""The parameter block of a call on rows of q.shape[3] columns in the kernels of head dim D.  `o` and `backward` (dO, dq, dk, dv)
+	as _t4() gives them; scratch and the bias gradient are the caller's to add."""
+	B, Sq, Hq, rows = q.shape
+	_, Sk, Hkv, _ = k.shape
+	seed, seed_dev = _seed_fields(seed, q.device)
+	b = (0, 0, 0, 0, 0, 0)
 	if bias is not None:
-		p.bias = bias.data_ptr()
-		p.bias_dtype = _BIAS_DTYPES[bias.dtype]
+		b_b, b_h = bias.shape[:2]
 		# broadcast rules of calc_bias_strides (_utils.py:169-190): size-1 axes get stride 0.
-		p.bias_stride_b = 0 if bias.shape[0] == 1 else bias.stride(0)
-		p.bias_stride_h = 0 if bias.shape[1] == 1 else bias.stride(1)
-		p.bias_stride_m = bias.stride(2)
 		# a bias with Hkv heads is read per KV group instead of being repeated to Hq heads
 		# (the facade materialises that repeat, flash_attention.py:161-164)
-		p.bias_group = 1 if (bias.shape[1] == Hkv and Hkv != Hq and bias.shape[1] != 1) else 0
-	if seqlens is not None:
-		p.seqlens = seqlens.data_ptr()
-	if window is not None:
-		left, right = window
-		p.has_window, p.window_left, p.window_right = 1, int(left), int(right)
-	p.softcap = float(softcap or 0.0)
-	if kv_lens is not None:
-		if kv_lens.dtype != torch.int32 or kv_lens.numel() != B or not kv_lens.is_contiguous():
-			raise ValueError("kv_lens must be a contiguous int32 tensor with one entry per batch row")
-		p.kv_lens = kv_lens.data_ptr()
+		b = (bias.data_ptr(), _BIAS_DTYPES[bias.dtype], 1 if (b_h == Hkv and Hkv != Hq and b_h != 1) else 0,
+		     0 if b_b == 1 else bias.stride(0), 0 if b_h == 1 else bias.stride(1), bias.stride(2))
+	if kv_lens is not None and (kv_lens.dtype != torch.int32 or kv_lens.numel() != B or not kv_lens.is_contiguous()):
+		raise ValueError("kv_lens must be a contiguous int32 tensor with one entry per batch row")
+	# (a bound beyond 2^30 is none at all; kept within the 32 bits of the field)
+	left, right = (0, 0) if window is None else (max(-1, min(int(w), 1 << 30)) for w in window)
+	dout, dq, dk, dv = backward
+	# (in the order of include/fa2.h)
+	return _lib.Fa2Params.from_buffer_copy(_lib.PACKED.pack(
+		_lib.PACKED.size, _DTYPES[q.dtype], B, Sq, Sk, Hq, Hkv, D, 1 if causal else 0, float(scale), float(p_drop), seed,
+		*_t4(q), *_t4(k), *_t4(v), *o, 0 if lse is None else lse.data_ptr(),
+		*b, 0 if seqlens is None else seqlens.data_ptr(),
+		*dout, *dq, *dk, *dv, 0, 0,  # (scratch)
+		seed_dev, 0 if kv_lens is None else kv_lens.data_ptr(),
+		0 if window is None else 1, left, right, float(softcap or 0.0),
+		0, 0, 0, 0,  # (dbias)
+		rows))
 
 
-def _fill_seed(p, seed, device):
+def _seed_fields(seed, device):
 	"""The dropout seed is a Python int (copied into the parameter block) or a one-element int64 tensor on the device,
 	which the kernels read there: a seed that is itself the result of device work - as a traced `dropout_seed` is in
 	the reference, an operand of the custom call (_forward_triton.py:553) - needs no host round trip."""
 	if isinstance(seed, torch.Tensor):
 		if seed.dtype != torch.int64 or seed.numel() != 1 or seed.device != device:
 			raise ValueError("a tensor dropout_seed must be a one-element int64 tensor on the device of q")
-		p.seed = 0
-		p.seed_dev = seed.data_ptr()
-	else:
-		p.seed = int(seed or 0) & 0xFFFFFFFFFFFFFFFF
-		p.seed_dev = None
+		return 0, seed.data_ptr()
+	return int(seed or 0) & 0xFFFFFFFFFFFFFFFF, 0
 
 
 def _prep_bias(bias):
@@ -165,22 +161,18 @@ def fwd(q, k, v, bias=None, seqlens=None, softmax_scale=None, dropout_prob=0.0, 
 	scale = 1.0 / math.sqrt(D0) if softmax_scale is None else softmax_scale
 	call = (bias, seqlens, scale, dropout_prob, causal, dropout_seed, kv_lens, window, softcap)
 	rows = D0 if D0 != D and _runs_unpadded(lib, 0, D, q, k, v, *call) else D  # columns of the rows the library is given
-	q, k, v = (_usable(_pad_d(x, rows)) for x in (q, k, v))
-	B, Sq, Hq, _ = q.shape
-	out = torch.empty((B, Sq, Hq, rows), dtype=q.dtype, device=q.device)
-	lse = torch.empty((B, Hq, Sq), dtype=torch.float32, device=q.device)
-	p = _lib.new_params()
-	_fill_common(p, q, k, v, *call)
-	p.D, p.head_dim = D, rows
-	p.o = _t4(out)
-	p.lse = lse.data_ptr()
+	q, k, v = _usable(_pad_d(q, rows)), _usable(_pad_d(k, rows)), _usable(_pad_d(v, rows))
+	out = torch.empty_like(q, memory_format=torch.contiguous_format)
+	lse = torch.empty((q.shape[0], q.shape[2], q.shape[1]), dtype=torch.float32, device=q.device)
+	p = _block(D, q, k, v, *call, _t4(out), lse)
+	ref = ctypes.byref(p)
 	# short query over many keys: scratch lets the library split the keys over workgroups
-	need = lib.fa2_fwd_scratch_bytes(ctypes.byref(p))
+	need = lib.fa2_fwd_scratch_bytes(ref)
 	if need:
 		scratch = torch.empty((need,), dtype=torch.uint8, device=q.device)
 		p.scratch = scratch.data_ptr()
 		p.scratch_bytes = need
-	_lib.check(lib.fa2_fwd(ctypes.byref(p), _stream_ptr(q.device)))
+	_lib.check(lib.fa2_fwd(ref, _stream_ptr(q.device)))
 	return (out if rows == D0 else out[..., :D0]), lse
 
 
@@ -197,16 +189,11 @@ def bwd(q, k, v, out, lse, dout, bias=None, seqlens=None, softmax_scale=None, dr
 	call = (bias, seqlens, scale, dropout_prob, causal, dropout_seed, kv_lens, window, softcap)
 	rows = D0 if D0 != D and _runs_unpadded(lib, 1, D, q, k, v, *call) else D
 	q, k, v, out, dout = (_usable(_pad_d(x, rows)) for x in (q, k, v, out, dout))
-	B, Sq, Hq, _ = q.shape
+	Sq = q.shape[1]
 	dq = torch.empty_like(q, memory_format=torch.contiguous_format)
 	dk = torch.empty_like(k, memory_format=torch.contiguous_format)
 	dv = torch.empty_like(v, memory_format=torch.contiguous_format)
-	p = _lib.new_params()
-	_fill_common(p, q, k, v, *call)
-	p.D, p.head_dim = D, rows
-	p.o = _t4(out)
-	p.lse = lse.data_ptr()
-	p.dout, p.dq, p.dk, p.dv = _t4(dout), _t4(dq), _t4(dk), _t4(dv)
+	p = _block(D, q, k, v, *call, _t4(out), lse, (_t4(dout), _t4(dq), _t4(dk), _t4(dv)))
 	# (the larger size, where it applies, lets the dK/dV kernel of a small grid split the q-heads of a group over workgroups)
 	need = max(lib.fa2_bwd_scratch_bytes(ctypes.byref(p)), lib.fa2_bwd_split_scratch_bytes(ctypes.byref(p)))
 	scratch = torch.empty((max(need, 256),), dtype=torch.uint8, device=q.device)
@@ -240,8 +227,8 @@ def dropout_mask(B, H, Sq, Sk, dropout_prob, dropout_seed, device) -> torch.Tens
 	p = _lib.new_params()
 	p.B, p.Hq, p.Hkv, p.Sq, p.Sk, p.D = B, H, H, Sq, Sk, 64
 	p.p_drop = float(dropout_prob)
-	_fill_seed(p, dropout_seed, torch.device(device))
-	_lib.check(lib.fa2_dropout_mask(ctypes.byref(p), keep.data_ptr(), _stream_ptr(device)))
+	p.seed, p.seed_dev = _seed_fields(dropout_seed, torch.device(device))
+	_lib.check(lib.fa2_dropout_mask(ctypes.byref(p), keep.data_ptr(), _stream_ptr(keep.device)))
 	return keep
 
 
@@ -260,19 +247,19 @@ class Plan:
 		scale = 1.0 / math.sqrt(D) if softmax_scale is None else softmax_scale
 		self.out = torch.empty((B, Sq, Hq, D), dtype=q.dtype, device=q.device)
 		self.lse = torch.empty((B, Hq, Sq), dtype=torch.float32, device=q.device)
-		p = self.params = _lib.new_params()
 		self.kv_lens = kv_lens
-		_fill_common(p, self.q, self.k, self.v, self.bias, seqlens, scale, dropout_prob, causal, dropout_seed, kv_lens, window, softcap)
 		self.seed = dropout_seed  # (a device-resident seed must outlive the plan's calls)
-		p.o = _t4(self.out)
-		p.lse = self.lse.data_ptr()
 		self.device = q.device
+		backward = (_NONE4, _NONE4, _NONE4, _NONE4)
 		if dout is not None:
 			self.dout = _usable(dout)
 			self.dq = torch.empty_like(self.q, memory_format=torch.contiguous_format)
 			self.dk = torch.empty_like(self.k, memory_format=torch.contiguous_format)
 			self.dv = torch.empty_like(self.v, memory_format=torch.contiguous_format)
-			p.dout, p.dq, p.dk, p.dv = _t4(self.dout), _t4(self.dq), _t4(self.dk), _t4(self.dv)
+			backward = (_t4(self.dout), _t4(self.dq), _t4(self.dk), _t4(self.dv))
+		p = self.params = _block(D, self.q, self.k, self.v, self.bias, seqlens, scale, dropout_prob, causal, dropout_seed, kv_lens, window, softcap,
+		                         _t4(self.out), self.lse, backward)
+		if dout is not None:
 			need = max(self.lib.fa2_bwd_scratch_bytes(ctypes.byref(p)), self.lib.fa2_bwd_split_scratch_bytes(ctypes.byref(p)))
 		else:
 			need = 0
