@@ -70,6 +70,7 @@ __global__ __launch_bounds__(256) void bwd_delta_kernel(const KArgs a) {
 // With 1 and 2 every workgroup of a KV group that walks in the same direction is at the same query tile at the same
 // time, whatever its key tile - the tiles of Q / dO they stream are then fetched from memory once per XCD.
 // What depends on the batch row only: valid rows / keys and the causal alignment, the dropout key.
+constexpr int kPlain = 0, kMasked = 1, kBlocks = 2;  // how a streamed tile is gone through (run_step of bwd_dkdv_tile)
 struct DkdvRow {
 	int sq_eff, sk_eff, off;
 	uint32_t drop_k0, drop_k1;
@@ -104,14 +105,11 @@ FA2_DEV DkdvRow dkdv_row(const KArgs& a, int b) {
 	return rw;
 }
 
-// K, V rows of this lane's key of key tile nt as B operands: the lane holds X[key][16 ks + 8 g .. + 7].
-template <typename T, int DE, int NW, bool COLS>
-FA2_DEV void dkdv_load_kv(const KArgs& a, int nt, int hk, int b, typename T::V8 (&kf)[DE / 16], typename T::V8 (&vf)[DE / 16]) {
+// K, V rows of key jcol (this lane's) as B operands: the lane holds X[key][16 ks + 8 g .. + 7].
+template <typename T, int DE, bool COLS>
+FA2_DEV void dkdv_load_kv(const KArgs& a, int jcol, int hk, int b, typename T::V8 (&kf)[DE / 16], typename T::V8 (&vf)[DE / 16]) {
 	typedef typename T::V8 V8;
-	const int tid = threadIdx.x, lane = tid & 63;
-	const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
-	const int g = lane >> 5, c = lane & 31;
-	const int jcol = nt * (NW * 32) + 32 * w + c;
+	const int g = (threadIdx.x & 63) >> 5;
 	int j = jcol < a.Sk ? jcol : a.Sk - 1;
 	const char* kp = a.k.ptr + (int64_t)b * a.k.sb + (int64_t)hk * a.k.sh + (int64_t)j * a.k.ss;
 	const char* vp = a.v.ptr + (int64_t)b * a.v.sb + (int64_t)hk * a.v.sh + (int64_t)j * a.v.ss;
@@ -185,12 +183,21 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 	const int r = a.Hq / a.Hkv;
 	const int sq_eff = rw.sq_eff, sk_eff = rw.sk_eff, off = rw.off;
 	const int n0 = nt * BN;
-	const int wn0 = n0 + 32 * w;
+	// A key tile that ends within its first or second 32 keys would leave three or two waves without work for as long as a full tile
+	// takes: there all four waves take the same one or two blocks of keys, each a quarter or a half of every streamed tile's rows, and
+	// their dK / dV are summed at the end.  (B64 S257 H16 D80 - three key tiles of which the last has one key, three row tiles of which the
+	// last has one row: forward and backward 389 -> 371 us; B32 H12 D64 of 256 to 511 tokens 193 -> 190.)
+	constexpr bool SHARES = KV_AGPR && !WALKS && NW == 4 && QB == 4;
+	const int blocks = (sk_eff - n0 + 31) >> 5;  // 32-key blocks with a valid key
+	const int share = SHARES && blocks == 1 ? 4 : (SHARES && blocks == 2 ? 2 : 1);
+	const int kblk = w & (4 / share - 1), rgrp = w / (4 / share);  // this wave's block of keys, its share of the rows
+	const int row0 = rgrp * (BMQ / share);                         // first row of that in a streamed tile
+	const int wn0 = n0 + 32 * kblk;
 	const int jcol = wn0 + c;  // this lane's key
 
 	// K, V rows of this lane's key as B operands: lane holds X[jcol][16ks + 8g .. +7]
 	V8 kf[KS], vf[KS];
-	dkdv_load_kv<T, DE, NW, COLS>(a, nt, hk, b, kf, vf);
+	dkdv_load_kv<T, DE, COLS>(a, jcol, hk, b, kf, vf);
 	// The fragments must have arrived before the loop over streamed tiles starts.  Otherwise the compiler places its
 	// waits for these loads (s_waitcnt vmcnt) at their first uses inside the loop - it does not see the wait that
 	// publishes a tile - where the same counter also counts the tile copies in flight: every step would then wait
@@ -325,11 +332,11 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 	constexpr int KR = KS < 8 ? KS : 8, DR = DB < 4 ? DB : 4;
 	int poff[KR];
 #pragma unroll
-	for (int ks = 0; ks < KR; ++ks) poff[ks] = tile_off<D>(c, 2 * ks + g);
+	for (int ks = 0; ks < KR; ++ks) poff[ks] = tile_off<D>(row0 + c, 2 * ks + g);
 	int toff[DR][2];
 	{
 		int i16 = lane & 15;
-		int trow = 4 * g + (i16 >> 2);
+		int trow = row0 + 4 * g + (i16 >> 2);
 		int tcol = 16 * ((lane >> 4) & 1) + 4 * (i16 & 3);
 #pragma unroll
 		for (int db = 0; db < DR; ++db) {
@@ -339,7 +346,7 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 		}
 	}
 
-	int soff = 16 * g;  // statistics: this half-wave's four rows of a quad (+ the buffer, flipped per step)
+	int soff = 16 * g + 4 * row0;  // statistics: this half-wave's four rows of a quad (+ the buffer, flipped per step)
 
 	// bias tile (rows of 128 keys): this lane's 8-byte piece of rows 4 g + i16 / 4 (+ 8) at its wave's 32 keys
 	int boffq[2] = {0, 0};
@@ -351,10 +358,11 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 		boffq[1] = tile_off<128>(trow + 8, col >> 3) + ((col & 4) << 1);
 	}
 
-	// One streamed tile of BMQ query rows of q-head hq.  MASKED = some (row, key)
-	// of this wave's 32 keys x BMQ rows is masked.
-	auto tile_body = [&](auto masked_tag, int hq, int m0) __attribute__((always_inline)) {
+	// NB blocks of 32 rows of a streamed tile of q-head hq, from the wave's first row (m0 of the sequence) on.  MASKED = some (row, key)
+	// of this wave's 32 keys x 32 NB rows is masked.
+	auto tile_body = [&](auto masked_tag, auto nb_tag, int hq, int m0) __attribute__((always_inline)) {
 		constexpr bool MASKED = decltype(masked_tag)::value;
+		constexpr int NB = decltype(nb_tag)::value;
 		const char* bias_base = nullptr;
 		if constexpr (BIAS) {
 			int hb = a.bias_group ? hk : hq;
@@ -362,7 +370,7 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 			int es = a.bias_dtype == 3 ? 4 : a.bias_dtype == 4 ? 1 : 2;
 			bias_base = a.bias + (int64_t)b * a.bias_sb + (int64_t)hb * a.bias_sh + (int64_t)jc * es;
 		}
-		// The tile's QB blocks of 32 rows go through three stages,
+		// The NB blocks of 32 rows go through three stages,
 		//   A(i): S_i = Q_i K^T, dP_i = dO_i V^T          (2 KS matrix products)
 		//   B(i): P_i, dS_i from S_i, dP_i, lse, delta      (elementwise, 16 values per lane)
 		//   C(i): dV^T += dO_i^T P_i, dK^T += Q_i^T dS_i   (4 DB matrix products)
@@ -653,8 +661,8 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 
 		auto stage = [&](auto k_tag) __attribute__((always_inline)) {
 			constexpr int k = decltype(k_tag)::value;
-			constexpr bool HAS_A = k < QB, HAS_B = k >= 1 && k - 1 < QB, HAS_C = k >= 2 && k - 2 < QB;
-			constexpr bool NEXT_A = k + 1 < QB, NEXT_B = k + 1 >= 1 && k < QB, NEXT_C = k + 1 >= 2 && k - 1 < QB;
+			constexpr bool HAS_A = k < NB, HAS_B = k >= 1 && k - 1 < NB, HAS_C = k >= 2 && k - 2 < NB;
+			constexpr bool NEXT_A = k + 1 < NB, NEXT_B = k + 1 >= 1 && k < NB, NEXT_C = k + 1 >= 2 && k - 1 < NB;
 			// One row block per step (head dim 256): nothing else is in flight, so the products of C start half a stage
 			// early - those of the block's first 16 rows (its slots 0 .. H - 1) run beside the elementwise math of its last
 			// 16 rows in the second half of stage 1, the rest in a stage 2 of half the length.
@@ -664,7 +672,7 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 			__builtin_amdgcn_sched_barrier(0);
 			// (a stage that starts with the elementwise math of a block whose last products - inline assembly - were the
 			// previous stage's last instructions: their results need their wait states)
-			if constexpr (S_VGPR && HAS_B && !HAS_A) asm volatile("s_nop 15" ::: "memory");
+			if constexpr ((S_VGPR || (KV_AGPR && NB == 1)) && HAS_B && !HAS_A) asm volatile("s_nop 15" ::: "memory");
 #pragma unroll
 			for (int j = 0; j < NS; ++j) {
 				// this slot's product of C, if any: block and slot index within that block's C
@@ -772,10 +780,10 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 		stage(std::integral_constant<int, 0>{});
 		stage(std::integral_constant<int, 1>{});
 		stage(std::integral_constant<int, 2>{});
-		if constexpr (QB + 1 >= 3) stage(std::integral_constant<int, 3>{});
-		if constexpr (QB + 1 >= 4) stage(std::integral_constant<int, 4>{});
-		if constexpr (QB + 1 >= 5) stage(std::integral_constant<int, 5>{});
-		static_assert(QB <= 4, "");
+		if constexpr (NB + 1 >= 3) stage(std::integral_constant<int, 3>{});
+		if constexpr (NB + 1 >= 4) stage(std::integral_constant<int, 4>{});
+		if constexpr (NB + 1 >= 5) stage(std::integral_constant<int, 5>{});
+		static_assert(NB <= 4, "");
 	};
 
 	// (q-head, first row) of the streamed tile the next step computes on: decoded once, when its copies are started
@@ -787,7 +795,9 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 	}
 
 	// One pipeline step: publish streamed tile `step`, start the copies of the next, compute.
-	auto run_step = [&](auto masked_tag, int step) {
+	// mode: kPlain no mask; kMasked; kBlocks masked, block by block and only those of the wave's share that have a valid row
+	auto run_step = [&](auto mode_tag, int step) {
+		constexpr int MODE = decltype(mode_tag)::value;
 		const int buf = (step - s_lo) & 1;
 		wait_async_loads();
 		__syncthreads();
@@ -803,14 +813,35 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 			issue_tile(step + 1, tb, nxt_m0, lds + (buf ^ 1) * (2 * TILE_BYTES), lds + (buf ^ 1) * (2 * TILE_BYTES) + TILE_BYTES);
 		}
 		{
-			const int hq = cur_hq, m0 = cur_m0;
+			const int hq = cur_hq, m0 = cur_m0 + row0;
+			// wave-uniform: nothing to do for (rows m0.., keys wn0..)?
+			const int rows = BMQ / share, last_row = m0 + rows - 1 < sq_eff - 1 ? m0 + rows - 1 : sq_eff - 1;
 			bool skip = false;
-			if constexpr (decltype(masked_tag)::value) {
-				// wave-uniform: nothing to do for (rows m0.., keys wn0..)?
-				int last_row = m0 + BMQ - 1 < sq_eff - 1 ? m0 + BMQ - 1 : sq_eff - 1;
-				skip = wn0 >= sk_eff || (wr >= 0 && wn0 > last_row + off + wr) || (wl >= 0 && wn0 + 31 < m0 + off - wl);
+			if constexpr (MODE != kPlain)
+				skip = wn0 >= sk_eff || m0 > last_row || (wr >= 0 && wn0 > last_row + off + wr) || (wl >= 0 && wn0 + 31 < m0 + off - wl);
+			if constexpr (MODE == kBlocks) {
+				if (!skip) {
+					const int nb = (last_row - m0 + 32) >> 5;
+					// (the offsets move along with the blocks and back)
+					auto move = [&](int by) __attribute__((always_inline)) {
+#pragma unroll
+						for (int ks = 0; ks < KR; ++ks) poff[ks] += by * (32 * D * 2);
+#pragma unroll
+						for (int db = 0; db < DR; ++db) {
+							toff[db][0] += by * (32 * D * 2);
+							toff[db][1] += by * (32 * D * 2);
+						}
+						soff += by * 128;
+					};
+					for (int i = 0; i < nb; ++i) {
+						tile_body(std::true_type{}, std::integral_constant<int, 1>{}, hq, m0 + 32 * i);
+						move(1);
+					}
+					move(-nb);
+				}
+			} else {
+				if (!skip) tile_body(std::integral_constant<bool, MODE == kMasked>{}, std::integral_constant<int, QB>{}, hq, m0);
 			}
-			if (!skip) tile_body(masked_tag, hq, m0);
 		}
 		// the other buffers next time
 #pragma unroll
@@ -855,45 +886,92 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 	if (wn0 + 32 > sk_eff) i_diag = nq;  // ragged key block: always masked
 	i_diag = i_diag < 0 ? 0 : (i_diag > nq ? nq : i_diag);
 	i_full = i_full < i_diag ? i_diag : (i_full > nq ? nq : i_full);
+	// Block by block: everything where waves share a block of keys, and a last tile of at most 64 valid rows.
+	int i_tail = nq;
+	if constexpr (SHARES) {
+		const int left = sq_eff - (q_lo + nq - 1) * BMQ;
+		i_tail = share > 1 ? 0 : (left <= BMQ / 2 && nq > 0 ? nq - 1 : nq);
+		i_diag = i_diag < i_tail ? i_diag : i_tail;
+		i_full = i_full < i_tail ? i_full : i_tail;
+	}
+	constexpr std::integral_constant<int, kPlain> plain;
+	constexpr std::integral_constant<int, kMasked> masked;
 	if (order == 0) {
 		for (int hi = 0; hi < r && nq > 0; ++hi) {
-			// (each of the three runs clipped to this workgroup's share of the steps)
+			// (each of the runs clipped to this workgroup's share of the steps)
 			int base = hi * nq;
 			auto clip = [&](int i) { int st = base + i; return st < s_lo ? s_lo : (st > s_hi ? s_hi : st); };
-			for (int st = clip(0); st < clip(i_diag); ++st) run_step(std::true_type{}, st);
-			for (int st = clip(i_diag); st < clip(i_full); ++st) run_step(std::false_type{}, st);
-			for (int st = clip(i_full); st < clip(nq); ++st) run_step(std::true_type{}, st);
+			for (int st = clip(0); st < clip(i_diag); ++st) run_step(masked, st);
+			for (int st = clip(i_diag); st < clip(i_full); ++st) run_step(plain, st);
+			for (int st = clip(i_full); st < clip(i_tail); ++st) run_step(masked, st);
+			if constexpr (SHARES) {
+				for (int st = clip(i_tail); st < clip(nq); ++st) run_step(std::integral_constant<int, kBlocks>{}, st);
+			}
 		}
 	} else {
 		// query tiles outermost: the same three runs, r steps per query tile, in the direction of the walk
 		const int pa = (order == 2 ? nq - i_full : i_diag) * r, pb = (order == 2 ? nq - i_diag : i_full) * r;
 		auto clip = [&](int st) { return st < s_lo ? s_lo : (st > s_hi ? s_hi : st); };
-		for (int st = clip(0); st < clip(pa); ++st) run_step(std::true_type{}, st);
-		for (int st = clip(pa); st < clip(pb); ++st) run_step(std::false_type{}, st);
-		for (int st = clip(pb); st < clip(steps); ++st) run_step(std::true_type{}, st);
+		for (int st = clip(0); st < clip(pa); ++st) run_step(masked, st);
+		for (int st = clip(pa); st < clip(pb); ++st) run_step(plain, st);
+		for (int st = clip(pb); st < clip(steps); ++st) run_step(masked, st);
 	}
 
 	// the last matrix products (issued as inline assembly) must have written dk / dv
 	asm volatile("s_nop 15\n\ts_nop 15\n\ts_nop 15" ::: "memory");
-	// epilogue: lane owns key jcol, four consecutive d per store
+	// The waves that share a block of keys leave dK / dV in LDS, value by value as their lanes hold them; the wave with the first rows,
+	// which stores the block, adds them up in order.  The others store the zeros of the key blocks beyond the valid keys.
+	constexpr int PIECE = 2 * DB * 4 * 1024;  // bytes of a wave
+	static_assert(!SHARES || 3 * PIECE <= 4 * TILE_BYTES, "");
+	if constexpr (SHARES) {
+		if (share > 1) {
+			__syncthreads();
+			if (rgrp > 0) {
+				FA2_LDS char* mine = lds + (w - 4 / share) * PIECE + lane * 16;
+#pragma unroll
+				for (int db = 0; db < DB; ++db)
+#pragma unroll
+					for (int aa = 0; aa < 4; ++aa) {
+						*(FA2_LDS f32x4*)(mine + (db * 4 + aa) * 1024) = f32x4{dk[db][4 * aa], dk[db][4 * aa + 1], dk[db][4 * aa + 2], dk[db][4 * aa + 3]};
+						*(FA2_LDS f32x4*)(mine + ((DB + db) * 4 + aa) * 1024) = f32x4{dv[db][4 * aa], dv[db][4 * aa + 1], dv[db][4 * aa + 2], dv[db][4 * aa + 3]};
+					}
+			}
+			__syncthreads();
+		}
+	}
+	const bool idle = SHARES && rgrp > 0;
+	// values 4 aa .. 4 aa + 3 of block db of dK (which = 0) or dV (1)
+	auto result = [&](int which, int db, int aa) __attribute__((always_inline)) {
+		f32x4 x;
+#pragma unroll
+		for (int e = 0; e < 4; ++e) x[e] = which ? dv[db][4 * aa + e] : dk[db][4 * aa + e];
+		if constexpr (SHARES) {
+			if (idle) x = f32x4{0.f, 0.f, 0.f, 0.f};
+			else
+				for (int y = 1; y < share; ++y) x += *(const FA2_LDS f32x4*)(lds + (w + (y - 1) * (4 / share)) * PIECE + lane * 16 + ((which * DB + db) * 4 + aa) * 1024);
+		}
+		return x;
+	};
+	// epilogue: lane owns key jst, four consecutive d per store
+	const int jst = n0 + 32 * w + c;
 	if (hsplit > 1) {
 		// partial sums over this workgroup's share of the steps, fp32 and unscaled, for the reduce kernel
-		if (jcol < a.Sk) {
-			float* pp = a.dkv_part + ((((int64_t)hsi * a.B + b) * a.Hkv + hk) * a.Sk + jcol) * (2 * D);
+		if (jst < a.Sk) {
+			float* pp = a.dkv_part + ((((int64_t)hsi * a.B + b) * a.Hkv + hk) * a.Sk + jst) * (2 * D);
 #pragma unroll
 			for (int db = 0; db < DB; ++db)
 #pragma unroll
 				for (int aa = 0; aa < 4; ++aa) {
 					int d0 = 32 * db + 8 * aa + 4 * g;
-					*(f32x4*)(pp + d0) = f32x4{dk[db][4 * aa], dk[db][4 * aa + 1], dk[db][4 * aa + 2], dk[db][4 * aa + 3]};
-					*(f32x4*)(pp + D + d0) = f32x4{dv[db][4 * aa], dv[db][4 * aa + 1], dv[db][4 * aa + 2], dv[db][4 * aa + 3]};
+					*(f32x4*)(pp + d0) = result(0, db, aa);
+					*(f32x4*)(pp + D + d0) = result(1, db, aa);
 				}
 		}
 		return;
 	}
-	if (jcol < a.Sk) {
-		char* dkp = a.dk.ptr + (int64_t)b * a.dk.sb + (int64_t)hk * a.dk.sh + (int64_t)jcol * a.dk.ss;
-		char* dvp = a.dv.ptr + (int64_t)b * a.dv.sb + (int64_t)hk * a.dv.sh + (int64_t)jcol * a.dv.ss;
+	if (jst < a.Sk) {
+		char* dkp = a.dk.ptr + (int64_t)b * a.dk.sb + (int64_t)hk * a.dk.sh + (int64_t)jst * a.dk.ss;
+		char* dvp = a.dv.ptr + (int64_t)b * a.dv.sb + (int64_t)hk * a.dv.sh + (int64_t)jst * a.dv.ss;
 		const float ks_ = a.scale;
 		const float vs_ = DROP ? a.drop_inv_keep : 1.f;
 #pragma unroll
@@ -902,12 +980,9 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 			for (int aa = 0; aa < 4; ++aa) {
 				if (COLS && 32 * db + 8 * aa >= a.hd) continue;
 				int d0 = 32 * db + 8 * aa + 4 * g;
-				u32x2 pk = {pack2<typename T::V2>(dk[db][4 * aa] * ks_, dk[db][4 * aa + 1] * ks_),
-				            pack2<typename T::V2>(dk[db][4 * aa + 2] * ks_, dk[db][4 * aa + 3] * ks_)};
-				*(u32x2*)(dkp + d0 * 2) = pk;
-				u32x2 pv = {pack2<typename T::V2>(dv[db][4 * aa] * vs_, dv[db][4 * aa + 1] * vs_),
-				            pack2<typename T::V2>(dv[db][4 * aa + 2] * vs_, dv[db][4 * aa + 3] * vs_)};
-				*(u32x2*)(dvp + d0 * 2) = pv;
+				const f32x4 xk = result(0, db, aa), xv = result(1, db, aa);
+				*(u32x2*)(dkp + d0 * 2) = u32x2{pack2<typename T::V2>(xk[0] * ks_, xk[1] * ks_), pack2<typename T::V2>(xk[2] * ks_, xk[3] * ks_)};
+				*(u32x2*)(dvp + d0 * 2) = u32x2{pack2<typename T::V2>(xv[0] * vs_, xv[1] * vs_), pack2<typename T::V2>(xv[2] * vs_, xv[3] * vs_)};
 			}
 	}
 }
@@ -1246,6 +1321,10 @@ __global__ __launch_bounds__(NW * 64, WPS) void bwd_dq_kernel(const KArgs a) {
 		constexpr bool MASKED = decltype(masked_tag)::value;
 #pragma unroll
 		for (int kb = 0; kb < KB; ++kb) {
+			// (a block of 32 keys that no row of the wave sees)
+			if constexpr (MASKED) {
+				if (n0 + 32 * kb > wave_jmax || n0 + 32 * kb + 31 < wave_lmin) continue;
+			}
 			f32x4 bv[BIAS && !BIAS_LDS ? QB : 1][4];
 			typename T::V4 bvl[BIAS_LDS ? 4 : 1];  // from LDS, kept in the element type until used (half the registers)
 			if constexpr (BIAS_LDS) {
