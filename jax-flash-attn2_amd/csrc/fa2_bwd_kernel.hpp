@@ -1023,7 +1023,7 @@ __global__ __launch_bounds__(NW * 64) void bwd_dkdv_kernel(const KArgs a) {
 			// a.interleave = e groups of an XCD advance together: e adjacent workgroups are the same key tile (see launch_order())
 			int e = a.interleave;
 			int sgi = j / (e * per_group), rem = j % (e * per_group);
-			grp = (sgi * e + rem % e) * 8 + xcd;
+			grp = group_on_xcd(a, sgi * e + rem % e, xcd);
 			within = rem / e;
 		} else {
 			grp = id / per_group;
@@ -1691,6 +1691,7 @@ hipError_t launch_bwd_v(KArgs& a, hipStream_t s) {
 	typedef BwdCfg<T, D> C;
 	int groups = a.B * a.Hkv;
 	a.xcd_remap = (groups % 8 == 0) ? 1 : 0;
+	a.xcd_ranges = DE < D && xcd_ranges_of(a);
 	if (BIAS && a.bias_sh == 0 && a.B % 8 == 0) a.xcd_remap = a.kv_lens ? 3 : 2;
 	// Delta and dQ both requested (the whole backward, or stages 1 + 4): the dQ kernel forms delta
 	// itself and runs first, the dK/dV kernel reads the delta it left in scratch.  Otherwise each
