@@ -239,6 +239,10 @@ int fa2_bwd_static(const fa2_params* p, void* hip_stream);
  * (_forward_triton.py:140-143). Uses B, Hq, Sq, Sk, p_drop, seed / seed_dev only. */
 int fa2_dropout_mask(const fa2_params* p, uint8_t* keep, void* hip_stream);
 
+/* lens[b] = number of non-zero bytes among the first S of row b of `mask` (rows `stride` bytes apart): the `seqlens` of a
+ * right-padded boolean validity mask [B, S] (the reference sums and packs on the host side, _forward_triton.py:499-510). */
+int fa2_mask_lengths(const uint8_t* mask, int64_t stride, int32_t B, int32_t S, int32_t* lens, void* hip_stream);
+
 /* Validate params exactly as fa2_fwd / fa2_bwd would, without launching
  * (host-only; usable without a GPU).  which: 0 = forward, 1 = backward. */
 int fa2_validate(const fa2_params* p, int which);

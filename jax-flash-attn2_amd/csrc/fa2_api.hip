@@ -507,6 +507,12 @@ int fa2_dropout_mask(const fa2_params* p, uint8_t* keep, void* hip_stream) {
 	return e == hipSuccess ? FA2_OK : FA2_EHIP;
 }
 
+int fa2_mask_lengths(const uint8_t* mask, int64_t stride, int32_t B, int32_t S, int32_t* lens, void* hip_stream) {
+	if (B <= 0 || S <= 0) return FA2_EINVAL_SHAPE;
+	if (!mask || !lens || ((uintptr_t)lens & 3)) return FA2_EINVAL_PTR;
+	return fa2::launch_mask_lengths(mask, stride, B, S, lens, (hipStream_t)hip_stream) == hipSuccess ? FA2_OK : FA2_EHIP;
+}
+
 const char* fa2_strerror(int code) {
 	switch (code) {
 		case FA2_OK: return "ok";

@@ -73,6 +73,7 @@ hipError_t launch_fwd(int dtype, int D, bool bias, bool drop, KArgs& a, hipStrea
 hipError_t launch_bwd(int dtype, int D, bool bias, bool drop, KArgs& a, hipStream_t s);
 hipError_t launch_dropout_mask(uint8_t* keep, int B, int H, int Sq, int Sk, uint32_t k0, uint32_t k1, uint32_t thr,
                                const uint32_t* seed_dev, hipStream_t s);
+hipError_t launch_mask_lengths(const uint8_t* mask, int64_t stride, int B, int S, int32_t* lens, hipStream_t s);
 
 // Per-(dtype, D) translation units provide these.
 #define FA2_DECL_FWD(TAG, DD) hipError_t launch_fwd_##TAG##_##DD(bool bias, bool drop, KArgs& a, hipStream_t s);

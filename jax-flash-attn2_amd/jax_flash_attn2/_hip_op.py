@@ -148,7 +148,14 @@ def _seqlens_from_mask(attention_mask, q):
 		return None
 	if attention_mask.dim() != 2:
 		raise ValueError("attention_mask must be a 2-D [batch, seq] right-padded validity mask; use bias for general masks")
-	return attention_mask.to(device=q.device).ne(0).sum(dim=1, dtype=torch.int32).contiguous()
+	m = attention_mask.to(device=q.device)
+	if m.dtype != torch.bool:
+		m = m.ne(0)
+	if not q.is_cuda or m.numel() == 0 or m.stride(1) != 1:
+		return m.sum(dim=1, dtype=torch.int32).contiguous()
+	lens = torch.empty((m.shape[0],), dtype=torch.int32, device=q.device)
+	_lib.check(_lib.load().fa2_mask_lengths(m.data_ptr(), m.stride(0), m.shape[0], m.shape[1], lens.data_ptr(), _stream_ptr(q.device)))
+	return lens
 
 
 def fwd(q, k, v, bias=None, seqlens=None, softmax_scale=None, dropout_prob=0.0, causal=False, dropout_seed=None, kv_lens=None,

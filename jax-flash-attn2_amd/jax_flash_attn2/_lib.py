@@ -82,6 +82,7 @@ EXPORTS = (
 	"fa2_bwd_split_scratch_bytes",
 	"fa2_fwd_scratch_bytes",
 	"fa2_dropout_mask",
+	"fa2_mask_lengths",
 	"fa2_validate",
 	"fa2_strerror",
 	"fa2_version",
@@ -128,6 +129,8 @@ def load() -> ctypes.CDLL:
 		lib.fa2_fwd_scratch_bytes.restype = ctypes.c_size_t
 		lib.fa2_dropout_mask.argtypes = [pp, ctypes.c_void_p, ctypes.c_void_p]
 		lib.fa2_dropout_mask.restype = ctypes.c_int
+		lib.fa2_mask_lengths.argtypes = [ctypes.c_void_p, ctypes.c_int64, ctypes.c_int32, ctypes.c_int32, ctypes.c_void_p, ctypes.c_void_p]
+		lib.fa2_mask_lengths.restype = ctypes.c_int
 		lib.fa2_validate.argtypes = [pp, ctypes.c_int]
 		lib.fa2_validate.restype = ctypes.c_int
 		lib.fa2_strerror.argtypes = [ctypes.c_int]
