@@ -122,7 +122,8 @@ FA2_DEV void dkdv_load_kv(const KArgs& a, int jcol, int hk, int b, typename T::V
 
 // WALKS: `order` is a run-time value (the paired kernel); otherwise the tile is walked head by head and `order_rt` is not looked at.
 // DE: columns of the products (DE < D: rows of a.hd <= DE columns in tiles of D, see the forward kernel).
-template <typename T, int D, int NW, int QB, bool BIAS, bool DROP, bool BIAS_T, bool CAP, bool WALKS, int DE = D>
+// BLK: block by block throughout, without the pipeline over the blocks of a tile, in half the registers: two workgroups per CU.
+template <typename T, int D, int NW, int QB, bool BIAS, bool DROP, bool BIAS_T, bool CAP, bool WALKS, int DE = D, bool BLK = false>
 FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int b, const int hsi, const int hsplit, const int order_rt,
                            const int rot, const DkdvRow& rw) {
 	const int order = WALKS ? order_rt : 0;
@@ -367,7 +368,7 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 		// elementwise math of B(k-1) - the vector ALU and the LDS work in the shadow of the
 		// matrix pipe.  A scheduling barrier after every slot pins that order.
 		constexpr int NSLOT = 2 * KS;     // = 4 DB
-		constexpr int PA = 4;             // read-ahead distance in slots
+		constexpr int PA = BLK ? 3 : 4;   // read-ahead distance in slots
 		constexpr int RING = PA + 1;
 		static_assert(NSLOT % 16 == 0 || NSLOT == 8 || (NSLOT == 12 && FOLD), "");
 		f32x16 s[2], dp[2];
@@ -822,9 +823,9 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 			bool skip = false;
 			if constexpr (MODE != kPlain)
 				skip = wn0 >= sk_eff || m0 > last_row || (wr >= 0 && wn0 > last_row + off + wr) || (wl >= 0 && wn0 + 31 < m0 + off - wl);
-			if constexpr (MODE == kBlocks) {
+			if constexpr (MODE == kBlocks || BLK) {
 				if (!skip) {
-					const int nb = (last_row - m0 + 32) >> 5;
+					const int nb = MODE == kPlain ? QB : (last_row - m0 + 32) >> 5;
 					// (the offsets move along with the blocks and back)
 					auto move = [&](int by) __attribute__((always_inline)) {
 #pragma unroll
@@ -835,9 +836,13 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 							toff[db][1] += by * (32 * D * 2);
 						}
 						soff += by * 128;
+						if constexpr (BIAS_LDS) {
+							boffq[0] += by * (32 * 256);
+							boffq[1] += by * (32 * 256);
+						}
 					};
 					for (int i = 0; i < nb; ++i) {
-						tile_body(std::true_type{}, std::integral_constant<int, 1>{}, hq, m0 + 32 * i);
+						tile_body(std::integral_constant<bool, MODE != kPlain>{}, std::integral_constant<int, 1>{}, hq, m0 + 32 * i);
 						move(1);
 					}
 					move(-nb);
@@ -995,8 +1000,8 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 // CAP: tanh soft-capping of the scores (see the forward kernel); the bias itself may then be absent
 // PAIR: the instantiation for launches that give a workgroup two key tiles (a.kv_pair); the launcher picks it only then,
 // so that every other launch runs the kernel with the one walk as a compile-time constant.
-template <typename T, int D, int NW, int QB, bool BIAS, bool DROP, bool BIAS_T, bool CAP = false, bool PAIR = false, int DE = D>
-__global__ __launch_bounds__(NW * 64) void bwd_dkdv_kernel(const KArgs a) {
+template <typename T, int D, int NW, int QB, bool BIAS, bool DROP, bool BIAS_T, bool CAP = false, bool PAIR = false, int DE = D, bool BLK = false>
+__global__ __launch_bounds__(NW * 64, BLK ? 2 : 1) void bwd_dkdv_kernel(const KArgs a) {
 	// (with the steps of a key tile split over workgroups: the parts of one key tile are adjacent)
 	int hk, b, within;
 	const int hsplit = a.kv_hsplit > 1 ? a.kv_hsplit : 1;
@@ -1035,7 +1040,7 @@ __global__ __launch_bounds__(NW * 64) void bwd_dkdv_kernel(const KArgs a) {
 	const DkdvRow rw = dkdv_row<DROP>(a, b);
 	if constexpr (!PAIR) {
 		// one key tile, head by head (early key tiles see the most query rows under a causal mask: first)
-		bwd_dkdv_tile<T, D, NW, QB, BIAS, DROP, BIAS_T, CAP, false, DE>(a, within, hk, b, hsi, hsplit, 0, 0, rw);
+		bwd_dkdv_tile<T, D, NW, QB, BIAS, DROP, BIAS_T, CAP, false, DE, BLK>(a, within, hk, b, hsi, hsplit, 0, 0, rw);
 	} else {
 		// Causal self-attention: key tile p streams every query tile from p up, so a workgroup takes tile p and tile
 		// ntiles - 1 - p one after the other - every workgroup then has the same number of steps (no CU waits for the
@@ -1766,20 +1771,39 @@ hipError_t launch_bwd_v(KArgs& a, hipStream_t s) {
 		// typed variant: bias in the element type of q, staged through LDS: it also needs 16-byte aligned rows of whole 16-byte pieces
 		bool typed = BIAS && a.bias_dtype == (std::is_same<T, BF16>::value ? 2 : 1);
 		if (!a.bias_lds) typed = false;
-		// with bias at D = 128 the streamed tiles are 64 rows, which leaves LDS room for the bias tiles
-		constexpr int QBV = (BIAS && D == 128) ? 2 : C::KV_QB;
-		if constexpr (BIAS) {
-			if (a.softcap > 0.f)
-				hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, C::KV_NW, QBV, true, DROP, false, true>), grid, block, 0, s, a);
-			else if (typed)
-				hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, C::KV_NW, QBV, true, DROP, true>), grid, block, 0, s, a);
+		// Head dim 64 on grids of at least two workgroups per CU: block by block in half the registers, two workgroups on a CU.  The one wave
+		// per SIMD of the pipelined form is bound by the issue of its elementwise stage and stands still while its workgroup starts and
+		// ends; two hide each other's.  Forward and backward, pipelined -> this: B32 H12 of 256 to 511 tokens 177 -> 159 us, B8 H16 S1024 200 ->
+		// 190, causal 144 -> 140, with dropout 315 -> 290, B8 H16 S2048 with a shared bias 842 -> 809, B2 S2048 with a bias per head 283 -> 267,
+		// B1 Hq32 Hkv8 S8191 in a window of 1024 389 -> 373.  Below that number of workgroups it is alone on its CU and slower (384
+		// of them, B4 Hq32 Hkv4 S1500 causal: 256 -> 284), and so it is against pairs of key tiles (B4 Hq16 Hkv4 S4096 causal 656 -> 732).
+		const bool blk = D == 64 && !a.kv_pair && (int64_t)grid.x >= 2 * kNumCU;
+		auto launch_dkdv = [&](auto blk_tag) {
+			constexpr bool BLK = decltype(blk_tag)::value;
+			// with bias at D = 128 the streamed tiles are 64 rows, which leaves LDS room for the bias tiles (and block by block for a second workgroup)
+			constexpr int QBV = (BIAS && (D == 128 || BLK)) ? 2 : C::KV_QB;
+			if constexpr (BIAS) {
+				if (a.softcap > 0.f)
+					hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, C::KV_NW, QBV, true, DROP, false, true, false, DE, BLK>), grid, block, 0, s, a);
+				else if (typed)
+					hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, C::KV_NW, QBV, true, DROP, true, false, false, DE, BLK>), grid, block, 0, s, a);
+				else
+					hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, C::KV_NW, QBV, true, DROP, false, false, false, DE, BLK>), grid, block, 0, s, a);
+			} else if (a.kv_pair) {
+				// (only instantiated where the launcher can choose it: no bias, head dim up to 128)
+				if constexpr (D <= 128 && !BLK)
+					hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, C::KV_NW, QBV, false, DROP, false, false, true, DE>), grid, block, 0, s, a);
+			} else {
+				hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, C::KV_NW, QBV, false, DROP, false, false, false, DE, BLK>), grid, block, 0, s, a);
+			}
+		};
+		if constexpr (D == 64) {
+			if (blk)
+				launch_dkdv(std::true_type{});
 			else
-				hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, C::KV_NW, QBV, true, DROP, false>), grid, block, 0, s, a);
-		} else if (a.kv_pair) {
-			// (only instantiated where the launcher can choose it: no bias, head dim up to 128)
-			if constexpr (D <= 128) hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, C::KV_NW, QBV, false, DROP, false, false, true, DE>), grid, block, 0, s, a);
+				launch_dkdv(std::false_type{});
 		} else {
-			hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, C::KV_NW, QBV, false, DROP, false, false, false, DE>), grid, block, 0, s, a);
+			launch_dkdv(std::false_type{});
 		}
 		if (hs > 1) {
 			int64_t total = (int64_t)a.B * a.Hkv * a.Sk * 2 * (D / 8);
