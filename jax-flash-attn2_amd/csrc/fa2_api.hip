@@ -378,9 +378,13 @@ static size_t fwd_scratch_bytes(const fa2_params* p) {
 }  // extern "C"
 
 namespace {
+// (of the padded rows, which are contiguous: whatever strides the short ones have, the answer is the same before and after
+// the caller copies them for their alignment)
 bool fwd_takes_ranges(const fa2_params* p) {
+	fa2_params padded = *p;
+	padded.q.stride_s = padded.q.stride_h = 0;
 	int whole;
-	return fwd_decode_waves(p, &whole) || fwd_scratch_bytes(p);
+	return fwd_decode_waves(&padded, &whole) || fwd_scratch_bytes(&padded);
 }
 }  // namespace
 

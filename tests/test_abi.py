@@ -237,3 +237,15 @@ def test_backward_split_scratch_only_on_small_grids():
 	assert need(4, 4096, 32, 8, causal=1)[0] == 0
 	n, base = need(1, 2048, 8, 8, causal=1)    # 16 steps: the 2 parts that fill the chip, no more
 	assert n == base + 2 * (1 * 8 * 2048 * 2 * 128 * 4)
+
+
+def test_short_rows_are_refused_alike_whatever_the_strides():
+	"""A forward of few query rows over 80 columns wants padded rows.  The answer must not change once the caller has copied
+	badly aligned or widely spaced rows into contiguous ones."""
+	for spacing in (80, 1 << 30):
+		p = _good_params()
+		p.B, p.Sq, p.Sk, p.Hq, p.Hkv, p.D, p.head_dim, p.causal = 64, 2, 4096, 16, 8, 128, 80, 0
+		for t in (p.q, p.k, p.v, p.o):
+			t.stride_h, t.stride_s, t.stride_b = 80, 16 * 80, 4096 * 16 * 80
+		p.q.stride_h = spacing
+		assert _rc(p, 0) == -10
