@@ -1,0 +1,62 @@
+"""NaN and infinity through the forwards that work on pieces of a key range (the split kernels and the decoding kernel): a row that
+sees a non-finite value must come out non-finite whatever the keys were cut into."""
+
+import ctypes
+
+import numpy as np
+import pytest
+import torch
+
+import fa2_oracle as O
+from _cases import f64, make_inputs
+from jax_flash_attn2 import _hip_op as op
+from jax_flash_attn2 import _lib
+
+pytestmark = pytest.mark.gpu
+
+
+def _scratch(q, k, v, causal=False, kv_lens=None):
+	return _lib.load().fa2_fwd_scratch_bytes(ctypes.byref(op._block(q.shape[3], q, k, v, None, None, 1.0, 0.0, causal, None, kv_lens)))
+
+
+# (B, Sq, Sk, Hq, Hkv, D, causal): 128-row workgroups on several ranges; ranges of the 64-row kernel with the q-heads packed; head
+# dim 256, which takes that kernel unpacked; the decoding kernel with units of several waves, and of few keys (257 .. 448)
+_PIECES = [
+	(1, 100, 2000, 8, 2, 128, True),
+	(1, 300, 1500, 4, 4, 64, False),
+	(1, 8, 4000, 8, 2, 128, False),
+	(1, 65, 2048, 2, 2, 256, True),
+	(1, 1, 1029, 32, 8, 128, False),
+	(2, 2, 300, 4, 2, 64, True),
+	(2, 1, 400, 4, 4, 256, False),
+]
+
+
+@pytest.mark.parametrize("B,Sq,Sk,Hq,Hkv,D,causal", _PIECES)
+@pytest.mark.parametrize("what", ["nan in one key", "infinity in one key", "nan in a query row", "infinity in a query row"])
+def test_non_finite_rows_stay_non_finite(B, Sq, Sk, Hq, Hkv, D, causal, what):
+	dtype = torch.bfloat16
+	q, k, v, _, _ = make_inputs(B, Sq, Sk, Hq, Hkv, D, dtype, seed=Sq + Sk)
+	bad = float("nan") if "nan" in what else float("inf")
+	key, row = Sk - 40, Sq // 2
+	if "key" in what:
+		q[..., 3] = q[..., 3].abs() + 0.1  # (of infinity: every row that sees the key scores +inf, whose softmax is NaN)
+		k[:, key, Hkv - 1, 3] = bad
+	else:
+		q[:, row, Hq - 1, 3] = bad
+		k[..., 3] = k[..., 3].abs() + 0.1
+	assert _scratch(q, k, v, causal) > 0, "this shape is meant to be cut into pieces"
+	o, lse = op.fwd(q.cuda(), k.cuda(), v.cuda(), causal=causal)
+	o = o.float().cpu()
+	hit = torch.zeros(B, Sq, Hq, dtype=torch.bool)
+	if "key" in what:
+		first = max(0, key - (Sk - Sq)) if causal else 0
+		hit[:, first:, Hq - Hq // Hkv :] = True
+	else:
+		hit[:, row, Hq - 1] = True
+	assert torch.isnan(o[hit]).all(), f"{int((~torch.isnan(o[hit])).sum())} finite values in rows that see {what}"
+	# and nothing else changed
+	for x in (q, k):
+		x[~torch.isfinite(x)] = 0.0
+	o_ref, _ = O.attention_fwd(f64(q), f64(k), f64(v), causal=causal)
+	assert np.abs(o[~hit].numpy() - torch.from_numpy(o_ref)[~hit].numpy()).max() <= 2e-2
