@@ -89,13 +89,24 @@ __global__ __launch_bounds__(DecodeCfg<D>::NW * 64) void fwd_decode_kernel(const
 	int share, f, f_end;
 	DecodePos pos;
 	if (a.decode_whole) {
-		// one unit per wave, and nobody else to store the zeros of a unit without keys
+		// one unit per wave, which also stores the zeros of a unit without keys
 		if (wid >= a.B * a.Hkv) return;
 		pos.b = wid / a.Hkv;
 		pos.hk = wid - pos.b * a.Hkv;
 		pos.t = 0;
 		pos.len = decode_len(a, pos.b);
-		pos.tiles = pos.len > 0 ? tiles_of(pos.len) : 1;
+		if (pos.len == 0) {
+			// nothing may be read here: the slots of an empty row of a cache can hold anything, and 0 times NaN is NaN
+			if (c < nrows) {
+				const int hh = c / a.Sq, i = c - hh * a.Sq, h = pos.hk * r + hh;
+				char* rp = a.o.ptr + (int64_t)pos.b * a.o.sb + (int64_t)h * a.o.sh + (int64_t)i * a.o.ss + 8 * g;
+#pragma unroll
+				for (int db = 0; db < DB; ++db) *(u32x2*)(rp + 32 * db) = u32x2{0u, 0u};
+				if (g == 0) a.lse[((int64_t)pos.b * a.Hq + h) * a.Sq + i] = -INFINITY;
+			}
+			return;
+		}
+		pos.tiles = tiles_of(pos.len);
 		share = f_end = pos.tiles;
 		f = 0;
 	} else if (!a.kv_lens) {
@@ -162,8 +173,7 @@ __global__ __launch_bounds__(DecodeCfg<D>::NW * 64) void fwd_decode_kernel(const
 	}
 	auto issue = [&](const DecodePos& p, int buf, bool with_q, int qbuf) __attribute__((always_inline)) {
 		const int n0 = p.t * KT;
-		int rows = p.len - n0 < KT ? p.len - n0 : KT;
-		rows = rows > 0 ? rows : 1;  // (a unit without keys: its only tile is masked as a whole)
+		const int rows = p.len - n0 < KT ? p.len - n0 : KT;
 		if (with_q) {
 			const char* qb = TileLoader<D, KT, 64>::uniform(a.q.ptr + (int64_t)p.b * a.q.sb + (int64_t)(p.hk * r) * a.q.sh);
 #pragma unroll

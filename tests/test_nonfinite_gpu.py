@@ -1,5 +1,6 @@
 """NaN and infinity through the forwards that work on pieces of a key range (the split kernels and the decoding kernel): a row that
-sees a non-finite value must come out non-finite whatever the keys were cut into."""
+sees a non-finite value must come out non-finite whatever the keys were cut into, and a value that no row may see - a slot of
+the cache beyond its row's length - must not come out at all."""
 
 import ctypes
 
@@ -8,7 +9,7 @@ import pytest
 import torch
 
 import fa2_oracle as O
-from _cases import f64, make_inputs
+from _cases import check_forward, f64, make_inputs
 from jax_flash_attn2 import _hip_op as op
 from jax_flash_attn2 import _lib
 
@@ -60,3 +61,36 @@ def test_non_finite_rows_stay_non_finite(B, Sq, Sk, Hq, Hkv, D, causal, what):
 		x[~torch.isfinite(x)] = 0.0
 	o_ref, _ = O.attention_fwd(f64(q), f64(k), f64(v), causal=causal)
 	assert np.abs(o[~hit].numpy() - torch.from_numpy(o_ref)[~hit].numpy()).max() <= 2e-2
+
+
+@pytest.mark.parametrize(
+	"B,Sq,Sk,Hq,Hkv,D,lens,cut",
+	[
+		# one wave a unit: few keys, and from 2048 units on
+		(3, 1, 200, 8, 2, 64, [0, 200, 7], False),
+		(2, 2, 192, 4, 2, 128, [0, 33], False),
+		(2, 1, 100, 4, 4, 256, [64, 0], False),
+		(128, 1, 300, 16, 16, 64, None, None),
+		# units of several waves; 128-row workgroups, unsplit and split
+		(4, 1, 700, 8, 2, 128, [700, 0, 31, 384], True),
+		(2, 130, 200, 2, 1, 128, [0, 70], False),
+		(2, 150, 1500, 4, 4, 128, [0, 40], True),
+	],
+)
+def test_slots_beyond_the_length_are_not_looked_at(B, Sq, Sk, Hq, Hkv, D, lens, cut):
+	dtype = torch.bfloat16
+	if lens is None:
+		lens = [int(x) for x in np.linspace(0, Sk, B)]
+	q, k, v, _, _ = make_inputs(B, Sq, Sk, Hq, Hkv, D, dtype, seed=B + Sk)
+	o_ref, lse_ref = O.attention_fwd(f64(q), f64(k), f64(v), kv_lens=lens)
+	for b, n in enumerate(lens):
+		k[b, n:] = float("nan")
+		v[b, n:] = float("nan")
+	kl = torch.tensor(lens, dtype=torch.int32, device="cuda:0")
+	if cut is not None:
+		assert bool(_scratch(q, k, v, kv_lens=kl)) == cut
+	o, lse = op.fwd(q.cuda(), k.cuda(), v.cuda(), kv_lens=kl)
+	check_forward(o, lse, o_ref, lse_ref, dtype, f"B{B} Sq{Sq} Sk{Sk} Hq{Hq} Hkv{Hkv} D{D} lens={lens}")
+	for b, n in enumerate(lens):
+		if n == 0:
+			assert not o[b].any() and torch.isneginf(lse[b]).all()
