@@ -75,6 +75,15 @@ def _usable(x: torch.Tensor) -> torch.Tensor:
 	return x
 
 
+def _usable_short(x: torch.Tensor) -> torch.Tensor:
+	"""The same for rows that are shorter than the kernels' head dim.  A padded copy of such rows would be in order whatever the
+	tensor is, so what the library refuses of it is copied too: a contiguous tensor that is not aligned, rows too far apart."""
+	sb, ss, sh, sd = x.stride()
+	if sd != 1 or (sb | ss | sh) & 7 or x.data_ptr() & 15 or ss > 0x7FFFFFFF // 256:
+		return x.clone(memory_format=torch.contiguous_format)
+	return x
+
+
 def _block(D, q, k, v, bias, seqlens, scale, p_drop, causal, seed, kv_lens=None, window=None, softcap=0.0, o=_NONE4, lse=None,
            backward=(_NONE4, _NONE4, _NONE4, _NONE4)):
 	"""The parameter block of a call on rows of q.shape[3] columns in the kernels of head dim D.  `o` and `backward` (dO, dq, dk, dv)
@@ -168,7 +177,7 @@ def fwd(q, k, v, bias=None, seqlens=None, softmax_scale=None, dropout_prob=0.0, 
 	scale = 1.0 / math.sqrt(D0) if softmax_scale is None else softmax_scale
 	call = (bias, seqlens, scale, dropout_prob, causal, dropout_seed, kv_lens, window, softcap)
 	rows = D0 if D0 != D and _runs_unpadded(lib, 0, D, q, k, v, *call) else D  # columns of the rows the library is given
-	q, k, v = _usable(_pad_d(q, rows)), _usable(_pad_d(k, rows)), _usable(_pad_d(v, rows))
+	q, k, v = (_usable(_pad_d(x, D)) if rows == D else _usable_short(x) for x in (q, k, v))
 	out = torch.empty_like(q, memory_format=torch.contiguous_format)
 	lse = torch.empty((q.shape[0], q.shape[2], q.shape[1]), dtype=torch.float32, device=q.device)
 	p = _block(D, q, k, v, *call, _t4(out), lse)
@@ -195,7 +204,7 @@ def bwd(q, k, v, out, lse, dout, bias=None, seqlens=None, softmax_scale=None, dr
 	scale = 1.0 / math.sqrt(D0) if softmax_scale is None else softmax_scale
 	call = (bias, seqlens, scale, dropout_prob, causal, dropout_seed, kv_lens, window, softcap)
 	rows = D0 if D0 != D and _runs_unpadded(lib, 1, D, q, k, v, *call) else D
-	q, k, v, out, dout = (_usable(_pad_d(x, rows)) for x in (q, k, v, out, dout))
+	q, k, v, out, dout = (_usable(_pad_d(x, D)) if rows == D else _usable_short(x) for x in (q, k, v, out, dout))
 	Sq = q.shape[1]
 	dq = torch.empty_like(q, memory_format=torch.contiguous_format)
 	dk = torch.empty_like(k, memory_format=torch.contiguous_format)

@@ -56,3 +56,30 @@ def test_infinite_last_column():
 	keep = [j for j in range(100) if j != 5]
 	o_ref, lse_ref = O.attention_fwd(f64(q), f64(k[:, keep]), f64(v[:, keep]))
 	check_forward(o, lse, o_ref, lse_ref, torch.bfloat16, "key of -inf")
+
+
+@pytest.mark.parametrize("how", ["two bytes into a buffer", "odd batch stride", "rows too far apart"])
+def test_short_rows_in_any_memory(how):
+	"""Tensors that are contiguous and yet not aligned, or whose rows lie further apart than the kernels address: padded rows were
+	copies in order, rows taken as they are have to be brought in order."""
+	B, S, H, D, dtype = 1, 300, 2, 80, torch.float16
+	q, k, v, do, _ = make_inputs(B, S, S, H, H, D, dtype, seed=4)
+
+	def placed(x):
+		x = x.cuda()
+		if how == "two bytes into a buffer":
+			return torch.nn.functional.pad(x.flatten(), (1, 0))[1:].view(x.shape)
+		if how == "odd batch stride":
+			return x.as_strided(x.shape, (x.numel() + 1, *x.stride()[1:]))
+		far = 0x7FFFFFFF // 256 + 8 - (0x7FFFFFFF // 256) % 8  # the first multiple of 8 beyond the limit
+		wide = torch.empty((S - 1) * far + H * D, dtype=dtype, device="cuda:0")
+		y = wide.as_strided(x.shape, (S * far, far, D, 1))
+		y.copy_(x)
+		return y
+
+	args = [placed(x) for x in (q, k, v, do)]
+	o, lse = op.fwd(*args[:3], causal=True)
+	grads = op.bwd(*args[:3], o, lse, args[3], causal=True)
+	a = [f64(x) for x in (q, k, v, do)]
+	check_forward(o, lse, *O.attention_fwd(*a[:3], causal=True), dtype, how)
+	check_grads(grads, O.attention_bwd(*a, causal=True), how)
