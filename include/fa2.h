@@ -182,7 +182,9 @@ int fa2_fwd(const fa2_params* p, void* hip_stream);
  * units to fill the chip - decoding, `Sq == 1` in flash_attention.py:239-242, from 512 keys, and
  * prompts at batch 1 with few heads from 1024 or 2048 keys: given `scratch` (256-byte aligned) of at least this many
  * bytes, fa2_fwd splits the keys into ranges handled by separate workgroups and merges the
- * partial results (same O and lse to rounding).  Without it the call runs unsplit. */
+ * partial results (same O and lse to rounding).  Without it the call runs unsplit.  The query reads the sizes, causal,
+ * has_window, softcap, p_drop, the strides of q, and whether bias, seqlens and kv_lens are given: fa2_fwd decides by the same
+ * fields, so the answer for a block that lacks one of them may be that of another plan. */
 size_t fa2_fwd_scratch_bytes(const fa2_params* p);
 
 /* dq, dk, dv from (q, k, v, o, lse, dO).  Replaces the `_attn_bwd_preprocess`

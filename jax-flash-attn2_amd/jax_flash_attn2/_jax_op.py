@@ -141,29 +141,34 @@ def _seed_operand(dropout_seed):
 	return jnp.stack([x.astype(jnp.uint32), jnp.zeros((), jnp.uint32)])
 
 
-def _size_query(q, k, cfg: _Cfg, fn_names):
-	"""max over the named host-only size queries of the library for these shapes (at least one aligned unit so that
-	the result buffer is never empty)."""
+def _size_query(ops: dict, cfg: _Cfg, fn_names):
+	"""max over the named host-only size queries of the library for these operands (at least one aligned unit so that
+	the result buffer is never empty).  The handler launches by the same fields, so all that the queries look at is set:
+	of the optional operands only whether they are there."""
 	from . import _lib
 
+	q, k = ops["q"], ops["k"]
 	p = _lib.new_params()
 	p.B, p.Sq, p.Hq, p.D = (int(x) for x in q.shape)
 	p.Sk, p.Hkv = int(k.shape[1]), int(k.shape[2])
 	p.causal = 1 if cfg.causal else 0  # (causal backward launches split further: their key tiles differ in length)
 	p.has_window = 1 if cfg.has_window else 0
 	p.softcap = float(cfg.softcap)
+	p.p_drop = float(cfg.dropout_p)
+	for name in ("bias", "seqlens", "kv_lens"):
+		setattr(p, name, 256 if ops[name].size else None)
 	lib = _lib.load()
 	return max([int(getattr(lib, n)(ctypes.byref(p))) for n in fn_names] + [256])
 
 
 def _fwd_call(ops: dict, cfg: _Cfg):
 	_register()
-	q, k = ops["q"], ops["k"]
+	q = ops["q"]
 	B, Sq, Hq, _ = q.shape
 	out_types = dict(
 		o=jax.ShapeDtypeStruct(q.shape, q.dtype),
 		lse=jax.ShapeDtypeStruct((B, Hq, Sq), jnp.float32),
-		scratch=jax.ShapeDtypeStruct((_size_query(q, k, cfg, ("fa2_fwd_scratch_bytes",)),), jnp.uint8),
+		scratch=jax.ShapeDtypeStruct((_size_query(ops, cfg, ("fa2_fwd_scratch_bytes",)),), jnp.uint8),
 	)
 	res = _ffi_call("fa2_fwd_ffi", tuple(out_types[n] for n in spec.FWD_RESULTS))(*[ops[n] for n in spec.FWD_OPERANDS], **_attr_dict(cfg))
 	res = dict(zip(spec.FWD_RESULTS, res))
@@ -175,7 +180,7 @@ def _bwd_call(ops: dict, cfg: _Cfg):
 	q, k, v = ops["q"], ops["k"], ops["v"]
 	B, Sq, Hq, _ = q.shape
 	Sk = k.shape[1]
-	scratch_bytes = _size_query(q, k, cfg, ("fa2_bwd_scratch_bytes", "fa2_bwd_split_scratch_bytes"))
+	scratch_bytes = _size_query(ops, cfg, ("fa2_bwd_scratch_bytes", "fa2_bwd_split_scratch_bytes"))
 	out_types = dict(
 		dq=jax.ShapeDtypeStruct(q.shape, q.dtype),
 		dk=jax.ShapeDtypeStruct(k.shape, k.dtype),

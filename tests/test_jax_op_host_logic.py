@@ -164,3 +164,45 @@ def test_other_head_dims_are_padded_and_cut(jop):
 	assert abs(float(calls[-1][2]["scale"]) - 80 ** -0.5) < 1e-7  # the scale keeps the true head dim
 	with pytest.raises(ValueError):
 		mod.flash_attention(*_qkv(D=320))
+
+
+@pytest.mark.parametrize("B,Sq,Sk,Hq,Hkv,D", [(1, 64, 16384, 8, 8, 128), (1, 300, 8192, 8, 2, 128), (8, 40, 2000, 32, 8, 128), (2, 2048, 2048, 4, 4, 64),
+                                              (1, 1, 1029, 32, 8, 128), (2, 100, 3000, 4, 4, 256), (1, 512, 512, 4, 4, 64)])
+@pytest.mark.parametrize("extra", ["", "bias", "mask", "dropout", "causal", "kv_lens", "2-D mask", "window"])
+def test_scratch_is_what_the_library_asks_for_with_the_operands_of_the_call(jop, B, Sq, Sk, Hq, Hkv, D, extra):
+	"""The scratch results hold what the library's queries give for the block that the handler fills from operands and attributes."""
+	import ctypes
+
+	from jax_flash_attn2 import _ffi_spec as spec
+	from jax_flash_attn2 import _lib
+
+	if extra == "2-D mask" and Sq != Sk:
+		pytest.skip("a 2-D mask wants as many keys as queries")
+	mod, calls = jop
+	kw = {
+		"": {},
+		"bias": dict(bias=np.zeros((1, 1, Sq, Sk), np.float16)),
+		"mask": dict(attention_mask=np.ones((1, 1, Sq, Sk), np.bool_)),
+		"dropout": dict(dropout_prob=0.1),
+		"causal": dict(causal=True),
+		"kv_lens": dict(kv_lens=[Sk] * B),
+		"2-D mask": dict(attention_mask=np.ones((B, Sk), np.int32)),
+		"window": dict(window_size=(100, 0)),
+	}[extra]
+	mod.flash_attention(*(np.zeros(s, np.float16) for s in ((B, Sq, Hq, D), (B, Sk, Hkv, D), (B, Sk, Hkv, D))), **kw)
+	mod._attention.pullback(np.zeros((B, Sq, Hq, D), np.float16))
+	lib = _lib.load()
+	for (name, operands, attrs, out_types, _), queries in zip(calls[-2:], (("fa2_fwd_scratch_bytes",), ("fa2_bwd_scratch_bytes", "fa2_bwd_split_scratch_bytes"))):
+		names, results, _ = spec.HANDLERS[name]
+		ops, p = dict(zip(names, operands)), _lib.new_params()
+		p.dtype, p.B, p.Sq, p.Sk, p.Hq, p.Hkv, p.D, p.head_dim = _lib.FA2_FP16, B, Sq, Sk, Hq, Hkv, D, D
+		p.causal, p.scale, p.p_drop, p.softcap = int(attrs["causal"]), float(attrs["scale"]), float(attrs["dropout_p"]), float(attrs["softcap"])
+		p.has_window, p.window_left, p.window_right = int(attrs["has_window"]), int(attrs["window_left"]), int(attrs["window_right"])
+		for t in ("q", "k", "v"):
+			b, s, h, d = ops[t].shape
+			f = getattr(p, t)
+			f.ptr, f.stride_b, f.stride_s, f.stride_h = ops[t].ctypes.data, s * h * d, h * d, d
+		for t in ("bias", "seqlens", "kv_lens"):
+			setattr(p, t, ops[t].ctypes.data if ops[t].size else None)
+		want = max([int(getattr(lib, n)(ctypes.byref(p))) for n in queries] + [256])
+		assert out_types[results.index("scratch")].shape == (want,), name
