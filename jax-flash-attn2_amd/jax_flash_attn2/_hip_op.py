@@ -32,6 +32,8 @@ _BIAS_DTYPES = {torch.float16: FA2_FP16, torch.bfloat16: FA2_BF16, torch.float32
 
 def _stream_ptr(device) -> int:
 	# (what torch.cuda.current_stream(device).cuda_stream gives, without building the stream object)
+	if device.type != "cuda":
+		raise ValueError(f"Expected a cuda device, but got: {device}")
 	return torch._C._cuda_getCurrentRawStream(device.index)
 
 

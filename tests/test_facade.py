@@ -107,3 +107,12 @@ def test_kernel_head_dim_padding_rule():
 	x = torch.ones(1, 2, 3, 80)
 	y = _hip_op._pad_d(x, 128)
 	assert y.shape == (1, 2, 3, 128) and float(y[..., 80:].abs().sum()) == 0.0 and _hip_op._pad_d(y, 128) is y
+
+
+def test_tensors_in_host_memory_are_refused_by_name():
+	"""The error that asking torch for the stream of such a device gives; nothing is launched."""
+	q = torch.zeros(1, 8, 2, 64, dtype=torch.float16)
+	with pytest.raises(ValueError, match="Expected a cuda device, but got: cpu"):
+		_hip_op.fwd(q, q, q)
+	with pytest.raises(ValueError, match="Expected a cuda device, but got: cpu"):
+		_hip_op.bwd(q, q, q, q, torch.zeros(1, 2, 8), q)
