@@ -95,18 +95,7 @@ __global__ __launch_bounds__(DecodeCfg<D>::NW * 64) void fwd_decode_kernel(const
 		pos.hk = wid - pos.b * a.Hkv;
 		pos.t = 0;
 		pos.len = decode_len(a, pos.b);
-		if (pos.len == 0) {
-			// nothing may be read here: the slots of an empty row of a cache can hold anything, and 0 times NaN is NaN
-			if (c < nrows) {
-				const int hh = c / a.Sq, i = c - hh * a.Sq, h = pos.hk * r + hh;
-				char* rp = a.o.ptr + (int64_t)pos.b * a.o.sb + (int64_t)h * a.o.sh + (int64_t)i * a.o.ss + 8 * g;
-#pragma unroll
-				for (int db = 0; db < DB; ++db) *(u32x2*)(rp + 32 * db) = u32x2{0u, 0u};
-				if (g == 0) a.lse[((int64_t)pos.b * a.Hq + h) * a.Sq + i] = -INFINITY;
-			}
-			return;
-		}
-		pos.tiles = tiles_of(pos.len);
+		pos.tiles = pos.len > 0 ? tiles_of(pos.len) : 1;
 		share = f_end = pos.tiles;
 		f = 0;
 	} else if (!a.kv_lens) {
@@ -173,7 +162,8 @@ __global__ __launch_bounds__(DecodeCfg<D>::NW * 64) void fwd_decode_kernel(const
 	}
 	auto issue = [&](const DecodePos& p, int buf, bool with_q, int qbuf) __attribute__((always_inline)) {
 		const int n0 = p.t * KT;
-		const int rows = p.len - n0 < KT ? p.len - n0 : KT;
+		int rows = p.len - n0 < KT ? p.len - n0 : KT;
+		rows = rows > 0 ? rows : 1;  // (a unit without keys: its only tile is masked as a whole)
 		if (with_q) {
 			const char* qb = TileLoader<D, KT, 64>::uniform(a.q.ptr + (int64_t)p.b * a.q.sb + (int64_t)(p.hk * r) * a.q.sh);
 #pragma unroll
@@ -256,6 +246,11 @@ __global__ __launch_bounds__(DecodeCfg<D>::NW * 64) void fwd_decode_kernel(const
 	// the columns' results: into O and lse when the unit lies inside this wave's share, else as a piece of it into scratch.  Pieces
 	// are numbered wave + unit: both only grow along the sequence, and each piece begins with a new wave, a new unit or both.
 	auto flush = [&](const DecodePos& p, bool whole) __attribute__((always_inline)) {
+		if (p.len == 0) {
+			// a unit without keys: the slot that was copied for it can hold anything, and 0 times NaN is NaN
+#pragma unroll
+			for (int db = 0; db < DB; ++db) oacc[db] = f32x4{0.f, 0.f, 0.f, 0.f};
+		}
 		const float l = column_sum(l_run);
 		const float inv = l > 0.f ? 1.f / l : 0.f;
 		const float lse = l > 0.f ? (m_run + log2_fast(l)) * kLn2 : -INFINITY;
