@@ -293,16 +293,37 @@ static int fwd_decode_waves(const fa2_params* p, int* whole) {
 	const int kt = p->D == 64 ? 64 : 32;
 	const int64_t tiles = (p->Sk + kt - 1) / kt, total = units * tiles;
 	if (total > 0x3fffffff) return 0;
-	// A wave takes about a microsecond per tile, the second launch 4.5: a unit of up to six tiles is left whole (at eight tiles of
-	// 32 keys, B1 Hkv8, 11.0 us against 10.8 in the 128-row kernel, which keeps that range; tiles of 64 keys 6.9 against 8.1),
-	// and so are the units where they fill all resident waves in whole rounds (B64 Hkv32 Sk2048: 283 us; B70, 2.2 rounds, 323 us
-	// whole) or are so many that the last round does not matter.
-	if (p->Sk <= 256 && tiles > 6) return 0;
-	*whole = p->Sk <= 256 || (units >= 2048 && (units % 1024 == 0 || units >= 16384));
+	const int64_t resident = p->D == 256 ? 512 : 1024;  // waves that run at once
+	const int64_t heads = (int64_t)p->B * p->Hq;        // workgroups of the general kernel, of which 512 run at once (256 at D = 256)
+	const int64_t rows = r * p->Sq;
+	if (p->Sk <= 256) {
+		// A wave takes about a microsecond per tile, so units of up to six tiles are left whole.  Six tiles, or four under more than eight
+		// rows, are whole tiles of the general kernel too, which is then as fast or faster unless the units are many: 8 kv-heads, D128, 16 rows,
+		// here and there, B8 Sk192 10.2 and 9.2 us, Sk160 9.1 and 9.3, Sk128 8.1 and 7.6, B64 Sk192 11.3 and 13.2; D256 B8 Sk192 14.3 and 13.2.
+		if (tiles > 6) return 0;
+		const bool many = heads > resident / 2 || units >= resident / 2;
+		if (!many && p->D != 64 && (tiles == 6 || (tiles == 4 && rows > 8))) return 0;
+		*whole = 1;
+		return (int)units;
+	}
+	// A few hundred keys under many rows: the general kernel runs all its workgroups at once (B40 H8 D128, 16 rows over 300 keys: 16.9 us;
+	// 18.5 here with whole units, 21.7 in shares).
+	if (p->D == 128 && rows > 8 && p->Sk <= 512 && units >= 192 && heads <= 512) return 0;
+	// Whole units or equal shares?  Whole units leave the last round of waves to less than the full stream of memory, unless it is nearly full:
+	// that costs so many us a tile, and a quarter of a tile's time where rows of different length may end early.  Shares cost the
+	// second launch, the partial results written and read, and with lengths the search for a wave's first tile.  From 2989
+	// calls (8 to 2560 units of 257 to 4000 keys, caches not in L2; us whole / shares): H8 D128 B64 Sk500 27.3 / 29.7, Sk2048 98.6 / 93.6;
+	// B96 Sk700 47.4 / 54.0; B192 Sk2048 271 / 271; D64 B64, 16 rows over 700 keys 21.3 / 28.8; D256 B80 Sk1000 144 / 116.
+	// The rule is within 0.6 % of the better of the two on average; what it replaced, shares below 2048 units, lost up to a third
+	// to the general kernel where these are many and the keys few (D64 B64 H8, 16 rows over 257 keys: 17.8 us against 12.1; whole 11.6).
+	const int64_t rem = units % resident;
+	double idle = rem == 0 ? 0.0 : p->D == 256 ? 2.0 - 0.0056 * rem : 1.25 - 0.0022 * rem;
+	idle = (idle > 0 ? idle : 0) + (p->kv_lens ? 0.25 : 0.0);
+	int64_t waves = resident < total ? resident : total;
+	const double merge = 3.4 + (p->kv_lens ? 3.7 : 0.0) + (waves + (units < waves ? units : waves)) * rows * p->D * 8 / 3.1e6;
+	*whole = idle * tiles < merge;
 	if (*whole) return (int)units;
 	// as many waves as are resident at once, down to a tile each (B1 Hkv8 Sk1029: 8.5 us, two tiles each 10.0), at most 63 a unit
-	int64_t waves = p->D == 256 ? 512 : 1024;
-	if (waves > total) waves = total;
 	return (int)(waves < 63 * units ? waves : 63 * units);
 }
 

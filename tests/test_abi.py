@@ -249,3 +249,29 @@ def test_short_rows_are_refused_alike_whatever_the_strides():
 			t.stride_h, t.stride_s, t.stride_b = 80, 16 * 80, 4096 * 16 * 80
 		p.q.stride_h = spacing
 		assert _rc(p, 0) == -10
+
+
+def test_decoding_takes_whole_units_or_equal_shares():
+	"""fa2_fwd_scratch_bytes of calls with few query rows: shares of the key tiles merge their pieces in scratch, a wave that takes a
+	whole (batch, kv-head) needs none."""
+	lib = _lib.load()
+
+	def need(B, Sk, D, lens=False, rows=1, Hkv=8):
+		p = _lib.new_params()
+		p.B, p.Sq, p.Sk, p.Hq, p.Hkv, p.D = B, rows, Sk, Hkv, Hkv, D
+		p.kv_lens = 256 if lens else None
+		return lib.fa2_fwd_scratch_bytes(ctypes.byref(p))
+
+	for D in (64, 128, 256):
+		assert need(1, 192, D) == 0 and need(1, 192, D, rows=16) == 0   # few keys: never cut
+		assert need(4, 1029, D) > 0 and need(4, 1029, D, lens=True) > 0  # few units: shares
+		full = 64 if D == 256 else 128                                   # B x 8 units: every wave that runs at once has one
+		assert need(full, 4000, D) == 0 and need(2 * full, 4000, D) == 0
+		assert need(full + 4, 4000, D) > 0                               # a second round that is nearly empty, over many keys
+		assert need(full, 300, D, lens=True) == 0                        # rows of different length matter over many keys only
+		assert need(full, 8192, D, lens=True) > 0
+	# half a round: whole units where a second launch costs more than the memory pipe that is not full
+	assert need(64, 500, 128) == 0 and need(64, 2048, 128) > 0
+	# many rows make the pieces expensive; at head dim 128 a few hundred keys under many rows take the general kernel, unsplit
+	assert need(64, 1000, 64, rows=16) == 0 and need(64, 2048, 64) > 0
+	assert need(40, 300, 128, rows=16) == 0

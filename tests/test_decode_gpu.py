@@ -36,6 +36,13 @@ pytestmark = pytest.mark.gpu
 		(70, 1, 330, 4, 2, 64, torch.bfloat16, False, "ramp"),
 		(150, 1, 300, 12, 12, 64, torch.float16, False, "ramp"),
 		(3, 1, 9001, 12, 12, 128, torch.bfloat16, False, "ramp"),
+		# whole units over more than 256 keys: half a round of waves, more than a round
+		(64, 1, 600, 8, 8, 128, torch.bfloat16, False, "ramp"),
+		(70, 4, 290, 16, 16, 64, torch.float16, True, None),
+		# sixteen rows over four and six tiles of 32 keys, and over a few hundred keys: left to the general kernel
+		(2, 16, 128, 4, 4, 128, torch.bfloat16, True, None),
+		(2, 4, 190, 8, 2, 256, torch.float16, True, [190, 0]),
+		(24, 16, 270, 8, 8, 128, torch.bfloat16, True, "ramp"),
 		# from 2048 units on every unit is one wave's
 		(130, 1, 270, 16, 16, 64, torch.bfloat16, False, "ramp"),
 	],
