@@ -184,7 +184,7 @@ int fa2_fwd(const fa2_params* p, void* hip_stream);
  * bytes, fa2_fwd splits the keys into ranges handled by separate workgroups and merges the
  * partial results (same O and lse to rounding).  Without it the call runs unsplit.  The query reads the sizes, causal,
  * has_window, softcap, p_drop, the strides of q, and whether bias, seqlens and kv_lens are given: fa2_fwd decides by the same
- * fields, so the answer for a block that lacks one of them may be that of another plan. */
+ * fields, so the answer for a block that lacks one of them may be that of another plan.  It is never more than 128 MiB. */
 size_t fa2_fwd_scratch_bytes(const fa2_params* p);
 
 /* dq, dk, dv from (q, k, v, o, lse, dO).  Replaces the `_attn_bwd_preprocess`

@@ -282,6 +282,17 @@ static bool fwd_pack_gqa(const fa2_params* p) {
 	return p->Hkv > 0 && p->Hq % p->Hkv == 0 && p->Hq > p->Hkv && (long)(p->Hq / p->Hkv) * p->Sq <= 64;
 }
 
+// The most scratch a forward asks for.  It binds the ranges of grids of 128-row workgroups that are more than half full over very many keys
+// (0.2 % of shapes spread over the logarithm of their sizes; 1 % longer on average there, 4 % at most by the plan's own estimate).
+constexpr size_t kFwdScratchMax = 128u << 20;
+
+// Scratch of fwd_decode_kernel for this many waves: the pieces (at most one per wave and one more per (batch, kv-head)), O and lse of a
+// unit's rows; where they are, per unit.
+static size_t fwd_decode_scratch(const fa2_params* p, int64_t waves) {
+	const size_t units = (size_t)p->B * (size_t)p->Hkv, rows = ((size_t)waves + units) * (size_t)(p->Hq / p->Hkv) * (size_t)p->Sq;
+	return (rows * ((size_t)p->D + 1) * sizeof(float) + units * 8 + 255) & ~(size_t)255;
+}
+
 // Few query rows in all, nothing but masks by position and key lengths: fwd_decode_kernel.  Returns the number of waves that
 // share the key tiles (0 = not this kernel); *whole: one (batch, kv-head) per wave, no scratch.
 static int fwd_decode_waves(const fa2_params* p, int* whole) {
@@ -321,10 +332,10 @@ static int fwd_decode_waves(const fa2_params* p, int* whole) {
 	idle = (idle > 0 ? idle : 0) + (p->kv_lens ? 0.25 : 0.0);
 	int64_t waves = resident < total ? resident : total;
 	const double merge = 3.4 + (p->kv_lens ? 3.7 : 0.0) + (waves + (units < waves ? units : waves)) * rows * p->D * 8 / 3.1e6;
-	*whole = idle * tiles < merge;
-	if (*whole) return (int)units;
 	// as many waves as are resident at once, down to a tile each (B1 Hkv8 Sk1029: 8.5 us, two tiles each 10.0), at most 63 a unit
-	return (int)(waves < 63 * units ? waves : 63 * units);
+	if (waves > 63 * units) waves = 63 * units;
+	*whole = idle * tiles < merge || fwd_decode_scratch(p, waves) > kFwdScratchMax;
+	return (int)(*whole ? units : waves);
 }
 
 static int fwd_split_plan(const fa2_params* p, int* split_len, int* tall) {
@@ -347,7 +358,8 @@ static int fwd_split_plan(const fa2_params* p, int* split_len, int* tall) {
 		const double part_us = (double)p->B * p->Hq * p->Sq * p->D * 8 / 2.8e6 * (mean / tiles);
 		int best = 1;
 		double best_us = tiles * (base <= 256 ? tile_us : (1.46 + (base - 256) / 256.0 * 0.7) * (even ? 1.0 : 0.6));
-		for (int n = 2; n <= 16 && n <= tiles / 2; ++n) {
+		const size_t range_bytes = (size_t)p->B * (size_t)p->Hq * (size_t)p->Sq * ((size_t)p->D + 1) * sizeof(float);
+		for (int n = 2; n <= 16 && n <= tiles / 2 && n * range_bytes <= kFwdScratchMax; ++n) {
 			const int64_t rounds = (base * n + 255) / 256;
 			const double us = rounds * ((tiles + n - 1) / n) * (even || rounds == 1 ? 1.0 : 0.85) * tile_us + 3 + n * part_us;
 			if (us < best_us) {
@@ -384,12 +396,7 @@ static size_t fwd_scratch_bytes(const fa2_params* p) {
 	if (p->has_window || p->softcap > 0.f) return 0;
 	int len;
 	int whole;
-	if (int waves = fwd_decode_waves(p, &whole)) {
-		if (whole) return 0;
-		// the pieces (at most one per wave and one more per (batch, kv-head)): O and lse of a unit's rows; where they are, per unit
-		const size_t units = (size_t)p->B * (size_t)p->Hkv, rows = (waves + units) * (size_t)(p->Hq / p->Hkv) * (size_t)p->Sq;
-		return (rows * ((size_t)p->D + 1) * sizeof(float) + units * 8 + 255) & ~(size_t)255;
-	}
+	if (int waves = fwd_decode_waves(p, &whole)) return whole ? 0 : fwd_decode_scratch(p, waves);
 	int tall, n = fwd_split_plan(p, &len, &tall);
 	if (n <= 1) return 0;
 	size_t rows = (size_t)n * (size_t)p->B * (size_t)p->Hq * (size_t)p->Sq;

@@ -3,7 +3,9 @@ include/fa2.h declares, the ctypes mirror of fa2_params has the C layout, and
 argument validation returns the documented codes.  No kernel is launched."""
 
 import ctypes
+import math
 import os
+import random
 import re
 import subprocess
 import sys
@@ -275,3 +277,21 @@ def test_decoding_takes_whole_units_or_equal_shares():
 	# many rows make the pieces expensive; at head dim 128 a few hundred keys under many rows take the general kernel, unsplit
 	assert need(64, 1000, 64, rows=16) == 0 and need(64, 2048, 64) > 0
 	assert need(40, 300, 128, rows=16) == 0
+
+
+def test_forward_scratch_is_bounded():
+	"""fa2_fwd_scratch_bytes never asks for more than 128 MiB, whatever the sizes."""
+	lib, rng = _lib.load(), random.Random(11)
+	log = lambda lo, hi: int(round(math.exp(rng.uniform(math.log(lo), math.log(hi)))))
+	most = 0
+	for _ in range(20000):
+		p = _lib.new_params()
+		p.Hkv = rng.choice([1, 2, 4, 8, 16])
+		p.B, p.Hq, p.Sq, p.Sk, p.D = log(1, 4096), p.Hkv * rng.choice([1, 1, 2, 4, 8]), rng.choice([1, log(1, 16), log(1, 8192)]), log(64, 200000), rng.choice([64, 128, 256])
+		p.causal, p.bias, p.kv_lens = rng.choice([0, 1]), rng.choice([None, None, 256]), rng.choice([None, 256])
+		most = max(most, lib.fa2_fwd_scratch_bytes(ctypes.byref(p)))
+	for B, Hq, Hkv, Sq, Sk, D in ((1, 16, 16, 2123, 119339, 128), (2200, 128, 8, 1, 100000, 256)):
+		p = _lib.new_params()
+		p.B, p.Hq, p.Hkv, p.Sq, p.Sk, p.D = B, Hq, Hkv, Sq, Sk, D
+		most = max(most, lib.fa2_fwd_scratch_bytes(ctypes.byref(p)))
+	assert 64 << 20 < most <= 128 << 20
