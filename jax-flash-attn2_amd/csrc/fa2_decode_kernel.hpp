@@ -267,7 +267,7 @@ __global__ __launch_bounds__(DecodeCfg<D>::NW * 64) void fwd_decode_kernel(const
 			float* rp = a.o_part + prow * D + 4 * g;
 #pragma unroll
 			for (int db = 0; db < DB; ++db) *(f32x4*)(rp + 16 * db) = f32x4{oacc[db][0] * inv, oacc[db][1] * inv, oacc[db][2] * inv, oacc[db][3] * inv};
-			if (g == 0) a.lse_part[prow] = l >= 0.f ? lse : l;  // (a NaN sum stays NaN: the combine kernel's weight of the piece)
+			if (g == 0) a.lse_part[prow] = l >= 0.f ? lse : INFINITY;  // (NaN: a weight of inf - inf in the combine kernel)
 		}
 	};
 
@@ -381,17 +381,17 @@ __global__ __launch_bounds__(256) void fwd_decode_combine_kernel(const KArgs a) 
 	tot = 0.f;
 #pragma unroll
 	for (int e = 0; e < 8; ++e) acc[e] = 0.f;
-	// (all groups, also those without a maximum: their sums are 0, or NaN)
-	const float ref = m > -INFINITY ? m : 0.f;
+	if (m > -INFINITY) {
 #pragma unroll
-	for (int x = 0; x < G; ++x) {
-		const float wgt = exp2_fast((smax[slot][x] - ref) * kLog2e);
-		tot += wgt * stot[slot][x];
-		f32x4 x0 = *(const f32x4*)&sacc[slot][x][part * 8], x1 = *(const f32x4*)&sacc[slot][x][part * 8 + 4];
+		for (int x = 0; x < G; ++x) {
+			const float wgt = exp2_fast((smax[slot][x] - m) * kLog2e);
+			tot += wgt * stot[slot][x];
+			f32x4 x0 = *(const f32x4*)&sacc[slot][x][part * 8], x1 = *(const f32x4*)&sacc[slot][x][part * 8 + 4];
 #pragma unroll
-		for (int e = 0; e < 4; ++e) {
-			acc[e] += wgt * x0[e];
-			acc[4 + e] += wgt * x1[e];
+			for (int e = 0; e < 4; ++e) {
+				acc[e] += wgt * x0[e];
+				acc[4 + e] += wgt * x1[e];
+			}
 		}
 	}
 	const int h = hk * r + n / a.Sq, i = n % a.Sq;

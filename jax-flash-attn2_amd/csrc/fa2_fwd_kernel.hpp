@@ -1059,7 +1059,8 @@ __global__ __launch_bounds__(NW * 64 * KW, WPS) void fwd_kernel(const KArgs a) {
 			if (i < a.Sq) {
 				int64_t row = (((int64_t)split * a.B + b) * a.Hq + hl[qb]) * a.Sq + i;
 				float* rp = a.o_part + row * D;
-				// (a row without keys in this range leaves its -inf only, one whose sum is NaN its NaN: the combine kernel does not look at its O)
+				// (a row without keys in this range leaves its -inf only: the combine kernel does not look at its O; one whose sum is
+				// NaN leaves +inf, against which its own weight is inf - inf, and with that the row is NaN)
 				for (int db = 0; db < DB && lt > 0.f; ++db)
 #pragma unroll
 					for (int aa = 0; aa < 4; ++aa) {
@@ -1068,7 +1069,7 @@ __global__ __launch_bounds__(NW * 64 * KW, WPS) void fwd_kernel(const KArgs a) {
 						*(f32x4*)(rp + 32 * db + 8 * aa + 4 * g) = o4;
 					}
 				if (g == 0) {
-					float lse = lt == 0.f ? -INFINITY : lt;
+					float lse = lt == 0.f ? -INFINITY : INFINITY;
 					if (lt > 0.f) lse = BIAS ? mrow[qb] + log2_fast(lt) * kLn2 : (mrow[qb] * c1 + log2_fast(lt)) * kLn2;
 					a.lse_part[row] = lse;
 				}
@@ -1117,8 +1118,7 @@ __global__ __launch_bounds__(256) void fwd_combine_kernel(const KArgs a) {
 	float m = -INFINITY, tot = 0.f;
 	float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 	if (live) {
-		// four ranges at a time, so that their loads are on their way together; of a range without keys for the row only lse is there,
-		// and of one whose sum is NaN (its weight, and with that the row, becomes NaN)
+		// four ranges at a time, so that their loads are on their way together; of a range without keys for the row only lse is there
 		for (int s0 = g; s0 < a.nsplit; s0 += 4 * G) {
 			float lse[4];
 			f32x4 x0[4], x1[4];
@@ -1166,17 +1166,17 @@ __global__ __launch_bounds__(256) void fwd_combine_kernel(const KArgs a) {
 		tot = 0.f;
 #pragma unroll
 		for (int e = 0; e < 8; ++e) acc[e] = 0.f;
-		// (all groups, also those without a maximum: their sums are 0, or NaN)
-		const float ref = m > -INFINITY ? m : 0.f;
+		if (m > -INFINITY) {
 #pragma unroll
-		for (int x = 0; x < G; ++x) {
-			const float wgt = exp2_fast((smax[slot][x] - ref) * kLog2e);
-			tot += wgt * stot[slot][x];
-			f32x4 x0 = *(const f32x4*)&sacc[slot][x][part * 8], x1 = *(const f32x4*)&sacc[slot][x][part * 8 + 4];
+			for (int x = 0; x < G; ++x) {
+				const float wgt = exp2_fast((smax[slot][x] - m) * kLog2e);
+				tot += wgt * stot[slot][x];
+				f32x4 x0 = *(const f32x4*)&sacc[slot][x][part * 8], x1 = *(const f32x4*)&sacc[slot][x][part * 8 + 4];
 #pragma unroll
-			for (int e = 0; e < 4; ++e) {
-				acc[e] += wgt * x0[e];
-				acc[4 + e] += wgt * x1[e];
+				for (int e = 0; e < 4; ++e) {
+					acc[e] += wgt * x0[e];
+					acc[4 + e] += wgt * x1[e];
+				}
 			}
 		}
 	}
