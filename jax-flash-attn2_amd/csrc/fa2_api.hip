@@ -346,18 +346,22 @@ static int fwd_split_plan(const fa2_params* p, int* split_len, int* tall) {
 		// rounds of the longest workgroup (less where a causal mask makes them unequal and they even out over
 		// several rounds), plus 3 us for the second launch and the partial results written and read.  Figures measured: a tile
 		// takes such a workgroup 1.07 us (0.8 at D = 64), partial results move at 2.8 TB/s; without ranges and with more than 256 workgroups
-		// the 128-row kernel runs two workgroups a CU and needs 1.46 to 2.2 us a tile.  B1 Hq32 Hkv8 D128, 100 rows over
+		// the 128-row kernel runs two workgroups a CU and needs 1.46 to 2.2 us a tile (1.05 to 1.8 at D = 64).  B1 Hq32 Hkv8 D128, 100 rows over
 		// 4000 keys: 71 us in one range, 44 in 2, 30 in 4, 24 in 8, 35 in 12 (16 ranges of the 64-row kernel: 36); B1 H4 S4096 D128
-		// causal: 61 / 42 / 54 us in 1 / 2 / 4; B2 Hq16 300 rows over 3000 keys: 55 / 36 / 44 us in 1 / 2 / 4.
+		// causal: 61 / 42 / 54 us in 1 / 2 / 4; B2 Hq16 300 rows over 3000 keys: 55 / 36 / 44 us in 1 / 2 / 4; B2 H12 D64, 2048 rows over
+		// 3048 keys (384 workgroups): 63 / 72 / 89 in 1 / 2 / 4.  Multi-head queries of 17 to 64 rows, half a workgroup or less, are here too:
+		// against the 64-row kernel's ranges B1 H8 D128 64 rows over 16384 keys 52 -> 25 us, B8 H16 32 rows over 4096 57 -> 49.
 		const int64_t base = (int64_t)p->B * p->Hq * ((p->Sq + 127) / 128);
 		if (base >= 512) return 1;
 		const int tiles = (p->Sk + 63) / 64;
+		// (eight tiles of D = 64 are too little for a second launch: B1 H8, 64 rows over 512 keys 10.3 us in one range, 10.9 in 2, 11.7 in 4)
+		if (p->D == 64 && tiles <= 8) return 1;
 		const double mean = p->causal && p->Sq <= p->Sk ? (p->Sk - 0.5 * p->Sq) / 64 : tiles;
 		const bool even = mean > 0.75 * tiles;
 		const double tile_us = p->D == 64 ? 0.8 : 1.07;
 		const double part_us = (double)p->B * p->Hq * p->Sq * p->D * 8 / 2.8e6 * (mean / tiles);
 		int best = 1;
-		double best_us = tiles * (base <= 256 ? tile_us : (1.46 + (base - 256) / 256.0 * 0.7) * (even ? 1.0 : 0.6));
+		double best_us = tiles * (base <= 256 ? tile_us : ((p->D == 64 ? 1.05 : 1.46) + (base - 256) / 256.0 * 0.7) * (even ? 1.0 : 0.6));
 		const size_t range_bytes = (size_t)p->B * (size_t)p->Hq * (size_t)p->Sq * ((size_t)p->D + 1) * sizeof(float);
 		for (int n = 2; n <= 16 && n <= tiles / 2 && n * range_bytes <= kFwdScratchMax; ++n) {
 			const int64_t rounds = (base * n + 255) / 256;

@@ -196,6 +196,8 @@ def test_forward_scratch_only_for_small_grids_over_many_keys():
 	assert need(1, 1024, 1024, 16, 64) == 0      # 256 row tiles over 16 key tiles: the same
 	assert need(1, 2048, 2048, 8, 64) > 0        # 256 row tiles over 32 key tiles: split
 	assert need(1, 1024, 1024, 8, 64) > 0        # 128 row tiles over 16 key tiles: split
+	assert need(1, 64, 512, 8, 64) == 0 and need(1, 64, 704, 8, 64) > 0  # head dim 64: eight key tiles are too few, eleven are not
+	assert need(2, 2048, 3048, 12, 64) == 0      # 384 workgroups of 128 rows: two a CU are faster than ranges
 
 
 def test_backward_split_scratch_only_on_small_grids():
