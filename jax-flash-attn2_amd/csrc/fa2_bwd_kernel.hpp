@@ -190,7 +190,8 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 	// last has one row: forward and backward 389 -> 371 us; B32 H12 D64 of 256 to 511 tokens 193 -> 190.)
 	constexpr bool SHARES = KV_AGPR && !WALKS && NW == 4 && QB == 4;
 	const int blocks = (sk_eff - n0 + 31) >> 5;  // 32-key blocks with a valid key
-	const int share = SHARES && blocks == 1 ? 4 : (SHARES && blocks == 2 ? 2 : 1);
+	// (not where the other waves' part of the rows is empty: B1 H8 S33 D128 backward 17.9 us shared, 15.4 not)
+	const int share = SHARES && blocks == 1 && sq_eff > BMQ / 4 ? 4 : (SHARES && blocks == 2 && sq_eff > BMQ / 2 ? 2 : 1);
 	const int kblk = w & (4 / share - 1), rgrp = w / (4 / share);  // this wave's block of keys, its share of the rows
 	const int row0 = rgrp * (BMQ / share);                         // first row of that in a streamed tile
 	const int wn0 = n0 + 32 * kblk;

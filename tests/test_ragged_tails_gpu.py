@@ -25,6 +25,10 @@ pytestmark = pytest.mark.gpu
 		(200, 384, 1, 1, False, [130, 300], None),   # lengths that end in the second tile: keys beyond them get zeros
 		(384, 384, 1, 1, True, [5, 384], None),
 		(420, 420, 2, 2, True, None, (70, 0)),
+		(33, 33, 2, 2, False, None, None),     # keys that waves would share, but only the first of them has rows; one row more
+		(64, 64, 2, 1, True, None, None),
+		(32, 20, 1, 1, False, None, None),
+		(33, 20, 2, 1, False, None, None),
 		(2100, 40, 16, 1, False, None, None),  # the steps of the one key tile split over workgroups
 	],
 )
