@@ -275,8 +275,6 @@ size_t fa2_bwd_split_scratch_bytes(const fa2_params* p) {
 	return hs > 1 ? base + bwd_split_part_bytes(p, hs) : 0;
 }
 
-// Key ranges for a split forward: few query rows (one row tile of 64), too few (batch, head)
-// pairs to fill the chip, many keys.  Returns the number of ranges (1 = no split).
 // the rows of all q-heads of a kv-head fit one row tile: they share one workgroup (and one pass over K, V)
 static bool fwd_pack_gqa(const fa2_params* p) {
 	return p->Hkv > 0 && p->Hq % p->Hkv == 0 && p->Hq > p->Hkv && (long)(p->Hq / p->Hkv) * p->Sq <= 64;
@@ -338,6 +336,8 @@ static int fwd_decode_waves(const fa2_params* p, int* whole) {
 	return (int)(*whole ? units : waves);
 }
 
+// Key ranges for a split forward: too few workgroups to fill the chip, many keys.  Returns the number of ranges (1 = no split) of
+// *split_len keys; *tall: in workgroups of 128 rows.
 static int fwd_split_plan(const fa2_params* p, int* split_len, int* tall) {
 	*split_len = 0;
 	*tall = 0;

@@ -7,8 +7,8 @@
 // over the chip, leave nobody waiting.  A wave streams its share through LDS tiles of its own, the next tile always on its
 // way, across the ends of units too; there is no barrier in the kernel.  Four waves keep 64 KiB a CU in flight (a plain read of
 // 150 MiB: 3.6 TB/s with 16 KiB a CU, 5.0 with 32, 5.5 with 64).  A unit that lies inside one share is stored directly, the
-// pieces of the others go through scratch to fwd_decode_combine_kernel (about 4.5 us: where a unit has few tiles, or there are
-// plenty of units, every unit is one wave's and there is no second launch).
+// pieces of the others go through scratch to fwd_decode_combine_kernel (3.4 us and more: where whole
+// units leave little of the last round of waves idle, every unit is one wave's and there is no second launch, see fwd_decode_waves()).
 // Measured against the split of fwd_kernel that these shapes took before (Hkv 8, D 128, half to all of the slots filled): B8 Hq32
 // Sk8192 57 -> 44 us (201 MB: 5.3 TB/s without the combine), B64 Hq16 Sk8000 630 -> 274 us (5.7 TB/s), B2 Hq64 Sk16000 58 -> 27 us,
 // B1 Hq32 Sk1029 16.4 -> 8.5 us.

@@ -1214,7 +1214,6 @@ struct FwdCfg {
 	static constexpr int BM = NW * QB * 32;
 };
 
-// Split forward: 2 waves x 32 rows per workgroup (the query is short), nsplit key ranges each.
 // Split forward of a longer query on a small grid: the 128-row workgroups of eight waves of launch_fwd_t, nsplit key ranges each.
 template <typename T, int D>
 hipError_t launch_fwd_tall_split_t(KArgs& a, hipStream_t s) {
@@ -1225,6 +1224,7 @@ hipError_t launch_fwd_tall_split_t(KArgs& a, hipStream_t s) {
 	return launch_fwd_combine_t<T, D>(a, s);
 }
 
+// Split forward of a short query, or with bias or dropout: 2 waves x 32 rows per workgroup, nsplit key ranges each.
 template <typename T, int D>
 hipError_t launch_fwd_split_t(bool bias, bool drop, KArgs& a, hipStream_t s) {
 	constexpr int NW = D == 256 ? 4 : 2, BM = NW * 32;  // (D = 256: four waves, the tile copies need the threads)
