@@ -32,9 +32,10 @@ _BIAS_DTYPES = {torch.float16: FA2_FP16, torch.bfloat16: FA2_BF16, torch.float32
 
 def _stream_ptr(device) -> int:
 	# (what torch.cuda.current_stream(device).cuda_stream gives, without building the stream object)
-	if device.type != "cuda":
+	index = device.index
+	if index is None:  # (a tensor in host memory)
 		raise ValueError(f"Expected a cuda device, but got: {device}")
-	return torch._C._cuda_getCurrentRawStream(device.index)
+	return torch._C._cuda_getCurrentRawStream(index)
 
 
 _NONE4 = (0, 0, 0, 0)  # an absent tensor
@@ -179,7 +180,10 @@ def fwd(q, k, v, bias=None, seqlens=None, softmax_scale=None, dropout_prob=0.0, 
 	scale = 1.0 / math.sqrt(D0) if softmax_scale is None else softmax_scale
 	call = (bias, seqlens, scale, dropout_prob, causal, dropout_seed, kv_lens, window, softcap)
 	rows = D0 if D0 != D and _runs_unpadded(lib, 0, D, q, k, v, *call) else D  # columns of the rows the library is given
-	q, k, v = (_usable(_pad_d(x, D)) if rows == D else _usable_short(x) for x in (q, k, v))
+	if rows == D:
+		q, k, v = _usable(_pad_d(q, D)), _usable(_pad_d(k, D)), _usable(_pad_d(v, D))
+	else:
+		q, k, v = _usable_short(q), _usable_short(k), _usable_short(v)
 	out = torch.empty_like(q, memory_format=torch.contiguous_format)
 	lse = torch.empty((q.shape[0], q.shape[2], q.shape[1]), dtype=torch.float32, device=q.device)
 	p = _block(D, q, k, v, *call, _t4(out), lse)
