@@ -341,7 +341,25 @@ static int fwd_decode_waves(const fa2_params* p, int* whole) {
 static int fwd_split_plan(const fa2_params* p, int* split_len, int* tall) {
 	*split_len = 0;
 	*tall = 0;
-	if (p->D <= 128 && !p->bias && !(p->p_drop > 0.f) && !fwd_pack_gqa(p)) {
+	const int tiles = (p->Sk + 63) / 64;
+	// Up to 64 rows a q-head fill half of a 128-row workgroup at most.  Over many keys the two-wave workgroups of the 64-row kernel, four of them a
+	// CU, have more of the memory's and the chip's time, and ranges beyond a row's length cost them little (here and in 128 rows): D64 B18 H8,
+	// 19 rows over 1880 keys 22 and 34 us, B8 Hq16 Hkv4, 60 over 14088 64 and 101; D128 B1 H4, 39 over 15090 17.4 and 26.1, with lengths
+	// B3 Hq64 Hkv32, 62 over 10371 134 and 180; but D128 B12 H1, 55 over 15914 without lengths 58 and 31.  Over 700 calls the
+	// rule is 0.8 % (D64) and 0.5 % (D128) from the better of the two on average; always 128 rows 10.7 and 1.9, always 64 rows 2.6 and 11.8.
+	// Above 256 workgroups of 128 rows the alternative is the unsplit kernel, at D128 over K / V beyond an XCD's L2 in workgroups of 256 rows
+	// (B18 Hq16 Hkv8, 55 over 5126: 139 and 232 us), and an odd number of 64-row tiles can leave fewer than 512 of these (D64 B17 H8, 176 over
+	// 5979 with lengths: 68 and 112; unsplit up to 64 % longer and never shorter in the 14 such calls of 500).
+	const int64_t heads = (int64_t)p->B * p->Hq, wide = heads * ((p->Sq + 127) / 128), narrow = heads * ((p->Sq + 63) / 64);
+	bool few_rows;
+	if (p->Sq > 64)
+		few_rows = p->D == 64 && tiles >= 32 && wide > 256 && narrow < 512;
+	else if (p->D == 64)
+		few_rows = tiles >= (heads < 32 ? 64 : heads < 64 ? 24 : 16);
+	else
+		few_rows = (tiles >= 128 && heads < 16) || (p->kv_lens && tiles >= 48 && heads >= 32) ||
+		           (heads > 256 && (int64_t)p->Sk * p->D * 4 > (p->causal ? 4 << 20 : 2 << 20));
+	if (p->D <= 128 && !p->bias && !(p->p_drop > 0.f) && !fwd_pack_gqa(p) && !few_rows) {
 		// Workgroups of 128 rows whose eight waves share the keys, one per CU: as many key ranges as make the estimate smallest - whole
 		// rounds of the longest workgroup (less where a causal mask makes them unequal and they even out over
 		// several rounds), plus 3 us for the second launch and the partial results written and read.  Figures measured: a tile
@@ -349,11 +367,9 @@ static int fwd_split_plan(const fa2_params* p, int* split_len, int* tall) {
 		// the 128-row kernel runs two workgroups a CU and needs 1.46 to 2.2 us a tile (1.05 to 1.8 at D = 64).  B1 Hq32 Hkv8 D128, 100 rows over
 		// 4000 keys: 71 us in one range, 44 in 2, 30 in 4, 24 in 8, 35 in 12 (16 ranges of the 64-row kernel: 36); B1 H4 S4096 D128
 		// causal: 61 / 42 / 54 us in 1 / 2 / 4; B2 Hq16 300 rows over 3000 keys: 55 / 36 / 44 us in 1 / 2 / 4; B2 H12 D64, 2048 rows over
-		// 3048 keys (384 workgroups): 63 / 72 / 89 in 1 / 2 / 4.  Multi-head queries of 17 to 64 rows, half a workgroup or less, are here too:
-		// against the 64-row kernel's ranges B1 H8 D128 64 rows over 16384 keys 52 -> 25 us, B8 H16 32 rows over 4096 57 -> 49.
-		const int64_t base = (int64_t)p->B * p->Hq * ((p->Sq + 127) / 128);
+		// 3048 keys (384 workgroups): 63 / 72 / 89 in 1 / 2 / 4.
+		const int64_t base = wide;
 		if (base >= 512) return 1;
-		const int tiles = (p->Sk + 63) / 64;
 		// (eight tiles of D = 64 are too little for a second launch: B1 H8, 64 rows over 512 keys 10.3 us in one range, 10.9 in 2, 11.7 in 4)
 		if (p->D == 64 && tiles <= 8) return 1;
 		const double mean = p->causal && p->Sq <= p->Sk ? (p->Sk - 0.5 * p->Sq) / 64 : tiles;
@@ -377,8 +393,7 @@ static int fwd_split_plan(const fa2_params* p, int* split_len, int* tall) {
 		return (tiles + per - 1) / per;
 	}
 	// workgroups of an unsplit launch of this kernel variant (row tiles of 64)
-	long base = fwd_pack_gqa(p) ? (long)p->B * p->Hkv : (long)p->B * p->Hq * ((p->Sq + 63) / 64);
-	int tiles = (p->Sk + 63) / 64;
+	long base = fwd_pack_gqa(p) ? (long)p->B * p->Hkv : (long)narrow;
 	// A query longer than one row tile (with bias or dropout, or at D = 256) runs unsplit on the 128-row kernel, which a quarter of the
 	// chip's worth of units already keeps busy over a short key range: the second launch pays from 16 key tiles on up to 128 units
 	// and from 32 above.

@@ -281,6 +281,26 @@ def test_decoding_takes_whole_units_or_equal_shares():
 	assert need(40, 300, 128, rows=16) == 0
 
 
+def test_ranges_of_few_rows_by_the_better_of_two_kernels():
+	"""Queries of up to 64 rows a q-head that share no keys: the 64-row kernel cuts the keys into up to 64 ranges of at least four tiles (1024
+	workgroups in all), the workgroups of 128 rows into 16 at most - recognised by their number."""
+	lib = _lib.load()
+
+	def ranges(B, Sq, Sk, H, D, lens=False):
+		p = _lib.new_params()
+		p.B, p.Sq, p.Sk, p.Hq, p.Hkv, p.D = B, Sq, Sk, H, H, D
+		p.kv_lens = 256 if lens else None
+		return lib.fa2_fwd_scratch_bytes(ctypes.byref(p)) // (B * Sq * H * (D + 1) * 4)
+
+	assert ranges(1, 40, 9000, 4, 64) > 16 >= ranges(1, 65, 9000, 4, 64)               # head dim 64, up to 64 rows
+	assert ranges(12, 60, 9000, 4, 64) == 21 and ranges(18, 19, 1880, 8, 64) == 6      # 48 and 144 heads
+	assert ranges(1, 39, 15090, 4, 128) > 16 >= ranges(1, 39, 8000, 4, 128) > 1        # head dim 128: few heads over very many keys
+	assert ranges(12, 55, 15914, 1, 128) > 16 >= ranges(16, 55, 15914, 1, 128)
+	assert ranges(4, 62, 10371, 8, 128, lens=True) > 16 >= ranges(4, 62, 10371, 8, 128)   # or rows of different length
+	assert ranges(18, 55, 5126, 16, 128) == 4 and ranges(18, 55, 4096, 16, 128) == 0   # 288 heads: unsplit, and in half empty workgroups of 256 rows
+	assert ranges(17, 176, 5979, 8, 64) == 3 and ranges(17, 200, 5979, 8, 64) == 0     # three 64-row tiles a head, and four
+
+
 def test_forward_scratch_is_bounded():
 	"""fa2_fwd_scratch_bytes never asks for more than 128 MiB, whatever the sizes."""
 	lib, rng = _lib.load(), random.Random(11)

@@ -29,6 +29,11 @@ pytestmark = pytest.mark.gpu
 		(1, 1030, 1030, 2, 1, 64, torch.float16, True, None, None, 0.0, False),
 		(2, 150, 1500, 4, 4, 128, torch.float16, False, [40, 1500], None, 0.0, False),
 		(1, 17, 1100, 4, 4, 64, torch.bfloat16, True, None, None, 0.0, False),
+		# up to 64 rows over many keys: ranges of the 64-row kernel (head dim 64; head dim 128 with few heads, and with lengths)
+		(1, 40, 4200, 4, 4, 64, torch.bfloat16, True, None, None, 0.0, False),
+		(2, 64, 1100, 32, 32, 64, torch.float16, False, [1100, 30], None, 0.0, False),
+		(1, 33, 8200, 2, 2, 128, torch.bfloat16, True, None, None, 0.0, False),
+		(4, 20, 3100, 8, 8, 128, torch.float16, False, [3100, 0, 1, 2000], None, 0.0, False),
 	],
 )
 def test_groups_and_ranges_of_keys(B, Sq, Sk, Hq, Hkv, D, dtype, causal, lens, window, p, bias):
