@@ -184,28 +184,6 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 	const int r = a.Hq / a.Hkv;
 	const int sq_eff = rw.sq_eff, sk_eff = rw.sk_eff, off = rw.off;
 	const int n0 = nt * BN;
-	// A key tile that ends within its first or second 32 keys would leave three or two waves without work for as long as a full tile
-	// takes: there all four waves take the same one or two blocks of keys, each a quarter or a half of every streamed tile's rows, and
-	// their dK / dV are summed at the end.  (B64 S257 H16 D80 - three key tiles of which the last has one key, three row tiles of which the
-	// last has one row: forward and backward 389 -> 371 us; B32 H12 D64 of 256 to 511 tokens 193 -> 190.)
-	constexpr bool SHARES = KV_AGPR && !WALKS && NW == 4 && QB == 4;
-	const int blocks = (sk_eff - n0 + 31) >> 5;  // 32-key blocks with a valid key
-	// (not where the other waves' part of the rows is empty: B1 H8 S33 D128 backward 17.9 us shared, 15.4 not)
-	const int share = SHARES && blocks == 1 && sq_eff > BMQ / 4 ? 4 : (SHARES && blocks == 2 && sq_eff > BMQ / 2 ? 2 : 1);
-	const int kblk = w & (4 / share - 1), rgrp = w / (4 / share);  // this wave's block of keys, its share of the rows
-	const int row0 = rgrp * (BMQ / share);                         // first row of that in a streamed tile
-	const int wn0 = n0 + 32 * kblk;
-	const int jcol = wn0 + c;  // this lane's key
-
-	// K, V rows of this lane's key as B operands: lane holds X[jcol][16ks + 8g .. +7]
-	V8 kf[KS], vf[KS];
-	dkdv_load_kv<T, DE, COLS>(a, jcol, hk, b, kf, vf);
-	f32x16 dk[DB], dv[DB];
-#pragma unroll
-	for (int db = 0; db < DB; ++db)
-#pragma unroll
-		for (int i = 0; i < 16; ++i) dk[db][i] = dv[db][i] = 0.f;
-
 	// Row i may look at keys i + off - win_left .. i + off + win_right (each bound only when >= 0; causal is
 	// win_right = 0), so key j is seen by rows j - off - win_right .. j - off + win_left.
 	const int wr = a.win_right, wl = a.win_left;
@@ -222,13 +200,39 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 		q_hi = e < q_hi ? e : q_hi;
 	}
 	if (n0 >= sk_eff) q_hi = q_lo;
+	const int nq = q_hi > q_lo ? q_hi - q_lo : 0;
+	const int steps = nq * r;
+	// A key tile that ends within its first or second 32 keys would leave three or two waves without work for as long as a full tile
+	// takes: there all four waves take the same one or two blocks of keys, each a quarter or a half of every streamed tile's rows, and
+	// their dK / dV are summed at the end.  The sum costs 2 us (5 at head dim 128) and the rows go block by block, so only where the
+	// workgroup has more than four tiles to stream, and rows in more than one share.  Backward, kernels without sharing and with it: B23
+	// Hq64 Hkv16 D64, 580 rows over 3 keys (20 tiles) 225 -> 179 us; B17 H8 D128, 1734 rows over 11 keys (14) 113 -> 94; B3 Hq16 Hkv8
+	// S158 D64 (4) 24.3 -> 22.7; B3 H2 D128, 111 rows over 5 keys (1) 17.2 -> 21.7; B64 H16 S257 D80 (3) 214 -> 219.
+	constexpr bool SHARES = KV_AGPR && !WALKS && NW == 4 && QB == 4;
+	const int blocks = (sk_eff - n0 + 31) >> 5;  // 32-key blocks with a valid key
+	const int first_row = wr >= 0 && n0 - off - wr > 0 ? n0 - off - wr : 0;
+	const bool many = SHARES && steps > 4 * hsplit;
+	const int share = many && blocks == 1 && first_row / (BMQ / 4) < (sq_eff - 1) / (BMQ / 4) ? 4
+	                : many && blocks == 2 && first_row / (BMQ / 2) < (sq_eff - 1) / (BMQ / 2) ? 2 : 1;
+	const int kblk = w & (4 / share - 1), rgrp = w / (4 / share);  // this wave's block of keys, its share of the rows
+	const int row0 = rgrp * (BMQ / share);                         // first row of that in a streamed tile
+	const int wn0 = n0 + 32 * kblk;
+	const int jcol = wn0 + c;  // this lane's key
+
+	// K, V rows of this lane's key as B operands: lane holds X[jcol][16ks + 8g .. +7]
+	V8 kf[KS], vf[KS];
+	dkdv_load_kv<T, DE, COLS>(a, jcol, hk, b, kf, vf);
+	f32x16 dk[DB], dv[DB];
+#pragma unroll
+	for (int db = 0; db < DB; ++db)
+#pragma unroll
+		for (int i = 0; i < 16; ++i) dk[db][i] = dv[db][i] = 0.f;
+
 	// rows that may see this lane's key: row_lo .. row_hi (none when the key itself is beyond the valid ones)
 	int row_lo = wr >= 0 ? jcol - off - wr : -(1 << 30);
 	int row_hi = sq_eff - 1;
 	if (wl >= 0) row_hi = jcol - off + wl < row_hi ? jcol - off + wl : row_hi;
 	if (jcol >= sk_eff) row_lo = 1 << 30;
-	const int nq = q_hi > q_lo ? q_hi - q_lo : 0;
-	const int steps = nq * r;
 	// this workgroup's share of the steps (all of them unless the launch splits the steps of a key tile over `hsplit` workgroups)
 	const int s_lo = hsplit > 1 ? (int)((int64_t)steps * hsi / hsplit) : 0;
 	const int s_hi = hsplit > 1 ? (int)((int64_t)steps * (hsi + 1) / hsplit) : steps;

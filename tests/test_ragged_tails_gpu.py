@@ -30,6 +30,15 @@ pytestmark = pytest.mark.gpu
 		(32, 20, 1, 1, False, None, None),
 		(33, 20, 2, 1, False, None, None),
 		(2100, 40, 16, 1, False, None, None),  # the steps of the one key tile split over workgroups
+		# more than four row tiles (or heads times row tiles): only there do waves share the keys, and only if more than one has rows
+		(641, 257, 1, 1, False, None, None),   # one block of keys
+		(600, 150, 2, 1, True, None, None),
+		(650, 192, 4, 2, False, [192, 140], None),   # two blocks; a row of the batch with one block
+		(769, 35, 1, 1, False, None, (300, 500)),
+		(130, 20, 6, 1, False, None, None),
+		(33, 20, 6, 1, True, None, None),      # rows 13 to 32 see keys: in two shares of 32 rows
+		(33, 1, 6, 1, True, None, None),       # one row does
+		(645, 645, 6, 1, True, None, None),    # five rows and keys in the last tiles
 	],
 )
 def test_ends_of_sequences(Sq, Sk, Hq, Hkv, causal, kv_lens, window, D, dtype):
