@@ -1306,8 +1306,10 @@ hipError_t launch_fwd_t(bool bias, bool drop, KArgs& a, hipStream_t s) {
 			// ... and two groups of four waves that take the key tiles of the workgroup's rows in turn: two waves per SIMD where
 			// there was one (B1 Hq32 Hkv8 D128, 1000 rows over 9000 keys: 233 -> 170 us; B1 H8 S4096 D128 81 -> 71 us, causal 79 -> 61;
 			// B2 H16 S1024 D64 with bias 23.4 -> 20.5; B4 H12 S197 D64 9.3 -> 8.9).  With up to three tiles the merge costs more
-			// than it saves (B1 H8 S128: 8.7 us alone, 10.1 in two groups); four groups spill.
-			if (a.Sk > 3 * kFwdBN && (D == 64 || !bias)) return launch_fwd_cfg<T, D, DE, 4, 1, 2>(bias, drop, a, s);
+			// than it saves (B1 H8 S128: 8.7 us alone, 10.1 in two groups; in a window a row tile sees that few whatever the number of keys:
+			// B26 Hq4 Hkv1 S243 D64, 61 keys a row, 9.2 and 10.1); four groups spill.
+			const int64_t seen = a.win_left >= 0 && a.win_right >= 0 ? (int64_t)a.win_left + a.win_right + 128 : a.Sk;
+			if (a.Sk > 3 * kFwdBN && seen > 3 * kFwdBN && (D == 64 || !bias)) return launch_fwd_cfg<T, D, DE, 4, 1, 2>(bias, drop, a, s);
 			return launch_fwd_cfg<T, D, DE, 4, 1>(bias, drop, a, s);
 		}
 		// Larger grids: two independent 128-row workgroups per CU instead of one of 256 rows - the same eight waves, but

@@ -34,6 +34,9 @@ pytestmark = pytest.mark.gpu
 		(2, 64, 1100, 32, 32, 64, torch.float16, False, [1100, 30], None, 0.0, False),
 		(1, 33, 8200, 2, 2, 128, torch.bfloat16, True, None, None, 0.0, False),
 		(4, 20, 3100, 8, 8, 128, torch.float16, False, [3100, 0, 1, 2000], None, 0.0, False),
+		# a window of which a row tile sees three tiles of keys, and one more
+		(2, 243, 243, 2, 1, 64, torch.bfloat16, True, None, (64, 0), 0.0, False),
+		(2, 243, 243, 2, 1, 64, torch.bfloat16, True, None, (65, 0), 0.0, False),
 	],
 )
 def test_groups_and_ranges_of_keys(B, Sq, Sk, Hq, Hkv, D, dtype, causal, lens, window, p, bias):
