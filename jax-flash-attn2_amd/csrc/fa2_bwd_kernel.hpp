@@ -206,8 +206,8 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 	// takes: there all four waves take the same one or two blocks of keys, each a quarter or a half of every streamed tile's rows, and
 	// their dK / dV are summed at the end.  The sum costs 2 us (5 at head dim 128) and the rows go block by block, so only where the
 	// workgroup has more than four tiles to stream, and rows in more than one share.  Backward, kernels without sharing and with it: B23
-	// Hq64 Hkv16 D64, 580 rows over 3 keys (20 tiles) 225 -> 179 us; B17 H8 D128, 1734 rows over 11 keys (14) 113 -> 94; B3 Hq16 Hkv8
-	// S158 D64 (4) 24.3 -> 22.7; B3 H2 D128, 111 rows over 5 keys (1) 17.2 -> 21.7; B64 H16 S257 D80 (3) 214 -> 219.
+	// Hq64 Hkv16 D64, 580 rows over 3 keys (20 tiles) 225 -> 179 us; B17 H8 D128, 1734 rows over 11 keys (14) 113 -> 94; B3 H8 D64,
+	// 535 rows over 158 keys (5) 24.3 -> 22.7; B3 H2 D128, 111 rows over 5 keys (1) 17.2 -> 21.7; with the forward B64 H16 S257 D80 (3) 348 -> 353.
 	constexpr bool SHARES = KV_AGPR && !WALKS && NW == 4 && QB == 4;
 	const int blocks = (sk_eff - n0 + 31) >> 5;  // 32-key blocks with a valid key
 	const int first_row = wr >= 0 && n0 - off - wr > 0 ? n0 - off - wr : 0;
