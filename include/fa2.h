@@ -181,7 +181,8 @@ int fa2_fwd(const fa2_params* p, void* hip_stream);
 /* Optional scratch for fa2_fwd.  Non-zero for many keys under too few query rows to fill the chip: decoding (`Sq == 1` in
  * flash_attention.py:239-242; up to 16 rows per kv-head, from 257 keys on, where equal shares of the key tiles are
  * estimated to be faster than whole (batch, kv-head) units), and fewer than 512 workgroups of 128 rows - of 64 at D = 256,
- * with bias or dropout, or where the q-heads of a kv-head have no more together - over enough keys for two launches to pay:
+ * with bias or dropout, where the q-heads of a kv-head have no more together, and where these are faster - over enough keys for
+ * two launches to pay:
  * given `scratch` (256-byte aligned) of at least this many bytes, fa2_fwd splits the keys into ranges handled by separate workgroups and merges the
  * partial results (same O and lse to rounding; a row that is NaN in one range is NaN).  Without it the call runs unsplit.  The query reads the sizes, causal,
  * has_window, softcap, p_drop, the strides of q, and whether bias, seqlens and kv_lens are given: fa2_fwd decides by the same
