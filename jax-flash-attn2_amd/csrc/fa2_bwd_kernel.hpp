@@ -205,13 +205,14 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 	// A key tile that ends within its first or second 32 keys would leave three or two waves without work for as long as a full tile
 	// takes: there all four waves take the same one or two blocks of keys, each a quarter or a half of every streamed tile's rows, and
 	// their dK / dV are summed at the end.  The sum costs 2 us (5 at head dim 128) and the rows go block by block, so only where the
-	// workgroup has more than four tiles to stream, and rows in more than one share.  Backward, kernels without sharing and with it: B23
+	// workgroup has more than four tiles to stream (two where every tile goes that way: B32 H12 D64 of 256 to 511 tokens, forward and
+	// backward 155.6 -> 154.2; the two meet at three tiles), and rows in more than one share.  Backward, kernels without sharing and with it: B23
 	// Hq64 Hkv16 D64, 580 rows over 3 keys (20 tiles) 225 -> 179 us; B17 H8 D128, 1734 rows over 11 keys (14) 113 -> 94; B3 H8 D64,
 	// 535 rows over 158 keys (5) 24.3 -> 22.7; B3 H2 D128, 111 rows over 5 keys (1) 17.2 -> 21.7; with the forward B64 H16 S257 D80 (3) 348 -> 353.
 	constexpr bool SHARES = KV_AGPR && !WALKS && NW == 4 && QB == 4;
 	const int blocks = (sk_eff - n0 + 31) >> 5;  // 32-key blocks with a valid key
 	const int first_row = wr >= 0 && n0 - off - wr > 0 ? n0 - off - wr : 0;
-	const bool many = SHARES && steps > 4 * hsplit;
+	const bool many = SHARES && steps > (BLK ? 2 : 4) * hsplit;
 	const int share = many && blocks == 1 && first_row / (BMQ / 4) < (sq_eff - 1) / (BMQ / 4) ? 4
 	                : many && blocks == 2 && first_row / (BMQ / 2) < (sq_eff - 1) / (BMQ / 2) ? 2 : 1;
 	const int kblk = w & (4 / share - 1), rgrp = w / (4 / share);  // this wave's block of keys, its share of the rows
