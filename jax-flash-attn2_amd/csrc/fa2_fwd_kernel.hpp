@@ -1305,11 +1305,14 @@ hipError_t launch_fwd_t(bool bias, bool drop, KArgs& a, hipStream_t s) {
 		if (wgs <= kNumCU) {
 			// ... and two groups of four waves that take the key tiles of the workgroup's rows in turn: two waves per SIMD where
 			// there was one (B1 Hq32 Hkv8 D128, 1000 rows over 9000 keys: 233 -> 170 us; B1 H8 S4096 D128 81 -> 71 us, causal 79 -> 61;
-			// B2 H16 S1024 D64 with bias 23.4 -> 20.5; B4 H12 S197 D64 9.3 -> 8.9).  With up to three tiles the merge costs more
-			// than it saves (B1 H8 S128: 8.7 us alone, 10.1 in two groups; in a window a row tile sees that few whatever the number of keys:
-			// B26 Hq4 Hkv1 S243 D64, 61 keys a row, 9.2 and 10.1); four groups spill.
+			// B2 H16 S1024 D64 with bias 23.4 -> 20.5).  With few tiles the merge costs more than it saves (B1 H8 S128: 8.7 us alone, 10.1 in two
+			// groups): up to three, five at D = 64 and four under a causal mask at D = 128, where it is not dropout or a bias that makes a
+			// tile long.  By tiles, two groups over one, 500 calls: D64 4 / 5 / 6 tiles 1.01 / 1.01 / 0.94, causal 1.06 / 1.00 / 0.98,
+			// dropout 0.97 / 0.96 / 0.92; D128 0.98 / 0.98 / 0.92, causal 1.02 / 0.96 / 0.93.  In a window a row tile sees few tiles whatever
+			// the number of keys (B26 Hq4 Hkv1 S243 D64, 61 keys a row, 9.2 and 10.1).  Four groups spill.
+			const int few = drop || bias ? 3 : D == 64 ? 5 : a.causal ? 4 : 3;
 			const int64_t seen = a.win_left >= 0 && a.win_right >= 0 ? (int64_t)a.win_left + a.win_right + 128 : a.Sk;
-			if (a.Sk > 3 * kFwdBN && seen > 3 * kFwdBN && (D == 64 || !bias)) return launch_fwd_cfg<T, D, DE, 4, 1, 2>(bias, drop, a, s);
+			if (a.Sk > few * kFwdBN && seen > few * kFwdBN && (D == 64 || !bias)) return launch_fwd_cfg<T, D, DE, 4, 1, 2>(bias, drop, a, s);
 			return launch_fwd_cfg<T, D, DE, 4, 1>(bias, drop, a, s);
 		}
 		// Larger grids: two independent 128-row workgroups per CU instead of one of 256 rows - the same eight waves, but

@@ -34,9 +34,15 @@ pytestmark = pytest.mark.gpu
 		(2, 64, 1100, 32, 32, 64, torch.float16, False, [1100, 30], None, 0.0, False),
 		(1, 33, 8200, 2, 2, 128, torch.bfloat16, True, None, None, 0.0, False),
 		(4, 20, 3100, 8, 8, 128, torch.float16, False, [3100, 0, 1, 2000], None, 0.0, False),
-		# a window of which a row tile sees three tiles of keys, and one more
-		(2, 243, 243, 2, 1, 64, torch.bfloat16, True, None, (64, 0), 0.0, False),
-		(2, 243, 243, 2, 1, 64, torch.bfloat16, True, None, (65, 0), 0.0, False),
+		# head dim 64 without bias and dropout: two groups from six tiles on; a window of which a row tile sees five tiles' keys, and one more
+		(2, 320, 320, 2, 2, 64, torch.float16, True, None, None, 0.0, False),
+		(2, 321, 321, 2, 2, 64, torch.float16, True, None, None, 0.0, False),
+		(2, 450, 450, 2, 1, 64, torch.bfloat16, True, None, (192, 0), 0.0, False),
+		(2, 450, 450, 2, 1, 64, torch.bfloat16, True, None, (193, 0), 0.0, False),
+		# head dim 128 under a causal mask: from five tiles on; rows without keys, a window that begins in the middle
+		(1, 500, 256, 2, 2, 128, torch.bfloat16, True, None, None, 0.0, False),
+		(1, 500, 257, 2, 2, 128, torch.bfloat16, True, None, None, 0.0, False),
+		(1, 600, 600, 2, 1, 128, torch.bfloat16, True, None, (200, 0), 0.0, False),
 	],
 )
 def test_groups_and_ranges_of_keys(B, Sq, Sk, Hq, Hkv, D, dtype, causal, lens, window, p, bias):
