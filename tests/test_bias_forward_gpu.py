@@ -1,0 +1,60 @@
+"""The forward whose tiles of bias go through LDS tries a tile without looking at the row maximum first: biases for which that stands, for
+which it fails now and then or on every tile, and references that no exponent may be formed against."""
+
+import numpy as np
+import pytest
+import torch
+
+from jax_flash_attn2 import _hip_op as op
+import fa2_oracle as O
+from _cases import check_forward, f64, make_inputs
+
+pytestmark = pytest.mark.gpu
+
+
+def _bias(kind, dtype, B, H, Sq, Sk):
+	"""[B, H, Sq, Sk] in float64"""
+	i, j = np.arange(Sq)[:, None], np.arange(Sk)[None, :]
+	lowest = torch.finfo(dtype).min
+	if kind == "flat":
+		x = 1.0 / (1.0 + abs(i - j))
+	elif kind == "steep":  # every tile raises the maximum by 32
+		x = 0.5 * (j - i)
+	elif kind == "one late key":  # far above the reference, in a tile that was tried without the maximum
+		x = np.where(j == Sk - 9, 30.0, 0.0) + 0.0 * i
+	elif kind == "first tiles hidden":  # the reference of the first tiles is the lowest finite value
+		x = np.where(j < min(Sk - 8, 150), lowest, 0.5) + 0.0 * i
+	elif kind == "rows hidden":  # uniform over all keys, in half of the rows of a wave; nothing in the other half is hidden
+		x = np.where(i % 2 == 0, lowest, 0.25) + 0.0 * j
+	else:
+		assert kind == "infinite"
+		x = np.where((i + j) % 3 == 0, -np.inf, 0.0)
+	return torch.from_numpy(np.broadcast_to(x, (B, H, Sq, Sk)).copy()).to(dtype)
+
+
+@pytest.mark.parametrize("kind", ["flat", "steep", "one late key", "first tiles hidden", "rows hidden", "infinite"])
+@pytest.mark.parametrize(
+	"B,Sq,Sk,Hq,Hkv,D,dtype,causal,p",
+	[
+		(1, 200, 448, 2, 1, 64, torch.bfloat16, False, 0.0),  # two groups of waves
+		(1, 328, 328, 2, 2, 64, torch.float16, True, 0.1),
+		(300, 40, 136, 1, 1, 64, torch.bfloat16, False, 0.0),  # one group, a last tile of eight keys
+		(1, 130, 264, 2, 2, 128, torch.float16, False, 0.0),
+		(1, 200, 264, 2, 2, 256, torch.bfloat16, True, 0.0),
+		(1, 100, 320, 2, 1, 256, torch.float16, False, 0.2),
+		(1, 8, 1024, 2, 2, 64, torch.bfloat16, False, 0.0),  # several ranges of keys, equal ones (a hidden row weighs them by their number)
+	],
+)
+def test_bias_that_rises_falls_and_hides(B, Sq, Sk, Hq, Hkv, D, dtype, causal, p, kind):
+	q, k, v, _, _ = make_inputs(B, Sq, Sk, Hq, Hkv, D, dtype, seed=Sq + D)
+	bias = _bias(kind, dtype, B, 1, Sq, Sk)
+	if kind == "infinite":
+		bias[..., 1] = 0.0  # (every row keeps a key)
+	o_ref, lse_ref = O.attention_fwd(f64(q), f64(k), f64(v), f64(bias), causal=causal, p_drop=p, seed=5)
+	o, lse = op.fwd(q.cuda(), k.cuda(), v.cuda(), bias.cuda(), dropout_prob=p, causal=causal, dropout_seed=5)
+	if kind == "rows hidden":  # (their logsumexp is the lowest finite value in the 24 bits of fp32: -3.39e38 to a part in 1e7)
+		hidden = lse_ref < -6e4
+		assert np.allclose(lse.float().cpu().numpy()[hidden], lse_ref[hidden], rtol=1e-6)
+		lse_ref = np.where(hidden, 0.0, lse_ref)
+		lse = torch.where(torch.from_numpy(hidden).cuda(), torch.zeros_like(lse), lse)
+	check_forward(o, lse, o_ref, lse_ref, dtype, f"{kind} B{B} Sq{Sq} Sk{Sk} D{D} causal={causal} p={p}")
