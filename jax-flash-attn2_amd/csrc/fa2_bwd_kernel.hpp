@@ -147,6 +147,9 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 	// dS = P * (dP accumulator).  The factor c1 = scale * log2(e) is applied to the fp32
 	// accumulator, as the reference scales the fp32 result of its dot (_backward_triton.py:554-559).
 	constexpr bool FOLD = KV_AGPR;
+	// (of the 256 registers of two waves per SIMD the compiler gives each file half: at 96 columns the accumulators and four of the six
+	// 16-column fragments of K and of V fill the 128 accumulation registers, the other two of each are in vector registers)
+	constexpr int KSA = BLK && 2 * KS * 4 + 2 * DB * 16 > 128 ? (128 - 2 * DB * 16) / 8 : KS;
 	// Head dim 64 with bias, no dropout (matrix products through the compiler's builtins): the chain of dP still starts
 	// from -delta of the block's rows - the start value is the four LDS reads of the statistics as they are, the
 	// subtraction per value goes away (one of about eight vector-ALU instructions per value of a kernel that is bound by them).
@@ -386,10 +389,15 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 		float bv[2][BIAS && !BIAS_LDS ? 16 : 1];  // [block parity]: bias values, fetched one stage ahead of their use
 		u32x2 bvr[2][BIAS_LDS ? 4 : 1];           // the same from LDS: [block parity][quad], 4 values of 16 bits
 
-		// fragment of product j of A(qb): even j -> Q (S), odd j -> dO (dP), k-step j / 2
+		// Product j of A: even j -> Q (S), odd j -> dO (dP), k-step j / 2.  Where registers are short (KSA < KS) the chain of S comes first and
+		// that of dP after it, so that the start values and the results of the two do not all live at once.
+		constexpr bool CHAINS = KSA < KS;
+		auto a_is_dp = [](int j) __attribute__((always_inline)) { return CHAINS ? j >= KS : (j & 1) != 0; };
+		auto a_step = [](int j) __attribute__((always_inline)) { return CHAINS ? j % KS : j >> 1; };
 		auto issue_A = [&](int qb, int j) __attribute__((always_inline)) {
 			// (poff carries the buffer; dO lies one tile behind Q)
-			afr[(qb * NSLOT + j) % RING] = *(const FA2_LDS V8*)(lds + poff[(j >> 1) % KR] + ((j >> 1) / KR) * 256 + ((j & 1) ? TILE_BYTES : 0) + qb * (32 * D * 2));
+			const int ks = a_step(j);
+			afr[(qb * NSLOT + j) % RING] = *(const FA2_LDS V8*)(lds + poff[ks % KR] + (ks / KR) * 256 + (a_is_dp(j) ? TILE_BYTES : 0) + qb * (32 * D * 2));
 		};
 		// fragment of product j of C(qb): half j / (2 DB); inside a half even -> dO^T (dV), odd -> Q^T (dK)
 		auto issue_C = [&](int qb, int j) __attribute__((always_inline)) {
@@ -400,7 +408,7 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 		// statistics of rows 8 aa + 4 g .. + 3 of block qb
 		auto issue_stat = [&](int qb, int aa) __attribute__((always_inline)) {
 			lse4[aa] = *(const FA2_LDS f32x4*)(stat + soff + (32 * qb + 8 * aa) * 4);
-			if constexpr (!FOLD_DEL) del4[aa] = *(const FA2_LDS f32x4*)(stat + soff + 2 * STAT_BYTES + (32 * qb + 8 * aa) * 4);
+			if constexpr (!FOLD_DEL && !CHAINS) del4[aa] = *(const FA2_LDS f32x4*)(stat + soff + 2 * STAT_BYTES + (32 * qb + 8 * aa) * 4);
 		};
 		// FOLD_DEL: -delta of rows 8 aa + 4 g .. + 3 of block qb, the start value of its chain of dP (read a stage ahead of the statistics)
 		f32x4 cdel4[FOLD_DEL ? 4 : 1];
@@ -452,21 +460,28 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 			}
 		};
 		auto mfma_A = [&](int qb, int j, f32x16& sa, f32x16& dpa) __attribute__((always_inline)) {
-			int ks = j >> 1, r = (qb * NSLOT + j) % RING;
+			int ks = a_step(j), r = (qb * NSLOT + j) % RING;
 			if constexpr (KV_AGPR) {
 				// the chains start from -lse and -delta of the block's rows (accumulator element i
 				// belongs to row 8 (i / 4) + 4 g + i % 4, which is element i % 4 of quarter i / 4)
 				if (j == 0) {
 					cstart[0] = __builtin_shufflevector(__builtin_shufflevector(lse4[0], lse4[1], 0, 1, 2, 3, 4, 5, 6, 7), __builtin_shufflevector(lse4[2], lse4[3], 0, 1, 2, 3, 4, 5, 6, 7), 0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
 					mfma32_vc(sa, afr[r], kf[ks], cstart[0]);
-				} else if (j == 1) {
+				} else if (ks == 0) {
 					cstart[1] = __builtin_shufflevector(__builtin_shufflevector(del4[0], del4[1], 0, 1, 2, 3, 4, 5, 6, 7), __builtin_shufflevector(del4[2], del4[3], 0, 1, 2, 3, 4, 5, 6, 7), 0, 1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15);
 					mfma32_vc(dpa, afr[r], vf[ks], cstart[1]);
 				}
-				else if (j & 1)
-					mfma32_va<true>(dpa, afr[r], vf[ks]);
-				else
-					mfma32_va<true>(sa, afr[r], kf[ks]);
+				else if (ks < KSA) {
+					if (a_is_dp(j))
+						mfma32_va<true>(dpa, afr[r], vf[ks]);
+					else
+						mfma32_va<true>(sa, afr[r], kf[ks]);
+				} else {
+					if (a_is_dp(j))
+						mfma32_va<false>(dpa, afr[r], vf[ks]);
+					else
+						mfma32_va<false>(sa, afr[r], kf[ks]);
+				}
 			} else if constexpr (S_VGPR) {
 				if (j == 0)
 					mfma32_vz(sa, afr[r], kf[ks]);
@@ -693,6 +708,9 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 						int cn = k == 1 ? j + PA - H : j + PA + H;
 						if (cn >= 0 && cn < NSLOT) issue_C(0, cn);
 					}
+					if constexpr (CHAINS && HAS_A) {
+						if (j >= KS - 4 && j < KS) del4[j - (KS - 4)] = *(const FA2_LDS f32x4*)(stat + soff + 2 * STAT_BYTES + (32 * k + 8 * (j - (KS - 4))) * 4);
+					}
 					// the start values of the chains of the next block, in the last four slots
 					if constexpr (FOLD && NEXT_A) {
 						if (j >= NSLOT - 4) issue_stat(k + 1, j - (NSLOT - 4));
@@ -731,7 +749,7 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 				// the destination) therefore stay allocated until two further products have been issued.
 				if constexpr (HAS_A && KV_AGPR) {
 					if (j == 2) asm volatile("; chain start of S still allocated" ::"v"(cstart[0]));
-					if (j == 3) asm volatile("; chain start of dP still allocated" ::"v"(cstart[1]));
+					if (j == (CHAINS ? KS + 2 : 3)) asm volatile("; chain start of dP still allocated" ::"v"(cstart[1]));
 				}
 				// the vector-ALU work below must not move above the product: for the products
 				// issued as inline assembly that order is what keeps a read of S / dP at least
@@ -797,7 +815,7 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 	// accumulation registers, where the inline-assembly products read them.)
 #pragma unroll
 	for (int ks = 0; ks < KS; ++ks) {
-		if constexpr (KV_AGPR)
+		if (KV_AGPR && ks < KSA)
 			asm volatile("; K / V fragment present" : "+a"(kf[ks]), "+a"(vf[ks]));
 		else
 			asm volatile("; K / V fragment present" : "+v"(kf[ks]), "+v"(vf[ks]));
@@ -1783,11 +1801,13 @@ hipError_t launch_bwd_v(KArgs& a, hipStream_t s) {
 		// 190, causal 144 -> 140, with dropout 315 -> 290, B8 H16 S2048 with a shared bias 842 -> 809, B2 S2048 with a bias per head 283 -> 267,
 		// B1 Hq32 Hkv8 S8191 in a window of 1024 389 -> 373.  Below that number of workgroups it is alone on its CU and slower (384
 		// of them, B4 Hq32 Hkv4 S1500 causal: 256 -> 284), and so it is against pairs of key tiles (B4 Hq16 Hkv4 S4096 causal 656 -> 732).
-		const bool blk = D == 64 && !a.kv_pair && (int64_t)grid.x >= 2 * kNumCU;
+		// Rows of 72 to 96 columns fit two workgroups a CU too, in tiles of 64 rows (128 would take 130 KiB of LDS): B64 H16 S257 D80
+		// 349 -> 303 us, B32 H16 S520 D88 444 -> 402, B7 H16 S1100 D96 333 -> 309, B8 H16 S1040 D72 causal 215 -> 202, B2 H16 S4096 D96 943 -> 925.
+		const bool blk = (D == 64 || DE < D) && !a.kv_pair && (int64_t)grid.x >= 2 * kNumCU;
 		auto launch_dkdv = [&](auto blk_tag) {
 			constexpr bool BLK = decltype(blk_tag)::value;
 			// with bias at D = 128 the streamed tiles are 64 rows, which leaves LDS room for the bias tiles (and block by block for a second workgroup)
-			constexpr int QBV = (BIAS && (D == 128 || BLK)) ? 2 : C::KV_QB;
+			constexpr int QBV = (BIAS && (D == 128 || BLK)) || (BLK && D == 128) ? 2 : C::KV_QB;
 			if constexpr (BIAS) {
 				if (a.softcap > 0.f)
 					hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, C::KV_NW, QBV, true, DROP, false, true, false, DE, BLK>), grid, block, 0, s, a);
@@ -1803,7 +1823,7 @@ hipError_t launch_bwd_v(KArgs& a, hipStream_t s) {
 				hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, C::KV_NW, QBV, false, DROP, false, false, false, DE, BLK>), grid, block, 0, s, a);
 			}
 		};
-		if constexpr (D == 64) {
+		if constexpr (D == 64 || DE < D) {
 			if (blk)
 				launch_dkdv(std::true_type{});
 			else

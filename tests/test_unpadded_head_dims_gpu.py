@@ -83,3 +83,31 @@ def test_short_rows_in_any_memory(how):
 	a = [f64(x) for x in (q, k, v, do)]
 	check_forward(o, lse, *O.attention_fwd(*a[:3], causal=True), dtype, how)
 	check_grads(grads, O.attention_bwd(*a, causal=True), how)
+
+
+@pytest.mark.parametrize("dtype,D", [(torch.bfloat16, 72), (torch.float16, 80), (torch.bfloat16, 96), (torch.float16, 88)])
+@pytest.mark.parametrize(
+	"Sq,Sk,kw",
+	[
+		(257, 257, {}),                                       # a row beyond the fourth tile, a key beyond the second key tile
+		(31, 513, {}),                                        # one block of rows
+		(96, 520, dict(causal=True)),                         # rows that see no key of the last key tile's end; a tile of one block
+		(545, 545, dict(causal=True, kv_lens=[545, 129])),
+		(640, 640, dict(causal=True, window=(99, 0))),
+	],
+)
+def test_short_rows_block_by_block(Sq, Sk, kw, dtype, D):
+	"""dK/dV on grids of at least two workgroups per CU: block by block in tiles of 64 rows."""
+	B, H = 2, 128
+	assert B * H * ((Sk + 127) // 128) >= 512
+	q, k, v, do, _ = make_inputs(B, Sq, Sk, H, H, D, dtype, seed=Sq + D)
+	kv_lens = kw.get("kv_lens")
+	kl = None if kv_lens is None else torch.tensor(kv_lens, dtype=torch.int32, device="cuda:0")
+	args = (None, None, None, 0.0, kw.get("causal", False), None, kl, kw.get("window"))
+	o, lse = op.fwd(q.cuda(), k.cuda(), v.cuda(), *args)
+	g = op.bwd(q.cuda(), k.cuda(), v.cuda(), o, lse, do.cuda(), *args)
+	for b, h in ((0, 0), (B - 1, H - 1)):
+		bs, hs = slice(b, b + 1), slice(h, h + 1)
+		want = O.attention_bwd(*[f64(x[bs, :, hs]) for x in (q, k, v, do)], causal=kw.get("causal", False), window=kw.get("window"),
+		                       kv_lens=None if kv_lens is None else kv_lens[bs])
+		check_grads([x[bs, :, hs] for x in g], want, f"Sq{Sq} Sk{Sk} D{D} {kw} b{b} h{h}")
