@@ -22,6 +22,11 @@ import typing as tp
 import torch
 
 from . import _lib
+
+try:
+	from . import _fa2_torch
+except ImportError as e:
+	raise ImportError(f"the extension module _fa2_torch is missing or does not load ({e}): build it with `make -C csrc` as libfa2_hip.so") from e
 from ._checks import check_shapes  # noqa: F401  (re-exported)
 from ._lib import FA2_BF16, FA2_FP16, FA2_FP32, FA2_MASK_U8
 
@@ -170,9 +175,30 @@ def _seqlens_from_mask(attention_mask, q):
 	return lens
 
 
+_bound = None
+
+
+def _entry_points():
+	"""The entry points of libfa2_hip.so as the extension module takes them."""
+	global _bound
+	lib = _lib.load()
+	if _bound is None:
+		names = ("fa2_fwd", "fa2_bwd", "fa2_validate", "fa2_fwd_scratch_bytes", "fa2_bwd_scratch_bytes", "fa2_bwd_split_scratch_bytes")
+		_bound = _fa2_torch.bind(*(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in names))
+	return _bound
+
+
 def fwd(q, k, v, bias=None, seqlens=None, softmax_scale=None, dropout_prob=0.0, causal=False, dropout_seed=None, kv_lens=None,
         window=None, softcap=0.0):
 	"""Returns (out [B,Sq,Hq,D] in q.dtype, lse [B,Hq,Sq] fp32 natural log)."""
+	if q.is_cuda:
+		# an ordinary call: plain tensors in order for the kernels (anything else: None, and what follows copies, pads or refuses)
+		res = _fa2_torch.forward(_entry_points(), q, k, v, bias, seqlens, softmax_scale, dropout_prob, causal, dropout_seed, kv_lens, window,
+		                         softcap, _stream_ptr(q.device))
+		if res.__class__ is int:
+			_lib.check(res)
+		elif res is not None:
+			return res
 	lib = _lib.load()
 	D0 = q.shape[-1]
 	D = _kernel_head_dim(D0)
@@ -203,6 +229,13 @@ def bwd(q, k, v, out, lse, dout, bias=None, seqlens=None, softmax_scale=None, dr
 	"""Returns (dq, dk, dv) in the dtypes of q, k, v; dk/dv summed over each KV group.  With `need_dbias` a fourth
 	result: the gradient of the additive bias, fp32, in the shape of `bias` (summed over the axes it is broadcast on;
 	those sums are atomic adds in the dQ kernel - see fa2_params.dbias - so the buffer is as small as the bias)."""
+	if q.is_cuda and not need_dbias:
+		res = _fa2_torch.backward(_entry_points(), q, k, v, bias, seqlens, softmax_scale, dropout_prob, causal, dropout_seed, kv_lens, window,
+		                          softcap, out, lse, dout, _stream_ptr(q.device))
+		if res.__class__ is int:
+			_lib.check(res)
+		elif res is not None:
+			return res
 	lib = _lib.load()
 	D0 = q.shape[-1]
 	D = _kernel_head_dim(D0)
@@ -363,7 +396,11 @@ def flash_attention(
 	if attention_mask is not None and attention_mask.dim() == 4:
 		assert bias is None, "Attention mask is not supported along with attention bias. Just use bias instead."
 		bias, attention_mask = _mask_operand(attention_mask, q), None
-	check_shapes(q, k, v, bias, attention_mask)
+	flags = _fa2_torch.checked(q, k, v, bias, attention_mask)
+	if not flags:
+		check_shapes(q, k, v, bias, attention_mask)
 	seqlens = _seqlens_from_mask(attention_mask, q)
+	if flags & 2:  # (nothing differentiates, batches or traces this call)
+		return fwd(q, k, v, bias, seqlens, softmax_scale, dropout_prob, causal, dropout_seed, kv_lens, window_size, softcap)[0]
 	return _FlashAttentionFn.apply(q, k, v, bias, seqlens, softmax_scale, dropout_prob, causal, dropout_seed, kv_lens, window_size, softcap,
 	                               bias_grad)

@@ -1,0 +1,192 @@
+"""The extension that makes the torch operator's calls fills the parameter block the Python code fills, for every form of a call that it
+takes, and leaves the others - and every error of an argument's form - to the Python code."""
+
+import ctypes
+import itertools
+import math
+
+import pytest
+import torch
+
+from jax_flash_attn2 import _fa2_torch, _hip_op as op, _lib
+from jax_flash_attn2._checks import check_shapes
+
+_CALL = ctypes.CFUNCTYPE(ctypes.c_int, ctypes.POINTER(_lib.Fa2Params), ctypes.c_void_p)
+
+
+class _Recorder:
+	"""Stands in for the two launching entry points; the others are the library's own."""
+
+	def __init__(self, rc=0):
+		self.rc, self.seen = rc, []
+		self.keep = _CALL(self._call)
+		lib = _lib.load()
+		at = ctypes.cast(self.keep, ctypes.c_void_p).value
+		rest = ("fa2_validate", "fa2_fwd_scratch_bytes", "fa2_bwd_scratch_bytes", "fa2_bwd_split_scratch_bytes")
+		self.bound = _fa2_torch.bind(at, at, *(ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in rest))
+
+	def _call(self, p, stream):
+		self.seen.append((_lib.Fa2Params.from_buffer_copy(p.contents), stream))
+		return self.rc
+
+
+def _x(*shape, dtype=torch.bfloat16, form="plain"):
+	B, S, H, D = shape
+	if form == "plain":
+		return torch.zeros(shape, dtype=dtype)
+	if form == "heads first":  # [B, H, S, D] in memory
+		return torch.zeros((B, H, S, D), dtype=dtype).transpose(1, 2)
+	if form == "slice":  # of fused rows, 16-byte aligned
+		return torch.zeros((B, S, H, 3 * D), dtype=dtype)[..., D : 2 * D]
+	if form == "one batch row":
+		return torch.zeros((1, S, H, D), dtype=dtype).expand(B, S, H, D)
+	if form == "reversed axes":
+		return torch.zeros((D, H, S, B), dtype=dtype).permute(3, 2, 1, 0)
+	assert form == "odd address"
+	n = B * S * H * D
+	return torch.zeros(n + 8, dtype=dtype)[1 : n + 1].view(shape)
+
+
+def _fields(p):
+	out = {}
+	for name, t in _lib.Fa2Params._fields_:
+		v = getattr(p, name)
+		out[name] = (v.ptr, v.stride_b, v.stride_s, v.stride_h) if t is _lib.Fa2Tensor else v
+	return out
+
+
+def _same(p, want, *own):
+	a, b = _fields(p), _fields(want)
+	for n in ("scratch", "scratch_bytes", *own):
+		a.pop(n), b.pop(n)
+	assert a == b
+
+
+def _scale(q, s):
+	return 1.0 / math.sqrt(q.shape[-1]) if s is None else s
+
+
+_SIZES = [(2, 5, 9, 4, 2, 64), (1, 1, 1029, 32, 8, 128), (2, 130, 130, 2, 2, 256), (1, 257, 257, 2, 1, 80), (1, 40, 40, 1, 1, 96)]
+_FORMS = ["plain", "heads first", "slice", "one batch row"]
+
+
+@pytest.mark.parametrize("B,Sq,Sk,Hq,Hkv,D", _SIZES)
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+def test_blocks_over_strides(B, Sq, Sk, Hq, Hkv, D, dtype):
+	rec = _Recorder()
+	for fq, fk in itertools.product(_FORMS, _FORMS):
+		q, k, v = _x(B, Sq, Hq, D, dtype=dtype, form=fq), _x(B, Sk, Hkv, D, dtype=dtype, form=fk), _x(B, Sk, Hkv, D, dtype=dtype)
+		call = (None, None, None, 0.0, True, None, None, None, 0.0)
+		res = _fa2_torch.forward(rec.bound, q, k, v, *call, 77)
+		Dk = op._kernel_head_dim(D)
+		usable = op._usable if D == Dk else op._usable_short
+		served = all(usable(x) is x for x in (q, k, v)) if D == Dk or op._runs_unpadded(_lib.load(), 0, Dk, q, k, v, None, None, 0.1, 0.0, True, None) else False
+		assert (res is not None) == served or (D != Dk and res is not None)
+		if res is None:
+			continue
+		out, lse = res
+		assert out.shape == q.shape and out.is_contiguous() and out.dtype == dtype and lse.shape == (B, Hq, Sq) and lse.dtype == torch.float32
+		p, stream = rec.seen[-1]
+		assert stream == 77
+		_same(p, op._block(Dk, q, k, v, None, None, _scale(q, None), 0.0, True, None, None, None, 0.0, op._t4(out), lse))
+		assert (p.scratch_bytes or 0) == _lib.load().fa2_fwd_scratch_bytes(ctypes.byref(p))
+		assert bool(p.scratch) == bool(p.scratch_bytes)
+		dout = _x(B, Sq, Hq, D, dtype=dtype, form=fq)
+		if usable(dout) is not dout:
+			continue
+		dq, dk, dv = _fa2_torch.backward(rec.bound, q, k, v, *call, out, lse, dout, 5)
+		p, stream = rec.seen[-1]
+		assert stream == 5 and dq.shape == q.shape and dk.shape == k.shape and dv.shape == v.shape
+		assert dq.is_contiguous() and dk.is_contiguous() and dv.is_contiguous()
+		_same(p, op._block(Dk, q, k, v, None, None, _scale(q, None), 0.0, True, None, None, None, 0.0, op._t4(out), lse,
+		                   (op._t4(dout), op._t4(dq), op._t4(dk), op._t4(dv))))
+		lib = _lib.load()
+		assert p.scratch and p.scratch_bytes == max(256, lib.fa2_bwd_scratch_bytes(ctypes.byref(p)), lib.fa2_bwd_split_scratch_bytes(ctypes.byref(p)))
+
+
+def _biases(B, Hq, Hkv, Sq, Sk):
+	for b, h in itertools.product((1, B), (1, Hkv, Hq)):
+		for dt in (torch.float16, torch.bfloat16, torch.float32, torch.uint8, torch.bool):
+			yield torch.zeros((b, h, Sq, Sk), dtype=dt)
+	yield torch.zeros((B, Hq, Sq, Sk + 5))[..., :Sk]
+	yield torch.zeros((1, 1, 1, Sk)).expand(B, Hq, Sq, Sk)
+
+
+def test_blocks_over_options():
+	rec = _Recorder()
+	B, Sq, Sk, Hq, Hkv, D = 2, 6, 10, 4, 2, 64
+	q, k, v = _x(B, Sq, Hq, D), _x(B, Sk, Hkv, D), _x(B, Sk, Hkv, D)
+	lens, seed = torch.full((B,), 3, dtype=torch.int32), torch.tensor([5])
+	full = dict(bias=None, seqlens=None, scale=None, p=0.0, causal=False, seed=None, kv_lens=None, window=None, softcap=0.0)
+	calls = [dict(full, bias=b) for b in _biases(B, Hq, Hkv, Sq, Sk)]
+	calls += [dict(full, seqlens=lens), dict(full, kv_lens=lens), dict(full, scale=0.3), dict(full, scale=2), dict(full, causal=True)]
+	calls += [dict(full, p=0.2, seed=s) for s in (None, 0, 7, -3, 1 << 63, (1 << 70) + 9, seed)]
+	calls += [dict(full, p=0), dict(full, softcap=30.0), dict(full, softcap=None), dict(full, softcap=5)]
+	calls += [dict(full, window=w) for w in ((3, 0), (-1, -1), (-7, 2), (1 << 40, -(1 << 70)), (1 << 70, 0))]
+	for c in calls:
+		res = _fa2_torch.forward(rec.bound, q, k, v, *c.values(), 0)
+		assert res is not None, c
+		want = dict(c, scale=_scale(q, c["scale"]), bias=op._prep_bias(c["bias"]))
+		_same(rec.seen[-1][0], op._block(D, q, k, v, *want.values(), op._t4(res[0]), res[1]))
+
+
+def test_what_is_left_to_the_python_code():
+	rec = _Recorder()
+	q = _x(1, 4, 2, 64)
+	plain = [None, None, None, 0.0, False, None, None, None, 0.0]
+
+	def served(*qkv, **change):
+		call = list(plain)
+		for i, x in change.values():
+			call[i] = x
+		return _fa2_torch.forward(rec.bound, *qkv, *call, 0) is not None
+
+	assert served(q, q, q)
+	assert not served(q, _x(1, 4, 2, 64, form="odd address"), q)
+	assert not served(_x(1, 4, 2, 64, form="reversed axes"), q, q)
+	for D in (32, 50, 72 + 4, 104, 200):
+		assert not served(*(_x(1, 4, 2, D) for _ in range(3)))
+	assert not served(*(x.float() for x in (q, q, q)))
+	assert not served(*(x.as_subclass(type("Other", (torch.Tensor,), {})) for x in (q, q, q)))
+	for i, x in [(0, torch.zeros(1, 1, 4, 4, dtype=torch.float64)), (0, torch.zeros(1, 1, 4, 4).mT), (0, torch.zeros(4, 4)), (2, torch.tensor(0.1)), (2, 1e300),
+	             (4, 1), (4, None), (5, 2.0), (5, True), (5, torch.tensor([1, 2])), (6, torch.tensor([4])), (6, torch.zeros(2, dtype=torch.int32)), (7, [1, 0]), (7, (1, 0, 0)),
+	             (7, (1.0, 0)), (8, True)]:
+		assert not served(q, q, q, change=(i, x)), (i, x)
+	assert len(rec.seen) == 1
+	# the code of an error comes back as a number
+	assert _fa2_torch.forward(_Recorder(rc=-12).bound, q, q, q, *plain, 0) == -12
+
+
+def _takes(*args):
+	try:
+		check_shapes(*args)
+	except Exception:
+		return False
+	return True
+
+
+def test_checks():
+	"""What the extension passes is what check_shapes() passes; a call that differentiates keeps its autograd function."""
+	z = torch.zeros
+	q = z(2, 4, 4, 64, dtype=torch.float16)
+	others = [q, z(2, 6, 2, 64, dtype=torch.float16), z(2, 4, 3, 64, dtype=torch.float16), z(1, 4, 4, 64, dtype=torch.float16), z(2, 4, 4, 32, dtype=torch.float16), z(2, 4, 4, 64),
+	          z(2, 4, 4, 64, dtype=torch.bfloat16)]
+	biases = [None, z(2, 4, 4, 4), z(1, 1, 4, 4), z(2, 2, 4, 6), z(3, 1, 4, 4), z(2, 3, 4, 4), z(2, 4, 4, 5)]
+	masks = [None, z(2, 4, dtype=torch.bool)]
+	for k, v, bias, mask in itertools.product(others, others, biases, masks):
+		assert bool(_fa2_torch.checked(q, k, v, bias, mask)) == _takes(q, k, v, bias, mask)
+	k = q.clone()
+	assert _fa2_torch.checked(q, k, q, None, None) == 3
+	k.requires_grad_()
+	assert _fa2_torch.checked(q, k, q, None, None) == 1
+	with torch.no_grad():
+		assert _fa2_torch.checked(q, k, q, None, None) == 3
+	bias = z(1, 1, 4, 4, requires_grad=True)
+	assert _fa2_torch.checked(q, q, q, bias, None) == 1
+	with torch.autograd.forward_ad.dual_level(), torch.no_grad():
+		dual = torch.autograd.forward_ad.make_dual(q, q.clone())
+		assert _fa2_torch.checked(q, dual, q, None, None) == 1
+	seen = []
+	torch.func.vmap(lambda x: (seen.append(_fa2_torch.checked(x, x, x, None, None)), x)[1])(z(3, 2, 4, 4, 64, dtype=torch.float16))
+	torch.jit.trace(lambda x: (seen.append(_fa2_torch.checked(x, x, x, None, None)), x * 1)[1], (q,), check_trace=False)
+	assert seen and all(not f & 2 for f in seen), seen
