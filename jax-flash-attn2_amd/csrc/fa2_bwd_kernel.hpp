@@ -984,7 +984,7 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 		}
 		return x;
 	};
-	// epilogue: lane owns key jst, four consecutive d per store
+	// epilogue: lane owns key jst, eight consecutive d per store (four of a partial result)
 	const int jst = n0 + 32 * w + c;
 	if (hsplit > 1) {
 		// partial sums over this workgroup's share of the steps, fp32 and unscaled, for the reduce kernel
@@ -1009,12 +1009,21 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 #pragma unroll
 		for (int db = 0; db < DB; ++db)
 #pragma unroll
-			for (int aa = 0; aa < 4; ++aa) {
+			for (int aa = 0; aa < 4; aa += 2) {
 				if (COLS && 32 * db + 8 * aa >= a.hd) continue;
-				int d0 = 32 * db + 8 * aa + 4 * g;
-				const f32x4 xk = result(0, db, aa), xv = result(1, db, aa);
-				*(u32x2*)(dkp + d0 * 2) = u32x2{pack2<typename T::V2>(xk[0] * ks_, xk[1] * ks_), pack2<typename T::V2>(xk[2] * ks_, xk[3] * ks_)};
-				*(u32x2*)(dvp + d0 * 2) = u32x2{pack2<typename T::V2>(xv[0] * vs_, xv[1] * vs_), pack2<typename T::V2>(xv[2] * vs_, xv[3] * vs_)};
+				u32x2 pk[2], pv[2];
+#pragma unroll
+				for (int u = 0; u < 2; ++u) {
+					const f32x4 xk = result(0, db, aa + u), xv = result(1, db, aa + u);
+					pk[u] = u32x2{pack2<typename T::V2>(xk[0] * ks_, xk[1] * ks_), pack2<typename T::V2>(xk[2] * ks_, xk[3] * ks_)};
+					pv[u] = u32x2{pack2<typename T::V2>(xv[0] * vs_, xv[1] * vs_), pack2<typename T::V2>(xv[2] * vs_, xv[3] * vs_)};
+				}
+				const u32x4 yk = pair_cols(pk[0], pk[1]), yv = pair_cols(pv[0], pv[1]);
+				const int col = 32 * db + 8 * (aa + g);
+				if (!COLS || col < a.hd) {
+					*(u32x4*)(dkp + col * 2) = yk;
+					*(u32x4*)(dvp + col * 2) = yv;
+				}
 			}
 	}
 }
@@ -1691,12 +1700,17 @@ __global__ __launch_bounds__(NW * 64, WPS) void bwd_dq_kernel(const KArgs a) {
 #pragma unroll
 			for (int db = 0; db < DB; ++db)
 #pragma unroll
-				for (int aa = 0; aa < 4; ++aa) {
+				for (int aa = 0; aa < 4; aa += 2) {
 					if (COLS && 32 * db + 8 * aa >= a.hd) continue;
 					const f32x16& x = dq[qb][db];
-					u32x2 pk = {pack2<typename T::V2>(x[4 * aa] * sc, x[4 * aa + 1] * sc),
-					            pack2<typename T::V2>(x[4 * aa + 2] * sc, x[4 * aa + 3] * sc)};
-					*(u32x2*)(rp + (32 * db + 8 * aa + 4 * g) * 2) = pk;
+					u32x2 pk[2];
+#pragma unroll
+					for (int u = 0; u < 2; ++u)
+						pk[u] = u32x2{pack2<typename T::V2>(x[4 * (aa + u)] * sc, x[4 * (aa + u) + 1] * sc),
+						              pack2<typename T::V2>(x[4 * (aa + u) + 2] * sc, x[4 * (aa + u) + 3] * sc)};
+					const u32x4 y = pair_cols(pk[0], pk[1]);
+					const int col = 32 * db + 8 * (aa + g);
+					if (!COLS || col < a.hd) *(u32x4*)(rp + col * 2) = y;
 				}
 		}
 	}

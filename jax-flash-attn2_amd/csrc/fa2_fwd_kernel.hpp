@@ -1131,7 +1131,7 @@ __global__ __launch_bounds__(NW * 64 * KW, WPS) void fwd_kernel(const KArgs a) {
 		}
 	}
 
-	// epilogue: normalise, store O (lane: row c, four consecutive d per store) and LSE
+	// epilogue: normalise, store O (lane: row c, eight consecutive d per store) and LSE
 	char* obase = a.o.ptr + (int64_t)b * a.o.sb + (int64_t)h * a.o.sh;
 #pragma unroll
 	for (int qb = 0; qb < QB; ++qb) {
@@ -1166,12 +1166,17 @@ __global__ __launch_bounds__(NW * 64 * KW, WPS) void fwd_kernel(const KArgs a) {
 #pragma unroll
 			for (int db = 0; db < DB; ++db)
 #pragma unroll
-				for (int aa = 0; aa < 4; ++aa) {
+				for (int aa = 0; aa < 4; aa += 2) {
 					if (COLS && 32 * db + 8 * aa >= a.hd) continue;
 					const f32x16& r = oacc[qb][db];
-					u32x2 pk = {pack2<typename T::V2>(r[4 * aa] * inv, r[4 * aa + 1] * inv),
-					            pack2<typename T::V2>(r[4 * aa + 2] * inv, r[4 * aa + 3] * inv)};
-					*(u32x2*)(rp + (32 * db + 8 * aa + 4 * g) * 2) = pk;
+					u32x2 pk[2];
+#pragma unroll
+					for (int u = 0; u < 2; ++u)
+						pk[u] = u32x2{pack2<typename T::V2>(r[4 * (aa + u)] * inv, r[4 * (aa + u) + 1] * inv),
+						              pack2<typename T::V2>(r[4 * (aa + u) + 2] * inv, r[4 * (aa + u) + 3] * inv)};
+					const u32x4 x = pair_cols(pk[0], pk[1]);
+					const int col = 32 * db + 8 * (aa + g);
+					if (!COLS || col < a.hd) *(u32x4*)(rp + col * 2) = x;
 				}
 			if (g == 0) {
 				float lse;
