@@ -403,15 +403,6 @@ __global__ __launch_bounds__(NW * 64 * KW, WPS) void fwd_kernel(const KArgs a) {
 		bias_base = a.bias + (int64_t)b * a.bias_sb + (int64_t)hb * a.bias_sh;
 	}
 	constexpr bool bias_lds = BIAS_LDS;
-	constexpr bool BIAS_FAST = BIAS_LDS && D != 128;
-	// The largest row sum of a tile that stands without the maximum, and how far (natural units) a tile that has looked at it may exceed the
-	// reference for the next one to be tried.  bfloat16 has the range of fp32, so that a bias that rises along the keys makes an attempt
-	// fail once in many tiles: B8 H16 S2048 D64, 1 / 2 / 4 / 32 a tile, 221 / 226 / 226 / 232 us -> 201 / 212 / 223 / 233 (with
-	// half precision's limits 217 / 229 / 283 / 233); half precision tries it where the maximum hardly moves (0 / 1 /
-	// 2 / 4 a tile 207 / 210 / 215 / 216 -> 196 / 217 / 220 / 224: what an attempt that is not made leaves is the addend).
-	constexpr bool WIDE = std::is_same<T, BF16>::value;
-	constexpr float kBiasFastSum = WIDE ? 0x1p40f : kFastSum, kBiasCalm = (WIDE ? 24.f : 2.f) * kLn2;
-	int bias_fast = 0, bias_first = 1;  // (scalar) try the path without the row maximum on the next tile; no tile yet
 	TileLoader<64, BM, NT> bload;
 	int brows = 0, boff_lane = 0, bkey16 = 0;
 	if constexpr (BIAS_LDS) {
@@ -457,41 +448,15 @@ __global__ __launch_bounds__(NW * 64 * KW, WPS) void fwd_kernel(const KArgs a) {
 		constexpr bool MASKED = decltype(masked_tag)::value;
 		// bias tile, fetched ahead of the matrix products
 		f32x4 bv[BIAS ? KB : 1][BIAS ? QB : 1][4];
-		// (BIAS_FAST: packed until it is the addend of the exponent, (bias - m) log2(e) - at head dim 64 formed beside the products of S,
-		// at 256, where there is no room for it as floats, as it is used)
-		constexpr bool EARLY_BIAS = BIAS_FAST && D == 64;
-		typename T::V4 bvp[BIAS_LDS ? KB : 1][4];
-		auto read_bias = [&]() __attribute__((always_inline)) {
+		if (BIAS_LDS && bias_lds) {
 			static_assert(!BIAS_LDS || QB == 1, "");
 #pragma unroll
 			for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
-				for (int aa = 0; aa < 4; ++aa)
-					bvp[kb][aa] = *(const FA2_LDS typename T::V4*)(lds + 4 * TILE_BYTES + boff_lane + (((kb * 4 + aa) << 4) ^ bkey16));
-		};
-		auto unpack_bias = [&]() __attribute__((always_inline)) {
-#pragma unroll
-			for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-				for (int aa = 0; aa < 4; ++aa) bv[kb][0][aa] = to_f32x4(bvp[kb][aa]);
-		};
-		const float nmb = -mrow[0] * kLog2e;
-		auto bias_addend = [&](int kb, int aa) __attribute__((always_inline)) {
-			f32x4 x = to_f32x4(bvp[kb][aa]);
-#pragma unroll
-			for (int e = 0; e < 4; ++e) x[e] = __builtin_fmaf(x[e], kLog2e, nmb);
-			return x;
-		};
-		if constexpr (BIAS_LDS) {
-			read_bias();
-			if constexpr (!BIAS_FAST) {
-				unpack_bias();
-			} else if constexpr (EARLY_BIAS) {
-#pragma unroll
-				for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-					for (int aa = 0; aa < 4; ++aa) bv[kb][0][aa] = bias_addend(kb, aa);
-			}
+				for (int aa = 0; aa < 4; ++aa) {
+					typename T::V4 x = *(const FA2_LDS typename T::V4*)(lds + 4 * TILE_BYTES + boff_lane + (((kb * 4 + aa) << 4) ^ bkey16));
+					bv[kb][0][aa] = to_f32x4(x);
+				}
 		} else if constexpr (BIAS) {
 #pragma unroll
 			for (int qb = 0; qb < QB; ++qb) {
@@ -691,51 +656,8 @@ __global__ __launch_bounds__(NW * 64 * KW, WPS) void fwd_kernel(const KArgs a) {
 #pragma unroll
 			for (int qb = 0; qb < QB; ++qb) lrow[qb] += lt[qb];
 		} else {
-			// The same fast path where the tiles of bias are in LDS: its exponent is one fused multiply-add of the score on top of the addend
-			// above.  A wave tries it as long as its last tile would have stood: a bias that rises along the keys (ALiBi
-			// with a steep slope) makes every attempt fail.  What bounds these forwards is the issue of the elementwise stage, of
-			// which the maximum is an instruction in seven and a chain: B8 H16 S2048 D64 with a shared bias 212 -> 194 us, B2 Hq16
-			// Hkv8 S2048 D256 with a bias per head 250 -> 218.  At head dim 128 it gains nothing (B2 Hq32 Hkv16 S4096 736 and 720 us,
-			// B2 H16 S2048 92.3 and 93.6): the stream of the bias and the products are as long there.
-			bool slow = true;
-			if constexpr (BIAS_FAST) {
-				if (bias_fast) {
-					const float c1l = c1 * kLog2e;
-					float ls4[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-					for (int kb = 0; kb < KB; ++kb)
-#pragma unroll
-						for (int hf = 0; hf < 2; ++hf) {
-							float pv[8];
-							if constexpr (!EARLY_BIAS) {
-								bv[kb][0][2 * hf] = bias_addend(kb, 2 * hf);
-								bv[kb][0][2 * hf + 1] = bias_addend(kb, 2 * hf + 1);
-							}
-#pragma unroll
-							for (int e = 0; e < 8; ++e) pv[e] = __builtin_fmaf(s[kb][0][8 * hf + e], c1l, bv[kb][0][2 * hf + (e >> 2)][e & 3]);
-#pragma unroll
-							for (int e = 0; e < 8; ++e) {
-								float p = exp2_fast(pv[e]);
-								if constexpr (MASKED) {
-									int j = n0 + 32 * kb + 8 * (2 * hf + (e >> 2)) + 4 * g + (e & 3);
-									p = ((j <= jmax[0]) & (j >= jmin[0])) ? p : 0.f;
-								}
-								ls4[e & 3] += p;
-								pv[e] = p;
-							}
-							pf[0][2 * kb + hf] = pack8<T>(pv[0], pv[1], pv[2], pv[3], pv[4], pv[5], pv[6], pv[7]);
-						}
-					const float lt = (ls4[0] + ls4[1]) + (ls4[2] + ls4[3]);
-					slow = __builtin_amdgcn_ballot_w64(!(lt <= kBiasFastSum)) != 0;
-					if (!slow) lrow[0] += lt;
-				}
-				if (slow) {
-					read_bias();
-					unpack_bias();
-				}
-			}
-#pragma unroll
-			for (int qb = 0; qb < QB && slow; ++qb) {
+			for (int qb = 0; qb < QB; ++qb) {
 				float mx4[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
 #pragma unroll
 				for (int kb = 0; kb < KB; ++kb)
@@ -761,7 +683,6 @@ __global__ __launch_bounds__(NW * 64 * KW, WPS) void fwd_kernel(const KArgs a) {
 				// P = exp2(x - m) may grow to 2^slack, which fp32 sums and 16-bit P hold without loss,
 				// and the O accumulators are left alone.
 				const float slack = kRescaleSlack * kLn2;
-				const bool calm = BIAS_FAST && __builtin_amdgcn_ballot_w64(mx > mrow[qb] + kBiasCalm) == 0;
 				if (__builtin_amdgcn_ballot_w64(mx > mrow[qb] + slack) != 0) {
 					float m_new = __builtin_fmaxf(mrow[qb], mx);
 					float m_use = m_new == -INFINITY ? 0.f : m_new;
@@ -796,11 +717,6 @@ __global__ __launch_bounds__(NW * 64 * KW, WPS) void fwd_kernel(const KArgs a) {
 							ls4[i & 3] += p;
 							s[kb][qb][i] = p;
 						}
-				}
-				// (every row of the wave has a reference, and the addend stays finite)
-				if constexpr (BIAS_FAST) {
-					bias_fast = __builtin_amdgcn_readfirstlane((calm || bias_first) && __builtin_amdgcn_ballot_w64(__builtin_fabsf(mrow[qb]) > 1e37f) == 0 ? 1 : 0);
-					bias_first = 0;
 				}
 				lrow[qb] += (ls4[0] + ls4[1]) + (ls4[2] + ls4[3]);
 				pack_p(qb);

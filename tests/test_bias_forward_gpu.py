@@ -1,5 +1,5 @@
-"""The forward whose tiles of bias go through LDS tries a tile without looking at the row maximum first: biases for which that stands, for
-which it fails now and then or on every tile, and references that no exponent may be formed against."""
+"""The forward with a bias: biases that leave the reference of a row alone, that raise it now and then or on every tile, and references
+that no exponent may be formed against."""
 
 import numpy as np
 import pytest
@@ -20,7 +20,7 @@ def _bias(kind, dtype, B, H, Sq, Sk):
 		x = 1.0 / (1.0 + abs(i - j))
 	elif kind == "steep":  # every tile raises the maximum by 32
 		x = 0.5 * (j - i)
-	elif kind == "one late key":  # far above the reference, in a tile that was tried without the maximum
+	elif kind == "one late key":  # far above the reference
 		x = np.where(j == Sk - 9, 30.0, 0.0) + 0.0 * i
 	elif kind == "first tiles hidden":  # the reference of the first tiles is the lowest finite value
 		x = np.where(j < min(Sk - 8, 150), lowest, 0.5) + 0.0 * i
@@ -58,3 +58,16 @@ def test_bias_that_rises_falls_and_hides(B, Sq, Sk, Hq, Hkv, D, dtype, causal, p
 		lse_ref = np.where(hidden, 0.0, lse_ref)
 		lse = torch.where(torch.from_numpy(hidden).cuda(), torch.zeros_like(lse), lse)
 	check_forward(o, lse, o_ref, lse_ref, dtype, f"{kind} B{B} Sq{Sq} Sk{Sk} D{D} causal={causal} p={p}")
+
+
+@pytest.mark.parametrize("D", [64, 128, 256])
+def test_values_near_the_largest_number(D):
+	"""A late key far above the reference, and values of V of 2^93 (bfloat16 has the range of fp32): no product of the two may pass
+	the fp32 range on the way to a result that is within it."""
+	B, Sq, Sk, H, dtype = 1, 72, 320, 2, torch.bfloat16
+	q, k, v, _, _ = make_inputs(B, Sq, Sk, H, H, D, dtype, seed=D)
+	bias = _bias("flat", dtype, B, 1, Sq, Sk)
+	bias[..., Sk - 9] = 25.0
+	o_ref, lse_ref = O.attention_fwd(f64(q), f64(k), f64(v), f64(bias))
+	o, lse = op.fwd(q.cuda(), k.cuda(), (v * 2.0**93).cuda(), bias.cuda())
+	check_forward(o.float() * 2.0**-93, lse, o_ref, lse_ref, dtype, f"D{D}")
