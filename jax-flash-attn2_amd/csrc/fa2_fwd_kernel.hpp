@@ -695,10 +695,12 @@ __global__ __launch_bounds__(NW * 64 * KW, WPS) void fwd_kernel(const KArgs a) {
 						for (int i = 0; i < 16; ++i) oacc[qb][db][i] *= alpha;
 				}
 				const float m_use = mrow[qb] == -INFINITY ? 0.f : mrow[qb];
-				// (x - m) log2(e) as one fused multiply-add, x log2(e) - m log2(e) - unless some row's reference is so
-				// large that m log2(e) leaves the fp32 range: a row whose keys all carry the finfo.min "mask" bias of
-				// the bf16 type (-3.39e38).  Such a wave (rare) subtracts first.
-				if (__builtin_amdgcn_ballot_w64(__builtin_fabsf(m_use) > 1e37f) == 0) {
+				// (x - m) log2(e) as one fused multiply-add, x log2(e) - m log2(e), whose addend is rounded: by up to 2^-7 at 1e5, as
+				// much as x itself is at that size, by 64 at -1e9 and 512 at -1e10 - a key that carries such a "mask" bias then had a P of
+				// infinity or 0 instead of 1 where it is the row's reference - and to infinity at the lowest bfloat16 (-3.39e38).
+				// A wave with a reference of that size (the first tiles of a row that is masked on the left, rows whose keys are all masked)
+				// subtracts first, which is exact for x near m.
+				if (__builtin_amdgcn_ballot_w64(__builtin_fabsf(m_use) > 1e5f) == 0) {
 					const float nm2 = -m_use * kLog2e;
 #pragma unroll
 					for (int kb = 0; kb < KB; ++kb)

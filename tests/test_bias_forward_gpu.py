@@ -71,3 +71,47 @@ def test_values_near_the_largest_number(D):
 	o_ref, lse_ref = O.attention_fwd(f64(q), f64(k), f64(v), f64(bias))
 	o, lse = op.fwd(q.cuda(), k.cuda(), (v * 2.0**93).cuda(), bias.cuda())
 	check_forward(o.float() * 2.0**-93, lse, o_ref, lse_ref, dtype, f"D{D}")
+
+
+# Masks that are spelt as a large negative number: beyond about 1e6 the product of a reference and log2(e) is rounded by more than an
+# exponent bears, from the lowest value / log2(e) on it leaves the fp32 range.
+_FILLS = [-1e6, -1e9, -1e10, -1e12, -1e30, None]  # (None: the lowest finite value)
+
+
+def _masked(fill, bias_dtype, Sq, Sk):
+	"""Two heads: in the first the keys of the first tiles are hidden, in the second all keys of every other row (their q is zero, so
+	that the oracle weighs these keys alike too; fp32 does so whatever q is, the bias absorbs the score)."""
+	fill = torch.finfo(bias_dtype).min if fill is None else fill
+	bias = _bias("flat", torch.float32, 1, 2, Sq, Sk)
+	bias[0, 0, :, :150] = fill
+	bias[0, 1, ::2] = fill
+	return bias.to(bias_dtype)
+
+
+def _masked_inputs(Sq, Sk, D, dtype):
+	q, k, v, do, _ = make_inputs(1, Sq, Sk, 2, 2, D, dtype, seed=D)
+	q[:, ::2, 1] = 0
+	return q, k, v, do
+
+
+_MASKED = [
+	(torch.bfloat16, torch.bfloat16, 320),  # tiles of bias in LDS
+	(torch.bfloat16, torch.bfloat16, 321),  # bias read value by value
+	(torch.float16, torch.float32, 320),
+]
+
+
+@pytest.mark.parametrize("fill", _FILLS)
+@pytest.mark.parametrize("D", [64, 128, 256])
+@pytest.mark.parametrize("dtype,bias_dtype,Sk", _MASKED)
+def test_large_negative_bias_as_a_mask(dtype, bias_dtype, Sk, D, fill):
+	Sq = 72
+	q, k, v, _ = _masked_inputs(Sq, Sk, D, dtype)
+	bias = _masked(fill, bias_dtype, Sq, Sk)
+	o_ref, lse_ref = O.attention_fwd(f64(q), f64(k), f64(v), f64(bias))
+	o, lse = op.fwd(q.cuda(), k.cuda(), v.cuda(), bias.cuda())
+	# (the logsumexp of a hidden row is the bias to the 24 bits of fp32)
+	assert np.allclose(lse[0, 1, ::2].cpu().numpy(), lse_ref[0, 1, ::2], rtol=1e-6)
+	lse[0, 1, ::2] = 0
+	lse_ref[0, 1, ::2] = 0
+	check_forward(o, lse, o_ref, lse_ref, dtype, f"D{D} {fill}")
