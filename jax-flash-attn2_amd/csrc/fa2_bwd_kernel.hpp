@@ -105,6 +105,12 @@ FA2_DEV DkdvRow dkdv_row(const KArgs& a, int b) {
 	return rw;
 }
 
+// With bias: -lse log2(e), the addend of the exponent of P = exp(x - lse).  A logsumexp beyond 2^24 comes from a row whose keys are all
+// masked by a large negative bias (or from a key that a large positive one forces): it holds nothing of the sum any more, and what
+// its product is rounded by is the exponent (up to 64 at 1e9, 512 at 1e10: P of infinity, times an incoming gradient that usually is 0).
+// Such a row passes no gradient on, as has been so at the lowest bfloat16.  (NaN: 3e38.)
+FA2_DEV float bias_exp_addend(float lse) { return __builtin_fabsf(lse) > 0x1p24f ? -INFINITY : __builtin_fminf(-lse * kLog2e, 3.0e38f); }
+
 // K, V rows of key jcol (this lane's) as B operands: the lane holds X[key][16 ks + 8 g .. + 7].
 template <typename T, int DE, bool COLS>
 FA2_DEV void dkdv_load_kv(const KArgs& a, int jcol, int hk, int b, typename T::V8 (&kf)[DE / 16], typename T::V8 (&vf)[DE / 16]) {
@@ -317,8 +323,9 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 	auto store_stat = [&](float x, int buf) {
 		if (tid < 2 * BMQ) {
 			int which = tid / BMQ;
-			// (kept finite: lse of a row whose keys all carry the finfo.min "mask" bias of the bf16 type is -3.39e38)
-			*(FA2_LDS float*)(stat + (2 * which + buf) * STAT_BYTES + stat_row * 4) = __builtin_fminf(x * stat_mul, 3.0e38f);
+			float y = __builtin_fminf(x * stat_mul, 3.0e38f);
+			if (BIAS && which == 0) y = bias_exp_addend(x);
+			*(FA2_LDS float*)(stat + (2 * which + buf) * STAT_BYTES + stat_row * 4) = y;
 		}
 	};
 
@@ -1222,9 +1229,8 @@ __global__ __launch_bounds__(NW * 64, WPS) void bwd_dq_kernel(const KArgs a) {
 		int64_t idx = ((int64_t)b * a.Hq + h) * a.Sq + ic;
 		float l = a.lse[idx];
 		// rows without any allowed key carry lse = -inf; their P is forced to 0 by the mask
-		// the addend of the fused multiply-add that forms the exponent, (x - lse) log2(e) = x log2(e) - lse log2(e); kept finite
-		// for a row whose keys all carry the finfo.min "mask" bias of the bf16 type (lse = -3.39e38: its P underflows to 0)
-		lse_r[qb] = __builtin_fminf(-l * kLog2e, 3.0e38f);
+		// the addend of the fused multiply-add that forms the exponent, (x - lse) log2(e) = x log2(e) - lse log2(e)
+		lse_r[qb] = BIAS ? bias_exp_addend(l) : __builtin_fminf(-l * kLog2e, 3.0e38f);
 		del_r[qb] = a.delta[idx];
 	}
 	int wave_jmin, wave_jmax, wave_lmin = kNoKey, wave_lmax = kNoKey;

@@ -1,4 +1,4 @@
-"""The forward with a bias: biases that leave the reference of a row alone, that raise it now and then or on every tile, and references
+"""The operator with a bias: biases that leave the reference of a row alone, that raise it now and then or on every tile, and references
 that no exponent may be formed against."""
 
 import numpy as np
@@ -7,7 +7,7 @@ import torch
 
 from jax_flash_attn2 import _hip_op as op
 import fa2_oracle as O
-from _cases import check_forward, f64, make_inputs
+from _cases import check_forward, check_grads, f64, make_inputs
 
 pytestmark = pytest.mark.gpu
 
@@ -115,3 +115,25 @@ def test_large_negative_bias_as_a_mask(dtype, bias_dtype, Sk, D, fill):
 	lse[0, 1, ::2] = 0
 	lse_ref[0, 1, ::2] = 0
 	check_forward(o, lse, o_ref, lse_ref, dtype, f"D{D} {fill}")
+
+
+@pytest.mark.parametrize("fill", [f for f in _FILLS if f != -1e6])
+@pytest.mark.parametrize("D,softcap", [(64, 0.0), (128, 0.0), (256, 0.0), (64, 20.0)])
+@pytest.mark.parametrize("dtype,bias_dtype,Sk", _MASKED)
+def test_gradients_of_a_large_negative_bias_as_a_mask(dtype, bias_dtype, Sk, D, softcap, fill):
+	"""A row whose keys are all hidden has a logsumexp that holds nothing of the sum any more: it passes no gradient on, whatever
+	gradient arrives at it, and it leaves the gradients of K and V to the other rows."""
+	Sq = 72
+	q, k, v, do = _masked_inputs(Sq, Sk, D, dtype)
+	bias = _masked(fill, bias_dtype, Sq, Sk)
+	a = [x.cuda() for x in (q, k, v)]
+	args = (bias.cuda(), None, None, 0.0, False, None, None, None, softcap)
+	o, lse = op.fwd(*a, *args)
+	got = op.bwd(*a, o, lse, do.cuda(), *args)
+	with_dbias = op.bwd(*a, o, lse, do.cuda(), *args, need_dbias=True)
+	do[:, ::2, 1] = 0
+	want = O.attention_bwd(f64(q), f64(k), f64(v), f64(do), f64(bias), softcap=softcap, return_dbias=True)
+	check_grads(got, want[:3], f"D{D} {fill}")
+	check_grads(with_dbias[:3], want[:3], f"D{D} {fill} with the gradient of the bias")
+	dbias = with_dbias[3].cpu().numpy()
+	assert np.isfinite(dbias).all() and O.rel_l2(dbias, want[3]) <= 1e-2
