@@ -1823,7 +1823,14 @@ hipError_t launch_bwd_v(KArgs& a, hipStream_t s) {
 		// of them, B4 Hq32 Hkv4 S1500 causal: 256 -> 284), and so it is against pairs of key tiles (B4 Hq16 Hkv4 S4096 causal 656 -> 732).
 		// Rows of 72 to 96 columns fit two workgroups a CU too, in tiles of 64 rows (128 would take 130 KiB of LDS): B64 H16 S257 D80
 		// 349 -> 303 us, B32 H16 S520 D88 444 -> 402, B7 H16 S1100 D96 333 -> 309, B8 H16 S1040 D72 causal 215 -> 202, B2 H16 S4096 D96 943 -> 925.
-		const bool blk = (D == 64 || DE < D) && !a.kv_pair && (int64_t)grid.x >= 2 * kNumCU;
+		// What they do not gain is balance: with all workgroups resident at once the longest two of a causal mask may share a CU, where one after the
+		// other the short ones fill up behind the long ones.  Backward, one workgroup a CU -> two, 512 workgroups: B4 H16 S1024 D80 causal 73.4 -> 81.4 us,
+		// of S2048 with key lengths 118 -> 125, in a window of 1791 112.5 -> 116; in one of 1023 104 -> 95, 1536 rows over 2048 keys 109 -> 104, four key tiles
+		// (B8 H16 S512 D96) 59 -> 54; 520 of them 140 -> 131.  With the steps split over workgroups up to 576: B1 Hkv8 S2048 Hq32 D80 127 -> 135, Hq128 394 -> 489, B4 Hq64
+		// Hkv8 S1000 D96 151 -> 174, B1 Hq144 Hkv12 S2000 (576) 577 -> 610, B8 Hq64 Hkv8 S512 (four tiles) 174 -> 182; two tiles 267 -> 240, 640 workgroups 664 -> 612.
+		const bool uneven = DE < D && a.win_right >= 0 && (a.win_left < 0 || 4 * (int64_t)a.win_left >= 3 * (int64_t)a.Sk) && 8 * (int64_t)a.Sq >= 7 * (int64_t)a.Sk;
+		const int64_t least = uneven && hs > 1 && a.kv_ntiles >= 4 ? 5 * kNumCU / 2 : uneven && hs == 1 && a.kv_ntiles >= 8 ? 2 * kNumCU + 1 : 2 * kNumCU;
+		const bool blk = (D == 64 || DE < D) && !a.kv_pair && (int64_t)grid.x >= least;
 		auto launch_dkdv = [&](auto blk_tag) {
 			constexpr bool BLK = decltype(blk_tag)::value;
 			// with bias at D = 128 the streamed tiles are 64 rows, which leaves LDS room for the bias tiles (and block by block for a second workgroup)

@@ -1,10 +1,12 @@
 """Head dims that run in the tiles of head dim 128 without padded copies of the operands: shortest and longest rows, query and key
 counts around the tiles, strided operands, and what surrounds the rows in memory (never read into a result, never written)."""
 
+import ctypes
+
 import pytest
 import torch
 
-from jax_flash_attn2 import _hip_op as op
+from jax_flash_attn2 import _hip_op as op, _lib
 import fa2_oracle as O
 from _cases import check_forward, check_grads, f64, make_inputs
 
@@ -21,7 +23,7 @@ pytestmark = pytest.mark.gpu
 		(1, 700, 700, 2, 2, 72, torch.bfloat16, True, None, (100, 0)),
 		(3, 1030, 1030, 32, 8, 80, torch.bfloat16, True, None, None),   # grids of more than one workgroup per CU
 		(8, 520, 5600, 16, 16, 96, torch.float16, False, None, None),   # keys of a head beyond what the smaller workgroups are for
-		(1, 2050, 2050, 64, 64, 88, torch.bfloat16, True, None, None),  # key tiles in pairs
+		(1, 2050, 2050, 64, 64, 88, torch.bfloat16, True, None, None),  # a bit more than two workgroups per CU
 	],
 )
 def test_short_rows_against_the_oracle(B, Sq, Sk, Hq, Hkv, D, dtype, causal, kv_lens, window):
@@ -111,3 +113,37 @@ def test_short_rows_block_by_block(Sq, Sk, kw, dtype, D):
 		want = O.attention_bwd(*[f64(x[bs, :, hs]) for x in (q, k, v, do)], causal=kw.get("causal", False), window=kw.get("window"),
 		                       kv_lens=None if kv_lens is None else kv_lens[bs])
 		check_grads([x[bs, :, hs] for x in g], want, f"Sq{Sq} Sk{Sk} D{D} {kw} b{b} h{h}")
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize(
+	"how,B,S,Hq,Hkv,D,window",
+	[
+		("split", 1, 2048, 32, 8, 80, None),                 # the steps of a key tile over several workgroups that leave partial sums
+		("split, blocks", 1, 2048, 32, 8, 80, (700, 0)),     # ... block by block
+		("split, blocks", 1, 2001, 32, 8, 96, (1000, 0)),    # ... a last key tile and a last row tile that are not whole
+		("blocks", 3, 1030, 40, 20, 72, None),               # block by block, two q-heads a kv-head
+		("one round", 4, 1024, 32, 16, 88, None),            # 512 workgroups of a causal mask: not block by block
+		("paired", 1, 2048, 32, 32, 88, None),               # two key tiles a workgroup
+		("paired", 1, 2030, 64, 32, 96, None),
+	],
+)
+def test_short_rows_by_the_plan_of_dkdv(how, B, S, Hq, Hkv, D, window, dtype):
+	q, k, v, do, _ = make_inputs(B, S, S, Hq, Hkv, D, dtype, seed=S + D)
+	qd, kd, vd, dod = (x.cuda() for x in (q, k, v, do))
+	# (the launcher's choice, from the sizes)
+	p, lib = op._block(128, q, k, v, None, None, 0.1, 0.0, True, None), _lib.load()
+	least, split = lib.fa2_bwd_scratch_bytes(ctypes.byref(p)), lib.fa2_bwd_split_scratch_bytes(ctypes.byref(p))
+	parts = (split - least) // (B * Hkv * S * 2 * 128 * 4) if split else 1
+	tiles = (S + 127) // 128
+	pairs, grid = (tiles + 1) // 2 * B * Hkv, B * Hkv * tiles * parts
+	assert (parts > 1) == ("split" in how)
+	assert (parts == 1 and window is None and tiles >= 16 and (pairs % 256 == 0 or pairs >= 2048)) == (how == "paired")
+	assert how == "paired" or (grid >= (512 if window else 640 if parts > 1 else 513)) == ("blocks" in how)
+	o, lse = op.fwd(qd, kd, vd, causal=True, window=window)
+	grads = op.bwd(qd, kd, vd, o, lse, dod, causal=True, window=window)
+	for b, hk in ((0, 0), (B - 1, Hkv - 1)):
+		r = Hq // Hkv
+		bs, hs, kv = slice(b, b + 1), slice(hk * r, hk * r + r), slice(hk, hk + 1)
+		a = [f64(x) for x in (q[bs, :, hs], k[bs, :, kv], v[bs, :, kv], do[bs, :, hs])]
+		check_grads([x[bs, :, y] for x, y in zip(grads, (hs, kv, kv))], O.attention_bwd(*a, causal=True, window=window), f"{how} S{S} D{D} b{b} hk{hk}")
