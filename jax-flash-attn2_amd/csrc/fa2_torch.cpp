@@ -55,6 +55,17 @@ float number(PyObject* o) {
 	return (float)x;
 }
 
+// An operand in other memory than q's is Python's to refuse (or to let pass: pinned host memory).
+const at::Tensor& beside(const at::Tensor& x, const at::Tensor& q) {
+	if (x.device() != q.device()) throw Other();
+	return x;
+}
+
+const int32_t* lengths(const at::Tensor& x, const at::Tensor& q, bool exact) {
+	if (beside(x, q).scalar_type() != at::kInt || !x.is_contiguous() || (exact ? x.numel() != q.size(0) : x.numel() < q.size(0))) throw Other();
+	return (const int32_t*)x.data_ptr();
+}
+
 // The kernels read 16 bytes at a time along the rows; anything else is copied first, by the Python code.
 fa2_tensor rows(const at::Tensor& x) {
 	const int64_t sb = x.stride(0), ss = x.stride(1), sh = x.stride(2);
@@ -101,11 +112,11 @@ void fill(fa2_params& p, const at::Tensor& q, const at::Tensor& k, const at::Ten
 	p.D = D <= 64 ? 64 : D <= 128 ? 128 : 256;
 	p.head_dim = (int32_t)D;
 	p.q = rows(q);
-	p.k = rows(k);
-	p.v = rows(v);
+	p.k = rows(beside(k, q));
+	p.v = rows(beside(v, q));
 
 	if (arg[0] != Py_None) {
-		const at::Tensor& bias = tensor(arg[0]);
+		const at::Tensor& bias = beside(tensor(arg[0]), q);
 		if (bias.dim() != 4 || bias.stride(3) != 1) throw Other();
 		p.bias = bias.data_ptr();
 		p.bias_dtype = bias_dtype(bias.scalar_type());
@@ -114,7 +125,7 @@ void fill(fa2_params& p, const at::Tensor& q, const at::Tensor& k, const at::Ten
 		p.bias_stride_h = bias.size(1) == 1 ? 0 : bias.stride(1);
 		p.bias_stride_m = bias.stride(2);
 	}
-	if (arg[1] != Py_None) p.seqlens = (const int32_t*)tensor(arg[1]).data_ptr();
+	if (arg[1] != Py_None) p.seqlens = lengths(tensor(arg[1]), q, false);
 	p.scale = arg[2] == Py_None ? (float)(1.0 / sqrt((double)D)) : number(arg[2]);
 	p.p_drop = number(arg[3]);
 	if (arg[4] != Py_True && arg[4] != Py_False) throw Other();
@@ -123,15 +134,11 @@ void fill(fa2_params& p, const at::Tensor& q, const at::Tensor& k, const at::Ten
 	} else if (PyLong_CheckExact(arg[5])) {
 		p.seed = PyLong_AsUnsignedLongLongMask(arg[5]);
 	} else {
-		const at::Tensor& seed = tensor(arg[5]);
-		if (seed.scalar_type() != at::kLong || seed.numel() != 1 || seed.device() != q.device()) throw Other();
+		const at::Tensor& seed = beside(tensor(arg[5]), q);
+		if (seed.scalar_type() != at::kLong || seed.numel() != 1) throw Other();
 		p.seed_dev = (const uint64_t*)seed.data_ptr();
 	}
-	if (arg[6] != Py_None) {
-		const at::Tensor& lens = tensor(arg[6]);
-		if (lens.scalar_type() != at::kInt || lens.numel() != p.B || !lens.is_contiguous()) throw Other();
-		p.kv_lens = (const int32_t*)lens.data_ptr();
-	}
+	if (arg[6] != Py_None) p.kv_lens = lengths(tensor(arg[6]), q, true);
 	if (arg[7] != Py_None) {
 		if (!PyTuple_CheckExact(arg[7]) || PyTuple_GET_SIZE(arg[7]) != 2) throw Other();
 		p.has_window = 1;
@@ -219,8 +226,9 @@ PyObject* backward(PyObject*, PyObject* const* arg, Py_ssize_t n) {
 		void* stream = PyLong_AsVoidPtr(arg[16]);
 		if (!stream && PyErr_Occurred()) throw python_error();
 		if (out.dim() != 4 || dout.dim() != 4) throw Other();
-		p.o = rows(out);
-		p.dout = rows(dout);
+		p.o = rows(beside(out, q));
+		p.dout = rows(beside(dout, q));
+		if (beside(lse, q).scalar_type() != at::kFloat || !lse.is_contiguous() || lse.numel() < (int64_t)p.B * p.Hq * p.Sq) throw Other();
 		p.lse = (float*)lse.data_ptr();
 		check_rows(lib, p, 1);
 		at::Tensor dq = like(q), dk = like(k), dv = like(v);

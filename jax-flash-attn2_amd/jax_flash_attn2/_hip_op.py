@@ -135,6 +135,18 @@ def _seed_fields(seed, device):
 	return int(seed or 0) & 0xFFFFFFFFFFFFFFFF, 0
 
 
+def _check_memory(q, seqlens=None, lse=None, **operands):
+	"""The kernels are given bare addresses: an operand in host memory or on another GPU would be a memory fault there, one of another
+	type wrong numbers.  (Pinned host memory has an address the GPU can read.)"""
+	B, Sq, Hq = q.shape[:3]
+	for name, x, dtype, n in (("seqlens", seqlens, torch.int32, B), ("lse", lse, torch.float32, B * Hq * Sq)):
+		if x is not None and (x.dtype != dtype or x.numel() < n or not x.is_contiguous()):
+			raise ValueError(f"{name} must be a contiguous {dtype} tensor with {n} entries")
+	for name, x in (*operands.items(), ("seqlens", seqlens), ("lse", lse)):
+		if x is not None and x.device != q.device and not (q.is_cuda and x.device.type == "cpu" and x.is_pinned()):
+			raise ValueError(f"{name} is on {x.device}, q on {q.device}")
+
+
 def _prep_bias(bias):
 	if bias is None:
 		return None
@@ -199,6 +211,7 @@ def fwd(q, k, v, bias=None, seqlens=None, softmax_scale=None, dropout_prob=0.0, 
 			_lib.check(res)
 		elif res is not None:
 			return res
+	_check_memory(q, seqlens, k=k, v=v, bias=bias, kv_lens=kv_lens)
 	lib = _lib.load()
 	D0 = q.shape[-1]
 	D = _kernel_head_dim(D0)
@@ -236,6 +249,7 @@ def bwd(q, k, v, out, lse, dout, bias=None, seqlens=None, softmax_scale=None, dr
 			_lib.check(res)
 		elif res is not None:
 			return res
+	_check_memory(q, seqlens, lse, k=k, v=v, bias=bias, kv_lens=kv_lens, out=out, dout=dout)
 	lib = _lib.load()
 	D0 = q.shape[-1]
 	D = _kernel_head_dim(D0)
@@ -294,6 +308,7 @@ class Plan:
 
 	def __init__(self, q, k, v, dout=None, bias=None, seqlens=None, softmax_scale=None, dropout_prob=0.0, causal=False,
 	             dropout_seed=None, kv_lens=None, window=None, softcap=0.0):
+		_check_memory(q, seqlens, k=k, v=v, bias=bias, kv_lens=kv_lens, dout=dout)
 		self.lib = _lib.load()
 		self.q, self.k, self.v = _usable(q), _usable(k), _usable(v)
 		self.bias = _prep_bias(bias)

@@ -190,3 +190,33 @@ def test_checks():
 	torch.func.vmap(lambda x: (seen.append(_fa2_torch.checked(x, x, x, None, None)), x)[1])(z(3, 2, 4, 4, 64, dtype=torch.float16))
 	torch.jit.trace(lambda x: (seen.append(_fa2_torch.checked(x, x, x, None, None)), x * 1)[1], (q,), check_trace=False)
 	assert seen and all(not f & 2 for f in seen), seen
+
+
+def test_operands_in_other_memory_are_refused():
+	"""An operand that is not where q is, lengths or a logsumexp of another type: nothing is launched, the Python code names it."""
+	rec = _Recorder()
+	q = _x(2, 4, 2, 64)
+	out, lse = torch.empty_like(q), torch.zeros(2, 2, 4)
+	lens = torch.full((2,), 3, dtype=torch.int32)
+	sound = dict(k=q, v=q, bias=torch.zeros(1, 1, 4, 4), seqlens=None, kv_lens=lens, out=out, lse=lse, dout=q)
+	cases = [(n, x.to("meta")) for n, x in sound.items() if x is not None] + [("seqlens", lens.to("meta"))]
+	cases += [("seqlens", lens.long()), ("seqlens", lens[:1]), ("kv_lens", lens.long()), ("lse", lse.double()), ("lse", lse.mT), ("lse", lse[:1])]
+
+	def block(d):
+		return (q, d["k"], d["v"], d["bias"], d["seqlens"], None, 0.0, False, None, d["kv_lens"], None, 0.0)
+
+	residuals = ("out", "lse", "dout")
+	assert _fa2_torch.forward(rec.bound, *block(sound), 0) is not None
+	assert _fa2_torch.backward(rec.bound, *block(sound), *(sound[n] for n in residuals), 0) is not None
+	assert len(rec.seen) == 2
+	for name, x in cases:
+		d = dict(sound, **{name: x})
+		if name not in residuals:
+			assert _fa2_torch.forward(rec.bound, *block(d), 0) is None, name
+			with pytest.raises(ValueError, match=name):
+				op.fwd(*block(d))
+		assert _fa2_torch.backward(rec.bound, *block(d), *(d[n] for n in residuals), 0) is None, name
+		b = block(d)
+		with pytest.raises(ValueError, match=name):
+			op.bwd(*b[:3], *(d[n] for n in residuals), *b[3:])
+	assert len(rec.seen) == 2
