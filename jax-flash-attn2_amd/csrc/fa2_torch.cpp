@@ -160,6 +160,7 @@ void check_rows(const Library& lib, const fa2_params& p, int which) {
 		if (t->stride_s > 0x7fffffff / 256) throw Other();
 }
 
+// Other threads run Python while outputs and scratch are allocated (which may be a hipMalloc) and the kernels are launched.
 struct NoGil {
 	PyThreadState* state = PyEval_SaveThread();
 	~NoGil() { PyEval_RestoreThread(state); }
@@ -188,18 +189,20 @@ PyObject* forward(PyObject*, PyObject* const* arg, Py_ssize_t n) {
 		fill(p, q, k, v, arg + 4);
 		void* stream = PyLong_AsVoidPtr(arg[13]);
 		if (!stream && PyErr_Occurred()) throw python_error();
-		check_rows(lib, p, 0);
-		at::Tensor out = like(q), lse = at::empty({p.B, p.Hq, p.Sq}, q.options().dtype(at::kFloat)), scratch;
-		p.o = rows(out);
-		p.lse = (float*)lse.data_ptr();
-		if (size_t need = lib.fwd_scratch(&p)) {
-			scratch = bytes(need, q);
-			p.scratch = scratch.data_ptr();
-			p.scratch_bytes = need;
-		}
+		at::Tensor out, lse, scratch;
 		int rc;
 		{
 			NoGil released;
+			check_rows(lib, p, 0);
+			out = like(q);
+			lse = at::empty({p.B, p.Hq, p.Sq}, q.options().dtype(at::kFloat));
+			p.o = rows(out);
+			p.lse = (float*)lse.data_ptr();
+			if (size_t need = lib.fwd_scratch(&p)) {
+				scratch = bytes(need, q);
+				p.scratch = scratch.data_ptr();
+				p.scratch_bytes = need;
+			}
 			rc = lib.fwd(&p, stream);
 		}
 		if (rc) return PyLong_FromLong(rc);
@@ -230,19 +233,22 @@ PyObject* backward(PyObject*, PyObject* const* arg, Py_ssize_t n) {
 		p.dout = rows(beside(dout, q));
 		if (beside(lse, q).scalar_type() != at::kFloat || !lse.is_contiguous() || lse.numel() < (int64_t)p.B * p.Hq * p.Sq) throw Other();
 		p.lse = (float*)lse.data_ptr();
-		check_rows(lib, p, 1);
-		at::Tensor dq = like(q), dk = like(k), dv = like(v);
-		p.dq = rows(dq);
-		p.dk = rows(dk);
-		p.dv = rows(dv);
-		const size_t least = lib.bwd_scratch(&p), split = lib.bwd_split_scratch(&p);
-		const size_t need = least > split ? least : split;
-		at::Tensor scratch = bytes(need > 256 ? need : 256, q);
-		p.scratch = scratch.data_ptr();
-		p.scratch_bytes = need > 256 ? need : 256;
+		at::Tensor dq, dk, dv, scratch;
 		int rc;
 		{
 			NoGil released;
+			check_rows(lib, p, 1);
+			dq = like(q);
+			dk = like(k);
+			dv = like(v);
+			p.dq = rows(dq);
+			p.dk = rows(dk);
+			p.dv = rows(dv);
+			const size_t least = lib.bwd_scratch(&p), split = lib.bwd_split_scratch(&p);
+			const size_t need = least > split ? least : split;
+			scratch = bytes(need > 256 ? need : 256, q);
+			p.scratch = scratch.data_ptr();
+			p.scratch_bytes = need > 256 ? need : 256;
 			rc = lib.bwd(&p, stream);
 		}
 		if (rc) return PyLong_FromLong(rc);

@@ -220,3 +220,16 @@ def test_operands_in_other_memory_are_refused():
 		with pytest.raises(ValueError, match=name):
 			op.bwd(*b[:3], *(d[n] for n in residuals), *b[3:])
 	assert len(rec.seen) == 2
+
+
+def test_other_threads_run_while_a_call_allocates_and_launches():
+	held = ctypes.cast(ctypes.pythonapi.PyGILState_Check, ctypes.c_void_p).value  # (1 where the calling thread holds the interpreter's lock)
+	rec = _Recorder()
+	at = ctypes.cast(rec.keep, ctypes.c_void_p).value
+	q = _x(1, 4, 2, 64)
+	call = (q, q, q, None, None, None, 0.0, False, None, None, None, 0.0)
+	# the size of the scratch is asked for between the allocation of the outputs and that of the scratch
+	out, lse = _fa2_torch.forward(_fa2_torch.bind(at, at, held, held, held, held), *call, 0)
+	assert not rec.seen[0][0].scratch
+	for entry, args in ((_fa2_torch.forward, (0,)), (_fa2_torch.backward, (out, lse, q, 0))):
+		assert isinstance(entry(_fa2_torch.bind(*[held] * 6), *call, *args), tuple)  # (an error code of 1 otherwise)
