@@ -4,6 +4,8 @@
 // backward of B1 H4 S64 137 -> 87).  Entry points are the same ones of include/fa2.h, given as addresses by whoever has opened
 // libfa2_hip.so (_lib.py).
 //
+// Nothing depends on it but time: where it is not built, or for another torch or Python, the Python code makes every call.
+//
 // A call that needs anything else - a copy of an operand for its alignment, a padded head dim, a bias of another type, a tensor
 // subclass - is left to the Python code (None is returned before anything has been launched), and so is every error of an argument's form.
 #define PY_SSIZE_T_CLEAN
@@ -326,4 +328,12 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_fa2_torch", nullptr, -1, methods,
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__fa2_torch() { return PyModule_Create(&module); }
+#define FA2_STRING_(x) #x
+#define FA2_STRING(x) FA2_STRING_(x)
+
+PyMODINIT_FUNC PyInit__fa2_torch() {
+	PyObject* m = PyModule_Create(&module);
+	// (FA2_TORCH_VERSION: from the Makefile.  Another torch may lay its tensors out otherwise and load this file all the same.)
+	if (m && PyModule_AddObject(m, "built_for", PyUnicode_FromFormat("%s %d.%d", FA2_STRING(FA2_TORCH_VERSION), PY_MAJOR_VERSION, PY_MINOR_VERSION))) Py_CLEAR(m);
+	return m;
+}

@@ -17,18 +17,35 @@ from __future__ import annotations
 
 import ctypes
 import math
+import sys
 import typing as tp
+import warnings
 
 import torch
 
 from . import _lib
-
-try:
-	from . import _fa2_torch
-except ImportError as e:
-	raise ImportError(f"the extension module _fa2_torch is missing or does not load ({e}): build it with `make -C csrc` as libfa2_hip.so") from e
 from ._checks import check_shapes  # noqa: F401  (re-exported)
 from ._lib import FA2_BF16, FA2_FP16, FA2_FP32, FA2_MASK_U8
+
+
+def _load_extension():
+	"""The extension that makes ordinary calls (csrc/fa2_torch.cpp), or None: the Python code below serves every call too, it only takes
+	longer about it.  It is built for one torch and one Python."""
+	here = f"{torch.__version__} {sys.version_info[0]}.{sys.version_info[1]}"
+	try:
+		from . import _fa2_torch as ext
+
+		built_for = getattr(ext, "built_for", None)
+		if built_for == here:
+			return ext
+		why = f"built for torch and Python {built_for}, not {here}"
+	except ImportError as e:
+		why = str(e)
+	warnings.warn(f"the extension _fa2_torch is not used ({why}): calls spend more time on the host; `make -C csrc` builds it", RuntimeWarning, stacklevel=3)
+	return None
+
+
+_fa2_torch = _load_extension()
 
 _DTYPES = {torch.float16: FA2_FP16, torch.bfloat16: FA2_BF16}
 # (a uint8 / bool `bias` is a boolean mask, one byte per position: see fa2_params.bias_dtype)
@@ -203,7 +220,7 @@ def _entry_points():
 def fwd(q, k, v, bias=None, seqlens=None, softmax_scale=None, dropout_prob=0.0, causal=False, dropout_seed=None, kv_lens=None,
         window=None, softcap=0.0):
 	"""Returns (out [B,Sq,Hq,D] in q.dtype, lse [B,Hq,Sq] fp32 natural log)."""
-	if q.is_cuda:
+	if _fa2_torch is not None and q.is_cuda:
 		# an ordinary call: plain tensors in order for the kernels (anything else: None, and what follows copies, pads or refuses)
 		res = _fa2_torch.forward(_entry_points(), q, k, v, bias, seqlens, softmax_scale, dropout_prob, causal, dropout_seed, kv_lens, window,
 		                         softcap, _stream_ptr(q.device))
@@ -242,7 +259,7 @@ def bwd(q, k, v, out, lse, dout, bias=None, seqlens=None, softmax_scale=None, dr
 	"""Returns (dq, dk, dv) in the dtypes of q, k, v; dk/dv summed over each KV group.  With `need_dbias` a fourth
 	result: the gradient of the additive bias, fp32, in the shape of `bias` (summed over the axes it is broadcast on;
 	those sums are atomic adds in the dQ kernel - see fa2_params.dbias - so the buffer is as small as the bias)."""
-	if q.is_cuda and not need_dbias:
+	if _fa2_torch is not None and q.is_cuda and not need_dbias:
 		res = _fa2_torch.backward(_entry_points(), q, k, v, bias, seqlens, softmax_scale, dropout_prob, causal, dropout_seed, kv_lens, window,
 		                          softcap, out, lse, dout, _stream_ptr(q.device))
 		if res.__class__ is int:
@@ -411,7 +428,7 @@ def flash_attention(
 	if attention_mask is not None and attention_mask.dim() == 4:
 		assert bias is None, "Attention mask is not supported along with attention bias. Just use bias instead."
 		bias, attention_mask = _mask_operand(attention_mask, q), None
-	flags = _fa2_torch.checked(q, k, v, bias, attention_mask)
+	flags = 0 if _fa2_torch is None else _fa2_torch.checked(q, k, v, bias, attention_mask)
 	if not flags:
 		check_shapes(q, k, v, bias, attention_mask)
 	seqlens = _seqlens_from_mask(attention_mask, q)

@@ -4,6 +4,9 @@ takes, and leaves the others - and every error of an argument's form - to the Py
 import ctypes
 import itertools
 import math
+import os
+import subprocess
+import sys
 
 import pytest
 import torch
@@ -233,3 +236,51 @@ def test_other_threads_run_while_a_call_allocates_and_launches():
 	assert not rec.seen[0][0].scratch
 	for entry, args in ((_fa2_torch.forward, (0,)), (_fa2_torch.backward, (out, lse, q, 0))):
 		assert isinstance(entry(_fa2_torch.bind(*[held] * 6), *call, *args), tuple)  # (an error code of 1 otherwise)
+
+
+@pytest.mark.parametrize("how", ["missing", "of another torch"])
+def test_without_the_extension(how):
+	"""Python makes every call, says so once and refuses what it did."""
+	code = """
+import sys, types, warnings
+import torch
+import jax_flash_attn2
+if sys.argv[1] == "missing":
+	sys.modules["jax_flash_attn2._fa2_torch"] = None
+else:
+	other = sys.modules["jax_flash_attn2._fa2_torch"] = jax_flash_attn2._fa2_torch = types.ModuleType("other")
+	other.built_for = "1.0 2.7"
+with warnings.catch_warnings(record=True) as seen:
+	warnings.simplefilter("always")
+	from jax_flash_attn2 import _hip_op as op
+assert op._fa2_torch is None
+assert [w.category for w in seen if "_fa2_torch" in str(w.message)] == [RuntimeWarning]
+q = torch.zeros(1, 4, 2, 64, dtype=torch.bfloat16)
+for args, error in (((q, q, q), ValueError), ((q, q[:, :, :, :8], q), AssertionError)):
+	try:
+		op.flash_attention(*args)
+	except error as e:
+		print(type(e).__name__, e)
+"""
+	env = dict(os.environ, PYTHONPATH=os.path.dirname(os.path.dirname(op.__file__)))
+	r = subprocess.run([sys.executable, "-c", code, how], env=env, capture_output=True, text=True, timeout=300)
+	assert r.returncode == 0, r.stderr
+	assert "ValueError Expected a cuda device" in r.stdout and "AssertionError key shape" in r.stdout
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [64, 80, 40])
+def test_the_python_code_makes_the_same_calls(monkeypatch, D):
+	g = torch.Generator(device="cuda").manual_seed(D)
+	q, do = (torch.empty(2, 130, 4, D, dtype=torch.float16, device="cuda").normal_(generator=g) for _ in range(2))
+	k, v = (torch.empty(2, 130, 2, D, dtype=torch.float16, device="cuda").normal_(generator=g) for _ in range(2))
+	for x in (q, k, v):
+		x.requires_grad_()
+	got = []
+	for ext in (_fa2_torch, None):
+		monkeypatch.setattr(op, "_fa2_torch", ext)
+		out = op.flash_attention(q, k, v, causal=True)
+		with torch.no_grad():
+			got.append((out, *torch.autograd.grad(out, (q, k, v), do), op.flash_attention(q, k, v, causal=True)))
+	for a, b in zip(*got):
+		assert torch.equal(a, b)
