@@ -261,12 +261,13 @@ PyObject* backward(PyObject*, PyObject* const* arg, Py_ssize_t n) {
 	END_HANDLE_TH_ERRORS
 }
 
-// checked(q, k, v, bias, attention_mask) -> 1: the shapes and types are in order (0: the Python code says what is not, or looks at what
-// this does not); + 2: nothing differentiates, batches or traces the call, so that no autograd function has to stand around it
+// checked(q, k, v, bias, attention_mask, *numbers) -> 1: the shapes and types are in order (0: the Python code says what is not, or
+// looks at what this does not); + 2: nothing differentiates, batches or traces the call, so that no autograd function has to stand around
+// it.  (`numbers`: the further arguments that may be tensors with a gradient.)
 PyObject* checked(PyObject*, PyObject* const* arg, Py_ssize_t n) {
 	HANDLE_TH_ERRORS
-	if (n != 5) {
-		PyErr_SetString(PyExc_TypeError, "checked takes 5 arguments");
+	if (n < 5) {
+		PyErr_SetString(PyExc_TypeError, "checked takes 5 arguments or more");
 		return nullptr;
 	}
 	try {
@@ -289,7 +290,9 @@ PyObject* checked(PyObject*, PyObject* const* arg, Py_ssize_t n) {
 		}
 		const bool transformed = c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode) ||
 		                         c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerBackMode);
-		const bool plain = !(grad && c10::GradMode::is_enabled()) && !forward_ad && !transformed && !torch::jit::tracer::isTracing();
+		bool numbers = true;
+		for (Py_ssize_t i = 5; i < n; ++i) numbers = numbers && (arg[i] == Py_None || PyFloat_CheckExact(arg[i]) || PyLong_CheckExact(arg[i]));
+		const bool plain = numbers && !(grad && c10::GradMode::is_enabled()) && !forward_ad && !transformed && !torch::jit::tracer::isTracing();
 		return PyLong_FromLong(plain ? 3 : 1);
 	} catch (const Other&) {
 		return PyLong_FromLong(0);

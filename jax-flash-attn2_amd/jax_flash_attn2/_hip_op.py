@@ -428,7 +428,7 @@ def flash_attention(
 	if attention_mask is not None and attention_mask.dim() == 4:
 		assert bias is None, "Attention mask is not supported along with attention bias. Just use bias instead."
 		bias, attention_mask = _mask_operand(attention_mask, q), None
-	flags = 0 if _fa2_torch is None else _fa2_torch.checked(q, k, v, bias, attention_mask)
+	flags = 0 if _fa2_torch is None else _fa2_torch.checked(q, k, v, bias, attention_mask, softmax_scale, dropout_prob, softcap)
 	if not flags:
 		check_shapes(q, k, v, bias, attention_mask)
 	seqlens = _seqlens_from_mask(attention_mask, q)

@@ -284,3 +284,15 @@ def test_the_python_code_makes_the_same_calls(monkeypatch, D):
 			got.append((out, *torch.autograd.grad(out, (q, k, v), do), op.flash_attention(q, k, v, causal=True)))
 	for a, b in zip(*got):
 		assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("which", ["softmax_scale", "dropout_prob", "softcap"])
+def test_a_number_that_requires_a_gradient_keeps_the_autograd_function(monkeypatch, which):
+	"""(The operator returns none for it, but its result is part of the graph.)"""
+	monkeypatch.setattr(op, "fwd", lambda q, *a: (torch.zeros_like(q), torch.zeros(1)))
+	q = _x(1, 4, 2, 64)
+	x = torch.tensor(0.5, requires_grad=True)
+	assert op.flash_attention(q, q, q, **{which: x}).requires_grad
+	assert not op.flash_attention(q, q, q, **{which: x.detach()}).requires_grad
+	with torch.no_grad():
+		assert not op.flash_attention(q, q, q, **{which: x}).requires_grad
