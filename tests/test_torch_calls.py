@@ -45,6 +45,9 @@ def _x(*shape, dtype=torch.bfloat16, form="plain"):
 		return torch.zeros((1, S, H, D), dtype=dtype).expand(B, S, H, D)
 	if form == "reversed axes":
 		return torch.zeros((D, H, S, B), dtype=dtype).permute(3, 2, 1, 0)
+	if form == "far rows":  # beyond what the kernels address short rows by
+		far = 0x7FFFFFFF // 256 // 8 * 8 + 8
+		return torch.empty((S - 1) * far + H * D, dtype=dtype).as_strided(shape, (S * far, far, D, 1))
 	assert form == "odd address"
 	n = B * S * H * D
 	return torch.zeros(n + 8, dtype=dtype)[1 : n + 1].view(shape)
@@ -70,41 +73,78 @@ def _scale(q, s):
 
 
 _SIZES = [(2, 5, 9, 4, 2, 64), (1, 1, 1029, 32, 8, 128), (2, 130, 130, 2, 2, 256), (1, 257, 257, 2, 1, 80), (1, 40, 40, 1, 1, 96)]
-_FORMS = ["plain", "heads first", "slice", "one batch row"]
+_FORMS = ["plain", "heads first", "slice", "one batch row", "odd address"]
+
+
+def _in_order(x, short):
+	"""Whether the kernels take the tensor as it lies (`short`: rows of fewer columns than theirs)."""
+	sb, ss, sh, sd = x.stride()
+	return sd == 1 and not (sb | ss | sh) % 8 and not x.data_ptr() % 16 and not (short and ss > 0x7FFFFFFF // 256)
+
+
+def _check_forward(rec, q, k, v):
+	B, Sq, Hq, D = q.shape
+	call = (None, None, None, 0.0, True, None, None, None, 0.0)
+	Dk, lib, launched = op._kernel_head_dim(D), _lib.load(), len(rec.seen)
+	res = _fa2_torch.forward(rec.bound, q, k, v, *call, 77)
+	want = (None, None, _scale(q, None), 0.0, True, None, None, None, 0.0)
+	served = all(_in_order(x, D < Dk) for x in (q, k, v)) and (D == Dk or op._runs_unpadded(lib, 0, Dk, q, k, v, *want))
+	assert (res is not None) == served and len(rec.seen) == launched + served
+	if not served:
+		return False
+	out, lse = res
+	assert out.shape == q.shape and out.is_contiguous() and out.dtype == q.dtype and lse.shape == (B, Hq, Sq) and lse.dtype == torch.float32
+	p, stream = rec.seen[-1]
+	assert stream == 77
+	_same(p, op._block(Dk, q, k, v, *want, op._t4(out), lse))
+	assert (p.scratch_bytes or 0) == lib.fa2_fwd_scratch_bytes(ctypes.byref(p))
+	assert bool(p.scratch) == bool(p.scratch_bytes)
+	return True
+
+
+def _check_backward(rec, q, k, v, out, dout):
+	B, Sq, Hq, D = q.shape
+	call = (None, None, None, 0.0, True, None, None, None, 0.0)
+	Dk, lib, launched = op._kernel_head_dim(D), _lib.load(), len(rec.seen)
+	lse = torch.zeros((B, Hq, Sq))
+	res = _fa2_torch.backward(rec.bound, q, k, v, *call, out, lse, dout, 5)
+	want = (None, None, _scale(q, None), 0.0, True, None, None, None, 0.0)
+	served = all(_in_order(x, D < Dk) for x in (q, k, v, out, dout)) and (D == Dk or op._runs_unpadded(lib, 1, Dk, q, k, v, *want))
+	assert (res is not None) == served and len(rec.seen) == launched + served
+	if not served:
+		return False
+	dq, dk, dv = res
+	p, stream = rec.seen[-1]
+	assert stream == 5 and dq.shape == q.shape and dk.shape == k.shape and dv.shape == v.shape
+	assert dq.is_contiguous() and dk.is_contiguous() and dv.is_contiguous()
+	_same(p, op._block(Dk, q, k, v, *want, op._t4(out), lse, (op._t4(dout), op._t4(dq), op._t4(dk), op._t4(dv))))
+	assert p.scratch and p.scratch_bytes == max(256, lib.fa2_bwd_scratch_bytes(ctypes.byref(p)), lib.fa2_bwd_split_scratch_bytes(ctypes.byref(p)))
+	return True
 
 
 @pytest.mark.parametrize("B,Sq,Sk,Hq,Hkv,D", _SIZES)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
 def test_blocks_over_strides(B, Sq, Sk, Hq, Hkv, D, dtype):
-	rec = _Recorder()
+	rec, served = _Recorder(), []
 	for fq, fk in itertools.product(_FORMS, _FORMS):
 		q, k, v = _x(B, Sq, Hq, D, dtype=dtype, form=fq), _x(B, Sk, Hkv, D, dtype=dtype, form=fk), _x(B, Sk, Hkv, D, dtype=dtype)
-		call = (None, None, None, 0.0, True, None, None, None, 0.0)
-		res = _fa2_torch.forward(rec.bound, q, k, v, *call, 77)
-		Dk = op._kernel_head_dim(D)
-		usable = op._usable if D == Dk else op._usable_short
-		served = all(usable(x) is x for x in (q, k, v)) if D == Dk or op._runs_unpadded(_lib.load(), 0, Dk, q, k, v, None, None, 0.1, 0.0, True, None) else False
-		assert (res is not None) == served or (D != Dk and res is not None)
-		if res is None:
-			continue
-		out, lse = res
-		assert out.shape == q.shape and out.is_contiguous() and out.dtype == dtype and lse.shape == (B, Hq, Sq) and lse.dtype == torch.float32
-		p, stream = rec.seen[-1]
-		assert stream == 77
-		_same(p, op._block(Dk, q, k, v, None, None, _scale(q, None), 0.0, True, None, None, None, 0.0, op._t4(out), lse))
-		assert (p.scratch_bytes or 0) == _lib.load().fa2_fwd_scratch_bytes(ctypes.byref(p))
-		assert bool(p.scratch) == bool(p.scratch_bytes)
-		dout = _x(B, Sq, Hq, D, dtype=dtype, form=fq)
-		if usable(dout) is not dout:
-			continue
-		dq, dk, dv = _fa2_torch.backward(rec.bound, q, k, v, *call, out, lse, dout, 5)
-		p, stream = rec.seen[-1]
-		assert stream == 5 and dq.shape == q.shape and dk.shape == k.shape and dv.shape == v.shape
-		assert dq.is_contiguous() and dk.is_contiguous() and dv.is_contiguous()
-		_same(p, op._block(Dk, q, k, v, None, None, _scale(q, None), 0.0, True, None, None, None, 0.0, op._t4(out), lse,
-		                   (op._t4(dout), op._t4(dq), op._t4(dk), op._t4(dv))))
-		lib = _lib.load()
-		assert p.scratch and p.scratch_bytes == max(256, lib.fa2_bwd_scratch_bytes(ctypes.byref(p)), lib.fa2_bwd_split_scratch_bytes(ctypes.byref(p)))
+		served.append(_check_forward(rec, q, k, v))
+		served.append(_check_forward(rec, q, v, k))
+		for fo in _FORMS:
+			o, do = _x(B, Sq, Hq, D, dtype=dtype), _x(B, Sq, Hq, D, dtype=dtype, form=fo)
+			served.append(_check_backward(rec, q, k, v, o, do))
+			served.append(_check_backward(rec, q, v, k, do, o))
+	assert any(served) and not all(served)
+
+
+@pytest.mark.parametrize("D", [64, 80])
+def test_blocks_of_rows_far_apart(D):
+	rec = _Recorder()
+	near, far = _x(1, 2, 1, D), _x(1, 2, 1, D, form="far rows")
+	for i in range(3):
+		assert _check_forward(rec, *(far if i == j else near for j in range(3))) == (D == 64)
+	for i in range(5):
+		assert _check_backward(rec, *(far if i == j else near for j in range(5))) == (D == 64)
 
 
 def _biases(B, Hq, Hkv, Sq, Sk):
