@@ -1132,9 +1132,8 @@ __global__ __launch_bounds__(256) void bwd_dkdv_reduce_kernel(const KArgs a, flo
 	u32x4 pk = {pack2<typename T::V2>(acc[0] * sc, acc[1] * sc), pack2<typename T::V2>(acc[2] * sc, acc[3] * sc),
 	            pack2<typename T::V2>(acc[4] * sc, acc[5] * sc), pack2<typename T::V2>(acc[6] * sc, acc[7] * sc)};
 	char* op_ = out.ptr + (int64_t)b * out.sb + (int64_t)hk * out.sh + (int64_t)key * out.ss + ch * 16;
-	// (rows of dk / dv need not be 16-byte aligned: two 8-byte stores)
-	*(u32x2*)op_ = u32x2{pk[0], pk[1]};
-	*(u32x2*)(op_ + 8) = u32x2{pk[2], pk[3]};
+	// (the C ABI takes dk and dv with rows that start on 16 bytes only)
+	*(u32x4*)op_ = pk;
 }
 
 // ---------------------------------------------------------------------------
@@ -1724,7 +1723,8 @@ __global__ __launch_bounds__(NW * 64, WPS) void bwd_dq_kernel(const KArgs a) {
 
 template <typename T, int D>
 struct BwdCfg {
-	// dK/dV: 4 waves x 32 keys; query rows streamed 64 (32 for D = 256) at a time
+	// dK/dV: 4 waves x 32 keys; query rows streamed 128 (32 for D = 256) at a time, 64 with bias at D = 128 and where the launcher goes block by
+	// block with bias or in tiles of D = 128
 	static constexpr int KV_NW = 4;
 	static constexpr int KV_QB = D <= 128 ? 4 : 1;
 	static constexpr int KV_BN = KV_NW * 32;
