@@ -1695,6 +1695,9 @@ __global__ __launch_bounds__(NW * 64, WPS) void bwd_dq_kernel(const KArgs a) {
 	for (int t = t_lo; t < t_full; ++t) step(std::false_type{}, t);
 	for (int t = t_full; t < ntiles; ++t) step(std::true_type{}, t);
 
+	// (Stored 16 bytes a lane as the other results are (pair_cols) the variants of head dim 64 without bias take 88 registers instead of 84 and the loop
+	// above is slower than what the stores gain: B64 H16 S257 59 -> 66 us, B32 H12 S511 55 -> 60, B16 Hq16 Hkv4 S1024 causal 70 -> 75, B8 H16 S2048 194 -> 204.)
+	constexpr bool HALVES = D == 64 && !BIAS;
 	char* obase = a.dq.ptr + (int64_t)b * a.dq.sb + (int64_t)h * a.dq.sh;
 #pragma unroll
 	for (int qb = 0; qb < QB; ++qb) {
@@ -1713,9 +1716,14 @@ __global__ __launch_bounds__(NW * 64, WPS) void bwd_dq_kernel(const KArgs a) {
 					for (int u = 0; u < 2; ++u)
 						pk[u] = u32x2{pack2<typename T::V2>(x[4 * (aa + u)] * sc, x[4 * (aa + u) + 1] * sc),
 						              pack2<typename T::V2>(x[4 * (aa + u) + 2] * sc, x[4 * (aa + u) + 3] * sc)};
-					const u32x4 y = pair_cols(pk[0], pk[1]);
-					const int col = 32 * db + 8 * (aa + g);
-					if (!COLS || col < a.hd) *(u32x4*)(rp + col * 2) = y;
+					if constexpr (HALVES) {
+						*(u32x2*)(rp + (32 * db + 8 * aa + 4 * g) * 2) = pk[0];
+						*(u32x2*)(rp + (32 * db + 8 * aa + 8 + 4 * g) * 2) = pk[1];
+					} else {
+						const u32x4 y = pair_cols(pk[0], pk[1]);
+						const int col = 32 * db + 8 * (aa + g);
+						if (!COLS || col < a.hd) *(u32x4*)(rp + col * 2) = y;
+					}
 				}
 		}
 	}
