@@ -82,7 +82,9 @@ typedef struct fa2_params {
 	/* Optional additive bias [B|1, Hq|Hkv|1, Sq, Sk], unit stride on Sk.
 	 * stride 0 on batch / head = broadcast (calc_bias_strides, _utils.py:151-193).
 	 * bias_group != 0: the head axis has Hkv entries and q-head h reads entry
-	 * h / (Hq/Hkv) (flash_attention.py:161-164 materialises this repeat).   */
+	 * h / (Hq/Hkv) (flash_attention.py:161-164 materialises this repeat).
+	 * A row whose keys are all masked by a large negative bias is the plain average of V; its lse is that bias, and beyond
+	 * 2^24, where fp32 keeps nothing of the sum beside it, the row passes no gradient on.   */
 	const void* bias;       /* NULL = no bias                              */
 	int32_t bias_dtype;     /* FA2_FP16 | FA2_BF16 | FA2_FP32, or FA2_MASK_U8: `bias` then points to a
 	                           boolean mask, one byte per position (0 = masked), same shape and stride

@@ -153,8 +153,8 @@ FA2_DEV float pair_sum(float x) {
 // Lanes l and l^32 hold four columns each of two blocks of eight columns of a row, x of the first and y of the second (the lower lane the
 // columns 0 .. 3): the lower lane gets the whole first block, the upper lane the second.
 // The kernels end with it: half as many stores, of 16 bytes, 32 bytes of a row next to each other instead of 16.  Where workgroups live for few steps their
-// stores are a part of the time: forward and backward B64 H16 S257 D80 302 -> 284 us, B8 H16 S2048 D64 with a shared bias 797 -> 773, B8 H16 S2048 D256
-// with dropout 1704 -> 1684, B4 Hq32 Hkv8 S4096 D128 0.7 % (O, dQ, dK and dV start every row on 16 bytes: the C ABI checks it).
+// stores are a part of the time: forward and backward B64 H16 S257 D80 302 -> 284 us, B8 H16 S2048 D64 with a shared bias 797 -> 789, B8 H16 S2048 D256
+// with dropout 1704 -> 1684 (O, dQ, dK and dV start every row on 16 bytes: the C ABI checks it).  Not dQ at head dim 64 without bias, see there.
 FA2_DEV u32x4 pair_cols(u32x2 x, u32x2 y) {
 	auto r0 = __builtin_amdgcn_permlane32_swap((int)x[0], (int)y[0], false, false);
 	auto r1 = __builtin_amdgcn_permlane32_swap((int)x[1], (int)y[1], false, false);
