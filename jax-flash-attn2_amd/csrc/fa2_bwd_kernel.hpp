@@ -1765,7 +1765,7 @@ hipError_t launch_bwd_v(KArgs& a, hipStream_t s) {
 		a.mtiles = (a.Sq + BM - 1) / BM;
 		a.interleave = a.xcd_remap == 1 ? launch_order(a, a.Hq / a.Hkv, groups / 8, (int64_t)a.Sk * DE * 4) : 1;
 		dim3 grid((unsigned)(a.mtiles * a.B * a.Hq)), block(NW * 64);
-		a.fold_half = fold_half_of(a, NW, (int64_t)grid.x, D == 64 || WPS == 2);
+		a.fold = fold_of(a, NW, (int64_t)grid.x, D == 64 || WPS == 2 ? 2 : 1);
 		if constexpr (BIAS) {
 			if (a.dbias && a.softcap > 0.f)
 				hipLaunchKernelGGL((bwd_dq_kernel<T, D, NW, C::DQ_QB, WPS, true, DROP, false, true, true>), grid, block, 0, s, a);

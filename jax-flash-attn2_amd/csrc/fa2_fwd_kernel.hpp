@@ -57,14 +57,12 @@ inline int launch_order(const KArgs& a, int heads, int per_xcd, int64_t stream_b
 	return e;
 }
 
-// Workgroup ids of the first half of a causal grid that runs two 4-wave workgroups per CU (see decode_block), else 0.
-// two_per_cu: the kernel variant leaves room for two workgroups on a CU (registers, LDS).  Measured with and without,
-// B2 Hq8 Hkv2 S4096 D128 forward 0.086 / 0.109 ms (unfolded, the two batch rows put their long tiles on the same CUs),
-// a single group B1 Hq8 S8192 0.163 / 0.168 ms.
-inline int fold_half_of(const KArgs& a, int nw, int64_t total, bool two_per_cu) {
-	if (!two_per_cu || nw != 4 || !a.causal || a.win_left >= 0 || a.xcd_remap > 1) return 0;
-	if (total <= kNumCU || total > 2 * kNumCU || total % 16) return 0;
-	return (int)(total / 2);
+// Workgroups of a causal grid that are all resident at once, several on a CU (see decode_block), else 0.  per_cu: workgroups of the kernel variant that fit
+// a CU (registers, LDS).  Measured with and without, two a CU: B2 Hq8 Hkv2 S4096 D128 forward 0.086 / 0.109 ms (unfolded, the two batch rows put their long
+// tiles on the same CUs), a single group B1 Hq8 S8192 0.163 / 0.168 ms; three and four a CU: B6 Hq16 Hkv4 S1000 D64 33.7 / 28.7 us, B8 33.5 / 40.9.
+inline int fold_of(const KArgs& a, int nw, int64_t total, int per_cu) {
+	if (nw != 4 || !a.causal || a.win_left >= 0 || a.xcd_remap > 1) return 0;
+	return total > kNumCU && total <= per_cu * kNumCU ? (int)total : 0;
 }
 
 // The i-th (batch, kv-head) group of an XCD.  Rows that are not whole 128-byte lines share lines with the rows of the next head: on
@@ -74,15 +72,20 @@ inline int xcd_ranges_of(const KArgs& a) { return a.hd % 64 != 0 && !a.seqlens &
 FA2_DEV int group_on_xcd(const KArgs& a, int i, int xcd) { return a.xcd_ranges ? xcd * ((a.B * a.Hkv) >> 3) + i : i * 8 + xcd; }
 
 FA2_DEV void decode_block(const KArgs& a, int& mt, int& h, int& b, int id = (int)blockIdx.x) {
-	if (a.fold_half && id >= a.fold_half) {
-		// A causal grid of two workgroups per CU, all resident at once: the first half of the workgroup ids takes the
-		// first place of every CU, the second half the second place in the same order of CUs.  The first half runs
-		// from the longest tile down; the second half is visited backwards, so that the CU with the longest tile of
-		// the first half gets the shortest of the second (on every XCD for itself when groups are placed by XCD).
-		if (a.xcd_remap)
-			id = (((a.fold_half >> 3) + ((a.fold_half >> 2) - 1 - (id >> 3))) << 3) | (id & 7);
-		else
-			id = a.fold_half + (2 * a.fold_half - 1 - id);
+	if (a.fold) {
+		// A causal grid whose workgroups are all resident at once: the first 256 workgroup ids take the first place of every CU, the next 256 the
+		// second place in the same order of CUs, and so on (32 ids of every XCD where groups are placed by XCD).  What counts is which of them share a CU.  Their
+		// tiles run from the longest down, so the second half of these layers is visited backwards, and the CU with the longest tiles of the
+		// first half gets the shortest of the second; of three layers the first stays, the second is turned by half its width and the third takes
+		// what makes the sum the same everywhere.
+		const int sh = a.xcd_remap ? 3 : 0, width = kNumCU >> sh, n = a.fold >> sh, layers = (n + width - 1) / width;
+		const int layer = (id >> sh) / width, base = layer * width, count = n - base < width ? n - base : width;
+		int pos = (id >> sh) - base;
+		if (layers == 3 && count == width && layer > 0)
+			pos = layer == 1 ? (pos + width / 2) % width : pos < width / 2 ? width - 1 - 2 * pos : 2 * width - 2 - 2 * pos;
+		else if (2 * layer >= layers)
+			pos = count - 1 - pos;
+		id = ((base + pos) << sh) | (id & ((1 << sh) - 1));
 	}
 	if (a.xcd_remap == 2) {
 		// A bias without a head axis is re-read by every head: one batch per XCD, and on an
@@ -189,7 +192,10 @@ __global__ __launch_bounds__(NW * 64 * KW, WPS) void fwd_kernel(const KArgs a) {
 	static_assert(!CAP || (BIAS && !BLDS && !SPLIT), "soft-capping runs on the plain path with bias");
 	typedef typename T::V8 V8;
 	constexpr int BM = NW * QB * 32;
-	constexpr int BN = kFwdBN;
+	// Block by block (tile_blocks): so few registers that four waves share a SIMD at head dim 64, three in rows of 72 to 96 columns - these in tiles
+	// of 32 keys, since three workgroups' tiles of 64 do not fit LDS.
+	constexpr bool BLK = !BIAS && QB == 1 && (D == 64 ? !SPLIT || WPS == 4 : COLS && WPS == 3);
+	constexpr int BN = BLK && D == 128 ? 32 : kFwdBN;
 	constexpr int KB = BN / 32;   // 32-key blocks per tile
 	constexpr int KS = DE / 16;   // MFMA k-steps along D
 	constexpr int DB = DE / 32;   // 32-wide blocks of the head dim
@@ -200,7 +206,7 @@ __global__ __launch_bounds__(NW * 64 * KW, WPS) void fwd_kernel(const KArgs a) {
 	// room: read from global memory one row per lane, a wave's load touches 32 cache lines.
 	constexpr bool BIAS_LDS = BIAS && BLDS && (D <= 128 || !SPLIT);
 	constexpr int BIAS_BYTES = BIAS_LDS ? BM * BN * 2 : 0;
-	static_assert(BN == 64, "bias tiles use the 64-element row geometry");
+	static_assert(!BIAS || BN == 64, "bias tiles use the 64-element row geometry");
 	constexpr int GROUP_BYTES = 4 * TILE_BYTES + 2 * BIAS_BYTES;
 	__shared__ __attribute__((aligned(1024))) char smem[KW * GROUP_BYTES];
 	// layout (per group of waves): K[0] K[1] V[0] V[1] bias[0] bias[1]
@@ -775,7 +781,7 @@ __global__ __launch_bounds__(NW * 64 * KW, WPS) void fwd_kernel(const KArgs a) {
 	// (Head dim 128 takes the same path in its four-wave workgroups, where two waves share a SIMD: B4 H32 S4096 causal forward 0.531 -> 0.511 ms,
 	// B8 S2048 0.307 -> 0.294 ms; nothing at S 8192 or without a causal mask, and the eight-wave workgroups of long context
 	// measured 0.4 % slower and stay on the plain tile body.  With dropout the generator's pieces need sixteen slots a phase.)
-	constexpr bool PIPE = (D == 256 || (D == 128 && !DROP)) && NW == 4 && QB == 1 && FOLD && (!SPLIT || KW > 1);
+	constexpr bool PIPE = !BLK && (D == 256 || (D == 128 && !DROP)) && NW == 4 && QB == 1 && FOLD && (!SPLIT || KW > 1);
 	auto tile_pipe = [&](int n0) {
 		if constexpr (PIPE) {
 			constexpr int NFR = KS;  // fragments = products of a phase: KS of K for a half, 2 sixteen-key steps x DB of V
@@ -958,6 +964,129 @@ __global__ __launch_bounds__(NW * 64 * KW, WPS) void fwd_kernel(const KArgs a) {
 		}
 	};
 
+	// A tile one block of 32 keys at a time, as little in registers as that needs: 126 at head dim 64 without dropout, 155 in rows of 72 to 96 columns, where
+	// the body above takes 183 and 210.  What a block costs its wave - 8 or 12 products, about 30 cycles of vector ALU a score, LDS reads - is close to the sum of the three
+	// when two waves share a SIMD, whatever order they are issued in; four waves (three) overlap them.  The softmax is the path without
+	// the row maximum, per block (see tile_pipe, which does the same with its halves).  Two fragments of K and of V ahead: four
+	// take more registers and gain nothing (B8 H16 S2048 148 and 152 us).  Four waves against the body above with two, forward alone: B32 H12 S511 with lengths
+	// 40.3 -> 32.7 us, B64 H16 S257 58.9 -> 42.7, B8 H16 S2048 165 -> 148, B4 Hq32 Hkv8 S4096 causal 347 -> 300, B8 H16 S1024 causal dropout 55 -> 46; three, D80:
+	// B64 H16 S257 73.7 -> 58.6, B32 S520 98.1 -> 85.5.  At head dim 128 three waves (168 registers) spill in the loop: c2 500 -> 621 us.
+	auto tile_blocks = [&](auto masked_tag, int n0) __attribute__((always_inline)) {
+		if constexpr (BLK) {
+			constexpr bool MASKED = decltype(masked_tag)::value;
+			constexpr int PF = 2, NV = 2 * DB;  // fragments ahead; fragments of V: 16-key step f / DB of the block, d-block f % DB
+#pragma unroll
+			for (int kb = 0; kb < KB; ++kb) {
+				const int j0 = n0 + 32 * kb;
+				// (a block that no row of the wave sees)
+				if constexpr (MASKED) {
+					if (j0 > wave_jmax || j0 + 31 < wave_lmin) continue;
+				}
+				f32x16 s;
+#pragma unroll
+				for (int i = 0; i < 16; ++i) s[i] = 0.f;
+				__builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+				for (int ks = 0; ks < KS; ++ks) {
+					V8 kf = *(const FA2_LDS V8*)(lds + koff[ks % KR] + kb * (32 * D * 2));
+					s = mfma32(kf, qf[0][ks], s);
+				}
+				__builtin_amdgcn_sched_group_barrier(0x100, PF, 0);
+#pragma unroll
+				for (int i = 0; i < KS - PF; ++i) {
+					__builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+					__builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+				}
+				__builtin_amdgcn_sched_group_barrier(0x008, PF, 0);
+				__builtin_amdgcn_sched_barrier(0);
+				u32x4 vfr[NV];
+				auto read_v = [&](int f) __attribute__((always_inline)) {
+					vfr[f] = lds_tr_issue_rt<D>(lds + voff[f % DB][0], lds + voff[f % DB][1], 2 * kb + f / DB);
+				};
+#pragma unroll
+				for (int f = 0; f < PF; ++f) read_v(f);
+				auto seen = [&](int i) __attribute__((always_inline)) {  // value i of the block is a key of the lane's row
+					const int j = j0 + 8 * (i >> 2) + 4 * g + (i & 3);
+					return (j <= jmax[0]) & (j >= jmin[0]);
+				};
+				V8 pf[2];
+				float ls4[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+				for (int hf = 0; hf < 2; ++hf) {
+					float pv[8];
+#pragma unroll
+					for (int e = 0; e < 8; ++e) pv[e] = __builtin_fmaf(s[8 * hf + e], c1, nmc[0]);
+#pragma unroll
+					for (int e = 0; e < 8; ++e) {
+						float p = exp2_fast(pv[e]);
+						if constexpr (MASKED) p = seen(8 * hf + e) ? p : 0.f;
+						ls4[e & 3] += p;
+						pv[e] = p;
+					}
+					pf[hf] = pack8<T>(pv[0], pv[1], pv[2], pv[3], pv[4], pv[5], pv[6], pv[7]);
+				}
+				float lt = (ls4[0] + ls4[1]) + (ls4[2] + ls4[3]);
+				// (a NaN sum - from inf or NaN inputs - also takes the other path, which propagates it)
+				const bool over = !(lt <= kFastSum) || (mrow[0] == -INFINITY && jmax[0] >= j0 && jmin[0] < j0 + 32);
+				if (__builtin_amdgcn_ballot_w64(over) != 0) {
+					float mx4[4] = {-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+#pragma unroll
+					for (int i = 0; i < 16; ++i) {
+						if constexpr (MASKED) s[i] = seen(i) ? s[i] : -INFINITY;
+						mx4[i & 3] = __builtin_fmaxf(mx4[i & 3], s[i]);
+					}
+					const float mx = pair_max(__builtin_fmaxf(__builtin_fmaxf(mx4[0], mx4[1]), __builtin_fmaxf(mx4[2], mx4[3])));
+					if (mx > mrow[0]) {
+						const float alpha = exp2_fast((mrow[0] - mx) * c1);
+						mrow[0] = mx;
+						nmc[0] = -mx * c1;
+						lrow[0] *= alpha;
+#pragma unroll
+						for (int db = 0; db < DB; ++db)
+#pragma unroll
+							for (int i = 0; i < 16; ++i) oacc[0][db][i] *= alpha;
+					}
+#pragma unroll
+					for (int e = 0; e < 4; ++e) ls4[e] = 0.f;
+#pragma unroll
+					for (int i = 0; i < 16; ++i) {
+						s[i] = exp2_fast(__builtin_fmaf(s[i], c1, nmc[0]));
+						ls4[i & 3] += s[i];
+					}
+#pragma unroll
+					for (int hf = 0; hf < 2; ++hf)
+						pf[hf] = pack8<T>(s[8 * hf], s[8 * hf + 1], s[8 * hf + 2], s[8 * hf + 3], s[8 * hf + 4], s[8 * hf + 5], s[8 * hf + 6], s[8 * hf + 7]);
+					lt = (ls4[0] + ls4[1]) + (ls4[2] + ls4[3]);
+				}
+				lrow[0] += lt;
+				if constexpr (DROP) {  // (on the packed P, as drop_p of the body above)
+#pragma unroll
+					for (int hf = 0; hf < 2; ++hf) {
+						uint32_t dw[2][2];
+						dropout_words_rowlane_half<!SPLIT>(j0 + 4 * g, (uint32_t)qrow[0], (uint32_t)hl[0], (uint32_t)b, drop_k0, drop_k1, hf, dw);
+						u32x4 x = __builtin_bit_cast(u32x4, pf[hf]);
+#pragma unroll
+						for (int m = 0; m < 4; ++m) x[m] = keep_pair16(x[m], dw[m >> 1][m & 1], a.drop_thr * 0x10001u);
+						pf[hf] = __builtin_bit_cast(V8, x);
+					}
+				}
+				__builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+				for (int f = 0; f < NV; ++f) {
+					if (f + PF < NV) read_v(f + PF);
+					oacc[0][f % DB] = mfma32(as_frag<T>(vfr[f]), pf[f / DB], oacc[0][f % DB]);
+				}
+#pragma unroll
+				for (int i = 0; i < NV - PF; ++i) {
+					__builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+					__builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+				}
+				__builtin_amdgcn_sched_group_barrier(0x008, PF, 0);
+				__builtin_amdgcn_sched_barrier(0);
+			}
+		}
+	};
+
 	// One pipeline step: publish tile t, start the copies of the group's next tile, compute.
 	auto step = [&](auto masked_tag, int t) {
 		const int n0 = t * BN;
@@ -978,7 +1107,9 @@ __global__ __launch_bounds__(NW * 64 * KW, WPS) void fwd_kernel(const KArgs a) {
 		bool skip = false;
 		if constexpr (decltype(masked_tag)::value) skip = n0 > wave_jmax || n0 + BN - 1 < wave_lmin;  // whole tile masked for this wave (uniform)
 		if (!skip) {
-			if constexpr (PIPE && !decltype(masked_tag)::value)
+			if constexpr (BLK)
+				tile_blocks(masked_tag, n0);
+			else if constexpr (PIPE && !decltype(masked_tag)::value)
 				tile_pipe(n0);
 			else
 				tile_body(masked_tag, n0);
@@ -1232,7 +1363,16 @@ hipError_t launch_fwd_tall_split_t(KArgs& a, hipStream_t s) {
 	a.mtiles = (a.Sq + 127) / 128;
 	a.xcd_remap = (a.B * a.Hkv % 8 == 0) ? 1 : 0;
 	a.interleave = 1;
-	hipLaunchKernelGGL((fwd_kernel<T, D, 4, 1, 1, false, false, true, false, false, 2>), dim3((unsigned)(a.mtiles * a.B * a.Hq * a.nsplit)), dim3(512), 0, s, a);
+	const dim3 grid((unsigned)(a.mtiles * a.B * a.Hq * a.nsplit)), block(512);
+	// (head dim 64: two such workgroups a CU where there are more than CUs, B1 Hq16 Hkv4, 700 rows over 5000 keys 38.7 -> 34.3 us; alone on its CU the form of
+	// fewer registers is no faster, 300 rows over 7000 keys 28.2 and 29.1)
+	if constexpr (D == 64) {
+		if ((int64_t)grid.x > kNumCU) {
+			hipLaunchKernelGGL((fwd_kernel<T, D, 4, 1, 4, false, false, true, false, false, 2>), grid, block, 0, s, a);
+			return launch_fwd_combine_t<T, D>(a, s);
+		}
+	}
+	hipLaunchKernelGGL((fwd_kernel<T, D, 4, 1, 1, false, false, true, false, false, 2>), grid, block, 0, s, a);
 	return launch_fwd_combine_t<T, D>(a, s);
 }
 
@@ -1272,14 +1412,16 @@ hipError_t launch_fwd_cfg(bool bias, bool drop, KArgs& a, hipStream_t s) {
 	a.interleave = a.xcd_remap ? launch_order(a, a.Hq / a.Hkv, groups / 8, (int64_t)a.Sk * DE * 4) : 1;
 	if (bias && a.bias_sh == 0 && a.B % 8 == 0) a.xcd_remap = a.kv_lens ? 3 : 2;
 	dim3 grid((unsigned)(a.mtiles * a.B * a.Hq)), block(NW * 64 * KW);
-	a.fold_half = KW == 1 ? fold_half_of(a, NW, (int64_t)grid.x, D == 64 || WPS == 2) : 0;
+	a.fold = fold_of(a, NW, (int64_t)grid.x, KW > 1 ? WPS / KW : D == 64 && WPS == 1 ? 2 : WPS);
 	const bool blds = bias && a.bias_lds;
 	// (head dim 128 with bias tiles has no LDS for a second group)
-	constexpr bool WITH_BIAS = D == 64 || (DE == D && KW == 1 && WPS == 1);
-	if constexpr (DE == D) {
+	constexpr bool WITH_BIAS = DE == D && (D == 64 || KW == 1) && WPS == 1, WITHOUT = D != 64 || WPS > 1;
+	if constexpr (DE == D && WITHOUT) {
 		if (!bias && drop) hipLaunchKernelGGL((fwd_kernel<T, D, NW, QB, WPS, false, true, false, false, false, KW>), grid, block, 0, s, a);
 	}
-	if (!bias && !drop) hipLaunchKernelGGL((fwd_kernel<T, D, NW, QB, WPS, false, false, false, false, false, KW, DE>), grid, block, 0, s, a);
+	if constexpr (WITHOUT) {
+		if (!bias && !drop) hipLaunchKernelGGL((fwd_kernel<T, D, NW, QB, WPS, false, false, false, false, false, KW, DE>), grid, block, 0, s, a);
+	}
 	if constexpr (WITH_BIAS) {
 		if (!bias)
 			;
@@ -1314,6 +1456,7 @@ hipError_t launch_fwd_t(bool bias, bool drop, KArgs& a, hipStream_t s) {
 		// A grid that leaves at least half of the chip idle (small batch x heads, short sequences): workgroups of
 		// 128 rows instead of 256, twice as many of them, still at most one per CU.
 		int64_t wgs = (int64_t)((a.Sq + 127) / 128) * a.B * a.Hq;
+		const int64_t seen = a.win_left >= 0 && a.win_right >= 0 ? (int64_t)a.win_left + a.win_right + 128 : a.Sk;  // keys of a row tile
 		if (wgs <= kNumCU) {
 			// ... and two groups of four waves that take the key tiles of the workgroup's rows in turn: two waves per SIMD where
 			// there was one (B1 Hq32 Hkv8 D128, 1000 rows over 9000 keys: 233 -> 170 us; B1 H8 S4096 D128 81 -> 71 us, causal 79 -> 61;
@@ -1321,10 +1464,17 @@ hipError_t launch_fwd_t(bool bias, bool drop, KArgs& a, hipStream_t s) {
 			// groups): up to three, five at D = 64 and four under a causal mask at D = 128, where it is not dropout or a bias that makes a
 			// tile long.  By tiles, two groups over one, 500 calls: D64 4 / 5 / 6 tiles 1.01 / 1.01 / 0.94, causal 1.06 / 1.00 / 0.98,
 			// dropout 0.97 / 0.96 / 0.92; D128 0.98 / 0.98 / 0.92, causal 1.02 / 0.96 / 0.93.  In a window a row tile sees few tiles whatever
-			// the number of keys (B26 Hq4 Hkv1 S243 D64, 61 keys a row, 9.2 and 10.1).  Four groups spill.
-			const int few = drop || bias ? 3 : D == 64 ? 5 : a.causal ? 4 : 3;
-			const int64_t seen = a.win_left >= 0 && a.win_right >= 0 ? (int64_t)a.win_left + a.win_right + 128 : a.Sk;
-			if (a.Sk > few * kFwdBN && seen > few * kFwdBN && (D == 64 || !bias)) return launch_fwd_cfg<T, D, DE, 4, 1, 2>(bias, drop, a, s);
+			// the number of keys (B26 Hq4 Hkv1 S243 D64, 61 keys a row, 9.2 and 10.1).
+			// At head dim 64, block by block, two groups from four tiles on (B2 Hq16 Hkv4 S512 causal 10.8 -> 10.0 us, S256 of B4 8.2 -> 8.0), three from
+			// seventeen (B1 Hq16 Hkv4 S2000 29.9 -> 28.4; at S1024 and below 1 to 6 % slower than two).  Four take 128 registers a wave and spill.
+			const int few = drop || bias || D == 64 || !a.causal ? 3 : 4;
+			const bool groups = a.Sk > few * kFwdBN && seen > few * kFwdBN;
+			if constexpr (D == 64) {
+				if (!bias && groups && seen > 16 * kFwdBN) return launch_fwd_cfg<T, D, DE, 4, 3, 3>(bias, drop, a, s);
+				if (!bias && groups) return launch_fwd_cfg<T, D, DE, 4, 2, 2>(bias, drop, a, s);
+				if (!bias) return launch_fwd_cfg<T, D, DE, 4, 4>(bias, drop, a, s);
+			}
+			if (groups && (D == 64 || !bias)) return launch_fwd_cfg<T, D, DE, 4, 1, 2>(bias, drop, a, s);
 			return launch_fwd_cfg<T, D, DE, 4, 1>(bias, drop, a, s);
 		}
 		// Larger grids: two independent 128-row workgroups per CU instead of one of 256 rows - the same eight waves, but
@@ -1343,8 +1493,25 @@ hipError_t launch_fwd_t(bool bias, bool drop, KArgs& a, hipStream_t s) {
 		const int64_t kv_limit = D == 64   ? (4 << 20)
 		                         : a.causal ? ((drop && wgs > 2 * kNumCU) ? (2 << 20) : (4 << 20))
 		                                    : (drop ? 1024 * D * 4 : (2 << 20));
-		if ((int64_t)a.Sk * DE * 4 <= kv_limit && (D == 64 || (!bias && !(a.softcap > 0.f))))
+		if ((int64_t)a.Sk * DE * 4 <= kv_limit && (D == 64 || (!bias && !(a.softcap > 0.f)))) {
+			if constexpr (D == 64) {
+				// Four waves a SIMD: four such workgroups a CU, or two of two groups each where the grid has no more than that (over
+				// ten tiles and more; B4 Hq16 Hkv4 S1000 29.3 -> 28.4 us against 30.2 with one group, causal 23.9 -> 21.6 against 24.9; at S400 14.0 -> 12.8 with one, 15.0
+				// with two) or seventeen of a window (B1 Hq16 Hkv4 S4000, 1024 keys a row 29.3 -> 28.4 against 29.5, 512 keys 20.3 -> 21.5 against 20.0).
+				if (!bias && wgs <= 2 * kNumCU && a.Sk > 9 * kFwdBN && (a.win_left < 0 || seen > 16 * kFwdBN)) return launch_fwd_cfg<T, D, DE, 4, 4, 2>(bias, drop, a, s);
+				if (!bias) return launch_fwd_cfg<T, D, DE, 4, 4>(bias, drop, a, s);
+			}
+			if constexpr (DE < D) {
+				// Three workgroups a CU from the first one beyond two a CU on.  Under a causal mask a grid of up to twice the resident workgroups waits for its
+				// longest tile, which takes longer with three on a CU: B4 Hq16 Hkv4 S2000 D96 (1024 workgroups) 75 -> 84 us; at S4000 there is nothing to gain (207 -> 211).
+				const bool tail = a.causal && (a.Sk > 2048 || (a.Sk > 1024 && wgs > 3 * kNumCU && wgs < 11 * kNumCU / 2));
+				if (wgs > 2 * kNumCU && !tail) return launch_fwd_cfg<T, D, DE, 4, 3>(bias, drop, a, s);
+			}
 			return launch_fwd_cfg<T, D, DE, 4, (D == 128 ? 2 : 1)>(bias, drop, a, s);
+		}
+	}
+	if constexpr (D == 64) {
+		if (!bias) return launch_fwd_cfg<T, D, DE, C::NW, 4>(bias, drop, a, s);
 	}
 	return launch_fwd_cfg<T, D, DE, C::NW, C::WPS>(bias, drop, a, s);
 }
