@@ -337,7 +337,7 @@ static int fwd_decode_waves(const fa2_params* p, int* whole) {
 }
 
 // Key ranges for a split forward: too few workgroups to fill the chip, many keys.  Returns the number of ranges (1 = no split) of
-// *split_len keys; *tall: in workgroups of 128 rows.
+// *split_len keys; *tall: in workgroups of 128 rows (1: of eight waves, one a CU; 2: of four, two a CU).
 static int fwd_split_plan(const fa2_params* p, int* split_len, int* tall) {
 	*split_len = 0;
 	*tall = 0;
@@ -387,8 +387,31 @@ static int fwd_split_plan(const fa2_params* p, int* split_len, int* tall) {
 				best_us = us;
 			}
 		}
-		const int per = (tiles + best - 1) / best;
 		*tall = 1;
+		if (p->D == 128 && !short_rows(p) && !p->kv_lens && !p->seqlens) {
+			// Or workgroups of four waves, two a CU: no barrier holds one up for the other, but there are twice as many partial results. Fitted
+			// to Hkv 8, 4200 to 14200 keys, of 384 to 512 such workgroups: a tile takes 0.67 us and 1.24 more with the share of the places that are
+			// taken, partial results 0.57 of the above. B1 Hq32 Hkv8, 1000 causal rows over 9000 / 14200 keys 174 / 261 -> 155 / 227 us in two ranges, 700 rows over
+			// 8200 140 -> 120, 600 rows over 3000 / 10200 in three 56 / 126 -> 45 / 112; B1 Hq8 Hkv2, 1500 over 6200 in five 64 -> 51. Workgroups of eight waves in one
+			// range take 6 % more than their estimate over many keys (1000 rows over 6200: 104 and 117); from three ranges on a tenth has to be gained (four,
+			// estimated as even: B1 H4 S4096 over 6200 57 and 61, B1 Hq16 Hkv4, 1000 over 3000 41 and 45). Not with lengths: a range beyond
+			// a row's length is a place wasted (B3 Hq8 Hkv2, 1000 rows over 3000 keys 51 and 60). (Rows of fewer columns run on the rows as they are.)
+			int pairs = 0;
+			double pairs_us = 0;
+			for (int n = 2; n <= 16 && n <= tiles / 2 && base * n <= 512 && n * range_bytes <= kFwdScratchMax; ++n) {
+				if (base * n < 384) continue;
+				const double us = (tiles + n - 1) / n * (0.67 + 1.24 * (base * n) / 512) + 3.5 + 0.57 * n * part_us;
+				if (!pairs || us < pairs_us) {
+					pairs = n;
+					pairs_us = us;
+				}
+			}
+			if (pairs && pairs_us < best_us * (pairs == 2 ? 1.06 : 0.9)) {
+				best = pairs;
+				*tall = 2;
+			}
+		}
+		const int per = (tiles + best - 1) / best;
 		*split_len = per * 64;
 		return (tiles + per - 1) / per;
 	}

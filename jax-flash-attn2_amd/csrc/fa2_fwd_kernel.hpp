@@ -781,7 +781,7 @@ __global__ __launch_bounds__(NW * 64 * KW, WPS) void fwd_kernel(const KArgs a) {
 	// (Head dim 128 takes the same path in its four-wave workgroups, where two waves share a SIMD: B4 H32 S4096 causal forward 0.531 -> 0.511 ms,
 	// B8 S2048 0.307 -> 0.294 ms; nothing at S 8192 or without a causal mask, and the eight-wave workgroups of long context
 	// measured 0.4 % slower and stay on the plain tile body.  With dropout the generator's pieces need sixteen slots a phase.)
-	constexpr bool PIPE = !BLK && (D == 256 || (D == 128 && !DROP)) && NW == 4 && QB == 1 && FOLD && (!SPLIT || KW > 1);
+	constexpr bool PIPE = !BLK && (D == 256 || (D == 128 && !DROP)) && NW == 4 && QB == 1 && FOLD && (!SPLIT || KW > 1 || WPS == 2);
 	auto tile_pipe = [&](int n0) {
 		if constexpr (PIPE) {
 			constexpr int NFR = KS;  // fragments = products of a phase: KS of K for a half, 2 sixteen-key steps x DB of V
@@ -1357,13 +1357,20 @@ struct FwdCfg {
 	static constexpr int BM = NW * QB * 32;
 };
 
-// Split forward of a longer query on a small grid: the 128-row workgroups of eight waves of launch_fwd_t, nsplit key ranges each.
+// Split forward of a longer query on a small grid: the 128-row workgroups of eight waves of launch_fwd_t, nsplit key ranges each; tall_split 2: those of four
+// waves, two a CU.
 template <typename T, int D>
 hipError_t launch_fwd_tall_split_t(KArgs& a, hipStream_t s) {
 	a.mtiles = (a.Sq + 127) / 128;
 	a.xcd_remap = (a.B * a.Hkv % 8 == 0) ? 1 : 0;
 	a.interleave = 1;
 	const dim3 grid((unsigned)(a.mtiles * a.B * a.Hq * a.nsplit)), block(512);
+	if constexpr (D == 128) {
+		if (a.tall_split == 2) {
+			hipLaunchKernelGGL((fwd_kernel<T, D, 4, 1, 2, false, false, true>), grid, dim3(256), 0, s, a);
+			return launch_fwd_combine_t<T, D>(a, s);
+		}
+	}
 	// (head dim 64: two such workgroups a CU where there are more than CUs, B1 Hq16 Hkv4, 700 rows over 5000 keys 38.7 -> 34.3 us; alone on its CU the form of
 	// fewer registers is no faster, 300 rows over 7000 keys 28.2 and 29.1)
 	if constexpr (D == 64) {

@@ -60,7 +60,7 @@ struct KArgs {
 	int pack_gqa;     // split forward: one workgroup holds the rows of all q-heads of a kv-head
 	float* o_part;    // [nsplit, B, Hq, Sq, D] fp32
 	float* lse_part;  // [nsplit, B, Hq, Sq] fp32
-	int tall_split;   // split forward: of a query longer than one row tile, in workgroups of 128 rows
+	int tall_split;   // split forward: of a query longer than one row tile, in workgroups of 128 rows (2: of four waves)
 	// few query rows in all (fwd_decode_kernel): number of waves that share the key tiles (0 = off);
 	// pieces of units in o_part / lse_part, and per (batch, kv-head) where its pieces are
 	// (decode_whole: one (batch, kv-head) per wave, no scratch)

@@ -42,6 +42,11 @@ BF, FP = torch.bfloat16, torch.float16
 		(40, 65, 129, 30, 6, 64, BF, False, None, None, 0.2),
 		# key ranges of workgroups that share a CU
 		(1, 700, 5000, 16, 4, 64, BF, True, None, None, 0.0),
+		# head dim 128, four waves a workgroup and two workgroups a CU: two ranges, three, five; rows that end before the last, a range of one tile with one key
+		(1, 1000, 5700, 24, 8, 128, BF, True, None, None, 0.0),
+		(1, 600, 2945, 32, 8, 128, FP, False, None, None, 0.0),
+		(1, 1500, 1601, 8, 2, 128, BF, True, None, None, 0.0),
+		(2, 1500, 1400, 6, 6, 128, FP, True, None, None, 0.0),
 	],
 )
 def test_blocks(B, Sq, Sk, Hq, Hkv, D, dtype, causal, lens, window, p):
