@@ -138,7 +138,7 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 	constexpr int BN = NW * 32;     // keys per workgroup
 	constexpr int BMQ = QB * 32;    // query rows per streamed tile
 	constexpr int KS = DE / 16;
-	constexpr int DB = DE / 32;
+	constexpr int DB = (DE + 31) / 32;
 	constexpr bool COLS = DE < D;
 	static_assert(!COLS || (!BIAS && !DROP), "");
 	constexpr int NT = NW * 64;
@@ -255,7 +255,7 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 	qload.init(a.q.ss, tid, BMQ, cols);
 	doload.init(a.dout.ss, tid, BMQ, cols);
 	if constexpr (COLS) {
-		for (int i = 0; i < 4; ++i) zero_cols<D, BMQ, NT>(lds + i * TILE_BYTES, tid, cols, DE / 8);
+		for (int i = 0; i < 4; ++i) zero_cols<D, BMQ, NT>(lds + i * TILE_BYTES, tid, cols, DB * 4);
 	}
 	TileLoader<128, BMQ, NT> bload;
 	if constexpr (BIAS_LDS) bload.init(a.bias_sm, tid);
@@ -383,9 +383,10 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 		// slots to complete and the LDS traffic is spread evenly), and its share of the
 		// elementwise math of B(k-1) - the vector ALU and the LDS work in the shadow of the
 		// matrix pipe.  A scheduling barrier after every slot pins that order.
-		constexpr int NSLOT = 2 * KS;     // = 4 DB
+		constexpr int NSLOT = 4 * DB, NA = 2 * KS;  // products of C and of A (80 columns: two slots without one of A)
 		constexpr int PA = BLK ? 3 : 4;   // read-ahead distance in slots
 		constexpr int RING = PA + 1;
+		static_assert(NA == NSLOT || BLK, "");
 		static_assert(NSLOT % 16 == 0 || NSLOT == 8 || (NSLOT == 12 && FOLD), "");
 		f32x16 s[2], dp[2];
 		u32x4 pbits[2][2], sbits[2][2];   // [block parity][16-row half]: P and dS packed to 16 bits
@@ -403,6 +404,7 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 		auto a_step = [](int j) __attribute__((always_inline)) { return CHAINS ? j % KS : j >> 1; };
 		auto issue_A = [&](int qb, int j) __attribute__((always_inline)) {
 			// (poff carries the buffer; dO lies one tile behind Q)
+			if (j >= NA) return;
 			const int ks = a_step(j);
 			afr[(qb * NSLOT + j) % RING] = *(const FA2_LDS V8*)(lds + poff[ks % KR] + (ks / KR) * 256 + (a_is_dp(j) ? TILE_BYTES : 0) + qb * (32 * D * 2));
 		};
@@ -467,6 +469,7 @@ FA2_DEV void bwd_dkdv_tile(const KArgs& a, const int nt, const int hk, const int
 			}
 		};
 		auto mfma_A = [&](int qb, int j, f32x16& sa, f32x16& dpa) __attribute__((always_inline)) {
+			if (j >= NA) return;
 			int ks = a_step(j), r = (qb * NSLOT + j) % RING;
 			if constexpr (KV_AGPR) {
 				// the chains start from -lse and -delta of the block's rows (accumulator element i
@@ -1150,17 +1153,19 @@ __global__ __launch_bounds__(NW * 64, WPS) void bwd_dq_kernel(const KArgs a) {
 	static_assert(!DBIAS || (BIAS && !BLDS), "the bias gradient is written on the plain path with bias");
 	typedef typename T::V8 V8;
 	constexpr int BM = NW * QB * 32;
-	constexpr int BN = kFwdBN;
+	// Block by block (tile_blocks), three waves a SIMD: rows of 72 and 80 columns, in tiles of 32 keys as in the forward
+	constexpr bool BLK = COLS && WPS == 3;
+	constexpr int BN = BLK ? 32 : kFwdBN;
 	constexpr int KB = BN / 32;
 	constexpr int KS = DE / 16;
-	constexpr int DB = DE / 32;
+	constexpr int DB = (DE + 31) / 32;
 	constexpr int NT = NW * 64;
 	constexpr int TILE_BYTES = BN * D * 2;
 
 	// bias tiles through LDS as in the forward kernel
 	constexpr bool BIAS_LDS = BIAS && BLDS;
 	constexpr int BIAS_BYTES = BIAS_LDS ? BM * BN * 2 : 0;
-	static_assert(BN == 64, "bias tiles use the 64-element row geometry");
+	static_assert(!BIAS || BN == 64, "bias tiles use the 64-element row geometry");
 	__shared__ __attribute__((aligned(1024))) char smem[4 * TILE_BYTES + 2 * BIAS_BYTES];
 	FA2_LDS char* lds = (FA2_LDS char*)smem;
 
@@ -1260,7 +1265,7 @@ __global__ __launch_bounds__(NW * 64, WPS) void bwd_dq_kernel(const KArgs a) {
 	kload.init(a.k.ss, tid, BN, cols);
 	vload.init(a.v.ss, tid, BN, cols);
 	if constexpr (COLS) {
-		for (int i = 0; i < 4; ++i) zero_cols<D, BN, NT>(lds + i * TILE_BYTES, tid, cols, DE / 8);
+		for (int i = 0; i < 4; ++i) zero_cols<D, BN, NT>(lds + i * TILE_BYTES, tid, cols, DB * 4);
 	}
 	if (ntiles > t_begin) {
 		int nb = t_begin * BN, bsel = t_begin & 1;
@@ -1346,7 +1351,8 @@ __global__ __launch_bounds__(NW * 64, WPS) void bwd_dq_kernel(const KArgs a) {
 
 	// (the offsets carry the buffer - K[1] / V[1] / bias[1] lie a power of two behind K[0] / V[0] / bias[0] -
 	// and are flipped after every tile, so that the reads need no address arithmetic in the loop)
-	constexpr int KR = KS < 8 ? KS : 8, DR = DB < 4 ? DB : 4;  // (chunks 16 and up: + 256 bytes as an immediate, see the dK/dV kernel)
+	// (block by block only the first transposed offset is kept: the others differ from it in bits of the chunk)
+	constexpr int KR = KS < 8 ? KS : 8, DR = BLK ? 1 : DB < 4 ? DB : 4;  // (chunks 16 and up: + 256 bytes as an immediate, see the dK/dV kernel)
 	int koff[KR];
 #pragma unroll
 	for (int ks = 0; ks < KR; ++ks) koff[ks] = tile_off<D>(c, 2 * ks + g) + (t_begin & 1) * TILE_BYTES;
@@ -1516,6 +1522,84 @@ __global__ __launch_bounds__(NW * 64, WPS) void bwd_dq_kernel(const KArgs a) {
 		}
 	};
 
+	// A tile of one block of 32 keys, as little in registers as that needs: 164 where the body above takes 212, so that three workgroups share a CU. What a block
+	// costs its wave is close to the sum of its 16 products, its vector ALU and its LDS reads when two waves share a SIMD; a third overlaps them.  Each
+	// product is pinned behind the read of the fragment two products further on; left to the compiler the chain of dP comes after that of S, with all its fragments
+	// waiting in registers.  Backward, two waves and three, D80: B64 H16 S257 209 -> 198 us, B32 S520 260 -> 249, B4 S4096 1324 -> 1293 (with the dK/dV
+	// kernel's share of 80 columns, 3 to 7 us of the first two).  In rows of 96 columns it takes 168 and gains nothing (B32 S520 D88 288 both, B7 S1100 D96 222
+	// both), and at head dim 64, where the body above fits three waves, four spill (B32 H12 S511 137 -> 193).
+	auto tile_blocks = [&](auto masked_tag, int n0) __attribute__((always_inline)) {
+		if constexpr (BLK) {
+			constexpr bool MASKED = decltype(masked_tag)::value;
+			constexpr int PF = 2, NA = 2 * KS, NC = 2 * DB;  // fragments ahead; products of S and dP in turn; 16-key steps x d-blocks of K^T
+			// The chain of dP starts from -delta, copied anew for each block: sixteen registers that hold it would cost a wave.
+			float nd = -del_r[0];
+			asm volatile("" : "+v"(nd));
+			f32x16 s, dp;
+#pragma unroll
+			for (int i = 0; i < 16; ++i) s[i] = 0.f, dp[i] = nd;
+			V8 fr[NA];
+			auto read_a = [&](int f) __attribute__((always_inline)) {  // k-step f / 2 of K (even f) or V (odd f)
+				const int ks = f >> 1;
+				fr[f] = *(const FA2_LDS V8*)(lds + koff[ks] + ((f & 1) ? 2 * TILE_BYTES : 0));
+			};
+			__builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+			for (int f = 0; f < PF; ++f) read_a(f);
+#pragma unroll
+			for (int f = 0; f < NA; ++f) {
+				if (f + PF < NA) read_a(f + PF);
+				if (f & 1)
+					dp = mfma32(fr[f], dof[0][f >> 1], dp);
+				else
+					s = mfma32(fr[f], qf[0][f >> 1], s);
+				asm volatile("" : "+v"(s), "+v"(dp));
+				__builtin_amdgcn_sched_barrier(0);
+			}
+			u32x4 kfr[NC];
+			auto read_k = [&](int f) __attribute__((always_inline)) {
+				const int t0 = toff[0][0] ^ ((f % DB) << 6);  // (eight rows further on, the key of the swizzle differs in bit 1)
+				kfr[f] = lds_tr_issue_rt<D>(lds + t0, lds + 8 * D * 2 + (t0 ^ 32), f / DB);
+			};
+#pragma unroll
+			for (int f = 0; f < PF; ++f) read_k(f);
+			// (keys of the lane's row, counted from the lane's first key of the block)
+			int jlast = jmax[0] - n0 - 4 * g, jfirst = jmin[0] - n0 - 4 * g;
+			if constexpr (MASKED) asm volatile("" : "+v"(jlast), "+v"(jfirst));
+			V8 dsf[2];
+#pragma unroll
+			for (int hf = 0; hf < 2; ++hf) {
+				float ds[8];
+#pragma unroll
+				for (int e = 0; e < 8; ++e) ds[e] = __builtin_fmaf(s[8 * hf + e], c1, lse_r[0]);
+#pragma unroll
+				for (int e = 0; e < 8; ++e) {
+					const int i = 8 * hf + e;
+					float p = exp2_fast(ds[e]);
+					if constexpr (MASKED) {
+						const int j = 8 * (i >> 2) + (i & 3);
+						p = ((j <= jlast) & (j >= jfirst)) ? p : 0.f;
+					}
+					ds[e] = p * dp[i];
+				}
+				dsf[hf] = pack8<T>(ds[0], ds[1], ds[2], ds[3], ds[4], ds[5], ds[6], ds[7]);
+			}
+			__builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+			for (int f = 0; f < NC; ++f) {
+				if (f + PF < NC) read_k(f + PF);
+				dq[0][f % DB] = mfma32(as_frag<T>(kfr[f]), dsf[f / DB], dq[0][f % DB]);
+			}
+#pragma unroll
+			for (int i = 0; i < NC - PF; ++i) {
+				__builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+				__builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+			}
+			__builtin_amdgcn_sched_group_barrier(0x008, PF, 0);
+			__builtin_amdgcn_sched_barrier(0);
+		}
+	};
+
 	// Head dim 256 runs one wave per SIMD, so the elementwise stage overlaps the matrix products only if the wave
 	// interleaves them itself (as the forward kernel does at this head dim).  A tile without masking goes as two halves
 	// of 32 keys through four phases,
@@ -1668,7 +1752,9 @@ __global__ __launch_bounds__(NW * 64, WPS) void bwd_dq_kernel(const KArgs a) {
 		bool skip = false;
 		if constexpr (decltype(masked_tag)::value) skip = n0 > wave_jmax || n0 + BN - 1 < wave_lmin;  // whole tile masked for this wave (uniform)
 		if (!skip) {
-			if constexpr (PIPE && !decltype(masked_tag)::value)
+			if constexpr (BLK)
+				tile_blocks(masked_tag, n0);
+			else if constexpr (PIPE && !decltype(masked_tag)::value)
 				tile_pipe(n0);
 			else
 				tile_body(masked_tag, n0);
@@ -1695,8 +1781,8 @@ __global__ __launch_bounds__(NW * 64, WPS) void bwd_dq_kernel(const KArgs a) {
 	for (int t = t_lo; t < t_full; ++t) step(std::false_type{}, t);
 	for (int t = t_full; t < ntiles; ++t) step(std::true_type{}, t);
 
-	// (Stored 16 bytes a lane as the other results are (pair_cols) the variants of head dim 64 without bias take 88 registers instead of 84 and the loop
-	// above is slower than what the stores gain: B64 H16 S257 59 -> 66 us, B32 H12 S511 55 -> 60, B16 Hq16 Hkv4 S1024 causal 70 -> 75, B8 H16 S2048 194 -> 204.)
+	// (Stored 16 bytes a lane as the other results are (pair_cols) the variants of head dim 64 without bias take 176 registers instead of 168, two
+	// workgroups a CU instead of three: B64 H16 S257 59 -> 66 us, B32 H12 S511 55 -> 60, B16 Hq16 Hkv4 S1024 causal 70 -> 75, B8 H16 S2048 194 -> 204.)
 	constexpr bool HALVES = D == 64 && !BIAS;
 	char* obase = a.dq.ptr + (int64_t)b * a.dq.sb + (int64_t)h * a.dq.sh;
 #pragma unroll
@@ -1760,12 +1846,12 @@ hipError_t launch_bwd_v(KArgs& a, hipStream_t s) {
 		constexpr int RPB = 256 / (D / 8);
 		hipLaunchKernelGGL((bwd_delta_kernel<T, D>), dim3((unsigned)((nrows + RPB - 1) / RPB)), dim3(256), 0, s, a);
 	}
-	auto launch_dq_cfg = [&](auto nw_tag, auto wps_tag) {
+	auto launch_dq_cfg = [&](auto nw_tag, auto wps_tag, auto de_tag) {
 		constexpr int NW = decltype(nw_tag)::value, BM = NW * C::DQ_QB * 32, WPS = decltype(wps_tag)::value;
 		a.mtiles = (a.Sq + BM - 1) / BM;
 		a.interleave = a.xcd_remap == 1 ? launch_order(a, a.Hq / a.Hkv, groups / 8, (int64_t)a.Sk * DE * 4) : 1;
 		dim3 grid((unsigned)(a.mtiles * a.B * a.Hq)), block(NW * 64);
-		a.fold = fold_of(a, NW, (int64_t)grid.x, D == 64 || WPS == 2 ? 2 : 1);
+		a.fold = fold_of(a, NW, (int64_t)grid.x, D == 64 && WPS == 1 ? (BIAS ? 2 : 3) : WPS);
 		if constexpr (BIAS) {
 			if (a.dbias && a.softcap > 0.f)
 				hipLaunchKernelGGL((bwd_dq_kernel<T, D, NW, C::DQ_QB, WPS, true, DROP, false, true, true>), grid, block, 0, s, a);
@@ -1778,24 +1864,31 @@ hipError_t launch_bwd_v(KArgs& a, hipStream_t s) {
 			else
 				hipLaunchKernelGGL((bwd_dq_kernel<T, D, NW, C::DQ_QB, WPS, true, DROP>), grid, block, 0, s, a);
 		} else {
-			hipLaunchKernelGGL((bwd_dq_kernel<T, D, NW, C::DQ_QB, WPS, false, DROP, false, false, false, DE>), grid, block, 0, s, a);
+			hipLaunchKernelGGL((bwd_dq_kernel<T, D, NW, C::DQ_QB, WPS, false, DROP, false, false, false, decltype(de_tag)::value>), grid, block, 0, s, a);
 		}
 	};
+	constexpr std::integral_constant<int, DE> de{};
 	auto launch_dq = [&]() {
 		if constexpr (C::DQ_NW == 8) {
 			// a grid that leaves at least half of the chip idle: workgroups of 128 rows instead of 256 (see the forward)
 			int64_t wgs = (int64_t)((a.Sq + 127) / 128) * a.B * a.Hq;
-			if (wgs <= kNumCU) return launch_dq_cfg(std::integral_constant<int, 4>{}, std::integral_constant<int, C::DQ_WPS>{});
+			if (wgs <= kNumCU) return launch_dq_cfg(std::integral_constant<int, 4>{}, std::integral_constant<int, C::DQ_WPS>{}, de);
 			// larger grids: two 128-row workgroups per CU where the K and V of a head fit an XCD's L2 (see the forward;
 			// the dQ kernel gains with and without a causal mask: D = 128 B8 S2048 causal 0.460 -> 0.418 ms, non-causal
 			// 0.784 -> 0.734 ms, B4 S4096 causal 0.770 -> 0.739 ms; D = 64 B32 S512 0.060 -> 0.051 ms); D = 128 with bias
 			// would spill within 256 registers
 			if constexpr (D == 64 || !BIAS) {
-				if ((int64_t)a.Sk * DE * 4 <= (4 << 20))
-					return launch_dq_cfg(std::integral_constant<int, 4>{}, std::integral_constant<int, (D == 128 ? 2 : 1)>{});
+				if ((int64_t)a.Sk * DE * 4 <= (4 << 20)) {
+					if constexpr (DE < D) {
+						constexpr std::integral_constant<int, 80> de80{};
+						if (a.hd <= 80 && wgs > 2 * kNumCU && !causal_tail(a, wgs)) return launch_dq_cfg(std::integral_constant<int, 4>{}, std::integral_constant<int, 3>{}, de80);
+						if (a.hd <= 80) return launch_dq_cfg(std::integral_constant<int, 4>{}, std::integral_constant<int, 2>{}, de80);
+					}
+					return launch_dq_cfg(std::integral_constant<int, 4>{}, std::integral_constant<int, (D == 128 ? 2 : 1)>{}, de);
+				}
 			}
 		}
-		launch_dq_cfg(std::integral_constant<int, C::DQ_NW>{}, std::integral_constant<int, C::DQ_WPS>{});
+		launch_dq_cfg(std::integral_constant<int, C::DQ_NW>{}, std::integral_constant<int, C::DQ_WPS>{}, de);
 	};
 	if (fused_delta) launch_dq();
 	if (a.stages & 2) {
@@ -1839,7 +1932,7 @@ hipError_t launch_bwd_v(KArgs& a, hipStream_t s) {
 		const bool uneven = DE < D && a.win_right >= 0 && (a.win_left < 0 || 4 * (int64_t)a.win_left >= 3 * (int64_t)a.Sk) && 8 * (int64_t)a.Sq >= 7 * (int64_t)a.Sk;
 		const int64_t least = uneven && hs > 1 && a.kv_ntiles >= 4 ? 5 * kNumCU / 2 : uneven && hs == 1 && a.kv_ntiles >= 8 ? 2 * kNumCU + 1 : 2 * kNumCU;
 		const bool blk = (D == 64 || DE < D) && !a.kv_pair && (int64_t)grid.x >= least;
-		auto launch_dkdv = [&](auto blk_tag) {
+		auto launch_dkdv = [&](auto blk_tag, auto de_tag) {
 			constexpr bool BLK = decltype(blk_tag)::value;
 			// with bias at D = 128 the streamed tiles are 64 rows, which leaves LDS room for the bias tiles (and block by block for a second workgroup)
 			constexpr int QBV = (BIAS && (D == 128 || BLK)) || (BLK && D == 128) ? 2 : C::KV_QB;
@@ -1855,16 +1948,23 @@ hipError_t launch_bwd_v(KArgs& a, hipStream_t s) {
 				if constexpr (D <= 128 && !BLK)
 					hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, C::KV_NW, QBV, false, DROP, false, false, true, DE>), grid, block, 0, s, a);
 			} else {
-				hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, C::KV_NW, QBV, false, DROP, false, false, false, DE, BLK>), grid, block, 0, s, a);
+				hipLaunchKernelGGL((bwd_dkdv_kernel<T, D, C::KV_NW, QBV, false, DROP, false, false, false, decltype(de_tag)::value, BLK>), grid, block, 0, s, a);
 			}
 		};
-		if constexpr (D == 64 || DE < D) {
-			if (blk)
-				launch_dkdv(std::true_type{});
+		if constexpr (DE < D) {
+			if (blk && a.hd <= 80)
+				launch_dkdv(std::true_type{}, std::integral_constant<int, 80>{});
+			else if (blk)
+				launch_dkdv(std::true_type{}, de);
 			else
-				launch_dkdv(std::false_type{});
+				launch_dkdv(std::false_type{}, de);
+		} else if constexpr (D == 64) {
+			if (blk)
+				launch_dkdv(std::true_type{}, de);
+			else
+				launch_dkdv(std::false_type{}, de);
 		} else {
-			launch_dkdv(std::false_type{});
+			launch_dkdv(std::false_type{}, de);
 		}
 		if (hs > 1) {
 			int64_t total = (int64_t)a.B * a.Hkv * a.Sk * 2 * (D / 8);

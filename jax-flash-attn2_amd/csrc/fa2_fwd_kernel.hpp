@@ -65,6 +65,11 @@ inline int fold_of(const KArgs& a, int nw, int64_t total, int per_cu) {
 	return total > kNumCU && total <= per_cu * kNumCU ? (int)total : 0;
 }
 
+// Rows of 72 to 96 columns, three workgroups a CU: a causal grid of these many workgroups of 128 rows waits for its longest tiles, which take longer
+// the more workgroups share a CU (forward, see launch_fwd_t; dQ of rows of 80, two and three a CU: B4 Hq16 Hkv4 S2000 with the dK/dV kernel 224 and 233 us, S4000
+// of 72 columns 684 and 690).
+inline bool causal_tail(const KArgs& a, int64_t wgs) { return a.causal && (a.Sk > 2048 || (a.Sk > 1024 && wgs > 3 * kNumCU && wgs < 11 * kNumCU / 2)); }
+
 // The i-th (batch, kv-head) group of an XCD.  Rows that are not whole 128-byte lines share lines with the rows of the next head: on
 // different XCDs both fetch such a line and write it in part, so there (and where all batch rows are equally long) an XCD takes adjacent
 // groups.  B64 S257 H16 D80, 160-byte rows: dK/dV 190.5 -> 180.9 us, dQ 109.8 -> 103.8, forward 89.0 -> 87.0.
@@ -198,7 +203,7 @@ __global__ __launch_bounds__(NW * 64 * KW, WPS) void fwd_kernel(const KArgs a) {
 	constexpr int BN = BLK && D == 128 ? 32 : kFwdBN;
 	constexpr int KB = BN / 32;   // 32-key blocks per tile
 	constexpr int KS = DE / 16;   // MFMA k-steps along D
-	constexpr int DB = DE / 32;   // 32-wide blocks of the head dim
+	constexpr int DB = (DE + 31) / 32;   // 32-wide blocks of the head dim
 	constexpr int NT = NW * 64;
 	constexpr int TILE_BYTES = BN * D * 2;
 
@@ -352,7 +357,7 @@ __global__ __launch_bounds__(NW * 64 * KW, WPS) void fwd_kernel(const KArgs a) {
 	kload.init(a.k.ss, tid, BN, cols);
 	vload.init(a.v.ss, tid, BN, cols);
 	if constexpr (COLS) {
-		for (int i = 0; i < 2; ++i) zero_cols<D, BN, NT>(lds + i * TILE_BYTES, tid, cols, DE / 8);  // (of V they only reach columns that are not stored)
+		for (int i = 0; i < 2; ++i) zero_cols<D, BN, NT>(lds + i * TILE_BYTES, tid, cols, DB * 4);  // (of V they only reach columns that are not stored)
 	}
 	// prologue: first K/V tile in flight while Q is fetched
 	if (ntiles > t_first) {
@@ -1511,8 +1516,10 @@ hipError_t launch_fwd_t(bool bias, bool drop, KArgs& a, hipStream_t s) {
 			if constexpr (DE < D) {
 				// Three workgroups a CU from the first one beyond two a CU on.  Under a causal mask a grid of up to twice the resident workgroups waits for its
 				// longest tile, which takes longer with three on a CU: B4 Hq16 Hkv4 S2000 D96 (1024 workgroups) 75 -> 84 us; at S4000 there is nothing to gain (207 -> 211).
-				const bool tail = a.causal && (a.Sk > 2048 || (a.Sk > 1024 && wgs > 3 * kNumCU && wgs < 11 * kNumCU / 2));
-				if (wgs > 2 * kNumCU && !tail) return launch_fwd_cfg<T, D, DE, 4, 3>(bias, drop, a, s);
+				// Up to four a CU are two rounds of either: B7 H16 S1100 D72 72 -> 76, but B10 S577 D80 41.4 -> 40.2, B20 S300 causal 25.9 -> 23.4.
+				const bool even = a.Sk > 1024 && wgs > 3 * kNumCU && wgs <= 4 * kNumCU;
+				if (wgs > 2 * kNumCU && !causal_tail(a, wgs) && !even && a.hd <= 80) return launch_fwd_cfg<T, D, 80, 4, 3>(bias, drop, a, s);
+				if (wgs > 2 * kNumCU && !causal_tail(a, wgs) && !even) return launch_fwd_cfg<T, D, DE, 4, 3>(bias, drop, a, s);
 			}
 			return launch_fwd_cfg<T, D, DE, 4, (D == 128 ? 2 : 1)>(bias, drop, a, s);
 		}
