@@ -1513,11 +1513,11 @@ hipError_t launch_fwd_t(bool bias, bool drop, KArgs& a, hipStream_t s) {
 				if (!bias && wgs <= 2 * kNumCU && a.Sk > 9 * kFwdBN && (a.win_left < 0 || seen > 16 * kFwdBN)) return launch_fwd_cfg<T, D, DE, 4, 4, 2>(bias, drop, a, s);
 				// ... and where a causal grid of up to four a CU would wait for its longest tiles, of more than 32 tiles of keys, which two groups go through in half
 				// the steps.  Two of one group a CU (the tile body above), four of one group, two of two groups: B1 Hq32 Hkv8 S2200 49.1 / 51.3 / 40.2 us, S3000
-				// 61.5 / 67.1 / 53.5, B1 Hq16 Hkv8 S7000 138 / 156 / 122, B2 Hq16 Hkv4 S3700 75.1 / 86.2 / 72.4.  From four a CU on they meet (B1 Hq32 Hkv8 S4096
-				// 89.9 / 82.5 / 84.7, B1 Hq32 S6000 170 / 164 / 168), at S2000 four are as fast (B2 Hq32 Hkv8 55.7 / 55.2; groups not by XCD, B3 Hq16 Hkv4 54.0 / 61.6), with
+				// 61.5 / 67.1 / 53.5, B1 Hq16 Hkv8 S7000 138 / 156 / 122, B2 Hq16 Hkv4 S3700 75.1 / 86.2 / 72.4.  At four a CU the one is 15 % slower or 3 % faster (B1 Hq32 Hkv16 S3973 89.2 / 95.6 / 84.0, B1 Hq32 Hkv8 S4096
+				// 89.9 / 82.5 / 84.7), beyond that they meet (B1 Hq32 Hkv8 S6000 170 / 164 / 168), at S2000 four are as fast (B2 Hq32 Hkv8 55.7 / 55.2; groups not by XCD, B3 Hq16 Hkv4 54.0 / 61.6), with
 				// dropout faster (B1 Hq32 Hkv16 S3973 127 / 149).
 				const bool chain = a.causal && a.win_left < 0 && !drop && a.Sk > 2048 && 8 * (int64_t)a.Sq >= 7 * (int64_t)a.Sk && (a.B * a.Hkv) % 8 == 0;
-				if (!bias && chain && wgs < 4 * kNumCU) return launch_fwd_cfg<T, D, DE, 4, 4, 2>(bias, drop, a, s);
+				if (!bias && chain && wgs <= 4 * kNumCU) return launch_fwd_cfg<T, D, DE, 4, 4, 2>(bias, drop, a, s);
 				if (!bias) return launch_fwd_cfg<T, D, DE, 4, 4>(bias, drop, a, s);
 			}
 			if constexpr (DE < D) {

@@ -26,9 +26,10 @@ BF, FP = torch.bfloat16, torch.float16
 		# two groups of waves a workgroup, two workgroups a CU: ten tiles and more
 		(2, 600, 590, 30, 10, 64, FP, True, None, None, 0.0),
 		(2, 300, 640, 48, 16, 64, BF, False, [640, 65], None, 0.1),
-		# ... and causal grids of up to four a CU over more than 32 tiles: the shortest, one short of four a CU, more keys than rows
+		# ... and causal grids of up to four a CU over more than 32 tiles: the shortest, more keys than rows, four a CU
 		(1, 2049, 2049, 32, 8, 64, BF, True, None, None, 0.0),
 		(1, 2100, 2200, 56, 8, 64, FP, True, None, None, 0.0),
+		(1, 4033, 4033, 32, 16, 64, BF, True, None, None, 0.0),
 		# one to three groups on a grid below the CU count: four, five, sixteen, seventeen tiles; the last group without a tile
 		(1, 130, 193, 3, 1, 64, BF, False, None, None, 0.0),
 		(2, 300, 257, 2, 2, 64, FP, True, None, None, 0.0),
