@@ -24,11 +24,12 @@ forgets what is pending at an unconditional branch; a v_mfma between `;;#ASMSTAR
       spill off (-mllvm -amdgpu-spill-vgpr-to-agpr=0); this rule is the check that no operand is left
       partly unwritten.  (Other instructions are not checked: under a divergent branch the compiler
       legitimately reads registers that are only written for the lanes that use them.)
-  R4  (loops that stream tiles: blocks the compiler marks `Depth=2` or deeper) no access to scratch memory, and no
-      `s_waitcnt vmcnt` that a matrix product follows in the same block - unless the block itself loads values from
-      global memory into registers (the variants that read bias or mask values one by one).  The counter behind
-      vmcnt also counts the direct-to-LDS copies of the next tile, which are issued at the start of a step: a spill
-      reload or a late wait for a value loaded before the loop makes every step wait for those copies.
+  R4  (loops that stream tiles: blocks of a loop that holds matrix products of its own, at any depth) no access to scratch
+      memory, and no `s_waitcnt vmcnt` that a matrix product follows in the same block with no `s_barrier` between them - unless
+      the loop itself reads bias or mask values one by one into registers.
+      The counter behind vmcnt also counts the direct-to-LDS copies of the next tile, which are issued at the start of a step,
+      behind the barrier that publishes the present one: a spill reload or a late wait for a value loaded before the loop makes
+      every step wait for those copies.
       A violation fails the build for the kernel variants without bias and without dropout (the first two boolean
       template arguments); for the other variants, whose register budget is tighter, it is printed as a note.
 A wait state is one instruction; `s_nop N` counts N + 1.
@@ -150,31 +151,32 @@ def lint(path: str):
 	return problems
 
 
-_DEPTH = re.compile(r"^(\.L[\w$]+):.*Depth=(\d+)")
+_LOOP = re.compile(r"(?:Header=(BB\w+) )?Depth=(\d+)")
+_BLOCK_START = re.compile(r"^(?:\.L([\w$]+):|; (%bb\.\d+):)(.*)$")
 
 
 def lint_loops(path: str):
 	"""Rule R4: nothing in a tile loop waits on the memory counter that the tile copies share."""
 	problems, notes = [], []
 	kernel = "?"
-	blocks = []  # (label, depth, [(ln, text)])
+	blocks = []  # (label, loop, [(ln, text)]); loop: the innermost one that the block belongs to, by its header
 	cur = None
 
 	def flush():
 		flags = re.findall(r"Lb([01])E", kernel)[:2]
 		strict = flags == ["0", "0"]
 		out = problems if strict else notes
-		# variants that read bias or mask values one by one load into registers inside the loops: their waits are their own
-		loads = any(t.startswith(("global_load_", "buffer_load_", "flat_load_")) and not t.startswith("global_load_lds")
-		            for _, depth, insts in blocks if depth >= 2 for _, t in insts)
-		for label, depth, insts in blocks:
-			if depth < 2 or loads:
-				continue
+		tile_loops = {loop for _, loop, insts in blocks if any(t.startswith("v_mfma") for _, t in insts)}
+		# loops that read bias or mask values one by one (of one or two bytes, among others) load into registers: their waits are their own
+		own = {loop for _, loop, insts in blocks if any(re.match(r"(global|buffer|flat)_load_[us](byte|short)", t) for _, t in insts)}
+		streaming = [b for b in blocks if b[1] in tile_loops - own]
+		for label, _, insts in streaming:
 			for i, (ln, t) in enumerate(insts):
 				if t.startswith(("scratch_load", "scratch_store")):
 					out.append(f"{path}:{ln}: {kernel}: R4: scratch access `{t.split(';')[0].strip()}` inside a tile loop ({label})")
 				elif t.startswith("s_waitcnt") and "vmcnt" in t:
-					if any(u.startswith("v_mfma") for _, u in insts[i + 1:]):
+					nxt = next((u for _, u in insts[i + 1:] if u.startswith(("v_mfma", "s_barrier"))), "")
+					if nxt.startswith("v_mfma"):
 						out.append(f"{path}:{ln}: {kernel}: R4: `{t}` ahead of matrix products inside a tile loop ({label})")
 
 	with open(path) as f:
@@ -189,13 +191,15 @@ def lint_loops(path: str):
 				flush()
 				blocks, cur = [], None
 				continue
-			md = _DEPTH.match(s)
-			if md:
-				cur = (md.group(1), int(md.group(2)), [])
-				blocks.append(cur)
-				continue
-			if _BLOCK.match(s):
-				cur = None  # a block outside any loop
+			mb = _BLOCK_START.match(s)
+			if mb:
+				ml = _LOOP.search(mb.group(3))
+				if not ml:
+					cur = None  # a block outside any loop
+				elif mb.group(1) or cur is None or cur[1] != ml.group(1):  # (a fall-through inside the loop goes on with its block)
+					# a header names no other header: it is its own
+					cur = ("." + "L" + mb.group(1) if mb.group(1) else mb.group(2), ml.group(1) or mb.group(1), [])
+					blocks.append(cur)
 				continue
 			if cur is not None and s and not s.startswith((";", ".")):
 				cur[2].append((ln, s))

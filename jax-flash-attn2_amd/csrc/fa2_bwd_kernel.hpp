@@ -1313,6 +1313,13 @@ __global__ __launch_bounds__(NW * 64, WPS) void bwd_dq_kernel(const KArgs a) {
 		}
 	}
 
+	// (all of these loads are waited for here: a wait left for the first use stands inside the loop over key tiles and stalls every step until
+	// the copies of the next tile have landed, see the forward kernel)
+#pragma unroll
+	for (int qb = 0; qb < QB; ++qb)
+#pragma unroll
+		for (int ks = 0; ks < KS; ++ks) asm volatile("; Q / dO fragment present" : "+v"(qf[qb][ks]), "+v"(dof[qb][ks]));
+
 	f32x16 dq[QB][DB];
 #pragma unroll
 	for (int qb = 0; qb < QB; ++qb)

@@ -104,3 +104,48 @@ def test_r4_waits_and_spills_inside_tile_loops(tmp_path):
 	assert L.lint_loops(_write(tmp_path, LOOP_CLEAN)) == ([], [])
 	# loops that load values from global memory into registers have waits of their own
 	assert L.lint_loops(_write(tmp_path, LOOP_BIAS_BY_VALUE)) == ([], [])
+
+
+# a loop that streams tiles without another around it, as the compiler marks it: the header names itself, the other blocks name the header
+FLAT_LOOP = """
+	.LBB0_1:                                ; =>This Inner Loop Header: Depth=1
+	s_waitcnt vmcnt(0)
+	s_barrier
+	s_cbranch_scc1 .LBB0_3
+	; %bb.2:                                ;   in Loop: Header=BB0_1 Depth=1
+	global_load_lds_dwordx4 v8, s[8:9]
+	.LBB0_3:                                ;   in Loop: Header=BB0_1 Depth=1
+	{late}
+	v_mfma_f32_32x32x16_bf16 v[0:15], v[4:7], v[16:19], v[0:15]
+	s_cbranch_scc1 .LBB0_1
+	; %bb.4:
+	s_waitcnt vmcnt(0)
+	v_mfma_f32_32x32x16_bf16 v[0:15], v[4:7], v[16:19], v[0:15]
+"""
+# ... and a loop without products of its own, which may do either
+OTHER_LOOP = """
+	.LBB0_1:                                ; =>This Loop Header: Depth=1
+	scratch_load_dword v9, off, off offset:4
+	s_waitcnt vmcnt(0)
+	.LBB0_2:                                ;   Parent Loop BB0_1 Depth=1
+	                                        ; =>  This Inner Loop Header: Depth=2
+	v_mfma_f32_32x32x16_bf16 v[0:15], v[4:7], v[16:19], v[0:15]
+	s_cbranch_scc1 .LBB0_2
+"""
+
+
+def test_r4_loops_that_stand_alone(tmp_path):
+	assert L.lint_loops(_write(tmp_path, FLAT_LOOP.format(late="s_nop 0"))) == ([], [])
+	for late in ("s_waitcnt vmcnt(3) lgkmcnt(3)", "scratch_load_dword v9, off, off offset:4", "scratch_store_dword off, v9, off"):
+		problems, notes = L.lint_loops(_write(tmp_path, FLAT_LOOP.format(late=late)))
+		assert len(problems) == 1 and "R4" in problems[0] and not notes
+		problems, notes = L.lint_loops(_write(tmp_path, FLAT_LOOP.format(late=late), KERNEL_DROP))
+		assert not problems and len(notes) == 1
+	assert L.lint_loops(_write(tmp_path, OTHER_LOOP)) == ([], [])
+
+
+def test_r4_one_value_a_lane_is_no_excuse(tmp_path):
+	# (the statistics of the next tile; only bias and mask values of one or two bytes are waited for product by product)
+	body = FLAT_LOOP.format(late="s_waitcnt vmcnt(0)").replace("s_barrier", "s_barrier\n\tglobal_load_dword v9, v[10:11], off")
+	assert len(L.lint_loops(_write(tmp_path, body))[0]) == 1
+	assert L.lint_loops(_write(tmp_path, body.replace("global_load_dword", "global_load_ubyte"))) == ([], [])
