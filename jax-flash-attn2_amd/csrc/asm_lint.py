@@ -31,7 +31,8 @@ forgets what is pending at an unconditional branch; a v_mfma between `;;#ASMSTAR
       behind the barrier that publishes the present one: a spill reload or a late wait for a value loaded before the loop makes
       every step wait for those copies.
       A violation fails the build for the kernel variants without bias and without dropout (the first two boolean
-      template arguments); for the other variants, whose register budget is tighter, it is printed as a note.
+      template arguments), at head dim 64 (the first number) also for those with dropout; for the other variants, whose register
+      budget is tighter, it is printed as a note.
 A wait state is one instruction; `s_nop N` counts N + 1.
 
 Usage: asm_lint.py FILE.s [FILE.s ...]   (exit status 1 and one line per violation)
@@ -164,7 +165,8 @@ def lint_loops(path: str):
 
 	def flush():
 		flags = re.findall(r"Lb([01])E", kernel)[:2]
-		strict = flags == ["0", "0"]
+		dim = re.search(r"ELi(\d+)E", kernel)
+		strict = flags[:1] == ["0"] and (flags == ["0", "0"] or (dim is not None and dim.group(1) == "64"))
 		out = problems if strict else notes
 		tile_loops = {loop for _, loop, insts in blocks if any(t.startswith("v_mfma") for _, t in insts)}
 		# loops that read bias or mask values one by one (of one or two bytes, among others) load into registers: their waits are their own

@@ -265,7 +265,8 @@ FA2_DEV void lds_dma16_so(uint32_t lane_off, const char* uniform_base, FA2_LDS c
 
 // COLS: rows in memory are shorter than the tile's (head dims that are not the tile's own): lanes whose chunk lies beyond the row
 // fetch nothing, and what the tile holds there stays as it is - zero where zero_cols() has been called.
-template <int D, int ROWS, int NTHREADS, bool COLS = false>
+// LEAN: no offsets are kept, each copy computes its own (two instructions): for variants that have no registers for them.
+template <int D, int ROWS, int NTHREADS, bool COLS = false, bool LEAN = false>
 struct TileLoader {
 	static constexpr int CPR = D / 8;
 	static constexpr int TOTAL = ROWS * CPR;
@@ -278,13 +279,13 @@ struct TileLoader {
 	static constexpr bool COMPACT = D >= 256 && NTHREADS % CPR == 0;
 	static constexpr int RPI = NTHREADS / CPR;
 	static constexpr int P = RPI >= 16 ? 1 : 16 / RPI;
-	static constexpr int NP = COMPACT ? (NIT < P ? NIT : P) : NIT;
-	uint32_t off[NP];
+	static constexpr int NP = LEAN ? 0 : COMPACT ? (NIT < P ? NIT : P) : NIT;
+	uint32_t off[NP > 0 ? NP : 1];
 	int rows_state;  // the offsets clamp rows to [0, rows_state)
 	int cols_state;  // ... and 16-byte chunks of a row to [0, cols_state)
 	int wave_slot;   // byte offset of this wave's 64 x 16 bytes inside a piece (scalar)
 	bool lane_on;    // COLS: this lane's chunk is inside the row (the same for every piece: pieces differ by whole 16-row blocks)
-	static_assert(!COLS || (!COMPACT && RPI % 16 == 0), "");
+	static_assert(!COLS || (!COMPACT && !LEAN && RPI % 16 == 0), "");
 
 	static FA2_DEV uint32_t offset_of(int it, int64_t stride_bytes, int tid, int rows_valid, int chunks_valid) {
 		int slot = it * NTHREADS + tid;
@@ -308,7 +309,7 @@ struct TileLoader {
 	FA2_DEV void fit(int64_t stride_bytes, int tid, int rows_valid, int chunks_valid = CPR) {
 		rows_valid = rows_valid < ROWS ? rows_valid : ROWS;
 		chunks_valid = chunks_valid < CPR ? chunks_valid : CPR;
-		if constexpr (COMPACT) {
+		if constexpr (COMPACT || LEAN) {
 			rows_state = rows_valid;
 			cols_state = chunks_valid;
 		} else {
@@ -330,7 +331,10 @@ struct TileLoader {
 	FA2_DEV void load(FA2_LDS char* tile, const char* gbase, int64_t stride_bytes, int rows_valid, int tid, int chunks_valid = CPR) {
 		fit(stride_bytes, tid, rows_valid, chunks_valid);
 		const char* ub = uniform(gbase);
-		if constexpr (COMPACT) {
+		if constexpr (LEAN) {
+#pragma unroll
+			for (int it = 0; it < NIT; ++it) lds_dma16_so(offset_of(it, stride_bytes, tid, rows_state, cols_state), ub, tile + it * NTHREADS * 16 + wave_slot);
+		} else if constexpr (COMPACT) {
 			if (rows_state == ROWS && cols_state == CPR) {
 #pragma unroll
 				for (int it = 0; it < NIT; ++it)

@@ -149,3 +149,13 @@ def test_r4_one_value_a_lane_is_no_excuse(tmp_path):
 	body = FLAT_LOOP.format(late="s_waitcnt vmcnt(0)").replace("s_barrier", "s_barrier\n\tglobal_load_dword v9, v[10:11], off")
 	assert len(L.lint_loops(_write(tmp_path, body))[0]) == 1
 	assert L.lint_loops(_write(tmp_path, body.replace("global_load_dword", "global_load_ubyte"))) == ([], [])
+
+
+def test_r4_is_strict_with_dropout_at_head_dim_64(tmp_path):
+	# (two groups of waves a workgroup bound to 128 registers once reloaded spilled values in each of their loops)
+	kernel = "_ZN3fa210fwd_kernelINS_4BF16ELi64ELi4ELi1ELi4ELb0ELb1ELb0ELb0ELb0ELi2ELi64EEEvNS_5KArgsE"
+	body = FLAT_LOOP.format(late="scratch_load_dword v9, off, off offset:4")
+	problems, notes = L.lint_loops(_write(tmp_path, body, kernel))
+	assert len(problems) == 1 and not notes
+	problems, notes = L.lint_loops(_write(tmp_path, body, kernel.replace("ELb0ELb1ELb0", "ELb1ELb1ELb0", 1)))
+	assert not problems and len(notes) == 1
