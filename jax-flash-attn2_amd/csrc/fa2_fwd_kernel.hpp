@@ -18,6 +18,7 @@
 #include "fa2_common.hpp"
 #include "fa2_decode_kernel.hpp"
 #include "fa2_kernels.hpp"
+#include "fa2_order.hpp"
 
 namespace fa2 {
 
@@ -32,7 +33,7 @@ constexpr float kRescaleSlack = 8.f;
 // without bias: largest partial row sum of one tile of P = exp2(c1 S - c1 m) taken without looking at
 // the row maximum (fp16 holds values up to 65504)
 constexpr float kFastSum = 16384.f;
-constexpr int kNumCU = 256;  // compute units of the MI355X (tile-size choice for small grids)
+constexpr int kNumCULog2 = 8, kNumCU = 1 << kNumCULog2;  // compute units of the MI355X (tile-size choice for small grids)
 
 // blockIdx.x -> (row tile, q-head, batch).  With xcd_remap the workgroups of
 // one (batch, kv-head) - which share K and V - are kept on one XCD (hardware
@@ -59,7 +60,9 @@ inline int launch_order(const KArgs& a, int heads, int per_xcd, int64_t stream_b
 
 // Workgroups of a causal grid that are all resident at once, several on a CU (see decode_block), else 0.  per_cu: workgroups of the kernel variant that fit
 // a CU (registers, LDS).  Measured with and without, two a CU: B2 Hq8 Hkv2 S4096 D128 forward 0.086 / 0.109 ms (unfolded, the two batch rows put their long
-// tiles on the same CUs), a single group B1 Hq8 S8192 0.163 / 0.168 ms; three and four a CU: B6 Hq16 Hkv4 S1000 D64 33.7 / 28.7 us, B8 33.5 / 40.9.
+// tiles on the same CUs), a single group B1 Hq8 S8192 0.163 / 0.168 ms; three and four a CU: B6 Hq16 Hkv4 S1000 D64 25.8 / 35.0 us, B8 28.0 / 41.9.
+// By row tile over all groups, against group by group as in a larger grid and turned in layers: B1 Hq24 Hkv12 S4328 D64 125.9 / 98.7, B6 H8 S1322 34.6 / 30.2,
+// B3 Hq16 Hkv4 S1384 D88 47.8 / 42.0; B5 Hq4 Hkv1 S2468 D128 with dQ and dK/dV 194 / 192.
 inline int fold_of(const KArgs& a, int nw, int64_t total, int per_cu) {
 	if (nw != 4 || !a.causal || a.win_left >= 0 || a.xcd_remap > 1) return 0;
 	return total > kNumCU && total <= per_cu * kNumCU ? (int)total : 0;
@@ -77,20 +80,19 @@ inline int xcd_ranges_of(const KArgs& a) { return a.hd % 64 != 0 && !a.seqlens &
 FA2_DEV int group_on_xcd(const KArgs& a, int i, int xcd) { return a.xcd_ranges ? xcd * ((a.B * a.Hkv) >> 3) + i : i * 8 + xcd; }
 
 FA2_DEV void decode_block(const KArgs& a, int& mt, int& h, int& b, int id = (int)blockIdx.x) {
+	const int r = a.Hq / a.Hkv;
 	if (a.fold) {
-		// A causal grid whose workgroups are all resident at once: the first 256 workgroup ids take the first place of every CU, the next 256 the
-		// second place in the same order of CUs, and so on (32 ids of every XCD where groups are placed by XCD).  What counts is which of them share a CU.  Their
-		// tiles run from the longest down, so the second half of these layers is visited backwards, and the CU with the longest tiles of the
-		// first half gets the shortest of the second; of three layers the first stays, the second is turned by half its width and the third takes
-		// what makes the sum the same everywhere.
-		const int sh = a.xcd_remap ? 3 : 0, width = kNumCU >> sh, n = a.fold >> sh, layers = (n + width - 1) / width;
-		const int layer = (id >> sh) / width, base = layer * width, count = n - base < width ? n - base : width;
-		int pos = (id >> sh) - base;
-		if (layers == 3 && count == width && layer > 0)
-			pos = layer == 1 ? (pos + width / 2) % width : pos < width / 2 ? width - 1 - 2 * pos : 2 * width - 2 - 2 * pos;
-		else if (2 * layer >= layers)
-			pos = count - 1 - pos;
-		id = ((base + pos) << sh) | (id & ((1 << sh) - 1));
+		// A causal grid whose workgroups are all resident at once (resident_position): what counts is which of them share a CU.  Their order is by row tile
+		// over all (batch, kv-head) groups - of the XCD, where groups are placed by XCD -, the longest tiles first; K and V of all groups are
+		// streamed at once anyway.
+		const int sh = a.xcd_remap ? 3 : 0, n = a.fold >> sh, per_tile = n / a.mtiles;
+		const int j = resident_position(id >> sh, n, kNumCULog2 - sh);
+		const int t = j / per_tile, rem = j % per_tile;
+		const int grp = a.xcd_remap ? group_on_xcd(a, rem / r, id & 7) : rem / r;
+		mt = a.mtiles - 1 - t;
+		b = grp / a.Hkv;
+		h = grp % a.Hkv * r + rem % r;
+		return;
 	}
 	if (a.xcd_remap == 2) {
 		// A bias without a head axis is re-read by every head: one batch per XCD, and on an
@@ -116,7 +118,6 @@ FA2_DEV void decode_block(const KArgs& a, int& mt, int& h, int& b, int id = (int
 		b = ((xcd - tile) & 7) + 8 * (u % nb8);
 		return;
 	}
-	int r = a.Hq / a.Hkv;
 	int per_group = a.mtiles * r;
 	int grp, within;
 	if (a.xcd_remap) {
