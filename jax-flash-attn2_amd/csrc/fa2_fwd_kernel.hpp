@@ -17,6 +17,7 @@
 
 #include "fa2_common.hpp"
 #include "fa2_decode_kernel.hpp"
+#include "fa2_fwd_form.hpp"
 #include "fa2_kernels.hpp"
 #include "fa2_order.hpp"
 
@@ -33,7 +34,6 @@ constexpr float kRescaleSlack = 8.f;
 // without bias: largest partial row sum of one tile of P = exp2(c1 S - c1 m) taken without looking at
 // the row maximum (fp16 holds values up to 65504)
 constexpr float kFastSum = 16384.f;
-constexpr int kNumCULog2 = 8, kNumCU = 1 << kNumCULog2;  // compute units of the MI355X (tile-size choice for small grids)
 
 // blockIdx.x -> (row tile, q-head, batch).  With xcd_remap the workgroups of
 // one (batch, kv-head) - which share K and V - are kept on one XCD (hardware
@@ -64,7 +64,7 @@ inline int launch_order(const KArgs& a, int heads, int per_xcd, int64_t stream_b
 // By row tile over all groups, against group by group as in a larger grid and turned in layers: B1 Hq24 Hkv12 S4328 D64 125.9 / 98.7, B6 H8 S1322 34.6 / 30.2,
 // B3 Hq16 Hkv4 S1384 D88 47.8 / 42.0; B5 Hq4 Hkv1 S2468 D128 with dQ and dK/dV 194 / 192.
 inline int fold_of(const KArgs& a, int nw, int64_t total, int per_cu) {
-	if (nw != 4 || !a.causal || a.win_left >= 0 || a.xcd_remap > 1) return 0;
+	if (nw != 4 || !a.causal || !window_is_open(a.Sk, a.win_left) || a.xcd_remap > 1) return 0;
 	return total > kNumCU && total <= per_cu * kNumCU ? (int)total : 0;
 }
 
@@ -1458,6 +1458,16 @@ hipError_t launch_fwd_cfg(bool bias, bool drop, KArgs& a, hipStream_t s) {
 	return hipGetLastError();
 }
 
+// Head dim 64 without bias, workgroups of 128 rows, one or several to a CU.
+template <typename T>
+hipError_t launch_fwd_64_t(bool drop, KArgs& a, hipStream_t s) {
+	const FwdForm f = fwd_form_64(a.B, a.Hq, a.Hkv, a.Sq, a.Sk, a.causal, a.win_left, a.win_right, drop);
+	if (f.groups == 3) return launch_fwd_cfg<T, 64, 64, 4, 3, 3>(false, drop, a, s);
+	if (f.groups == 2 && f.waves == 2) return launch_fwd_cfg<T, 64, 64, 4, 2, 2>(false, drop, a, s);
+	if (f.groups == 2) return launch_fwd_cfg<T, 64, 64, 4, 4, 2>(false, drop, a, s);
+	return launch_fwd_cfg<T, 64, 64, 4, 4>(false, drop, a, s);
+}
+
 // DE < D: rows of a.hd <= DE columns in the tiles of head dim D, without bias and dropout, one range of keys (the C ABI checks)
 template <typename T, int D, int DE = D>
 hipError_t launch_fwd_t(bool bias, bool drop, KArgs& a, hipStream_t s) {
@@ -1473,24 +1483,18 @@ hipError_t launch_fwd_t(bool bias, bool drop, KArgs& a, hipStream_t s) {
 		// A grid that leaves at least half of the chip idle (small batch x heads, short sequences): workgroups of
 		// 128 rows instead of 256, twice as many of them, still at most one per CU.
 		int64_t wgs = (int64_t)((a.Sq + 127) / 128) * a.B * a.Hq;
-		const int64_t seen = a.win_left >= 0 && a.win_right >= 0 ? (int64_t)a.win_left + a.win_right + 128 : a.Sk;  // keys of a row tile
 		if (wgs <= kNumCU) {
 			// ... and two groups of four waves that take the key tiles of the workgroup's rows in turn: two waves per SIMD where
 			// there was one (B1 Hq32 Hkv8 D128, 1000 rows over 9000 keys: 233 -> 170 us; B1 H8 S4096 D128 81 -> 71 us, causal 79 -> 61;
 			// B2 H16 S1024 D64 with bias 23.4 -> 20.5).  With few tiles the merge costs more than it saves (B1 H8 S128: 8.7 us alone, 10.1 in two
-			// groups): up to three, five at D = 64 and four under a causal mask at D = 128, where it is not dropout or a bias that makes a
-			// tile long.  By tiles, two groups over one, 500 calls: D64 4 / 5 / 6 tiles 1.01 / 1.01 / 0.94, causal 1.06 / 1.00 / 0.98,
-			// dropout 0.97 / 0.96 / 0.92; D128 0.98 / 0.98 / 0.92, causal 1.02 / 0.96 / 0.93.  In a window a row tile sees few tiles whatever
-			// the number of keys (B26 Hq4 Hkv1 S243 D64, 61 keys a row, 9.2 and 10.1).
-			// At head dim 64, block by block, two groups from four tiles on (B2 Hq16 Hkv4 S512 causal 10.8 -> 10.0 us, S256 of B4 8.2 -> 8.0), three from
-			// seventeen (B1 Hq16 Hkv4 S2000 29.9 -> 28.4; at S1024 and below 1 to 6 % slower than two).  Four take 128 registers a wave and spill.
-			const int few = drop || bias || D == 64 || !a.causal ? 3 : 4;
-			const bool groups = a.Sk > few * kFwdBN && seen > few * kFwdBN;
+			// groups): up to three, four under a causal mask at D = 128, where it is not dropout or a bias that makes a tile long.  By tiles, two groups
+			// over one, 500 calls, D128 4 / 5 / 6 tiles 0.98 / 0.98 / 0.92, causal 1.02 / 0.96 / 0.93.  In a window a row tile sees few tiles whatever
+			// the number of keys (B26 Hq4 Hkv1 S243 D64, 61 keys a row, 9.2 and 10.1).  Head dim 64 without bias: fwd_form_64.
 			if constexpr (D == 64) {
-				if (!bias && groups && seen > 16 * kFwdBN) return launch_fwd_cfg<T, D, DE, 4, 3, 3>(bias, drop, a, s);
-				if (!bias && groups) return launch_fwd_cfg<T, D, DE, 4, 2, 2>(bias, drop, a, s);
-				if (!bias) return launch_fwd_cfg<T, D, DE, 4, 4>(bias, drop, a, s);
+				if (!bias) return launch_fwd_64_t<T>(drop, a, s);
 			}
+			const int few = drop || bias || !a.causal ? 3 : 4;
+			const bool groups = fwd_seen_keys(a.Sk, a.win_left, a.win_right) > few * kFwdBN;
 			if (groups && (D == 64 || !bias)) return launch_fwd_cfg<T, D, DE, 4, 1, 2>(bias, drop, a, s);
 			return launch_fwd_cfg<T, D, DE, 4, 1>(bias, drop, a, s);
 		}
@@ -1512,18 +1516,7 @@ hipError_t launch_fwd_t(bool bias, bool drop, KArgs& a, hipStream_t s) {
 		                                    : (drop ? 1024 * D * 4 : (2 << 20));
 		if ((int64_t)a.Sk * DE * 4 <= kv_limit && (D == 64 || (!bias && !(a.softcap > 0.f)))) {
 			if constexpr (D == 64) {
-				// Four waves a SIMD: four such workgroups a CU, or two of two groups each where the grid has no more than that (over
-				// ten tiles and more; B4 Hq16 Hkv4 S1000 29.3 -> 28.4 us against 30.2 with one group, causal 23.9 -> 21.6 against 24.9; at S400 14.0 -> 12.8 with one, 15.0
-				// with two) or seventeen of a window (B1 Hq16 Hkv4 S4000, 1024 keys a row 29.3 -> 28.4 against 29.5, 512 keys 20.3 -> 21.5 against 20.0).
-				if (!bias && wgs <= 2 * kNumCU && a.Sk > 9 * kFwdBN && (a.win_left < 0 || seen > 16 * kFwdBN)) return launch_fwd_cfg<T, D, DE, 4, 4, 2>(bias, drop, a, s);
-				// ... and where a causal grid of up to four a CU would wait for its longest tiles, of more than 32 tiles of keys, which two groups go through in half
-				// the steps.  Two of one group a CU (the tile body above), four of one group, two of two groups: B1 Hq32 Hkv8 S2200 49.1 / 51.3 / 40.2 us, S3000
-				// 61.5 / 67.1 / 53.5, B1 Hq16 Hkv8 S7000 138 / 156 / 122, B2 Hq16 Hkv4 S3700 75.1 / 86.2 / 72.4.  At four a CU the one is 15 % slower or 3 % faster (B1 Hq32 Hkv16 S3973 89.2 / 95.6 / 84.0, B1 Hq32 Hkv8 S4096
-				// 89.9 / 82.5 / 84.7), beyond that they meet (B1 Hq32 Hkv8 S6000 170 / 164 / 168), at S2000 four are as fast (B2 Hq32 Hkv8 55.7 / 55.2; groups not by XCD, B3 Hq16 Hkv4 54.0 / 61.6), with
-				// dropout faster (B1 Hq32 Hkv16 S3973 127 / 149).
-				const bool chain = a.causal && a.win_left < 0 && !drop && a.Sk > 2048 && 8 * (int64_t)a.Sq >= 7 * (int64_t)a.Sk && (a.B * a.Hkv) % 8 == 0;
-				if (!bias && chain && wgs <= 4 * kNumCU) return launch_fwd_cfg<T, D, DE, 4, 4, 2>(bias, drop, a, s);
-				if (!bias) return launch_fwd_cfg<T, D, DE, 4, 4>(bias, drop, a, s);
+				if (!bias) return launch_fwd_64_t<T>(drop, a, s);
 			}
 			if constexpr (DE < D) {
 				// Three workgroups a CU from the first one beyond two a CU on.  Under a causal mask a grid of up to twice the resident workgroups waits for its

@@ -10,6 +10,8 @@
 
 namespace fa2 {
 
+constexpr int kNumCULog2 = 8, kNumCU = 1 << kNumCULog2;  // compute units of the MI355X
+
 // n workgroups, the longest first, on 1 << log2_width compute units: the position in that order of the workgroup that arrives as the i-th.  The first
 // 1 << log2_width arrivals take the first place of every unit, the next as many the second place in the same order of units, and so on; what counts is the
 // sum over the places of a unit.  Units that get nothing of a last layer that is not full hold the longest workgroups, and the order of units starts from them.  The first

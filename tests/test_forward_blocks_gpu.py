@@ -23,6 +23,10 @@ BF, FP = torch.bfloat16, torch.float16
 		(4, 250, 300, 128, 8, 64, BF, True, None, None, 0.0),
 		(6, 250, 250, 64, 16, 80, FP, True, None, None, 0.0),
 		(5, 129, 129, 61, 61, 96, BF, True, None, None, 0.0),
+		# ... in a window that hides less than a third of the keys, or none
+		(5, 600, 600, 28, 7, 64, FP, True, None, (400, 0), 0.0),
+		(5, 257, 257, 40, 8, 64, BF, True, None, (1000, 0), 0.1),
+		(5, 250, 300, 64, 16, 88, BF, True, None, (200, 0), 0.0),
 		# two groups of waves a workgroup, two workgroups a CU: ten tiles and more
 		(2, 600, 590, 30, 10, 64, FP, True, None, None, 0.0),
 		(2, 300, 640, 48, 16, 64, BF, False, [640, 65], None, 0.1),

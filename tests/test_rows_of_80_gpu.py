@@ -30,6 +30,7 @@ BF, FP = torch.bfloat16, torch.float16
 		(1, 2100, 2100, 36, 36, 80, BF, True, None, None),
 		# three layers of workgroups that are all resident
 		(6, 250, 250, 64, 16, 80, BF, True, None, None),
+		(6, 250, 250, 64, 16, 80, FP, True, None, (170, 0)),
 	],
 )
 def test_against_the_oracle(B, Sq, Sk, Hq, Hkv, D, dtype, causal, kv_lens, window):
