@@ -1,10 +1,13 @@
 """The forward block by block (head dim 64, and rows of 72 to 96 columns), three and four workgroups a CU: grids whose workgroups are all resident at
 once and whose parts are visited backwards, two and three groups of waves on the keys of a row tile, ragged blocks of keys."""
 
+import ctypes
+
 import pytest
 import torch
 
 from jax_flash_attn2 import _hip_op as op
+from jax_flash_attn2 import _lib
 import fa2_oracle as O
 from _cases import check_forward, f64, make_inputs
 
@@ -12,10 +15,24 @@ pytestmark = pytest.mark.gpu
 BF, FP = torch.bfloat16, torch.float16
 
 
+def _check(B, Sq, Sk, Hq, Hkv, D, dtype, causal, lens, window, p, ranges=None, qk_scale=None):
+	"""ranges: into how many parts the keys of a row tile are meant to be cut (0: the call is meant to run unsplit)."""
+	q, k, v, _, _ = make_inputs(B, Sq, Sk, Hq, Hkv, D, dtype, seed=Sq + Sk, qk_scale=qk_scale)
+	kw = dict(causal=causal, kv_lens=lens, window=window, p_drop=p, seed=5)
+	q_, k_, v_ = q.cuda(), k.cuda(), v.cuda()
+	kl = None if lens is None else torch.tensor(lens, dtype=torch.int32, device="cuda:0")
+	if ranges is not None:
+		n = _lib.load().fa2_fwd_scratch_bytes(ctypes.byref(op._block(D, q_, k_, v_, None, None, 1.0, p, causal, 5, kl, window)))
+		assert n == (ranges * B * Hq * Sq * (D + 1) * 4 + 255) // 256 * 256
+	o, lse = op.fwd(q_, k_, v_, None, None, None, p, causal, 5, kl, window)
+	o_ref, lse_ref = O.attention_fwd(f64(q), f64(k), f64(v), None, **kw)
+	check_forward(o, lse, o_ref, lse_ref, dtype, f"B{B} Sq{Sq} Sk{Sk} Hq{Hq} Hkv{Hkv} D{D} qk_scale={qk_scale} {kw}")
+
+
 @pytest.mark.parametrize(
 	"B,Sq,Sk,Hq,Hkv,D,dtype,causal,lens,window,p",
 	[
-		# causal grids that are all resident: 264 workgroups (two layers), 768 (three whole ones), 640, 700 (the last one short), 1024 (four); by XCD and not
+		# causal grids that are all resident: 264 workgroups (two layers), 768 (three whole ones, twice), 700 and 610 (the last one short), 1024 (four); by XCD and not
 		(2, 300, 300, 44, 11, 64, BF, True, None, None, 0.0),
 		(8, 130, 130, 48, 6, 64, FP, True, None, None, 0.0),
 		(8, 257, 257, 32, 4, 64, BF, True, None, None, 0.0),
@@ -34,13 +51,6 @@ BF, FP = torch.bfloat16, torch.float16
 		(1, 2049, 2049, 32, 8, 64, BF, True, None, None, 0.0),
 		(1, 2100, 2200, 56, 8, 64, FP, True, None, None, 0.0),
 		(1, 4033, 4033, 32, 16, 64, BF, True, None, None, 0.0),
-		# one to three groups on a grid below the CU count: four, five, sixteen, seventeen tiles; the last group without a tile
-		(1, 130, 193, 3, 1, 64, BF, False, None, None, 0.0),
-		(2, 300, 257, 2, 2, 64, FP, True, None, None, 0.0),
-		(1, 1100, 1024, 2, 2, 64, BF, True, None, None, 0.0),
-		(1, 1100, 1025, 2, 2, 64, FP, True, None, None, 0.1),
-		(2, 1200, 1200, 2, 1, 64, BF, True, [1200, 0], None, 0.0),
-		(1, 1300, 1300, 2, 1, 64, FP, True, None, (900, 0), 0.0),
 		# more than two workgroups a CU: blocks of keys that only some rows see, lengths, a window, rows without keys, one key
 		(9, 257, 257, 20, 20, 80, FP, False, None, None, 0.0),
 		(9, 200, 97, 32, 8, 72, BF, True, [97, 96, 64, 33, 32, 31, 1, 0, 97], None, 0.0),
@@ -48,22 +58,86 @@ BF, FP = torch.bfloat16, torch.float16
 		(9, 300, 300, 20, 5, 64, BF, True, None, (33, 0), 0.0),
 		(70, 33, 1, 16, 2, 64, FP, False, None, None, 0.0),
 		(40, 65, 129, 30, 6, 64, BF, False, None, None, 0.2),
-		# key ranges of workgroups that share a CU
-		(1, 700, 5000, 16, 4, 64, BF, True, None, None, 0.0),
-		# head dim 128, four waves a workgroup and two workgroups a CU: two ranges, three, five; rows that end before the last, a range of one tile with one key
-		(1, 1000, 5700, 24, 8, 128, BF, True, None, None, 0.0),
-		(1, 600, 2945, 32, 8, 128, FP, False, None, None, 0.0),
-		(1, 1500, 1601, 8, 2, 128, BF, True, None, None, 0.0),
-		(2, 1500, 1400, 6, 6, 128, FP, True, None, None, 0.0),
 	],
 )
 def test_blocks(B, Sq, Sk, Hq, Hkv, D, dtype, causal, lens, window, p):
-	q, k, v, _, _ = make_inputs(B, Sq, Sk, Hq, Hkv, D, dtype, seed=Sq + Sk)
-	kw = dict(causal=causal, kv_lens=lens, window=window, p_drop=p, seed=5)
-	kl = None if lens is None else torch.tensor(lens, dtype=torch.int32, device="cuda:0")
-	o, lse = op.fwd(q.cuda(), k.cuda(), v.cuda(), None, None, None, p, causal, 5, kl, window)
-	o_ref, lse_ref = O.attention_fwd(f64(q), f64(k), f64(v), None, **kw)
-	check_forward(o, lse, o_ref, lse_ref, dtype, f"B{B} Sq{Sq} Sk{Sk} Hq{Hq} Hkv{Hkv} D{D} {kw}")
+	_check(B, Sq, Sk, Hq, Hkv, D, dtype, causal, lens, window, p)
+
+
+@pytest.mark.parametrize(
+	"B,Sq,Sk,Hq,Hkv,dtype,causal,lens,window,p",
+	[
+		# head dim 64, at most one workgroup a CU, keys in one range: one group of waves (three tiles), two (four, five, sixteen), three (seventeen and more)
+		(1, 130, 192, 3, 1, BF, False, None, None, 0.0),
+		(1, 130, 193, 3, 1, BF, False, None, None, 0.0),
+		(2, 300, 257, 2, 2, FP, True, None, None, 0.0),
+		(2, 900, 1024, 14, 7, BF, True, None, None, 0.0),
+		(2, 900, 1025, 14, 7, FP, True, None, None, 0.0),
+		(1, 2000, 2000, 16, 4, BF, True, None, None, 0.0),
+		# ... the same without a causal mask, with dropout
+		(2, 900, 1025, 14, 7, BF, False, None, None, 0.0),
+		(1, 1100, 1024, 16, 16, FP, True, None, None, 0.1),
+		(1, 1100, 1025, 16, 16, FP, True, None, None, 0.1),
+		(1, 1100, 1150, 16, 16, BF, False, None, None, 0.2),
+		# ... rows without keys; lengths that leave the second, or the third, of three groups without a tile
+		(2, 1200, 1200, 12, 4, BF, True, [1200, 0], None, 0.0),
+		(2, 900, 1025, 14, 7, FP, False, [64, 65], None, 0.0),
+		(2, 900, 1025, 14, 7, BF, False, [128, 129], None, 0.1),
+		# ... windows of which a row tile sees three, four, sixteen and seventeen tiles' keys, and one that begins in the middle
+		(2, 450, 450, 2, 1, BF, True, None, (64, 0), 0.0),
+		(2, 450, 450, 2, 1, BF, True, None, (65, 0), 0.0),
+		(2, 1300, 1300, 2, 1, FP, True, None, (896, 0), 0.0),
+		(2, 1300, 1300, 2, 1, FP, True, None, (897, 0), 0.0),
+	],
+)
+def test_groups_of_waves_on_a_range_of_keys(B, Sq, Sk, Hq, Hkv, dtype, causal, lens, window, p):
+	assert (Sq + 127) // 128 * B * Hq <= 256
+	_check(B, Sq, Sk, Hq, Hkv, 64, dtype, causal, lens, window, p, ranges=0)
+
+
+@pytest.mark.parametrize(
+	"Sq,Sk,Hq,Hkv,D,dtype,causal,ranges",
+	[
+		# head dim 64: workgroups that share a CU
+		(700, 5000, 16, 4, 64, BF, True, 5),
+		# head dim 128, four waves a workgroup and two workgroups a CU (these are 384 to 512 in all): two ranges, three, of which the last ends with one key in its last
+		# tile, and five, of which the first rows see no key of the last
+		(1000, 5700, 24, 8, 128, BF, True, 2),
+		(600, 2945, 32, 8, 128, FP, False, 3),
+		(1500, 6200, 8, 2, 128, BF, True, 5),
+		(1100, 4097, 10, 5, 128, FP, True, 5),
+		# ... and of eight waves, one a CU
+		(1500, 1601, 8, 2, 128, BF, True, 2),
+	],
+)
+def test_ranges_of_keys(Sq, Sk, Hq, Hkv, D, dtype, causal, ranges):
+	_check(1, Sq, Sk, Hq, Hkv, D, dtype, causal, None, None, 0.0, ranges)
+
+
+@pytest.mark.parametrize("qk_scale", [2.1, 4.2])
+@pytest.mark.parametrize(
+	"B,Sq,Sk,Hq,Hkv,D,dtype,causal,lens,p",
+	[
+		# block by block: a later block raises the reference of a row that has one.  Rows of 72 to 96 columns; one group of waves (four a SIMD, few tiles), two
+		# (two and four waves a SIMD), three; with dropout
+		(9, 257, 257, 20, 20, 80, FP, False, None, 0.0),
+		(9, 257, 300, 20, 5, 72, BF, True, None, 0.0),
+		(9, 257, 257, 20, 20, 96, BF, False, [257, 1, 33, 64, 65, 0, 200, 256, 97], 0.0),
+		(8, 257, 257, 32, 4, 64, BF, True, None, 0.0),
+		(9, 257, 257, 20, 20, 64, FP, False, None, 0.1),
+		(1, 130, 192, 3, 1, 64, FP, False, None, 0.1),
+		(2, 200, 520, 2, 2, 64, BF, False, None, 0.1),
+		(2, 600, 700, 30, 10, 64, FP, True, None, 0.1),
+		(2, 900, 1100, 14, 7, 64, BF, False, None, 0.0),
+		(1, 1100, 1100, 16, 16, 64, FP, True, None, 0.2),
+		# on key ranges of two workgroups a CU
+		(1, 700, 5000, 16, 4, 64, FP, True, None, 0.0),
+		(1, 600, 2945, 32, 8, 128, BF, False, None, 0.0),
+	],
+)
+def test_large_scores(B, Sq, Sk, Hq, Hkv, D, dtype, causal, lens, p, qk_scale):
+	"""Scores within about +-20 and +-80 at qk_scale 2.1 and 4.2."""
+	_check(B, Sq, Sk, Hq, Hkv, D, dtype, causal, lens, None, p, qk_scale=qk_scale)
 
 
 def test_256_row_workgroups_beyond_the_l2():

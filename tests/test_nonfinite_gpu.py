@@ -20,11 +20,12 @@ def _scratch(q, k, v, causal=False, kv_lens=None):
 	return _lib.load().fa2_fwd_scratch_bytes(ctypes.byref(op._block(q.shape[3], q, k, v, None, None, 1.0, 0.0, causal, None, kv_lens)))
 
 
-# (B, Sq, Sk, Hq, Hkv, D, causal): 128-row workgroups on several ranges; ranges of the 64-row kernel with the q-heads packed; head
+# (B, Sq, Sk, Hq, Hkv, D, causal): 128-row workgroups on several ranges, and of four waves, two a CU, on five; ranges of the 64-row kernel with the q-heads packed; head
 # dim 256, which takes that kernel unpacked; the decoding kernel with units of several waves, and of few keys (257 .. 448)
 _PIECES = [
 	(1, 100, 2000, 8, 2, 128, True),
 	(1, 300, 1500, 4, 4, 64, False),
+	(1, 1500, 6200, 8, 2, 128, True),
 	(1, 8, 4000, 8, 2, 128, False),
 	(1, 65, 2048, 2, 2, 256, True),
 	(1, 1, 1029, 32, 8, 128, False),

@@ -34,9 +34,13 @@ pytestmark = pytest.mark.gpu
 		(2, 64, 1100, 32, 32, 64, torch.float16, False, [1100, 30], None, 0.0, False),
 		(1, 33, 8200, 2, 2, 128, torch.bfloat16, True, None, None, 0.0, False),
 		(4, 20, 3100, 8, 8, 128, torch.float16, False, [3100, 0, 1, 2000], None, 0.0, False),
-		# head dim 64 without bias and dropout: two groups from six tiles on; a window of which a row tile sees five tiles' keys, and one more
+		# head dim 64 without bias: two groups from four tiles on; a window of which a row tile sees three tiles' keys, and one more
+		(2, 192, 192, 2, 2, 64, torch.float16, True, None, None, 0.0, False),
+		(2, 193, 193, 2, 2, 64, torch.float16, True, None, None, 0.0, False),
 		(2, 320, 320, 2, 2, 64, torch.float16, True, None, None, 0.0, False),
 		(2, 321, 321, 2, 2, 64, torch.float16, True, None, None, 0.0, False),
+		(2, 450, 450, 2, 1, 64, torch.bfloat16, True, None, (64, 0), 0.0, False),
+		(2, 450, 450, 2, 1, 64, torch.bfloat16, True, None, (65, 0), 0.0, False),
 		(2, 450, 450, 2, 1, 64, torch.bfloat16, True, None, (192, 0), 0.0, False),
 		(2, 450, 450, 2, 1, 64, torch.bfloat16, True, None, (193, 0), 0.0, False),
 		# head dim 128 under a causal mask: from five tiles on; rows without keys, a window that begins in the middle
