@@ -36,13 +36,14 @@ inline FwdForm fwd_form_64(int B, int Hq, int Hkv, int Sq, int Sk, bool causal, 
 	// with two) or seventeen of a window (B1 Hq16 Hkv4 S4000, 1024 keys a row 29.3 -> 28.4 against 29.5, 512 keys 20.3 -> 21.5 against 20.0).
 	const bool open = window_is_open(Sk, win_left);
 	if (wgs <= 2 * kNumCU && Sk > 9 * 64 && (open || seen > 16 * 64)) return {2, 4};
-	// ... and where a causal grid of up to four a CU would wait for its longest tiles, of more than 32 tiles of keys, which two groups go through in half
-	// the steps.  Two of one group a CU (the tile body), four of one group, two of two groups: B1 Hq32 Hkv8 S2200 49.1 / 51.3 / 40.2 us, S3000
-	// 61.5 / 67.1 / 53.5, B1 Hq16 Hkv8 S7000 138 / 156 / 122, B2 Hq16 Hkv4 S3700 75.1 / 86.2 / 72.4.  At four a CU the one is 15 % slower or 3 % faster (B1 Hq32 Hkv16 S3973 89.2 / 95.6 / 84.0, B1 Hq32 Hkv8 S4096
-	// 89.9 / 82.5 / 84.7), beyond that they meet (B1 Hq32 Hkv8 S6000 170 / 164 / 168), at S2000 four are as fast (B2 Hq32 Hkv8 55.7 / 55.2; groups not by XCD, B3 Hq16 Hkv4 54.0 / 61.6), with
-	// dropout faster (B1 Hq32 Hkv16 S3973 127 / 149).
-	const bool chain = causal && open && !drop && Sk > 2048 && 8 * (int64_t)Sq >= 7 * (int64_t)Sk && (int64_t)B * Hkv % 8 == 0;
-	if (chain && wgs <= 4 * kNumCU) return {2, 4};
+	// ... and where a causal grid would wait for its longest tiles, of more than 32 tiles of keys, which two groups go through in half the steps.  Two of one group a CU (the tile
+	// body) / four of one group / two of two groups: B1 Hq32 Hkv8 S2200 45.5 / 47.3 / 37.9 us, S3000 61 / 67 / 53, B1 Hq16 Hkv8 S7000 140 / 158 / 122, B2 Hq16 Hkv4 S3700 76 / 87 / 72,
+	// B1 Hq24 Hkv12 S4328 121 / 97 / 77, B1 Hq16 Hkv4 S6000 141 / 128 / 100; at four a CU B1 Hq32 Hkv16 S3973 88 / 97 / 83, B1 Hq32 Hkv8 S4096 90 / 83 / 85.  With dropout four of one
+	// group are faster up to there (S3973 152 / 127 / 133).  Up to five and a half a CU more than 64 tiles: B1 Hq32 Hkv8 S4200 94 / 105 / 89, B1 Hq16 Hkv8 S9000 200 / 224 / 189, with
+	// dropout 350 / 355 / 315, S11000 281 / 290 / 273, B1 Hq32 Hkv8 S5700 (5.6 a CU) 157 / 155 / 156, S6000 170 / 166 / 170; but B2 H24 S3200 89 / 75 / 81, B4 H16 S2400 67 / 57 / 65.
+	const bool chain = causal && open && 8 * (int64_t)Sq >= 7 * (int64_t)Sk;
+	if (chain && wgs <= 4 * kNumCU && Sk > 2048 && !drop) return {2, 4};
+	if (chain && wgs > 4 * kNumCU && 2 * wgs <= 11 * kNumCU && Sk > 4096) return {2, 4};
 	return {1, 4};
 }
 

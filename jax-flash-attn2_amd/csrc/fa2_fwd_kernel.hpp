@@ -118,24 +118,12 @@ FA2_DEV void decode_block(const KArgs& a, int& mt, int& h, int& b, int id = (int
 		b = ((xcd - tile) & 7) + 8 * (u % nb8);
 		return;
 	}
-	int per_group = a.mtiles * r;
-	int grp, within;
-	if (a.xcd_remap) {
-		int xcd = id & 7, j = id >> 3;
-		// a.interleave = e groups of an XCD advance together: e r adjacent workgroups are the same row tile (see launch_order())
-		int e = a.interleave;
-		int sgi = j / (e * per_group), rem = j % (e * per_group);
-		int t = rem / (e * r), rem2 = rem % (e * r);
-		grp = group_on_xcd(a, sgi * e + rem2 / r, xcd);
-		within = t * r + rem2 % r;
-	} else {
-		grp = id / per_group;
-		within = id % per_group;
-	}
-	int hk = grp % a.Hkv;
+	// (a.interleave groups advance together, see launch_order() and groups_together())
+	const Place p = place_of(a.xcd_remap ? id >> 3 : id, (a.B * a.Hkv) >> (a.xcd_remap ? 3 : 0), r, a.mtiles, a.interleave);
+	const int grp = a.xcd_remap ? group_on_xcd(a, p.group, id & 7) : p.group;
 	b = grp / a.Hkv;
-	mt = a.mtiles - 1 - within / r;
-	h = hk * r + within % r;
+	mt = a.mtiles - 1 - p.tile;
+	h = grp % a.Hkv * r + p.head;
 }
 
 // four consecutive bias values bias[row][col..col+3] as floats.  dtype 4: the row holds bytes of a boolean
@@ -1430,6 +1418,10 @@ hipError_t launch_fwd_cfg(bool bias, bool drop, KArgs& a, hipStream_t s) {
 	if (bias && a.bias_sh == 0 && a.B % 8 == 0) a.xcd_remap = a.kv_lens ? 3 : 2;
 	dim3 grid((unsigned)(a.mtiles * a.B * a.Hq)), block(NW * 64 * KW);
 	a.fold = fold_of(a, NW, (int64_t)grid.x, KW > 1 ? WPS / KW : D == 64 && WPS == 1 ? 2 : WPS);
+	if constexpr (D == 64 && NW == 4 && WPS > 1) {
+		if (!bias && a.causal && window_is_open(a.Sk, a.win_left) && !a.fold && (int64_t)grid.x > kNumCU)
+			a.interleave = groups_together(a.xcd_remap ? groups / 8 : groups, a.Hq / a.Hkv, a.xcd_remap, (int64_t)grid.x, (int64_t)a.Sk * D * 4);
+	}
 	const bool blds = bias && a.bias_lds;
 	// (head dim 128 with bias tiles has no LDS for a second group)
 	constexpr bool WITH_BIAS = DE == D && (D == 64 || KW == 1) && WPS == 1, WITHOUT = D != 64 || WPS > 1;

@@ -44,6 +44,13 @@ def _check(B, Sq, Sk, Hq, Hkv, D, dtype, causal, lens, window, p, ranges=None, q
 		(5, 600, 600, 28, 7, 64, FP, True, None, (400, 0), 0.0),
 		(5, 257, 257, 40, 8, 64, BF, True, None, (1000, 0), 0.1),
 		(5, 250, 300, 64, 16, 88, BF, True, None, (200, 0), 0.0),
+		# causal grids that are not: all groups advance together (by XCD and not), or as many as leave the last ones fewer
+		(8, 600, 600, 32, 8, 64, FP, True, None, None, 0.0),
+		(9, 600, 600, 28, 7, 64, BF, True, None, None, 0.1),
+		(9, 600, 600, 28, 7, 64, BF, True, None, (500, 0), 0.0),
+		(36, 130, 130, 30, 30, 64, BF, True, None, None, 0.0),
+		(35, 130, 140, 30, 30, 64, FP, True, None, None, 0.0),
+		(63, 130, 130, 20, 5, 64, BF, True, None, None, 0.0),
 		# two groups of waves a workgroup, two workgroups a CU: ten tiles and more
 		(2, 600, 590, 30, 10, 64, FP, True, None, None, 0.0),
 		(2, 300, 640, 48, 16, 64, BF, False, [640, 65], None, 0.1),
@@ -146,3 +153,14 @@ def test_256_row_workgroups_beyond_the_l2():
 	heads = [0, 131, 263]
 	o_ref, lse_ref = O.attention_fwd(f64(q[:, :, heads]), f64(k), f64(v), None, causal=True)
 	check_forward(o[:, :, heads], lse[:, heads], o_ref, lse_ref, BF)
+
+
+@pytest.mark.parametrize("S,Hq,Hkv", [(4100, 32, 16), (2300, 36, 12), (4100, 33, 3)])
+def test_two_groups_of_waves_on_grids_that_are_not_resident(S, Hq, Hkv):
+	q, k, v, _, _ = make_inputs(1, S, S, Hq, Hkv, 64, BF, seed=S + Hq)
+	o, lse = op.fwd(q.cuda(), k.cuda(), v.cuda(), None, None, None, 0.0, True, 0)
+	r = Hq // Hkv
+	for j in (0, Hkv // 2, Hkv - 1):
+		heads = slice(j * r, j * r + min(r, 3))
+		o_ref, lse_ref = O.attention_fwd(f64(q[:, :, heads]), f64(k[:, :, j : j + 1]), f64(v[:, :, j : j + 1]), None, causal=True)
+		check_forward(o[:, :, heads], lse[:, heads], o_ref, lse_ref, BF, f"S{S} Hq{Hq} Hkv{Hkv} group {j}")

@@ -56,3 +56,17 @@ def test_tiles_of_keys(lib):
 		assert _form(lib, 2, 4, 2, 130, causal=False, Sk=n) == form
 	for n, form in ((576, (1, 4)), (577, (2, 4))):
 		assert _form(lib, 2, 100, 100, 130, causal=False, Sk=n) == form
+
+
+def test_causal_grids_that_wait_for_their_longest_tiles(lib):
+	one, two = (1, 4), (2, 4)
+	# up to four workgroups a CU over more than 2048 keys, without dropout; groups placed by XCD or not
+	for B, Hq, Hkv in ((1, 40, 8), (1, 36, 9)):
+		assert _form(lib, B, Hq, Hkv, 2048) == one and _form(lib, B, Hq, Hkv, 2049) == two and _form(lib, B, Hq, Hkv, 2049, drop=True) == one
+	assert _form(lib, 1, 32, 8, 4096) == two and _form(lib, 1, 32, 8, 4096, drop=True) == one and _form(lib, 1, 36, 9, 4096) == one
+	# up to five and a half over more than 4096
+	for drop in (False, True):
+		assert _form(lib, 1, 32, 8, 4097, drop=drop) == two and _form(lib, 1, 32, 8, 5632, drop=drop) == two and _form(lib, 1, 32, 8, 5633, drop=drop) == one
+	assert _form(lib, 2, 24, 24, 3200) == one
+	# not where rows see about as many keys each
+	assert _form(lib, 1, 32, 8, 3500, Sk=4000) == two and _form(lib, 1, 32, 8, 3499, Sk=4000) == one and _form(lib, 1, 32, 8, 3000, causal=False) == one

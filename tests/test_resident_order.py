@@ -1,5 +1,6 @@
-"""The order of a causal grid whose workgroups are all resident at once (csrc/fa2_order.hpp), compiled for the host: every workgroup is
-visited once, and no compute unit has much more work than the best split of the same workgroups over as many places."""
+"""The orders of a grid's workgroups (csrc/fa2_order.hpp), compiled for the host.  Of a causal grid whose workgroups are all resident at once: every workgroup is
+visited once, and no compute unit has much more work than the best split of the same workgroups over as many places.  Of groups that advance together: each
+workgroup once, the longest first, and as many groups at a time as the rule says."""
 
 import ctypes
 import heapq
@@ -11,13 +12,29 @@ import pytest
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "jax-flash-attn2_amd", "csrc")
 
 
+SRC = """
+#include "fa2_order.hpp"
+extern "C" int position(int i, int n, int w) { return fa2::resident_position(i, n, w); }
+extern "C" void place(int i, int groups, int heads, int tiles, int together, int* out) {
+	const fa2::Place p = fa2::place_of(i, groups, heads, tiles, together);
+	out[0] = p.group, out[1] = p.tile, out[2] = p.head;
+}
+extern "C" int together(int groups, int heads, int by_xcd, long long wgs, long long kv_bytes) { return fa2::groups_together(groups, heads, by_xcd, wgs, kv_bytes); }
+"""
+
+
 @pytest.fixture(scope="module")
-def position(tmp_path_factory):
+def lib(tmp_path_factory):
 	d = tmp_path_factory.mktemp("order")
 	src, out = d / "order.cc", d / "order.so"
-	src.write_text('#include "fa2_order.hpp"\nextern "C" int position(int i, int n, int w) { return fa2::resident_position(i, n, w); }\n')
+	src.write_text(SRC)
 	subprocess.check_call([os.environ.get("CXX", "c++"), "-std=c++17", "-O1", "-shared", "-fPIC", "-I", CSRC, "-o", str(out), str(src)])
-	f = ctypes.CDLL(str(out)).position
+	return ctypes.CDLL(str(out))
+
+
+@pytest.fixture(scope="module")
+def position(lib):
+	f = lib.position
 	f.argtypes, f.restype = [ctypes.c_int] * 3, ctypes.c_int
 	return f
 
@@ -58,3 +75,32 @@ def test_no_unit_has_much_more_than_its_share(position, B, Hq, Hkv, S):
 	ours, best, mean = _loads(position, B, Hq, Hkv, S)
 	# (mean: where it is beyond any split, the longest workgroups alone are; three places of which the last is taken by a few are the worst of the rule)
 	assert ours <= 1.2 * max(best, mean), (ours, best, mean)
+
+
+@pytest.mark.parametrize("groups,heads,tiles,together", [(1, 1, 1, 1), (5, 1, 7, 1), (5, 3, 7, 2), (7, 4, 3, 7), (135, 1, 2, 8), (17, 2, 9, 6), (8, 8, 5, 3)])
+def test_groups_that_advance_together(lib, groups, heads, tiles, together):
+	out, seen, last = (ctypes.c_int * 3)(), set(), (0, 0)
+	for i in range(groups * heads * tiles):
+		lib.place(i, groups, heads, tiles, together, out)
+		group, tile, head = out
+		assert 0 <= group < groups and 0 <= tile < tiles and 0 <= head < heads
+		seen.add((group, tile, head))
+		at = (group // together, tile)  # each block of groups from its longest tiles down
+		assert at >= last
+		last = at
+	assert len(seen) == groups * heads * tiles
+
+
+def test_how_many_advance_together(lib):
+	def f(groups, heads, by_xcd, wgs, kv_bytes):
+		return lib.together(groups, heads, int(by_xcd), ctypes.c_longlong(wgs), ctypes.c_longlong(kv_bytes))
+
+	# up to eight workgroups a CU: all, of an XCD as long as their K and V are within 16 MiB
+	assert f(780, 1, False, 2048, 1 << 22) == 780 and f(16, 1, True, 2048, 1 << 20) == 16 and f(16, 1, True, 2048, (1 << 20) + 1) == 4
+	# beyond: evened out
+	assert f(780, 1, False, 2049, 1 << 18) == 60 and f(9, 1, True, 2049, 1 << 20) == 5 and f(9, 1, True, 2049, 2 << 20) == 3 and f(63, 4, False, 8000, 1 << 20) == 16
+	for groups in range(1, 200):
+		for heads in (1, 2, 4, 8, 16, 64):
+			for by_xcd in (False, True):
+				for wgs in (300, 2048, 2049, 1 << 20):
+					assert 1 <= f(groups, heads, by_xcd, wgs, 3 << 19) <= groups
