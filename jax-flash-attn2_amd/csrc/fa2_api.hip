@@ -394,8 +394,17 @@ static int fwd_split_plan(const fa2_params* p, int* split_len, int* tall) {
 			// taken, partial results 0.57 of the above. B1 Hq32 Hkv8, 1000 causal rows over 9000 / 14200 keys 174 / 261 -> 155 / 227 us in two ranges, 700 rows over
 			// 8200 140 -> 120, 600 rows over 3000 / 10200 in three 56 / 126 -> 45 / 112; B1 Hq8 Hkv2, 1500 over 6200 in five 64 -> 51. Workgroups of eight waves in one
 			// range take 6 % more than their estimate over many keys (1000 rows over 6200: 104 and 117); from three ranges on a tenth has to be gained (four,
-			// estimated as even: B1 H4 S4096 over 6200 57 and 61, B1 Hq16 Hkv4, 1000 over 3000 41 and 45). Not with lengths: a range beyond
-			// a row's length is a place wasted (B3 Hq8 Hkv2, 1000 rows over 3000 keys 51 and 60). (Rows of fewer columns run on the rows as they are.)
+			// estimated as even: B1 H4 S4096 over 6200 57 and 61, B1 Hq16 Hkv4, 1000 over 3000 41 and 45).
+			// All this with rows that do not fill their last wave, whose tiles all take the masked path: a workgroup of eight waves alone on its CU waits for that wave.
+			// Where rows are a multiple of 32 it takes 15 % less (B1 Hq64 Hkv16 over 3000 keys, 384 rows 47.5 us, 370 rows 55.8), workgroups that share a CU
+			// nothing less. Two ranges then gain nothing (47.5 -> 54.5; 512 rows of B4 H12 48 -> 58, B1 Hq32 Hkv8, 1024 over 7500 123 -> 130, over 13000 206 -> 211), three do
+			// (B1 Hq40 Hkv8, 512 over 4000 59.5 -> 55.4), more only over many keys (five, B1 Hq24 Hkv8, 512 over 7500 62.6 -> 59.2; four, B1 Hq20 Hkv5, 640 over 4000 40.9 -> 43.2), and
+			// over more where groups are not placed by XCD and every range is read on all of them (five, B1 H14, 896 over 7500 64 -> 70, over 13000 115 -> 109). There two
+			// ranges lose otherwise too (1000 rows of Hq25 Hkv5 over 3000 56 -> 62, of Hq30 Hkv10 over 7500 137 -> 141, over 13000 232 -> 230), and with more than three groups
+			// an XCD (368 rows of B2 Hq32 Hkv16 over 3000 56 -> 60, over 11000 174 -> 183; three, 409 of B3 Hq16 Hkv8 over 7033 120 -> 97).
+			// Fewer than 384 leave too many CUs with one: 288 of 96 x 3, 22.3 and 23.3, 72 x 4, 41 and 44; 320 of 80 x 4, 52.5 and 57, 160 x 2, 38.9 and 39.8; 352 of
+			// 176 x 2, 36 and 41, 43.6 and 42.9.  Not with lengths: a range beyond a row's length is a place wasted (B3 Hq8 Hkv2, 1000 rows over
+			// 3000 keys 51 and 60). (Rows of fewer columns run on the rows as they are.)
 			int pairs = 0;
 			double pairs_us = 0;
 			for (int n = 2; n <= 16 && n <= tiles / 2 && base * n <= 512 && n * range_bytes <= kFwdScratchMax; ++n) {
@@ -406,7 +415,10 @@ static int fwd_split_plan(const fa2_params* p, int* split_len, int* tall) {
 					pairs_us = us;
 				}
 			}
-			if (pairs && pairs_us < best_us * (pairs == 2 ? 1.06 : 0.9)) {
+			const bool whole = p->Sq % 32 == 0;
+			const bool by_xcd = (int64_t)p->B * p->Hkv % 8 == 0, far = tiles >= 160;
+			const bool ok = pairs == 2 ? !whole && (by_xcd ? (int64_t)p->B * p->Hkv <= 24 : far) : pairs == 3 || !whole || far || (by_xcd && tiles >= 100);
+			if (pairs && ok && pairs_us < best_us * (pairs == 2 ? 1.06 : 0.9)) {
 				best = pairs;
 				*tall = 2;
 			}
