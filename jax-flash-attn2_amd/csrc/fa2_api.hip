@@ -163,6 +163,7 @@ void fill(const fa2_params* p, KArgs& a) {
 	a.Sk = p->Sk;
 	a.Hq = p->Hq;
 	a.Hkv = p->Hkv;
+	a.group_heads = p->Hq / p->Hkv;
 	a.causal = p->causal ? 1 : 0;
 	// causal caps the right bound at 0, as the reference does (refrence_call.py:36-37)
 	a.win_left = p->has_window && p->window_left >= 0 ? p->window_left : -1;

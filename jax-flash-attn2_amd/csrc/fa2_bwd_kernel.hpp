@@ -1170,8 +1170,8 @@ __global__ __launch_bounds__(NW * 64, WPS) void bwd_dq_kernel(const KArgs a) {
 	FA2_LDS char* lds = (FA2_LDS char*)smem;
 
 	int mt, h, b;
-	decode_block(a, mt, h, b);
-	const int hk = h / (a.Hq / a.Hkv);
+	decode_block<BIAS>(a, mt, h, b);
+	const int hk = h / a.group_heads;
 	const int tid = threadIdx.x, lane = tid & 63;
 	// the wave index as an explicitly scalar value: everything derived from it (tile bounds, loop trip counts,
 	// "nothing to do for this wave") then stays in scalar registers and scalar branches
@@ -1861,6 +1861,7 @@ hipError_t launch_bwd_v(KArgs& a, hipStream_t s) {
 		// (head dim 64 without bias fits three; B6 H16 S1000 causal, with the dK/dV kernel, 88.7 -> 84.1 us, nothing from S2000 on)
 		const int per_cu = D == 64 && WPS == 1 ? (BIAS || a.Sk > 1536 ? 2 : 3) : WPS;
 		a.fold = fold_of(a, NW, (int64_t)grid.x, per_cu);
+		if (a.fold) a.interleave = a.xcd_remap ? groups / 8 : groups;
 		if constexpr (BIAS) {
 			if (a.dbias && a.softcap > 0.f)
 				hipLaunchKernelGGL((bwd_dq_kernel<T, D, NW, C::DQ_QB, WPS, true, DROP, false, true, true>), grid, block, 0, s, a);

@@ -79,51 +79,45 @@ inline bool causal_tail(const KArgs& a, int64_t wgs) { return a.causal && (a.Sk 
 inline int xcd_ranges_of(const KArgs& a) { return a.hd % 64 != 0 && !a.seqlens && !a.kv_lens; }
 FA2_DEV int group_on_xcd(const KArgs& a, int i, int xcd) { return a.xcd_ranges ? xcd * ((a.B * a.Hkv) >> 3) + i : i * 8 + xcd; }
 
+// BIAS: the grid may be placed for a bias without a head axis.
+template <bool BIAS>
 FA2_DEV void decode_block(const KArgs& a, int& mt, int& h, int& b, int id = (int)blockIdx.x) {
-	const int r = a.Hq / a.Hkv;
-	if (a.fold) {
-		// A causal grid whose workgroups are all resident at once (resident_position): what counts is which of them share a CU.  Their order is by row tile
-		// over all (batch, kv-head) groups - of the XCD, where groups are placed by XCD -, the longest tiles first; K and V of all groups are
-		// streamed at once anyway.
-		const int sh = a.xcd_remap ? 3 : 0, n = a.fold >> sh, per_tile = n / a.mtiles;
-		const int j = resident_position(id >> sh, n, kNumCULog2 - sh);
-		const int t = j / per_tile, rem = j % per_tile;
-		const int grp = a.xcd_remap ? group_on_xcd(a, rem / r, id & 7) : rem / r;
-		mt = a.mtiles - 1 - t;
-		b = grp / a.Hkv;
-		h = grp % a.Hkv * r + rem % r;
-		return;
+	const int sh = a.xcd_remap ? 3 : 0;
+	if constexpr (BIAS) {
+		if (a.xcd_remap == 2) {
+			// A bias without a head axis is re-read by every head: one batch per XCD, and on an
+			// XCD the heads of one row tile next to each other, so that the tile of bias they all
+			// read is fetched into that XCD's L2 once.
+			int xcd = id & 7, j = id >> 3;
+			int per_batch = a.mtiles * a.Hq;
+			b = (j / per_batch) * 8 + xcd;
+			int rem = j % per_batch;
+			mt = a.mtiles - 1 - rem / a.Hq;
+			h = rem % a.Hq;
+			return;
+		}
+		if (a.xcd_remap == 3) {
+			// The same sharing of a head-less bias, for batch rows of different key lengths: the unit (batch, row tile)
+			// with its heads adjacent stays on one XCD, but the units of one batch go round the XCDs (batch b, tile t
+			// on XCD (b + t) % 8), so that a short batch row does not leave its XCD idle.
+			int xcd = id & 7, j = id >> 3;
+			int u = j / a.Hq, nb8 = a.B >> 3;
+			int tile = u / nb8;
+			h = j % a.Hq;
+			mt = a.mtiles - 1 - tile;
+			b = ((xcd - tile) & 7) + 8 * (u % nb8);
+			return;
+		}
 	}
-	if (a.xcd_remap == 2) {
-		// A bias without a head axis is re-read by every head: one batch per XCD, and on an
-		// XCD the heads of one row tile next to each other, so that the tile of bias they all
-		// read is fetched into that XCD's L2 once.
-		int xcd = id & 7, j = id >> 3;
-		int per_batch = a.mtiles * a.Hq;
-		b = (j / per_batch) * 8 + xcd;
-		int rem = j % per_batch;
-		mt = a.mtiles - 1 - rem / a.Hq;
-		h = rem % a.Hq;
-		return;
-	}
-	if (a.xcd_remap == 3) {
-		// The same sharing of a head-less bias, for batch rows of different key lengths: the unit (batch, row tile)
-		// with its heads adjacent stays on one XCD, but the units of one batch go round the XCDs (batch b, tile t
-		// on XCD (b + t) % 8), so that a short batch row does not leave its XCD idle.
-		int xcd = id & 7, j = id >> 3;
-		int u = j / a.Hq, nb8 = a.B >> 3;
-		int tile = u / nb8;
-		h = j % a.Hq;
-		mt = a.mtiles - 1 - tile;
-		b = ((xcd - tile) & 7) + 8 * (u % nb8);
-		return;
-	}
-	// (a.interleave groups advance together, see launch_order() and groups_together())
-	const Place p = place_of(a.xcd_remap ? id >> 3 : id, (a.B * a.Hkv) >> (a.xcd_remap ? 3 : 0), r, a.mtiles, a.interleave);
+	// a.interleave groups (of an XCD, where groups are placed by XCD) advance together: launch_order(), groups_together().  On a causal grid whose workgroups are
+	// all resident at once all do, and what counts is which workgroups share a CU (resident_position).
+	int j = id >> sh;
+	if (a.fold) j = resident_position(j, a.fold >> sh, kNumCULog2 - sh);
+	const Place p = place_of(j, (a.B * a.Hkv) >> sh, a.group_heads, a.mtiles, a.interleave);
 	const int grp = a.xcd_remap ? group_on_xcd(a, p.group, id & 7) : p.group;
 	b = grp / a.Hkv;
 	mt = a.mtiles - 1 - p.tile;
-	h = grp % a.Hkv * r + p.head;
+	h = grp % a.Hkv * a.group_heads + p.head;
 }
 
 // four consecutive bias values bias[row][col..col+3] as floats.  dtype 4: the row holds bytes of a boolean
@@ -219,12 +213,12 @@ __global__ __launch_bounds__(NW * 64 * KW, WPS) void fwd_kernel(const KArgs a) {
 			h = (id2 % a.Hkv) * (a.Hq / a.Hkv);
 			mt = 0;
 		} else {
-			decode_block(a, mt, h, b, (int)blockIdx.x / a.nsplit);
+			decode_block<BIAS>(a, mt, h, b, (int)blockIdx.x / a.nsplit);
 		}
 	} else {
-		decode_block(a, mt, h, b);
+		decode_block<BIAS>(a, mt, h, b);
 	}
-	const int hk = h / (a.Hq / a.Hkv);
+	const int hk = h / a.group_heads;
 	const int tid = KW == 1 ? threadIdx.x : threadIdx.x & (NT - 1), lane = tid & 63;  // (of the group)
 	// the wave index as an explicitly scalar value: everything derived from it (tile bounds, loop trip counts,
 	// "nothing to do for this wave") then stays in scalar registers and scalar branches
@@ -1418,6 +1412,7 @@ hipError_t launch_fwd_cfg(bool bias, bool drop, KArgs& a, hipStream_t s) {
 	if (bias && a.bias_sh == 0 && a.B % 8 == 0) a.xcd_remap = a.kv_lens ? 3 : 2;
 	dim3 grid((unsigned)(a.mtiles * a.B * a.Hq)), block(NW * 64 * KW);
 	a.fold = fold_of(a, NW, (int64_t)grid.x, KW > 1 ? WPS / KW : D == 64 && WPS == 1 ? 2 : WPS);
+	if (a.fold) a.interleave = a.xcd_remap ? groups / 8 : groups;
 	if constexpr (D == 64 && NW == 4 && WPS > 1) {
 		if (!bias && a.causal && window_is_open(a.Sk, a.win_left) && !a.fold && (int64_t)grid.x > kNumCU)
 			a.interleave = groups_together(a.xcd_remap ? groups / 8 : groups, a.Hq / a.Hkv, a.xcd_remap, (int64_t)grid.x, (int64_t)a.Sk * D * 4);

@@ -53,6 +53,7 @@ struct KArgs {
 	int kv_pair, kv_ntiles;
 	int fold;        // forward / dQ: number of workgroups of a causal grid that are all resident at once (0 = it is another; see decode_block())
 	int interleave;  // this many (batch, kv-head) groups (with xcd_remap 1: of an XCD) advance through their tiles together
+	int group_heads; // q-heads of a kv-head
 	int stages;      // backward: bit 0 delta, bit 1 dK/dV, bit 2 dQ
 	int dq_makes_delta;  // the dQ kernel computes delta itself (and stores it for the dK/dV kernel)
 	// split forward (0 / 1 = off): key ranges of split_len keys, partial results in scratch
