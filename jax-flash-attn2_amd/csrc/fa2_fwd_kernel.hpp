@@ -3,8 +3,9 @@
 // (jax_flash_attn2/flash_attention_triton/_forward_triton.py:60-164, 213-459).
 //
 // One workgroup = NW waves = one tile of BM = NW*QB*32 query rows of one
-// (batch, q-head).  K/V tiles of BN = 64 keys are streamed through a double
-// buffer in LDS by direct global->LDS loads.  Everything is computed
+// (batch, q-head).  K/V tiles of BN = 64 keys (32 for rows of 72 to 96 columns
+// with three workgroups a CU) are streamed through a double buffer in LDS by
+// direct global->LDS loads.  Everything is computed
 // transposed so that no intermediate ever leaves registers:
 //   S^T[kv, q] = K[kv, :] . Q[q, :]      A = K fragment from LDS, B = Q in registers
 //   O^T[d,  q] = V^T[d, kv] . P^T[kv, q] A = V through transposed LDS reads,
